@@ -9,8 +9,9 @@ A case is a dict of plain values. Its ``path`` names the entry point:
   gram     ``sync.gram``: worker x worker products as a pass of their own (up to sixteen workers)
 
 ``listed()`` holds the fixed cases, ``draw(rng)`` makes another one of the same ranges, ``prepare`` builds what the
-program holds before the call, ``run`` is one pass, ``work`` the bytes and operations one pass cannot do without and
-``tolerance`` how far another correct implementation at the same precision may differ.
+program holds before the call, ``run`` is one pass, ``work`` the bytes and operations one pass cannot do without,
+``tolerance`` how far another correct implementation at the same precision may differ and ``exact`` the same pass in
+64-bit arithmetic.
 """
 import math
 import random
@@ -398,3 +399,135 @@ def tolerance(case):
     if case["path"] == "gram":
         return {"rel": 4e-7, "max": 8e-7} if case["grads"] == "bf16" and case["K"] > 7 else {"rel": 1e-14, "max": 1e-13}
     return {"rel": 4e-7, "max": 2e-6}
+
+
+# -------------------------------------------------------------------------------------------------------------- exact
+def _sums64(case, grads, halves, agg):
+    """Statistics row of a span: the four sums of the halves and the aggregate, every worker's norm, every pair's product."""
+    row = torch.zeros(40, dtype=torch.float64, device=DEVICE)
+    a, b = halves
+    row[:4] = torch.stack([(a * b).sum(), (a * a).sum(), (b * b).sum(), (agg * agg).sum()])
+    if case["stats"] in ("full", "gram"):
+        row[4:4 + len(grads)] = torch.stack([(g * g).sum() for g in grads])
+    if case["stats"] == "gram":
+        pairs = [(grads[i] * g).sum() for i in range(len(grads)) for g in grads[i + 1:]]
+        row[4 + len(grads):4 + len(grads) + len(pairs)] = torch.stack(pairs) if pairs else row[:0]
+    return row
+
+
+def _update64(opt, group, step, g, p, state):
+    """One optimizer step on the 64-bit slices p and state, in place."""
+    lr, wd = opt["groups"][group]["lr"], opt["groups"][group]["weight_decay"]
+    if opt["kind"] == "sgd":
+        state[0].mul_(opt["momentum"]).add_(g + wd * p)
+        p.sub_(lr * state[0])
+        return
+    b1, b2 = opt["betas"]
+    if opt["kind"] == "adamw":
+        p.mul_(1 - lr * wd)
+    else:
+        g = g + wd * p
+    state[0].mul_(b1).add_(g, alpha=1 - b1)
+    state[1].mul_(b2).add_(g * g, alpha=1 - b2)
+    second = state[1]
+    if opt.get("amsgrad", False):
+        second = state[2].copy_(torch.maximum(state[2], state[1]))
+    denom = second.sqrt().div_(math.sqrt(1 - b2 ** step)).add_(opt["eps"])
+    p.sub_(state[0] / denom * (lr / (1 - b1 ** step)))
+
+
+def _step64(case, spans, grads, agg, param, state):
+    """The sync step on 64-bit copies, span by span: the aggregate into agg, the update into param and state.
+    Returns the statistics rows. ``spans``: (first element, elements, [(start, group)], ...)."""
+    opt, rows, norm2 = _opt(case), [], 0.0
+    b = _batches(case)
+    half = [[x / (sum(b[h::2]) or 1) for x in b[h::2]] for h in (0, 1)]
+    for off, n, *_ in spans:
+        g = [t[off:off + n].double() for t in grads]
+        agg[off:off + n] = sum(x * (w / sum(b)) for x, w in zip(g, b))
+        if case["stats"] != "none" or case["clip"]:
+            halves = [sum((x * w for x, w in zip(g[h::2], half[h])), torch.zeros_like(g[0])) for h in (0, 1)]
+            rows.append(_sums64(case, g, halves, agg[off:off + n]))
+            norm2 += float(rows[-1][3])
+    if case["clip"]:
+        coef = case["clip"] / (math.sqrt(norm2) + 1e-6)
+        for off, n, *_ in spans:
+            agg[off:off + n].mul_(min(1.0, coef))
+    if opt is not None:
+        for off, n, bounds, *_ in spans:
+            ends = [start for start, _ in bounds[1:]] + [n]
+            for (start, group), end in zip(bounds, ends):
+                sl = slice(off + start, off + end)
+                _update64(opt, group, _Fill.STEP + 1, agg[sl], param[sl], [t[sl] for t in state])
+    return rows
+
+
+def _exact_arenas(case, eng):
+    state = [s.double() for s in (eng.state1, eng.state2, eng.state3)[:eng.n_state]]
+    param = eng.param.double()
+    agg = eng.agg.double() if eng.agg is not None else torch.zeros_like(param)
+    rows = _step64(case, eng.layout.spans, eng.grads, agg, param, state)
+    out = {"param": param, "replicas": [param.clone() for _ in eng.fanout]}
+    if case["aggregate"]:
+        out["aggregate"] = agg
+    for j, t in enumerate(state):
+        if eng.moments is not None:
+            shape = eng.moments.way(j).shape
+            t = torch.nn.functional.pad(t, (0, shape.numel() - t.numel())).view(shape)
+        out[f"state{j}"] = t
+    return out, rows
+
+
+def _exact_engine(case, s):
+    out, rows = _exact_arenas(case, s["engine"])
+    if case["stats"] != "none":
+        out["rows"] = torch.stack(rows)
+    if case["stats"] == "gram":
+        out["gram"] = _gram64([torch.cat([g[o:o + n] for o, n, *_ in s["engine"].layout.spans]) for g in s["engine"].grads])
+    return out
+
+
+def _exact_hooks(case, s):
+    out, rows = _exact_arenas(case, s["engine"])
+    out["rows"] = rows
+    return out
+
+
+def _exact_bucket(case, s):
+    param = None if s["param"] is None else s["param"].double()
+    state = [t.double() for t in s["state"]]
+    agg = torch.zeros(case["elements"], dtype=torch.float64, device=DEVICE)
+    bounds = s["span"].bounds or [(0, 0)]
+    rows = _step64(case, [(0, case["elements"], bounds)], s["grads"], agg, param, state)
+    return {"aggregate": agg, "param": param, "state": state, "row": rows[0] if rows else None}
+
+
+def _exact_shard(case, s):
+    param, state = s["param"].double(), [t.double() for t in s["state"]]
+    opt, layout, off = _opt(case), FlatLayout(_specs(case)), 0
+    for spec, g0 in zip(_specs(case), layout.param_offset):
+        sl = slice(off, off + spec.numel)
+        _update64(opt, spec.group, _Fill.STEP + 1, s["grads"][g0:g0 + spec.numel].double(), param[sl], [t[sl] for t in state])
+        off += -(-spec.numel // 128) * 128
+    return {"param": param, "state": state}
+
+
+def _gram64(grads):
+    out = torch.zeros(len(grads), len(grads), dtype=torch.float64, device=DEVICE)
+    for a, x in enumerate(grads):
+        x = x.double()
+        for b in range(a + 1):
+            out[a, b] = out[b, a] = (x * grads[b].double()).sum()
+    return out
+
+
+def _exact_gram(case, s):
+    return _gram64(s["grads"])
+
+
+_EXACT = {"engine": _exact_engine, "hooks": _exact_hooks, "bucket": _exact_bucket, "shard": _exact_shard, "gram": _exact_gram}
+
+
+def exact(case, seed):
+    """What ``run`` returns for these inputs, in 64-bit torch operations."""
+    return _EXACT[case["path"]](case, prepare(case, seed))
