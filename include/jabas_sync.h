@@ -340,6 +340,11 @@ int jabas_gram(const void* const* grads, int32_t K, int32_t grad_dtype,
 int jabas_clip_coef(const double* stats_rows, uint32_t n_rows, double max_norm, double eps,
                     float* coef_out, jabas_stream_t stream);
 
+/* K x K Gram matrix (K * K doubles, row by row, symmetric) out of statistics rows of level JABAS_STATS_GRAM: the rows
+ * summed in a fixed order (fp64), the norms on the diagonal, JABAS_STAT_PAIR(K, a, b) beside it. n_rows may be 0 (zeros).
+ * K <= JABAS_STATS_GRAM_MAX_K. Reads the rows only: no pass over the gradients. */
+int jabas_gram_from_rows(const double* stats_rows, uint32_t n_rows, int32_t K, double* gram_out, jabas_stream_t stream);
+
 /* SGD step with a ready fp32 gradient (torch 1.8.1 optim/_functional.sgd as used by
  * examples/resnet50/main.py:351-359, examples/faster_r_cnn/train.py:266-276).
  * momentum_buf may be NULL when momentum == 0. */

@@ -550,12 +550,28 @@ def gram(grads, stream=None, workspace=None):
     return out.view(L.GRAM_MAX_K, L.GRAM_MAX_K)[:K, :K]
 
 
+def _device_rows(t):
+    """Whether a kernel can read the statistics rows as they are: whole contiguous fp64 rows in GPU memory of a
+    plain tensor (not one that stands for others while a function transform or a tracer runs)."""
+    return (type(t) is torch.Tensor and t.is_cuda and t.dtype == torch.float64 and t.is_contiguous()
+            and 0 < t.numel() < L.STATS_STRIDE << 32 and t.numel() % L.STATS_STRIDE == 0 and not t.is_neg()
+            and not torch.compiler.is_compiling() and not torch._C._functorch.is_functorch_wrapped_tensor(t))
+
+
 def gram_from_stats(stats_rows, K):
     """K x K Gram matrix (float64, on the rows' device) of the worker gradients from statistics rows of level
     'gram', summed over the rows (one row per span or bucket): the diagonal from the per-VSW norms, the rest
-    from the pair slots. No launch of its own: the sums came out of the pass that aggregated the gradients."""
+    from the pair slots. No pass over the gradients: the sums came out of the one that aggregated them; rows on the
+    GPU are summed and unfolded by one small launch on the current stream (``jabas_gram_from_rows``)."""
     if not 1 <= K <= L.STATS_GRAM_MAX_K:
         raise ValueError(f"rows of level 'gram' exist for 1..{L.STATS_GRAM_MAX_K} workers, not {K}")
+    if _device_rows(stats_rows):
+        n_rows = stats_rows.numel() // L.STATS_STRIDE
+        with torch.cuda.device(stats_rows.device):
+            out = torch.empty(K, K, dtype=torch.float64, device=stats_rows.device)
+            L.check(L.lib().jabas_gram_from_rows(stats_rows.data_ptr(), n_rows, K, out.data_ptr(), _stream_ptr()),
+                    "jabas_gram_from_rows")
+        return out
     total = stats_rows.detach().reshape(-1, L.STATS_STRIDE).to(torch.float64).sum(dim=0)
     out = torch.empty(K, K, dtype=torch.float64, device=total.device)
     for a in range(K):

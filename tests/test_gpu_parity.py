@@ -1002,3 +1002,28 @@ def test_plan_with_nothing_but_empty_spans(gpu):
     assert plan.run(sync.make_step_args((1, 1), torch.float32, stats=False, opt=SGD, step=2)) is None
     torch.cuda.synchronize()
     assert torch.equal(p, torch.ones(16, device=gpu)) and torch.count_nonzero(m) == 0
+
+
+@pytest.mark.parametrize("K", [1, 2, 5, 8])
+@pytest.mark.parametrize("n_rows", [1, 2, 16, 17, 63, 1025])
+def test_gram_from_rows_on_the_device(gpu, K, n_rows):
+    """The launch that sums rows of level 'gram' and unfolds them against the torch path the host takes: fewer rows
+    than waves, one more, many. Both add n_rows doubles of at most m in some order: n_rows * 2**-53 * n_rows * m apart
+    at most."""
+    from jabas_amd import sync, _lib as L
+    rows = torch.randn(n_rows, L.STATS_STRIDE, dtype=torch.float64, generator=torch.Generator().manual_seed(K + n_rows))
+    want = sync.gram_from_stats(rows, K)
+    dev = rows.to(gpu)
+    got = sync.gram_from_stats(dev, K)
+    assert got.shape == (K, K) and got.is_contiguous() and torch.equal(got, got.t())
+    bound = n_rows * n_rows * 2.0 ** -53 * float(rows.abs().max())
+    assert float((got.cpu() - want).abs().max()) <= bound
+    assert torch.equal(sync.gram_from_stats(dev, K), got)                              # the same call, the same bits
+    strided = torch.cat([dev, dev], dim=1)[:, :L.STATS_STRIDE]                         # not whole rows in memory
+    assert float((sync.gram_from_stats(strided, K).cpu() - want).abs().max()) <= bound
+    assert torch.equal(sync.gram_from_stats(dev[:0], K), torch.zeros(K, K, dtype=torch.float64, device=gpu))
+    with pytest.raises(ValueError):
+        sync.gram_from_stats(dev, 9)
+    assert L.lib().jabas_gram_from_rows(None, 1, K, dev.data_ptr(), None) == L.ERR_NULL
+    assert L.lib().jabas_gram_from_rows(dev.data_ptr(), 1, 9, dev.data_ptr(), None) == L.ERR_K
+    assert L.lib().jabas_gram_from_rows(dev.data_ptr() + 4, 1, K, dev.data_ptr(), None) == L.ERR_ALIGN
