@@ -1,8 +1,8 @@
 // K x K Gram matrix of the K worker gradients of one span: gram[a][b] = sum_e g_a[e]*g_b[e].
 // Fixed order of operations: bit-identical run to run.
 //   few workers    grid-stride over 4-element vectors, exact fp64 products of the fp32 (or widened bf16) values,
-//                  K(K+1)/2 fp64 accumulators per thread on the vector ALU, wave64 shuffle tree -> LDS -> one
-//                  packed partial row per workgroup (K <= 5 for fp32 gradients, K <= 7 for bf16);
+//                  K(K+1)/2 fp64 accumulators per thread on the vector ALU, summed over the wave on the fp64 matrix
+//                  cores -> LDS -> one packed partial row per workgroup (K <= 3 for fp32 gradients, K <= 7 for bf16);
 //   more, to 16    fp32 gradients: fp64 matrix cores, v_mfma_f64_4x4x4 over 4 x 4 blocks of worker pairs, fed
 //                  from registers (gram_mfma_kernel below), still exact products and fp64 sums;
 //                  bf16 gradients: bf16 matrix cores, exact fp32 products, fp32 running sums over short runs,
@@ -11,7 +11,7 @@
 #include "jabas_internal.h"
 
 #ifndef JABAS_GRAM_VALU_MAX_K
-#define JABAS_GRAM_VALU_MAX_K 5
+#define JABAS_GRAM_VALU_MAX_K 3
 #endif
 
 namespace jabas {
@@ -20,9 +20,10 @@ namespace {
 #ifndef JABAS_GRAM_VALU_MAX_K_BF16
 #define JABAS_GRAM_VALU_MAX_K_BF16 7
 #endif
-// Up to here the vector-ALU kernel, beyond it the matrix cores. Measured on 86.6 M elements: fp32 K = 5: 5.95
-// against 4.96 TB/s, K = 6: 5.54 against 5.94, K = 8: 5.45 against 6.01; bf16 gradients K = 6: 5.83 against 5.81,
-// K = 8: 5.45 against 6.0.
+// Up to here the vector-ALU kernel, beyond it the matrix cores. Both, on 25.6 M / 1.2 M elements, whole call in us:
+// fp32 K = 3: 54.3 / 10.7 against 53.7 / 11.6, K = 4: 71.8 / 13.3 against 69.3 / 12.3, K = 5: 93.2 / 16.5 against
+// 91.3 / 13.1. bf16 gradients change at eight workers, where the matrix cores' sums are fp32 over short runs: up to
+// seven every sum stays fp64.
 constexpr int gram_valu_max_k(int grad_dtype) { return grad_dtype == JABAS_BF16 ? JABAS_GRAM_VALU_MAX_K_BF16 : JABAS_GRAM_VALU_MAX_K; }
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -38,7 +39,13 @@ template <> struct GramLoad<JABAS_F32> {
         return __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(static_cast<const float*>(base) + e));
     }
     static __device__ __forceinline__ float elem(const Raw& r, int i) { return r[i]; }
-    static __device__ __forceinline__ Raw from(const float (&x)[4]) { return Raw{x[0], x[1], x[2], x[3]}; }
+    // elements of the vector at e that lie in [lo, hi), zeros for the others: nothing outside the span is read
+    static __device__ __forceinline__ Raw edge(const void* base, uint64_t e, uint64_t lo, uint64_t hi) {
+        Raw r;
+#pragma unroll
+        for (int i = 0; i < EPT; ++i) r[i] = (e + i >= lo && e + i < hi) ? static_cast<const float*>(base)[e + i] : 0.0f;
+        return r;
+    }
     static __device__ __forceinline__ void vec(const void* base, uint64_t e, float (&x)[4]) {
         const f32x4 r = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(static_cast<const float*>(base) + e));
         x[0] = r.x; x[1] = r.y; x[2] = r.z; x[3] = r.w;
@@ -47,18 +54,6 @@ template <> struct GramLoad<JABAS_F32> {
 };
 template <> struct GramLoad<JABAS_BF16> {
     static constexpr int EPT = 4;
-    using Raw = u32x2;
-    static __device__ __forceinline__ Raw raw(const void* base, uint64_t e) {
-        return __builtin_nontemporal_load(reinterpret_cast<const u32x2*>(static_cast<const uint16_t*>(base) + e));
-    }
-    static __device__ __forceinline__ float elem(const Raw& r, int i) {
-        const uint32_t w = i < 2 ? r.x : r.y;
-        return bits_to_float((i & 1) ? (w & 0xffff0000u) : (w << 16));
-    }
-    static __device__ __forceinline__ Raw from(const float (&x)[4]) {       // values that came from bf16: exact
-        return Raw{(__builtin_bit_cast(uint32_t, x[0]) >> 16) | (__builtin_bit_cast(uint32_t, x[1]) & 0xffff0000u),
-                   (__builtin_bit_cast(uint32_t, x[2]) >> 16) | (__builtin_bit_cast(uint32_t, x[3]) & 0xffff0000u)};
-    }
     static __device__ __forceinline__ void vec(const void* base, uint64_t e, float (&x)[4]) {
         const u32x2 r = __builtin_nontemporal_load(reinterpret_cast<const u32x2*>(static_cast<const uint16_t*>(base) + e));
         x[0] = bits_to_float(r.x << 16); x[1] = bits_to_float(r.x & 0xffff0000u);
@@ -107,60 +102,69 @@ __global__ void __launch_bounds__(kBlock) gram_kernel(const SpanDev sp, double* 
         }
     }
 
-    __shared__ double red[kWaves][NP];
+    // Sum of every product over the wave's lanes on the fp64 matrix cores: lane j + 4 b + 16 i supplies entry (j, i) of
+    // product b of v_mfma_f64_4x4x4 as the left operand and (i, j) as the right one. With ones on the other side the first
+    // adds lanes 16 apart (entry (j, *) of its result is the sum over i), the second the four j: every lane 4 b + j of
+    // the last row holds the sum of the lanes with its b. Multiplying by one is exact, the sums are fp64. Two instructions
+    // per product, where a tree of wave shuffles takes twelve LDS permutations: 1.2 M elements, whole call, K = 5 fp32
+    // 22.0 -> 16.5 us, K = 7 bf16 34.8 -> 24.4.
+    __shared__ double red[kWaves][4][NP];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
     for (int i = 0; i < NP; ++i) {
-        double v = acc[i];
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
-        if (lane == 0) red[wave][i] = v;
+        const double q = __builtin_amdgcn_mfma_f64_4x4x4f64(acc[i], 1.0, 0.0, 0, 0, 0);
+        const double v = __builtin_amdgcn_mfma_f64_4x4x4f64(1.0, q, 0.0, 0, 0, 0);
+        if ((lane & 51) == 0) red[wave][lane >> 2][i] = v;
     }
     __syncthreads();
     if (threadIdx.x < NP) {
-        double s = red[0][threadIdx.x];
+        double s = 0.0;
 #pragma unroll
-        for (int w = 1; w < kWaves; ++w) s += red[w][threadIdx.x];
+        for (int w = 0; w < kWaves; ++w)
+            s += ((red[w][0][threadIdx.x] + red[w][1][threadIdx.x]) + red[w][2][threadIdx.x]) + red[w][3][threadIdx.x];
         partials[static_cast<uint64_t>(blockIdx.x) * JABAS_GRAM_STRIDE + threadIdx.x] = s;
     }
 }
 
-// Sums the workgroup rows and writes the symmetric matrix. 256 threads: thread (value, part) adds rows
-// part, part + 16, ... of one packed entry in increasing order, the 16 parts of an entry sit in one
-// 16-lane row and are combined by a fixed DPP pattern, so the result does not depend on timing. (One
-// wave walking all rows of its entry one after the other took 0.23 ms for 1024 rows: more than the
-// Gram kernel itself.)
-constexpr int kGramFinalizeBlock = 256;
+// Sums the workgroup rows and writes the symmetric matrix. E is the power of two that holds a row's products: thread
+// (part, entry) adds packed entry `entry` of rows part, part + 1024 / E, ... in that order, the parts of a wave are added
+// by a fixed butterfly and the 16 waves in order: the result does not depend on timing. Neighbouring lanes read
+// neighbouring entries of one row; with lanes along the rows a load touched as many lines as lanes, and 1024 rows of 28
+// entries cost one compute unit about 10 us (1.2 M elements, K = 7 bf16, whole call: 24.4 -> 13.7 us).
+constexpr int kGramFinalizeBlock = 1024, kGramFinalizeWaves = kGramFinalizeBlock / 64;
+static_assert(JABAS_GRAM_VALU_MAX_K * (JABAS_GRAM_VALU_MAX_K + 1) / 2 <= 32, "one slot per product");
+static_assert(JABAS_GRAM_VALU_MAX_K_BF16 * (JABAS_GRAM_VALU_MAX_K_BF16 + 1) / 2 <= 32, "one slot per product");
+template <int E>
 __global__ void __launch_bounds__(kGramFinalizeBlock) gram_finalize_kernel(int K, const double* partials, unsigned grid,
                                                                          double* gram_out) {
+    constexpr unsigned kParts = kGramFinalizeBlock / E;
+    __shared__ double wave_sum[kGramFinalizeWaves][E];
     const int np = K * (K + 1) / 2;
-    const int t = threadIdx.x;
+    const int t = threadIdx.x, v = t % E;
+    double s = 0.0;
+    if (v < np) {
+#pragma unroll 16
+        for (unsigned b = t / E; b < grid; b += kParts) s += partials[static_cast<uint64_t>(b) * JABAS_GRAM_STRIDE + v];
+    }
+#pragma unroll
+    for (int off = 32; off >= E; off >>= 1) s += __shfl_xor(s, off, 64);
+    if ((t & 63) < E) wave_sum[t >> 6][v] = s;
     if (t < JABAS_GRAM_STRIDE) gram_out[t] = 0.0;
     __syncthreads();
-    const int part = t & 15;
-    for (int v0 = 0; v0 < np; v0 += kGramFinalizeBlock / 16) {
-        const int v = v0 + (t >> 4);
-        double s = 0.0;
-        if (v < np) {
-#pragma unroll 8
-            for (unsigned b = part; b < grid; b += 16) s += partials[static_cast<uint64_t>(b) * JABAS_GRAM_STRIDE + v];
-        }
-        s += dpp_move<0xB1, 0xf>(s);     // quad_perm [1,0,3,2]
-        s += dpp_move<0x4E, 0xf>(s);     // quad_perm [2,3,0,1]
-        s += dpp_move<0x141, 0xf>(s);    // row_half_mirror
-        s += dpp_move<0x140, 0xf>(s);    // row_mirror
-        if (v < np && part == 0) {
-            int a = 0;
-            while ((a + 1) * (a + 2) / 2 <= v) ++a;  // packed index v = a*(a+1)/2 + b, b <= a
-            const int b = v - a * (a + 1) / 2;
-            gram_out[a * JABAS_GRAM_MAX_K + b] = s;
-            gram_out[b * JABAS_GRAM_MAX_K + a] = s;
-        }
+    if (t < np) {
+        s = wave_sum[0][t];
+#pragma unroll
+        for (int w = 1; w < kGramFinalizeWaves; ++w) s += wave_sum[w][t];
+        int a = 0;
+        while ((a + 1) * (a + 2) / 2 <= t) ++a;          // packed index t = a*(a+1)/2 + b, b <= a
+        const int b = t - a * (a + 1) / 2;
+        gram_out[a * JABAS_GRAM_MAX_K + b] = s;
+        gram_out[b * JABAS_GRAM_MAX_K + a] = s;
     }
 }
 
 
-// ---- K >= 5: fp64 matrix cores, 4 x 4 blocks ----------------------------------------------------------
+// ---- K >= 4: fp64 matrix cores, 4 x 4 blocks ----------------------------------------------------------
 // The Gram matrix is a contraction over the elements, X X^T with X the K x N matrix of the workers'
 // gradients. The workers are cut into G = ceil(K / 4) groups of four; v_mfma_f64_4x4x4 (four independent
 // 4 x 4 x 4 products per instruction) forms, for one pair of groups (ga <= gb), the 4 x 4 block of products
@@ -175,18 +179,15 @@ __global__ void __launch_bounds__(kGramFinalizeBlock) gram_finalize_kernel(int K
 #ifndef JABAS_GRAM_RUN_F32
 #define JABAS_GRAM_RUN_F32 2
 #endif
-#ifndef JABAS_GRAM_RUN_BF16
-#define JABAS_GRAM_RUN_BF16 4
-#endif
-// 64-element blocks a wave loads before it multiplies (bf16 vectors are half as long: twice as many in flight)
-template <int DT> struct GramRun { static constexpr int value = DT == JABAS_BF16 ? JABAS_GRAM_RUN_BF16 : JABAS_GRAM_RUN_F32; };
+// 64-element blocks in a run of a wave
+constexpr int kGramRunBlocks = JABAS_GRAM_RUN_F32;
 
-template <int DT, int G>
+template <int G>
 __global__ void __launch_bounds__(kBlock) gram_mfma_kernel(const SpanDev sp, int K, double* partials) {
-    using L = GramLoad<DT>;
+    using L = GramLoad<JABAS_F32>;
     constexpr int P = G * (G + 1) / 2;
-    constexpr int kGramRunBlocks = GramRun<DT>::value;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    constexpr uint64_t kRun = static_cast<uint64_t>(kGramRunBlocks) * 64;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wi = lane & 3;                           // worker inside its group
     const uint32_t lane_off = static_cast<uint32_t>(lane >> 2) * 4u;
     const void* base[G];
@@ -199,31 +200,19 @@ __global__ void __launch_bounds__(kBlock) gram_mfma_kernel(const SpanDev sp, int
     double acc[P];
 #pragma unroll
     for (int p = 0; p < P; ++p) acc[p] = 0.0;
-    const uint64_t n_blocks = (sp.hi + 63) / 64;
-    const uint64_t n_runs = (n_blocks + kGramRunBlocks - 1) / kGramRunBlocks;
+    // Runs that lie wholly in the span are [first, last); at most two others hold its ends.
+    const uint64_t n_runs = (sp.hi + kRun - 1) / kRun, first = (sp.lo + kRun - 1) / kRun;
+    const uint64_t last = sp.hi / kRun > first ? sp.hi / kRun : first;
     const uint64_t n_waves = static_cast<uint64_t>(gridDim.x) * kWaves;
-    for (uint64_t run = static_cast<uint64_t>(blockIdx.x) * kWaves + wave; run < n_runs; run += n_waves) {
-        typename L::Raw x[kGramRunBlocks][G];
+    auto load = [&](uint64_t run, L::Raw (&x)[kGramRunBlocks][G]) {
 #pragma unroll
-        for (int u = 0; u < kGramRunBlocks; ++u) {
-            const uint64_t e = (run * kGramRunBlocks + u) * 64 + lane_off;
-            const bool whole = e >= sp.lo && e + 4 <= sp.hi;
+        for (int u = 0; u < kGramRunBlocks; ++u)
 #pragma unroll
-            for (int g = 0; g < G; ++g) {
-                if (whole) {
-                    // a lane beyond the last worker reads worker 0's vector (the same line another lane of the
-                    // wave reads anyway) and drops it when it multiplies: the wave stays on one path and no
-                    // load waits for another
-                    x[u][g] = L::raw(base[g], e);
-                } else {                             // a vector across the span's first or last element
-                    float y[4];
-#pragma unroll
-                    for (int i = 0; i < 4; ++i)
-                        y[i] = (live[g] && e + i >= sp.lo && e + i < sp.hi) ? L::one(base[g], e + i) : 0.0f;
-                    x[u][g] = L::from(y);
-                }
-            }
-        }
+            // a lane beyond the last worker reads worker 0's vector (the same line another lane of the
+            // wave reads anyway) and drops it when it multiplies: no load waits for another
+            for (int g = 0; g < G; ++g) x[u][g] = L::raw(base[g], run * kRun + u * 64 + lane_off);
+    };
+    auto multiply = [&](const L::Raw (&x)[kGramRunBlocks][G]) {
 #pragma unroll
         for (int u = 0; u < kGramRunBlocks; ++u)
 #pragma unroll
@@ -238,6 +227,38 @@ __global__ void __launch_bounds__(kBlock) gram_mfma_kernel(const SpanDev sp, int
                     for (int gb = ga; gb < G; ++gb, ++p)
                         acc[p] = __builtin_amdgcn_mfma_f64_4x4x4f64(d[ga], d[gb], acc[p], 0, 0, 0);
             }
+    };
+    // Bound by HBM reads. Two runs in flight per wave, the next one's loads issued before this one is multiplied; only whole
+    // runs, so that the loop has no edge path. 25.6 M elements, whole call: K = 8 133.3 -> 122.8 us (6.66 TB/s), K = 12
+    // 197.4 -> 189.1 (6.49); runs half as long or twice as long lose 2-5 %.
+    const uint64_t id = static_cast<uint64_t>(blockIdx.x) * kWaves + wave;
+    L::Raw x[kGramRunBlocks][G], y[kGramRunBlocks][G];
+    uint64_t run = first + id;
+    if (run < last) {
+        load(run, x);
+        while (true) {
+            const bool more = (run += n_waves) < last;
+            if (more) load(run, y);
+            multiply(x);
+            if (!more) break;
+            const bool again = (run += n_waves) < last;
+            if (again) load(run, x);
+            multiply(y);
+            if (!again) break;
+        }
+    }
+    // The ends go to the last waves, which have a run less when the runs do not come out even.
+    const uint64_t n_ends = first + (n_runs > last ? n_runs - last : 0);
+    for (uint64_t r = n_waves - 1 - id; r < n_ends; r += n_waves) {
+        const uint64_t e0 = (r < first ? r : last + (r - first)) * kRun + lane_off;
+#pragma unroll
+        for (int u = 0; u < kGramRunBlocks; ++u) {
+            const uint64_t e = e0 + u * 64;
+            const bool whole = e >= sp.lo && e + L::EPT <= sp.hi;
+#pragma unroll
+            for (int g = 0; g < G; ++g) x[u][g] = whole ? L::raw(base[g], e) : L::edge(base[g], e, sp.lo, sp.hi);
+        }
+        multiply(x);
     }
     // The instruction's contraction index is lane / 16 and its four independent products are indexed by
     // (lane / 4) % 4; entry (i, j) of product b sits in lane j + 4 b + 16 i. Which of a lane's elements meets
@@ -448,16 +469,17 @@ template <int K>
 int launch_gram_k(int grad_dtype, const SpanDev& sp, double* partials, unsigned grid, hipStream_t stream) {
     if (grad_dtype == JABAS_BF16)
         return static_cast<int>(launch_kernel(gram_kernel<K, JABAS_BF16>, dim3(grid), dim3(kBlock), 0, stream, sp, partials));
-    return static_cast<int>(launch_kernel(gram_kernel<K, JABAS_F32>, dim3(grid), dim3(kBlock), 0, stream, sp, partials));
+    if constexpr (K <= JABAS_GRAM_VALU_MAX_K)
+        return static_cast<int>(launch_kernel(gram_kernel<K, JABAS_F32>, dim3(grid), dim3(kBlock), 0, stream, sp, partials));
+    return -1;
 }
 
-template <int DT>
 int launch_gram_mfma(int K, const SpanDev& sp, double* partials, unsigned grid, hipStream_t stream) {
     switch ((K + 3) / 4) {
-        case 1: return static_cast<int>(launch_kernel(gram_mfma_kernel<DT, 1>, dim3(grid), dim3(kBlock), 0, stream, sp, K, partials));
-        case 2: return static_cast<int>(launch_kernel(gram_mfma_kernel<DT, 2>, dim3(grid), dim3(kBlock), 0, stream, sp, K, partials));
-        case 3: return static_cast<int>(launch_kernel(gram_mfma_kernel<DT, 3>, dim3(grid), dim3(kBlock), 0, stream, sp, K, partials));
-        case 4: return static_cast<int>(launch_kernel(gram_mfma_kernel<DT, 4>, dim3(grid), dim3(kBlock), 0, stream, sp, K, partials));
+        case 1: return static_cast<int>(launch_kernel(gram_mfma_kernel<1>, dim3(grid), dim3(kBlock), 0, stream, sp, K, partials));
+        case 2: return static_cast<int>(launch_kernel(gram_mfma_kernel<2>, dim3(grid), dim3(kBlock), 0, stream, sp, K, partials));
+        case 3: return static_cast<int>(launch_kernel(gram_mfma_kernel<3>, dim3(grid), dim3(kBlock), 0, stream, sp, K, partials));
+        case 4: return static_cast<int>(launch_kernel(gram_mfma_kernel<4>, dim3(grid), dim3(kBlock), 0, stream, sp, K, partials));
         default: return -1;
     }
 }
@@ -467,7 +489,7 @@ int launch_gram_mfma(int K, const SpanDev& sp, double* partials, unsigned grid, 
 int launch_gram(int K, int grad_dtype, const SpanDev& sp, double* partials, unsigned grid, hipStream_t stream) {
     if (K > gram_valu_max_k(grad_dtype))
         return grad_dtype == JABAS_BF16 ? launch_gram_bf16_mfma(K, sp, partials, grid, stream)
-                                        : launch_gram_mfma<JABAS_F32>(K, sp, partials, grid, stream);
+                                        : launch_gram_mfma(K, sp, partials, grid, stream);
     switch (K) {
         case 1: return launch_gram_k<1>(grad_dtype, sp, partials, grid, stream);
         case 2: return launch_gram_k<2>(grad_dtype, sp, partials, grid, stream);
@@ -476,7 +498,6 @@ int launch_gram(int K, int grad_dtype, const SpanDev& sp, double* partials, unsi
         case 5: return launch_gram_k<5>(grad_dtype, sp, partials, grid, stream);
         case 6: return launch_gram_k<6>(grad_dtype, sp, partials, grid, stream);
         case 7: return launch_gram_k<7>(grad_dtype, sp, partials, grid, stream);
-        case 8: return launch_gram_k<8>(grad_dtype, sp, partials, grid, stream);
         default: return -1;
     }
 }
@@ -498,8 +519,11 @@ int launch_gram_finalize(int K, int grad_dtype, double* partials, unsigned grid,
         return static_cast<int>(launch_kernel(gram_mfma_finalize_kernel, dim3(1), dim3(kGramMfmaFinalizeBlock), 0, stream, K,
                                               static_cast<const double*>(partials), grid, gram_out));
     }
-    return static_cast<int>(launch_kernel(gram_finalize_kernel, dim3(1), dim3(kGramFinalizeBlock), 0, stream, K,
-                                          static_cast<const double*>(partials), grid, gram_out));
+    const double* rows = partials;
+    const dim3 one(1), block(kGramFinalizeBlock);
+    if (K <= 3) return static_cast<int>(launch_kernel(gram_finalize_kernel<8>, one, block, 0, stream, K, rows, grid, gram_out));
+    if (K <= 5) return static_cast<int>(launch_kernel(gram_finalize_kernel<16>, one, block, 0, stream, K, rows, grid, gram_out));
+    return static_cast<int>(launch_kernel(gram_finalize_kernel<32>, one, block, 0, stream, K, rows, grid, gram_out));
 }
 
 }  // namespace jabas
