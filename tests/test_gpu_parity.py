@@ -293,6 +293,30 @@ def test_gram(gpu, K, dtype):
         assert torch.equal(G, G.t())
 
 
+@pytest.mark.parametrize("dtype,K", [(torch.float32, 1), (torch.float32, 3), (torch.float32, 4), (torch.float32, 5),
+                                     (torch.float32, 12), (torch.bfloat16, 2), (torch.bfloat16, 5), (torch.bfloat16, 7)])
+def test_gram_at_the_edges_of_runs_and_routes(gpu, dtype, K):
+    """One element, one less and one more than a run, starts inside a vector, one run more than the waves of a full
+    grid; and a worker with infinities and NaN reaches no product but its own. fp64 sums of n exact products in any
+    order: n * 2**-53 * |g_a| |g_b| apart at most."""
+    from jabas_amd import sync
+    for n, skew in ((1, 0), (1, 3), (127, 0), (128, 0), (129, 1), (253, 3), (257, 0), (4096 * 128 + 1, 0), (4097 * 128 + 3, 3)):
+        hg = _host_grads(K, n, 70 + K, dtype=dtype)
+        G = sync.gram([_dev(t, gpu, skew) for t in hg]).cpu()
+        wide = torch.stack([t.double() for t in hg])
+        norm = wide.norm(dim=1)
+        bound = 2.0 * (n + 2) * 2.0 ** -53 * torch.outer(norm, norm)
+        assert bool(((G - wide @ wide.t()).abs() <= bound).all()), f"K={K} n={n} skew={skew}"
+    if K > 1:
+        hg = _host_grads(K, 5003, 90 + K, dtype=dtype)
+        clean = sync.gram([_dev(t, gpu, 0) for t in hg])
+        hg[1][17], hg[1][4000] = float("inf"), float("nan")
+        G = sync.gram([_dev(t, gpu, 0) for t in hg])
+        keep = [k for k in range(K) if k != 1]
+        assert torch.equal(G[keep][:, keep], clean[keep][:, keep])
+        assert bool(G[1].isnan().all()) and bool(G[:, 1].isnan().all())
+
+
 def test_gram_limits_and_determinism(gpu):
     from jabas_amd import sync, _lib as L
     g = [torch.zeros(4096, device=gpu) for _ in range(17)]
