@@ -11,6 +11,8 @@ import ctypes as C
 
 import numpy as np
 import torch
+from torch.overrides import _get_current_function_mode_stack
+from torch.utils._device import DeviceContext
 
 from . import _lib as L
 
@@ -550,12 +552,22 @@ def gram(grads, stream=None, workspace=None):
     return out.view(L.GRAM_MAX_K, L.GRAM_MAX_K)[:K, :K]
 
 
+def _watched():
+    """Whether operations on tensors are recorded or replaced at the moment (torch.jit.trace, torch.compile, make_fx,
+    any dispatch or function mode but the one of torch.set_default_device): a launch through the C ABI is not seen
+    by what does so, and its output would enter a recorded graph as memory that nobody writes."""
+    if torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._len_torch_dispatch_stack():
+        return True
+    return torch._C._len_torch_function_stack() > 0 and any(
+        not isinstance(mode, DeviceContext) for mode in _get_current_function_mode_stack())
+
+
 def _device_rows(t):
     """Whether a kernel can read the statistics rows as they are: whole contiguous fp64 rows in GPU memory of a
-    plain tensor (not one that stands for others while a function transform or a tracer runs)."""
-    return (type(t) is torch.Tensor and t.is_cuda and t.dtype == torch.float64 and t.is_contiguous()
+    plain tensor (not one that stands for others in a function transform) while nothing records the operations."""
+    return (not _watched() and type(t) is torch.Tensor and t.is_cuda and t.dtype == torch.float64 and t.is_contiguous()
             and 0 < t.numel() < L.STATS_STRIDE << 32 and t.numel() % L.STATS_STRIDE == 0 and not t.is_neg()
-            and not torch.compiler.is_compiling() and not torch._C._functorch.is_functorch_wrapped_tensor(t))
+            and not torch._C._functorch.is_functorch_wrapped_tensor(t))
 
 
 def gram_from_stats(stats_rows, K):

@@ -641,3 +641,43 @@ def test_step_scalar_block_holds_the_constants_a_plain_call_derives():
     span = _span(5000, opt=True)
     args.scalars_dev = 0x7f0000001008
     assert lib.jabas_sync_bucket(C.byref(span), None, C.byref(args), None, None, 0, None) == L.ERR_ALIGN
+
+
+def test_rows_are_not_read_behind_a_recorder():
+    """A launch through the C ABI is not in a recorded graph: under every recorder gram_from_stats has to stay torch
+    operations, so that the recording answers for other rows too."""
+    import torch
+    from torch.fx.experimental.proxy_tensor import make_fx
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+    from jabas_amd import sync
+
+    seen = []
+
+    def total(rows):
+        seen.append(sync._watched())
+        return sync.gram_from_stats(rows, 2)
+
+    class Pass(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    class PassBelow(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    rows, other = (torch.randn(3, L.STATS_STRIDE, dtype=torch.float64, generator=torch.Generator().manual_seed(i)) for i in (1, 2))
+    want = total(other)
+    assert seen == [False]
+    recorded = [torch.jit.trace(total, rows, check_trace=False)]
+    recorded += [make_fx(total, tracing_mode=mode)(rows) for mode in ("real", "fake", "symbolic")]
+    assert seen[1:] == [True] * 4
+    for graph in recorded:
+        assert torch.equal(graph(other), want)
+    del seen[:]
+    for mode in (Pass(), PassBelow()):
+        with mode:
+            assert torch.equal(total(other), want)
+    with torch.device("cpu"):                     # the mode of torch.set_default_device replaces no operation on rows
+        assert torch.equal(total(other), want)
+    assert seen == [True, True, False]

@@ -1051,3 +1051,16 @@ def test_gram_from_rows_on_the_device(gpu, K, n_rows):
     assert L.lib().jabas_gram_from_rows(None, 1, K, dev.data_ptr(), None) == L.ERR_NULL
     assert L.lib().jabas_gram_from_rows(dev.data_ptr(), 1, 9, dev.data_ptr(), None) == L.ERR_K
     assert L.lib().jabas_gram_from_rows(dev.data_ptr() + 4, 1, K, dev.data_ptr(), None) == L.ERR_ALIGN
+
+
+def test_gram_from_rows_recorded(gpu):
+    """Recordings of gram_from_stats answer for rows they were not made with. Four rows of small whole numbers: every sum is exact."""
+    from torch.fx.experimental.proxy_tensor import make_fx
+    from jabas_amd import sync, _lib as L
+    rows, other = (torch.randint(-99, 99, (4, L.STATS_STRIDE), generator=torch.Generator().manual_seed(i)).double().to(gpu) for i in (1, 2))
+    want = sync.gram_from_stats(other, 3)
+    for graph in (torch.jit.trace(lambda r: sync.gram_from_stats(r, 3), rows, check_trace=False),
+                  make_fx(lambda r: sync.gram_from_stats(r, 3))(rows)):
+        stale = torch.full((3, 3), float("nan"), dtype=torch.float64, device=gpu)       # left in the block an unwritten output would get
+        del stale
+        assert torch.equal(graph(other), want)
