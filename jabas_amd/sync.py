@@ -562,12 +562,19 @@ def _watched():
         not isinstance(mode, DeviceContext) for mode in _get_current_function_mode_stack())
 
 
+def _plain(t):
+    """Whether the values of ``t`` are what its memory holds: not a subclass, not one that stands for others in a function
+    transform, no lazy negation, no zeros without memory, no list of tensors."""
+    return type(t) is torch.Tensor and not (
+        t.is_neg() or t.is_nested or t._is_zerotensor() or torch._is_functional_tensor(t)
+        or torch._C._functorch.is_functorch_wrapped_tensor(t))
+
+
 def _device_rows(t):
     """Whether a kernel can read the statistics rows as they are: whole contiguous fp64 rows in GPU memory of a
-    plain tensor (not one that stands for others in a function transform) while nothing records the operations."""
-    return (not _watched() and type(t) is torch.Tensor and t.is_cuda and t.dtype == torch.float64 and t.is_contiguous()
-            and 0 < t.numel() < L.STATS_STRIDE << 32 and t.numel() % L.STATS_STRIDE == 0 and not t.is_neg()
-            and not torch._C._functorch.is_functorch_wrapped_tensor(t))
+    plain tensor while nothing records the operations on it."""
+    return (not _watched() and _plain(t) and t.is_cuda and t.dtype == torch.float64 and t.layout == torch.strided
+            and t.is_contiguous() and 0 < t.numel() < L.STATS_STRIDE << 32 and t.numel() % L.STATS_STRIDE == 0)
 
 
 def gram_from_stats(stats_rows, K):

@@ -681,3 +681,23 @@ def test_rows_are_not_read_behind_a_recorder():
     with torch.device("cpu"):                     # the mode of torch.set_default_device replaces no operation on rows
         assert torch.equal(total(other), want)
     assert seen == [True, True, False]
+
+
+@pytest.mark.filterwarnings("ignore::UserWarning")
+def test_rows_without_values_of_their_own_are_not_plain():
+    """Tensors that are strided, contiguous and of the right type and size, but whose memory is not their values."""
+    import torch
+    from jabas_amd import sync
+
+    rows = torch.randn(3, L.STATS_STRIDE, dtype=torch.float64, generator=torch.Generator().manual_seed(3))
+    assert sync._plain(rows) and sync._plain(rows[1]) and sync._plain(rows.detach().requires_grad_())
+    zeros = torch._efficientzerotensor(3, L.STATS_STRIDE, dtype=torch.float64)
+    negated = torch._neg_view(rows)
+    nested = torch.nested.nested_tensor([rows, rows])
+    functional = torch._to_functional_tensor(rows)
+    assert not any(sync._plain(t) for t in (zeros, negated, nested, functional, torch.nn.Parameter(rows)))
+    torch.func.vmap(lambda r: torch.tensor(0.0) if not sync._plain(r) else 1 / 0)(rows)
+    assert torch.equal(sync.gram_from_stats(zeros, 2), torch.zeros(2, 2, dtype=torch.float64))
+    assert torch.equal(sync.gram_from_stats(negated, 2), -sync.gram_from_stats(rows, 2))
+    with pytest.raises(RuntimeError):
+        sync.gram_from_stats(nested, 2)

@@ -1064,3 +1064,15 @@ def test_gram_from_rows_recorded(gpu):
         stale = torch.full((3, 3), float("nan"), dtype=torch.float64, device=gpu)       # left in the block an unwritten output would get
         del stale
         assert torch.equal(graph(other), want)
+
+
+@pytest.mark.filterwarnings("ignore::UserWarning")
+def test_gram_from_rows_that_hold_no_memory(gpu):
+    """Zeros without memory are summed like any others; a list of row tensors is refused."""
+    from jabas_amd import sync, _lib as L
+    zeros = torch._efficientzerotensor(3, L.STATS_STRIDE, dtype=torch.float64, device=gpu)
+    assert torch.equal(sync.gram_from_stats(zeros, 2), torch.zeros(2, 2, dtype=torch.float64, device=gpu))
+    rows = torch.ones(3, L.STATS_STRIDE, dtype=torch.float64, device=gpu)
+    assert torch.equal(sync.gram_from_stats(torch._neg_view(rows), 2), torch.full((2, 2), -3.0, dtype=torch.float64, device=gpu))
+    with pytest.raises(RuntimeError):
+        sync.gram_from_stats(torch.nested.nested_tensor([rows, rows]), 2)
