@@ -2,7 +2,7 @@
 // Fixed order of operations: bit-identical run to run.
 //   few workers    grid-stride over 4-element vectors, exact fp64 products of the fp32 (or widened bf16) values,
 //                  K(K+1)/2 fp64 accumulators per thread on the vector ALU, summed over the wave on the fp64 matrix
-//                  cores -> LDS -> one packed partial row per workgroup (K <= 3 for fp32 gradients, K <= 7 for bf16);
+//                  cores -> LDS -> one packed partial row per workgroup (K <= 5 for fp32 gradients, K <= 7 for bf16);
 //   more, to 16    fp32 gradients: fp64 matrix cores, v_mfma_f64_4x4x4 over 4 x 4 blocks of worker pairs, fed
 //                  from registers (gram_mfma_kernel below), still exact products and fp64 sums;
 //                  bf16 gradients: bf16 matrix cores, exact fp32 products, fp32 running sums over short runs,
@@ -11,7 +11,7 @@
 #include "jabas_internal.h"
 
 #ifndef JABAS_GRAM_VALU_MAX_K
-#define JABAS_GRAM_VALU_MAX_K 3
+#define JABAS_GRAM_VALU_MAX_K 5
 #endif
 
 namespace jabas {
@@ -20,10 +20,14 @@ namespace {
 #ifndef JABAS_GRAM_VALU_MAX_K_BF16
 #define JABAS_GRAM_VALU_MAX_K_BF16 7
 #endif
-// Up to here the vector-ALU kernel, beyond it the matrix cores. Both, on 25.6 M / 1.2 M elements, whole call in us:
-// fp32 K = 3: 54.3 / 10.7 against 53.7 / 11.6, K = 4: 71.8 / 13.3 against 69.3 / 12.3, K = 5: 93.2 / 16.5 against
-// 91.3 / 13.1. bf16 gradients change at eight workers, where the matrix cores' sums are fp32 over short runs: up to
-// seven every sum stays fp64.
+// Up to here the vector-ALU kernel, beyond it the matrix cores. Both on fp32 gradients of 65 k / 300 k / 1.2 M / 25.6 M /
+// 67 M / 100 M elements, whole call in us, vector ALU against matrix cores:
+//   K = 4   5.9 / 7.1 /  9.3 /  68.5 / 165.5 / 244.3   against   5.9 / 8.1 / 10.2 /  69.7 / 180.6 / 260.9
+//   K = 5   5.9 / 7.6 / 10.2 /  85.6 / 218.6 / 327.1   against   6.2 / 9.0 / 11.9 /  90.1 / 227.7 / 329.0
+//   K = 6   6.1 / 9.6 / 13.4 / 101.1 / 260.1 / 395.5   against   6.3 / 9.2 / 12.2 / 102.5 / 261.0 / 381.8
+//   K = 7   6.5 / 10.2 / 14.8 / 117.8 / 325.8 / 473.3  against   6.4 / 9.3 / 12.7 / 116.7 / 298.2 / 440.1
+// The vector ALU also sums in chains a sixteenth as long: 100 M elements are 1e-16 off against 5e-15. bf16 gradients change
+// at eight workers, where the matrix cores' sums are fp32 over short runs: up to seven every sum stays fp64.
 constexpr int gram_valu_max_k(int grad_dtype) { return grad_dtype == JABAS_BF16 ? JABAS_GRAM_VALU_MAX_K_BF16 : JABAS_GRAM_VALU_MAX_K; }
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -164,7 +168,7 @@ __global__ void __launch_bounds__(kGramFinalizeBlock) gram_finalize_kernel(int K
 }
 
 
-// ---- K >= 4: fp64 matrix cores, 4 x 4 blocks ----------------------------------------------------------
+// ---- K >= 6: fp64 matrix cores, 4 x 4 blocks ----------------------------------------------------------
 // The Gram matrix is a contraction over the elements, X X^T with X the K x N matrix of the workers'
 // gradients. The workers are cut into G = ceil(K / 4) groups of four; v_mfma_f64_4x4x4 (four independent
 // 4 x 4 x 4 products per instruction) forms, for one pair of groups (ga <= gb), the 4 x 4 block of products
@@ -173,7 +177,7 @@ __global__ void __launch_bounds__(kGramFinalizeBlock) gram_finalize_kernel(int K
 // (a wave reads 256 contiguous bytes of each worker) and feeds round r of every pair from registers,
 // A = element r of its vector of group ga, B = element r of its vector of group gb: no LDS, no shuffles,
 // G(G+1)/2 running sums per lane instead of K(K+1)/2 register pairs per thread (which is what limits the
-// vector-ALU form to K <= 8). Products of widened fp32 values are exact in fp64 and the order is fixed.
+// vector-ALU form to few workers). Products of widened fp32 values are exact in fp64 and the order is fixed.
 // Per 64 elements: 4 G(G+1)/2 MFMAs and 4 G conversions per wave, against 36 fp64 multiply-adds and 8
 // conversions PER ELEMENT AND THREAD at K = 8 on the vector ALU.
 #ifndef JABAS_GRAM_RUN_F32

@@ -1076,3 +1076,18 @@ def test_gram_from_rows_that_hold_no_memory(gpu):
     assert torch.equal(sync.gram_from_stats(torch._neg_view(rows), 2), torch.full((2, 2), -3.0, dtype=torch.float64, device=gpu))
     with pytest.raises(RuntimeError):
         sync.gram_from_stats(torch.nested.nested_tensor([rows, rows]), 2)
+
+
+@pytest.mark.parametrize("K", [3, 4, 5])
+def test_gram_of_few_workers_rounds_in_short_chains(gpu, K):
+    """2**25 elements of 1 + d and 1 - d, d = 2**-22: products 1 +- 2**-21 + 2**-44 and 1 - 2**-44. A thread sums 128 of
+    them, exactly (seven bits and 45). What follows rounds at most 50 times (wave 8, workgroup 8, rows of a part 16, parts
+    of a wave 2, waves 16). In chains of 2048 products, as long as a wave's sums on the matrix cores are, the 2**-44 is lost
+    from a sum of 512 on: 4e-14 off."""
+    from jabas_amd import sync
+    n, d = 1 << 25, 2.0 ** -22
+    G = sync.gram([torch.full((n,), 1 - d if k % 2 else 1 + d, dtype=torch.float32, device=gpu) for k in range(K)]).cpu()
+    for a in range(K):
+        for b in range(K):
+            exact = n * (1 - d * d if (a + b) % 2 else 1 - 2 * d + d * d if a % 2 else 1 + 2 * d + d * d)
+            assert abs(float(G[a, b]) - exact) <= 50 * 2.0 ** -53 * exact, (a, b)
