@@ -154,7 +154,11 @@ def lib():
                 "or `make -C jabas_amd/csrc` (needs hipcc). There is no CPU fallback.")
         handle = C.CDLL(LIB_PATH)
         for name, (res, args) in SIGNATURES.items():
-            fn = getattr(handle, name)
+            try:
+                fn = getattr(handle, name)
+            except AttributeError:
+                raise RuntimeError(f"{LIB_PATH} has no {name}: it was built from older sources; build it again "
+                                   "(`make -C jabas_amd/csrc`)") from None
             fn.restype = res
             fn.argtypes = args
         _lib = handle

@@ -701,3 +701,12 @@ def test_rows_without_values_of_their_own_are_not_plain():
     assert torch.equal(sync.gram_from_stats(negated, 2), -sync.gram_from_stats(rows, 2))
     with pytest.raises(RuntimeError):
         sync.gram_from_stats(nested, 2)
+
+
+def test_library_without_an_entry_point_is_refused_by_name(monkeypatch):
+    """A library of an older build lacks an entry point that the package calls."""
+    monkeypatch.setattr(L, "_lib", None)
+    monkeypatch.setitem(L.SIGNATURES, "jabas_of_a_later_build", (C.c_int, []))
+    with pytest.raises(RuntimeError, match="jabas_of_a_later_build.*build it again"):
+        L.lib()
+    assert L._lib is None
