@@ -2,7 +2,7 @@
 """Benchmark of the fused per-GPU gradient-sync step on one MI355X.
 
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--workload NAME] [--no-all] [--no-cpu] [--no-extras]
-                    [--cpu-seconds S] [--calibrate-copy] [--flat-moments]
+                    [--cpu-seconds S] [--calibrate-copy] [--flat-moments] [--details FILE]
 
 A step is one fused sync step (batch-weighted aggregate of the K VSW gradient buckets
 + the similarity statistics where the configuration asks for them + optimizer update) over
@@ -17,10 +17,10 @@ Prints ONE JSON line: metric sync_step_GBps = algorithmic bytes per step / time 
 with a "roofline" object (HBM-bound; achieved = algorithmic bytes per launch / mean launch
 duration = HIP-event time of the timed region on the launching stream / its launches) and a
 "cpu_baseline" object (the reference's unfused PyTorch structure timed on this box's host
-cores, rank 0 only, a bounded number of whole steps). Every entry of "workloads" carries
-its own figures of both, the step as the reference's calling convention reaches it (one
-hook call per bucket and VSW: one launch per bucket, per 64 MiB of buckets, per step), and the neighbouring launches
-(without statistics, with full statistics rows).
+cores, rank 0 only, a bounded number of whole steps). Every entry of "workloads" carries the time of its own
+step, of the step as the reference's calling convention reaches it (one hook call per bucket and VSW: one launch
+per bucket, per 64 MiB of buckets, per step), and of the neighbouring launches (without statistics, with full
+statistics rows). The line is kept short enough to be recorded whole; --details FILE writes everything measured.
 """
 import argparse
 import gc
@@ -680,6 +680,24 @@ def cpu_baseline(cfg, torch, budget_s):
                        f"torch.optim single-tensor loop), median of {iters} whole steps after 1 warm-up")
 
 
+def _digits(x, n=4):
+    return float(f"{x:.{n}g}") if isinstance(x, float) else x
+
+
+def printed_line(out):
+    """The line of a run: the headline's figures whole, beside them one time in ms per leg."""
+    line = dict(out)
+    line["workloads"] = rows = []
+    for r in out["workloads"]:
+        row = {k: _digits(r[k]) for k in ("workload", "ms_per_step", "GBps", "pct_hbm_peak")}
+        row["legs_ms"] = {k: _digits(v["ms_per_step"]) for k, v in r.items() if isinstance(v, dict) and "ms_per_step" in v}
+        rows.append(row)
+    line["like_for_like"] = {k: _digits(v["ms_per_step"]) for k, v in out["like_for_like"].items() if v}
+    line["gram_launches"] = {f"{g['grad_dtype']}_K{g['K']}_ms": _digits(g["ms_per_step"]) for g in out["gram_launches"] or []}
+    del line["statistics_launches"], line["reference_profile_metrics_resnet50"]
+    return json.dumps(line)
+
+
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
@@ -691,6 +709,7 @@ def main():
     ap.add_argument("--no-extras", action="store_true",
                     help="per workload only the timed steps and the instrumented launches (a kernel trace of such a "
                          "run holds one kind of launch per kernel name and grid)")
+    ap.add_argument("--details", metavar="FILE", help="write every figure of the run to FILE (JSON)")
     ap.add_argument("--cpu-seconds", type=float, default=20.0,
                     help="CPU time the headline's baseline may take; the other workloads get a third each")
     ap.add_argument("--bucket-launches", type=int, default=0, metavar="S",
@@ -831,7 +850,10 @@ def main():
         "device": guarded("device_info", lambda: device_info(device, torch)),
         "failures": failures,
     }
-    print(json.dumps(out))
+    if args.details:
+        with open(args.details, "w") as f:
+            json.dump(out, f, indent=1)
+    print(printed_line(out))
 
 
 if __name__ == "__main__":

@@ -102,3 +102,28 @@ def test_tracked_hbm_traffic_covers_every_workload_at_its_algorithmic_bytes():
         assert abs(entry["algorithmic_bytes"] - want) <= 1e-5 * want, (cfg.name, entry["algorithmic_bytes"], want)
         assert 1.0 <= entry["hbm_bytes_per_launch"] / want <= 1.02, cfg.name
         assert bench.measured_traffic(cfg.name) == entry["hbm_bytes_per_launch"]
+
+
+def test_benchmark_line_is_short_and_keeps_the_headline():
+    """What records a run keeps less than 10 000 characters of its output, the progress lines (about 2000) after the line."""
+    import json
+    import os
+    import sys
+    sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
+    import bench
+    leg = {name: 1.0 / 3.0 for name in ("ms_per_step", "GBps", "pct_hbm_peak", "wall_ms_per_step", "host_us_per_step")}
+    work = dict(workload="faster_rcnn_r50_fpn", elements=41885910, batches=[4, 2, 2], **leg,
+                **{f"hook_path_per_bucket_{i}_streams": dict(leg) for i in range(17)}, failed_leg=None)
+    out = dict(metric="sync_step_GBps", value=17728.0 / 3.0, unit="GB/s", n_gpus=1, ms_per_step=2.2689967346191406, failures={},
+               config=dict(workload="vit_l16"), roofline=leg, workloads=[work] * 5, reference_profile_metrics_resnet50=None,
+               like_for_like=dict(vit_b16=None, vit=leg), statistics_launches=[leg] * 8, gram_launches=None)
+    line = bench.printed_line(out)
+    assert len(line) < 7000 and "\n" not in line
+    got = json.loads(line)
+    for key in ("metric", "value", "unit", "n_gpus", "ms_per_step", "config", "roofline", "failures"):
+        assert got[key] == out[key]
+    assert len(got["workloads"]) == 5 and got["workloads"][0]["legs_ms"]["hook_path_per_bucket_0_streams"] == 0.3333
+    assert got["like_for_like"] == {"vit": 0.3333} and got["gram_launches"] == {}
+    out["gram_launches"] = [dict(K=4, grad_dtype="f32", **leg)]
+    assert json.loads(bench.printed_line(out))["gram_launches"] == {"f32_K4_ms": 0.3333}
+    assert out["workloads"] == [work] * 5
