@@ -585,11 +585,13 @@ def gram_from_stats(stats_rows, K):
     if not 1 <= K <= L.STATS_GRAM_MAX_K:
         raise ValueError(f"rows of level 'gram' exist for 1..{L.STATS_GRAM_MAX_K} workers, not {K}")
     if _device_rows(stats_rows):
-        n_rows = stats_rows.numel() // L.STATS_STRIDE
-        with torch.cuda.device(stats_rows.device):
-            out = torch.empty(K, K, dtype=torch.float64, device=stats_rows.device)
-            L.check(L.lib().jabas_gram_from_rows(stats_rows.data_ptr(), n_rows, K, out.data_ptr(), _stream_ptr()),
-                    "jabas_gram_from_rows")
+        dev = stats_rows.device
+        if dev.index != torch.cuda.current_device():
+            with torch.cuda.device(dev):
+                return gram_from_stats(stats_rows, K)
+        out = torch.empty(K, K, dtype=torch.float64, device=dev)
+        L.check(L.lib().jabas_gram_from_rows(stats_rows.data_ptr(), stats_rows.numel() // L.STATS_STRIDE, K, out.data_ptr(),
+                                             _stream_ptr()), "jabas_gram_from_rows")
         return out
     total = stats_rows.detach().reshape(-1, L.STATS_STRIDE).to(torch.float64).sum(dim=0)
     out = torch.empty(K, K, dtype=torch.float64, device=total.device)
