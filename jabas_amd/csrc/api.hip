@@ -421,8 +421,8 @@ __global__ void __launch_bounds__(64) clip_coef_kernel(const double* rows, uint3
 
 // K x K matrix of the workers' products out of rows of level JABAS_STATS_GRAM: one workgroup sums the rows (wave w
 // takes rows w, w + 16, ... in order, lane = slot, so a wave reads one whole row per load), adds the 16 sums of a slot in
-// wave order and unfolds the norms and pair slots. Bound by its launch: torch operations on the same rows are K (K + 1) / 2
-// element copies, 0.39 ms of launches for eight workers (K = 8, 1.2 M elements: step and matrix 364 -> 41 us).
+// wave order and unfolds the norms and pair slots. Bound by its launch (1.8 us for one row): torch operations on the same
+// rows are a sum and K * K element copies (K = 8, 1.2 M elements: step and matrix 364 -> 41 us).
 constexpr int kGramRowsBlock = 1024;
 __global__ void __launch_bounds__(kGramRowsBlock) gram_from_rows_kernel(const double* rows, uint32_t n_rows, int K, double* out) {
     __shared__ double sums[kGramRowsBlock / 64][kStatsStride];

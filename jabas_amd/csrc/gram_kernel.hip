@@ -108,10 +108,10 @@ __global__ void __launch_bounds__(kBlock) gram_kernel(const SpanDev sp, double* 
 
     // Sum of every product over the wave's lanes on the fp64 matrix cores: lane j + 4 b + 16 i supplies entry (j, i) of
     // product b of v_mfma_f64_4x4x4 as the left operand and (i, j) as the right one. With ones on the other side the first
-    // adds lanes 16 apart (entry (j, *) of its result is the sum over i), the second the four j: every lane 4 b + j of
-    // the last row holds the sum of the lanes with its b. Multiplying by one is exact, the sums are fp64. Two instructions
-    // per product, where a tree of wave shuffles takes twelve LDS permutations: 1.2 M elements, whole call, K = 5 fp32
-    // 22.0 -> 16.5 us, K = 7 bf16 34.8 -> 24.4.
+    // adds lanes 16 apart (entry (j, *) of its result is the sum over i), the second the four j: every lane then holds the
+    // sum of the 16 lanes with its b, and lanes 0, 4, 8 and 12 write the four. Multiplying by one is exact, the sums are
+    // fp64. Two instructions per product, where a tree of wave shuffles takes twelve LDS permutations: 1.2 M elements,
+    // whole call, K = 5 fp32 22.0 -> 16.5 us, K = 7 bf16 34.8 -> 24.4 (10.2 and 13.5 with the finalize below).
     __shared__ double red[kWaves][4][NP];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
@@ -233,8 +233,11 @@ __global__ void __launch_bounds__(kBlock) gram_mfma_kernel(const SpanDev sp, int
             }
     };
     // Bound by HBM reads. Two runs in flight per wave, the next one's loads issued before this one is multiplied; only whole
-    // runs, so that the loop has no edge path. 25.6 M elements, whole call: K = 8 133.3 -> 122.8 us (6.66 TB/s), K = 12
-    // 197.4 -> 189.1 (6.49); runs half as long or twice as long lose 2-5 %.
+    // runs, so that the loop has no edge path. Whole call, one run in flight -> two, 25.6 M elements: K = 6 106.0 -> 102.5
+    // us, K = 8 135.2 -> 124.5 (6.57 TB/s), K = 12 197.5 -> 189.0 (6.49), K = 13 226.8 -> 220.5, K = 16 259.1 -> 256.8;
+    // 100 M: K = 8 502 -> 490, K = 12 743 -> 732, K = 16 991 -> 990. Over 240 random sizes from 65 k to 100 M: K = 6..8
+    // 1.00-1.08 times as fast by decade half, K = 9..12 0.99-1.05 (0.99 around 600 k), K = 13..16 1.00-1.05. Runs half as
+    // long or twice as long lose 2-5 %.
     const uint64_t id = static_cast<uint64_t>(blockIdx.x) * kWaves + wave;
     L::Raw x[kGramRunBlocks][G], y[kGramRunBlocks][G];
     uint64_t run = first + id;
@@ -349,9 +352,6 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef u32x4 __attribute__((aligned(8))) u32x4_a8;     // element 0 of a bf16 buffer is 8-byte aligned, not more
 
 // 128-element blocks a wave loads before it multiplies, by number of groups
-#ifndef JABAS_GRAM_RUN_BF16_G1
-#define JABAS_GRAM_RUN_BF16_G1 2
-#endif
 #ifndef JABAS_GRAM_RUN_BF16_G2
 #define JABAS_GRAM_RUN_BF16_G2 2
 #endif
@@ -362,7 +362,7 @@ typedef u32x4 __attribute__((aligned(8))) u32x4_a8;     // element 0 of a bf16 b
 #define JABAS_GRAM_RUN_BF16_G4 4
 #endif
 constexpr int gram_bf16_run(int G) {
-    return G == 1 ? JABAS_GRAM_RUN_BF16_G1 : G == 2 ? JABAS_GRAM_RUN_BF16_G2 : G == 3 ? JABAS_GRAM_RUN_BF16_G3 : JABAS_GRAM_RUN_BF16_G4;
+    return G == 2 ? JABAS_GRAM_RUN_BF16_G2 : G == 3 ? JABAS_GRAM_RUN_BF16_G3 : JABAS_GRAM_RUN_BF16_G4;
 }
 constexpr int kGramBf16FlushRuns = 128;
 
@@ -459,9 +459,9 @@ __global__ void __launch_bounds__(kBlock) gram_bf16_mfma_kernel(const SpanDev sp
     }
 }
 
+static_assert(JABAS_GRAM_VALU_MAX_K >= 4 && JABAS_GRAM_VALU_MAX_K_BF16 >= 4, "the matrix-core kernels start at two groups");
 int launch_gram_bf16_mfma(int K, const SpanDev& sp, double* partials, unsigned grid, hipStream_t stream) {
     switch ((K + 3) / 4) {
-        case 1: return static_cast<int>(launch_kernel(gram_bf16_mfma_kernel<1>, dim3(grid), dim3(kBlock), 0, stream, sp, K, partials));
         case 2: return static_cast<int>(launch_kernel(gram_bf16_mfma_kernel<2>, dim3(grid), dim3(kBlock), 0, stream, sp, K, partials));
         case 3: return static_cast<int>(launch_kernel(gram_bf16_mfma_kernel<3>, dim3(grid), dim3(kBlock), 0, stream, sp, K, partials));
         case 4: return static_cast<int>(launch_kernel(gram_bf16_mfma_kernel<4>, dim3(grid), dim3(kBlock), 0, stream, sp, K, partials));
@@ -480,7 +480,6 @@ int launch_gram_k(int grad_dtype, const SpanDev& sp, double* partials, unsigned 
 
 int launch_gram_mfma(int K, const SpanDev& sp, double* partials, unsigned grid, hipStream_t stream) {
     switch ((K + 3) / 4) {
-        case 1: return static_cast<int>(launch_kernel(gram_mfma_kernel<1>, dim3(grid), dim3(kBlock), 0, stream, sp, K, partials));
         case 2: return static_cast<int>(launch_kernel(gram_mfma_kernel<2>, dim3(grid), dim3(kBlock), 0, stream, sp, K, partials));
         case 3: return static_cast<int>(launch_kernel(gram_mfma_kernel<3>, dim3(grid), dim3(kBlock), 0, stream, sp, K, partials));
         case 4: return static_cast<int>(launch_kernel(gram_mfma_kernel<4>, dim3(grid), dim3(kBlock), 0, stream, sp, K, partials));
