@@ -323,25 +323,45 @@ const LaunchFn kLaunch[JABAS_MAX_K] = {launch_fused_k1,  launch_fused_k2,  launc
 
 // Second level of the statistics reduction: sums partial rows in a fixed order.
 //   stripes == 0  rows [s*in_stripes, (s+1)*in_stripes) of `in` -> row s of `out`
-//   stripes >= 1  stripe j = blockIdx.x of the chunk rows of span s = blockIdx.y -> row s*stripes + j
-// Thread t adds rows t, t+256, ... in increasing order; the 256 per-thread sums then go
-// through the fixed wave tree and a wave-order sum, so the result does not depend on the
-// machine or on timing. A span with many chunks is cut into stripes (one workgroup each,
-// then one more launch over the stripe rows) because a single workgroup reads its rows at
-// the bandwidth of one CU.
-constexpr int kFinalizeBlock = 256;
-constexpr uint32_t kStripeRows = 512;        // chunk rows one workgroup sums in the striped launch
+//   stripes >= 1  stripe j = blockIdx.z of the chunk rows of span s = blockIdx.y -> row s*stripes + j
+// A workgroup sums four neighbouring slots (blockIdx.x) of its rows: lane = slot + 4 * row, so a wave's load covers
+// 32 contiguous bytes of sixteen rows, and a row of any width costs the time of its four widest. Thread (slot, class)
+// adds rows class, class + 256, ... in increasing order, sixteen loads in flight; the 256 sums of a slot meet by row
+// rotations, one LDS table and a second round of the same. The order depends on the number of rows alone, so the sums
+// that two statistics levels share are the same bits, on any machine.
+// Bound by latency: one trip to memory per sixteen (or four) rows of a class and the launch. Lanes along the rows with a
+// wave tree per slot, as it was, cost 2.1 us for 147 rows of 4 doubles, 5.6 us for 294 rows of 40, 9.4 us in two launches
+// beyond 2560 rows; this one 2.4, 3.8 and (3200 rows of 4, one launch) 4.5. Fourteen buckets through the hooks, fp32 K = 4:
+// 960 -> 897 us, 25 M elements, K = 6 with pair products: 243 -> 226 us.
+constexpr int kFinalizeBlock = 1024;
+constexpr int kFinalizeSlots = 4;
+constexpr uint32_t kFinalizeClasses = kFinalizeBlock / kFinalizeSlots;
+constexpr uint32_t kStripeRows = 1024;        // chunk rows one workgroup sums in the striped launch
 constexpr uint32_t kMaxStripes = 32;
-constexpr uint32_t kSingleLaunchRows = 2560; // up to here one workgroup per span finishes in about 6 us
-constexpr uint32_t kMaxStatsSpans = 65535;   // spans index the y dimension of the finalize grid
-template <int NS>
+constexpr uint32_t kSingleLaunchRows = 6144;  // up to here one workgroup per span and four slots (15.4 k rows: 9.9 us)
+constexpr uint32_t kMaxStatsSpans = 65535;    // spans index the y dimension of the finalize grid
+
+// Adds U rows of a class to acc, first row r, no row at or beyond c1 (c1 > 0): the loads are issued together, those beyond
+// the end repeat the last row and are dropped.
+template <int U>
+__device__ __forceinline__ void add_rows(const double* col, uint32_t ns, uint32_t r, uint32_t c1, double& acc) {
+    double v[U];
+#pragma unroll
+    for (int i = 0; i < U; ++i) {
+        const uint32_t c = r + i * kFinalizeClasses;
+        v[i] = col[static_cast<uint64_t>(c < c1 ? c : c1 - 1) * ns];
+    }
+#pragma unroll
+    for (int i = 0; i < U; ++i) acc += r + i * kFinalizeClasses < c1 ? v[i] : 0.0;
+}
+
 __global__ void __launch_bounds__(kFinalizeBlock) finalize_stats_kernel(const uint32_t* chunk_prefix, uint32_t n_chunks,
                                                                         uint32_t use_inline, uint32_t stripes,
-                                                                        uint32_t in_stripes, uint32_t out_stride,
+                                                                        uint32_t in_stripes, uint32_t ns, uint32_t out_stride,
                                                                         const double* in, double* out) {
-    // input rows are compact (NS doubles each, the width of the level); output rows have out_stride slots, the unused ones 0
-    __shared__ double red[kFinalizeBlock / 64][NS];
-    const uint32_t s = blockIdx.y, j = blockIdx.x, t = threadIdx.x;
+    // input rows are compact (ns doubles each, the width of the level); output rows have out_stride slots, the unused ones 0
+    __shared__ double table[kFinalizeBlock / 16][kFinalizeSlots];
+    const uint32_t s = blockIdx.y, j = blockIdx.z, t = threadIdx.x;
     uint32_t c0, c1, o;
     if (stripes == 0) {
         c0 = s * in_stripes;
@@ -355,51 +375,44 @@ __global__ void __launch_bounds__(kFinalizeBlock) finalize_stats_kernel(const ui
         c1 = c0 + per < b1 ? c0 + per : b1;
         o = s * stripes + j;
     }
-    double acc[NS];
-#pragma unroll
-    for (int i = 0; i < NS; ++i) acc[i] = 0.0;
-#pragma unroll 2
-    for (uint32_t c = c0 + t; c < c1; c += kFinalizeBlock) {
-        const double* row = in + static_cast<uint64_t>(c) * NS;
-#pragma unroll
-        for (int i = 0; i < NS; ++i) acc[i] += row[i];
-    }
-    const int lane = t & 63, wave = t >> 6;
-#pragma unroll
-    for (int i = 0; i < NS; ++i) {
-        const double v = wave_sum_to_lane63(acc[i]);
-        if (lane == 63) red[wave][i] = v;
-    }
-    __syncthreads();
-    if (t < out_stride) {
-        double sum = 0.0;
-        if (t < NS) {
-            sum = red[0][t];
-#pragma unroll
-            for (int w = 1; w < kFinalizeBlock / 64; ++w) sum += red[w][t];
+    const uint32_t slot = blockIdx.x * kFinalizeSlots + (t & (kFinalizeSlots - 1));
+    const double* col = in + (slot < ns ? slot : ns - 1);
+    double acc = 0.0;
+    for (uint32_t base = c0; base < c1;) {       // uniform over the workgroup
+        const uint32_t r = base + t / kFinalizeSlots;
+        if (c1 - base > 4 * kFinalizeClasses) {
+            add_rows<16>(col, ns, r, c1, acc);
+            base += 16 * kFinalizeClasses;
+        } else {
+            add_rows<4>(col, ns, r, c1, acc);
+            base += 4 * kFinalizeClasses;
         }
-        out[static_cast<uint64_t>(o) * out_stride + t] = sum;
+    }
+    acc += dpp_move<0x128, 0xf>(acc);            // row_ror:8, row_ror:4: the four classes of a 16-lane row, per slot
+    acc += dpp_move<0x124, 0xf>(acc);
+    if ((t & 15) < kFinalizeSlots) table[t >> 4][t & 15] = acc;
+    __syncthreads();
+    double* row = out + static_cast<uint64_t>(o) * out_stride;
+    if (t < 64) {                                // one wave: 64 entries of a slot, four per lane, then over the lanes
+        const int e = t >> 2, v = t & (kFinalizeSlots - 1);
+        double sum = table[e][v];
+#pragma unroll
+        for (int i = 1; i < kFinalizeBlock / 256; ++i) sum += table[16 * i + e][v];
+        sum += dpp_move<0x128, 0xf>(sum);
+        sum += dpp_move<0x124, 0xf>(sum);
+        sum += __shfl_xor(sum, 16);
+        sum += __shfl_xor(sum, 32);
+        if (t < kFinalizeSlots && slot < ns) row[slot] = sum;
+    } else if (blockIdx.x == 0) {
+        for (uint32_t i = ns + t - 64; i < out_stride; i += kFinalizeBlock - 64) row[i] = 0.0;
     }
 }
 
-template <int NS>
-hipError_t launch_finalize(dim3 grid, hipStream_t stream, const KArgs& a, uint32_t stripes, uint32_t in_stripes,
-                           uint32_t out_stride, const double* in, double* out) {
-    return launch_kernel(finalize_stats_kernel<NS>, grid, dim3(kFinalizeBlock), 0, stream, a.chunk_prefix, a.n_chunks,
-                         a.use_inline, stripes, in_stripes, out_stride, in, out);
-}
-// One instantiation per row width: 4 (similarity sums), 4 + K, K = 1..16, and 4 + K + K(K-1)/2 for K <= 8
-// (7, 10, 14, 19: among the widths of the full rows; 25, 32, 40).
-hipError_t finalize(int ns, dim3 grid, hipStream_t stream, const KArgs& a, uint32_t stripes, uint32_t in_stripes,
+hipError_t finalize(uint32_t ns, uint32_t grid_stripes, hipStream_t stream, const KArgs& a, uint32_t stripes, uint32_t in_stripes,
                     uint32_t out_stride, const double* in, double* out) {
-    switch (ns) {
-#define JABAS_FIN(n) case n: return launch_finalize<n>(grid, stream, a, stripes, in_stripes, out_stride, in, out);
-        JABAS_FIN(4) JABAS_FIN(5) JABAS_FIN(6) JABAS_FIN(7) JABAS_FIN(8) JABAS_FIN(9) JABAS_FIN(10) JABAS_FIN(11) JABAS_FIN(12)
-        JABAS_FIN(13) JABAS_FIN(14) JABAS_FIN(15) JABAS_FIN(16) JABAS_FIN(17) JABAS_FIN(18) JABAS_FIN(19) JABAS_FIN(20) JABAS_FIN(25)
-        JABAS_FIN(32) JABAS_FIN(40)
-#undef JABAS_FIN
-        default: return hipErrorInvalidValue;
-    }
+    const dim3 grid((ns + kFinalizeSlots - 1) / kFinalizeSlots, a.n_span, grid_stripes);
+    return launch_kernel(finalize_stats_kernel, grid, dim3(kFinalizeBlock), 0, stream, a.chunk_prefix, a.n_chunks, a.use_inline,
+                         stripes, in_stripes, ns, out_stride, in, out);
 }
 
 inline uint32_t stripes_for(uint32_t max_span_chunks) {
@@ -467,15 +480,14 @@ int run_fused(KArgs& a, const JabasStepArgs* s, uint32_t max_span_chunks, double
     }
     if (stats) {
         const uint32_t st = stripes_for(max_span_chunks);
-        const int ns = stats_row_width(s->K, stats);                // width of the partial rows
+        const uint32_t ns = static_cast<uint32_t>(stats_row_width(s->K, stats));      // width of the partial rows
         hipError_t err;
         if (st == 1) {
-            err = finalize(ns, dim3(1, a.n_span), stream, a, 1u, 0u, kStatsStride, a.partials, stats_out);
+            err = finalize(ns, 1, stream, a, 1u, 0u, kStatsStride, a.partials, stats_out);
         } else {
             double* level2 = a.partials + static_cast<uint64_t>(a.n_chunks) * ns;
-            err = finalize(ns, dim3(st, a.n_span), stream, a, st, 0u, static_cast<uint32_t>(ns), a.partials, level2);
-            if (err == hipSuccess)
-                err = finalize(ns, dim3(1, a.n_span), stream, a, 0u, st, kStatsStride, level2, stats_out);
+            err = finalize(ns, st, stream, a, st, 0u, ns, a.partials, level2);
+            if (err == hipSuccess) err = finalize(ns, 1, stream, a, 0u, st, kStatsStride, level2, stats_out);
         }
         if (err != hipSuccess) return JABAS_ERR_LAUNCH;
     }

@@ -1097,3 +1097,37 @@ def test_gram_of_few_workers_rounds_in_short_chains(gpu, K):
         for b in range(K):
             exact = n * (1 - d * d if (a + b) % 2 else 1 - 2 * d + d * d if a % 2 else 1 + 2 * d + d * d)
             assert abs(float(G[a, b]) - exact) <= 50 * 2.0 ** -53 * exact, (a, b)
+
+
+@pytest.mark.parametrize("rows", [1, 255, 257, 1024, 1025, 4097, 6144, 6145])
+@pytest.mark.parametrize("K,level", [(4, "similarity"), (5, "full"), (8, "gram"), (16, "full")])
+def test_statistics_over_many_chunks_are_exact(gpu, K, level, rows):
+    """Small whole numbers and weights that are powers of two: every sum is exact in fp64 in any order, so the row has to be
+    the integer result whatever the number of chunk rows (the edges of the second level's batches and of its split into
+    stripes) and the width of the row; scratch and output start as NaN."""
+    from jabas_amd import sync, _lib as L
+    chunk = 1024 * (2 if K <= 4 else 4)                        # 256 threads x 4 elements x tiles
+    n = chunk * (rows - 1) + 5
+    n = min(n, 1 << 24)
+    gen = torch.Generator(device=gpu).manual_seed(rows + K)
+    grads = [torch.randint(-3, 4, (n,), generator=gen, device=gpu).to(torch.bfloat16) for _ in range(K)]
+    batches = (4, 2, 1, 3, 2)[:K] if K == 5 else (1,) * K
+    args = sync.make_step_args(batches, torch.bfloat16, stats=level)
+    for k in range(K):                                         # powers of two instead of the batch quotients
+        args.weight[k] = args.half_weight[k] = 0.25
+    ws = sync.Workspace.for_span(n, torch.bfloat16, gpu)
+    ws.buf.fill_(float("nan"))
+    ws.stats.fill_(float("nan"))
+    row = sync.sync_bucket(sync.SpanSpec(grads), args, workspace=ws)
+    g = torch.stack(grads).float()
+    quarter = [(g[h::2].sum(0) * 0.25).double() for h in (0, 1)]
+    agg = (g.sum(0) * 0.25).double()
+    want = torch.zeros(L.STATS_STRIDE, dtype=torch.float64, device=gpu)
+    want[:4] = torch.stack([(quarter[0] * quarter[1]).sum(), (quarter[0] ** 2).sum(), (quarter[1] ** 2).sum(), (agg ** 2).sum()])
+    if level != "similarity":
+        want[4:4 + K] = torch.stack([(x.double() ** 2).sum() for x in g])
+    if level == "gram":
+        for a in range(K):
+            for b in range(a + 1, K):
+                want[L.stat_pair(K, a, b)] = (g[a].double() * g[b].double()).sum()
+    assert torch.equal(row, want)
