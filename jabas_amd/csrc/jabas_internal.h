@@ -15,8 +15,14 @@ namespace jabas {
 // buffer compact (higher HBM rate) and cut the ramp-up / drain of a launch; kernels that carry many
 // statistics have low occupancy and a long epilogue, and do better with more work per workgroup.
 // Measured per kernel family (A/B builds of the whole library, every shape passes the parity suite):
-//   full statistics rows          256 threads x 2 tiles (K <= 4) or 4 tiles (K > 4); 64, 128, 512 and
-//                                 1024 threads were all slower (-2 ... -15 %)
+//   full statistics rows          256 threads x 2 tiles (K <= 4) or 4 tiles (K = 5..8); 64, 128, 512 and
+//                                 1024 threads were all slower (-2 ... -15 %). K = 5..8 with full rows alone would be
+//                                 2-3 % faster at 2 tiles, but shares its chunks with the pair products, whose 25..40
+//                                 sums per workgroup make 2 tiles 11-14 % slower (K = 8 bf16, 25 and 90 M elements)
+//   full rows, K > 8              256 threads x 2 tiles: these kernels hold one tile in flight and two or three waves
+//                                 per SIMD, and half the work per workgroup keeps the streamed window compact and
+//                                 the last round of workgroups short: ResNet-50 K = 16 bf16 254 -> 232 us, K = 12
+//                                 fp32 SGD 25 M elements 307 -> 291, K = 16 fp32 Adam 60 M 957 -> 940 (1 tile: K = 16 bf16 240)
 //   similarity sums only          256 threads x 2 tiles: with four sums the K > 4 kernels fit 4 waves per SIMD
 //                                 with two tiles of loads in flight
 //   plain with optimizer, K > 4   256 threads x 2 tiles: +1 % over 512 x 1 and 512 x 2, +3 % over 256 x 4;
@@ -51,6 +57,9 @@ namespace jabas {
 #ifndef JABAS_CHUNK_TILES_MANYK
 #define JABAS_CHUNK_TILES_MANYK 2
 #endif
+#ifndef JABAS_CHUNK_TILES_FULL_MANYK
+#define JABAS_CHUNK_TILES_FULL_MANYK 2
+#endif
 #ifndef JABAS_CHUNK_TILES_SIM_MANYK
 #define JABAS_CHUNK_TILES_SIM_MANYK 2
 #endif
@@ -80,6 +89,7 @@ __host__ __device__ constexpr int launch_block(int K, int grad_dtype, int opt_cl
 }
 __host__ __device__ constexpr int launch_chunk_tiles(int K, int /*grad_dtype*/, int opt_class, int stats) {
     if (stats == 2) return K > 4 ? JABAS_CHUNK_TILES_SIM_MANYK : JABAS_CHUNK_TILES_SIM_LO;
+    if (stats && K > 8) return JABAS_CHUNK_TILES_FULL_MANYK;
     if (K > 4) return (stats || opt_class == 0) ? kMaxChunkTiles : JABAS_CHUNK_TILES_MANYK;
     if (!stats && opt_class >= 2) return JABAS_CHUNK_TILES_PLAIN_LO;
     return kMinChunkTiles;
@@ -93,7 +103,8 @@ __host__ __device__ constexpr int stats_row_width(int K, int stats) {
 constexpr int imin(int a, int b) { return a < b ? a : b; }
 // Fewest elements a chunk of a launch with statistics covers (one partial row per chunk): sizes workspaces.
 constexpr int kMinStatsChunkElems = 4 * imin(imin(JABAS_BLOCK * JABAS_CHUNK_TILES_LO, JABAS_BLOCK * JABAS_CHUNK_TILES_SIM_LO),
-                                             JABAS_BLOCK_SIM_MANYK * JABAS_CHUNK_TILES_SIM_MANYK);
+                                             imin(JABAS_BLOCK_SIM_MANYK * JABAS_CHUNK_TILES_SIM_MANYK,
+                                                  JABAS_BLOCK * JABAS_CHUNK_TILES_FULL_MANYK));
 // Fewest elements any chunk covers, over all shapes: sizes blobs that must fit every launch.
 constexpr int kMinChunkElems = imin(imin(kMinStatsChunkElems, 4 * JABAS_BLOCK_SGD * JABAS_CHUNK_TILES_LO),
                                     4 * imin(imin(JABAS_BLOCK * JABAS_CHUNK_TILES_PLAIN_LO, JABAS_BLOCK * JABAS_CHUNK_TILES_LO),

@@ -1106,7 +1106,7 @@ def test_statistics_over_many_chunks_are_exact(gpu, K, level, rows):
     the integer result whatever the number of chunk rows (the edges of the second level's batches and of its split into
     stripes) and the width of the row; scratch and output start as NaN."""
     from jabas_amd import sync, _lib as L
-    chunk = 1024 * (2 if K <= 4 else 4)                        # 256 threads x 4 elements x tiles
+    chunk = 1024 * (4 if 4 < K <= 8 else 2)                    # 256 threads x 4 elements x tiles
     n = chunk * (rows - 1) + 5
     n = min(n, 1 << 24)
     gen = torch.Generator(device=gpu).manual_seed(rows + K)
