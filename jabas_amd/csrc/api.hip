@@ -355,8 +355,8 @@ __device__ __forceinline__ void add_rows(const double* col, uint32_t ns, uint32_
     for (int i = 0; i < U; ++i) acc += r + i * kFinalizeClasses < c1 ? v[i] : 0.0;
 }
 
-__global__ void __launch_bounds__(kFinalizeBlock) finalize_stats_kernel(const uint32_t* chunk_prefix, uint32_t n_chunks,
-                                                                        uint32_t use_inline, uint32_t stripes,
+__global__ void __launch_bounds__(kFinalizeBlock) finalize_stats_kernel(const uint32_t* chunk_prefix, uint32_t n_rows,
+                                                                        uint32_t split_log2, uint32_t use_inline, uint32_t stripes,
                                                                         uint32_t in_stripes, uint32_t ns, uint32_t out_stride,
                                                                         const double* in, double* out) {
     // input rows are compact (ns doubles each, the width of the level); output rows have out_stride slots, the unused ones 0
@@ -368,8 +368,8 @@ __global__ void __launch_bounds__(kFinalizeBlock) finalize_stats_kernel(const ui
         c1 = c0 + in_stripes;
         o = s;
     } else {
-        uint32_t b0 = 0, b1 = n_chunks;
-        if (!use_inline) { b0 = chunk_prefix[s]; b1 = chunk_prefix[s + 1]; }
+        uint32_t b0 = 0, b1 = n_rows;
+        if (!use_inline) { b0 = chunk_prefix[s] << split_log2; b1 = chunk_prefix[s + 1] << split_log2; }
         const uint32_t per = (b1 - b0 + stripes - 1) / stripes;
         c0 = b0 + j * per < b1 ? b0 + j * per : b1;
         c1 = c0 + per < b1 ? c0 + per : b1;
@@ -408,11 +408,11 @@ __global__ void __launch_bounds__(kFinalizeBlock) finalize_stats_kernel(const ui
     }
 }
 
-hipError_t finalize(uint32_t ns, uint32_t grid_stripes, hipStream_t stream, const KArgs& a, uint32_t stripes, uint32_t in_stripes,
+hipError_t finalize(uint32_t ns, uint32_t grid_stripes, hipStream_t stream, const KArgs& a, uint32_t n_rows, uint32_t stripes, uint32_t in_stripes,
                     uint32_t out_stride, const double* in, double* out) {
     const dim3 grid((ns + kFinalizeSlots - 1) / kFinalizeSlots, a.n_span, grid_stripes);
-    return launch_kernel(finalize_stats_kernel, grid, dim3(kFinalizeBlock), 0, stream, a.chunk_prefix, a.n_chunks, a.use_inline,
-                         stripes, in_stripes, ns, out_stride, in, out);
+    return launch_kernel(finalize_stats_kernel, grid, dim3(kFinalizeBlock), 0, stream, a.chunk_prefix, n_rows, a.split_log2,
+                         a.use_inline, stripes, in_stripes, ns, out_stride, in, out);
 }
 
 inline uint32_t stripes_for(uint32_t max_span_chunks) {
@@ -460,34 +460,44 @@ __global__ void __launch_bounds__(kGramRowsBlock) gram_from_rows_kernel(const do
     }
 }
 
-int run_fused(KArgs& a, const JabasStepArgs* s, uint32_t max_span_chunks, double* stats_out, void* workspace,
+int run_fused(KArgs& a, const JabasStepArgs* s, uint32_t tiles, uint32_t max_span_chunks, double* stats_out, void* workspace,
               size_t workspace_bytes, hipStream_t stream) {
     const int oc = opt_class_of(s->opt_kind);
     const int stats = s->stats;                  // level, checked by fill_kargs
+    const uint32_t ns = static_cast<uint32_t>(stats_row_width(s->K, stats));      // width of the partial rows
+    // workgroups of the launch: a span by value has no chunk table, its last chunk's idle workgroups are left out
+    a.split_log2 = launch_split_log2(s->K, s->grad_dtype, oc, stats, a.n_chunks);
+    auto workgroups = [&] {
+        if (!a.use_inline) return static_cast<uint64_t>(a.n_chunks) << a.split_log2;
+        return chunks_of_tiles(tiles, a.chunk_tiles >> a.split_log2);
+    };
     if (stats) {
         if (!stats_out) return JABAS_ERR_NULL;
         if (a.n_span > kMaxStatsSpans) return JABAS_ERR_SIZE;     // before anything is launched: no half-done step
         if (!workspace || reinterpret_cast<uintptr_t>(workspace) % 8) return JABAS_ERR_WORKSPACE;
-        // one compact partial row per chunk and per (span, stripe), as wide as the level's rows are
-        if (workspace_bytes < workspace_rows(a.n_chunks, a.n_span) * stats_row_width(s->K, stats) * sizeof(double))
-            return JABAS_ERR_WORKSPACE;
+        // one compact partial row per workgroup and per (span, stripe), as wide as the level's rows are; scratch that holds
+        // a row per chunk only gets one workgroup per chunk
+        const auto fits = [&] { return workspace_bytes >= workspace_rows(workgroups(), a.n_span) * ns * sizeof(double); };
+        if (!fits()) a.split_log2 = 0;
+        if (!fits()) return JABAS_ERR_WORKSPACE;
         if (reinterpret_cast<uintptr_t>(stats_out) % 8) return JABAS_ERR_ALIGN;
     }
+    if (workgroups() > 0x7fffffffull) a.split_log2 = 0;
+    const uint32_t n_rows = static_cast<uint32_t>(workgroups());
     a.partials = static_cast<double*>(workspace);
     if (a.n_chunks) {
-        const int err = kLaunch[s->K - 1](s->grad_dtype, oc, stats, a.dyn != nullptr, a, a.n_chunks, stream);
+        const int err = kLaunch[s->K - 1](s->grad_dtype, oc, stats, a.dyn != nullptr, a, n_rows, stream);
         if (err != 0) return JABAS_ERR_LAUNCH;
     }
     if (stats) {
-        const uint32_t st = stripes_for(max_span_chunks);
-        const uint32_t ns = static_cast<uint32_t>(stats_row_width(s->K, stats));      // width of the partial rows
+        const uint32_t st = stripes_for(a.use_inline ? n_rows : max_span_chunks << a.split_log2);
         hipError_t err;
         if (st == 1) {
-            err = finalize(ns, 1, stream, a, 1u, 0u, kStatsStride, a.partials, stats_out);
+            err = finalize(ns, 1, stream, a, n_rows, 1u, 0u, kStatsStride, a.partials, stats_out);
         } else {
-            double* level2 = a.partials + static_cast<uint64_t>(a.n_chunks) * ns;
-            err = finalize(ns, st, stream, a, st, 0u, ns, a.partials, level2);
-            if (err == hipSuccess) err = finalize(ns, 1, stream, a, 0u, st, kStatsStride, level2, stats_out);
+            double* level2 = a.partials + static_cast<uint64_t>(n_rows) * ns;
+            err = finalize(ns, st, stream, a, n_rows, st, 0u, ns, a.partials, level2);
+            if (err == hipSuccess) err = finalize(ns, 1, stream, a, n_rows, 0u, st, kStatsStride, level2, stats_out);
         }
         if (err != hipSuccess) return JABAS_ERR_LAUNCH;
     }
@@ -711,7 +721,12 @@ JABAS_API size_t jabas_plan_workspace_bytes(const void* host_blob) {
     if (!host_blob) return 0;
     PlanHeader h;
     if (!read_plan_header(host_blob, &h)) return 0;
-    const uint32_t rows = h.shape[1].n_chunks > h.shape[2].n_chunks ? h.shape[1].n_chunks : h.shape[2].n_chunks;
+    uint64_t rows = 0;                           // of the level with the most workgroups
+    for (const int level : {JABAS_STATS_FULL, JABAS_STATS_SIMILARITY}) {
+        const uint64_t n = h.shape[level].n_chunks;
+        const uint64_t wg = n << launch_split_log2(h.K, h.grad_dtype, opt_class_of(h.opt_kind), level, n);
+        rows = wg > rows ? wg : rows;
+    }
     return workspace_rows(rows, h.n_span) * kStatsStride * sizeof(double);
 }
 
@@ -749,7 +764,7 @@ JABAS_API int jabas_sync_fused(const void* plan_host, const void* plan_dev, cons
     a.n_chunks = ps.n_chunks;
     a.chunk_tiles = ps.chunk_tiles;
     a.use_inline = 0;
-    return run_fused(a, args, ps.max_span_chunks, stats_out, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
+    return run_fused(a, args, 0, ps.max_span_chunks, stats_out, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
 }
 
 JABAS_API int jabas_sync_bucket(const JabasSpan* span, const JabasBound* bounds_dev, const JabasStepArgs* args,
@@ -777,7 +792,7 @@ JABAS_API int jabas_sync_bucket(const JabasSpan* span, const JabasBound* bounds_
     a.chunk_tiles = launch_chunk_tiles(args->K, args->grad_dtype, oc, stats);
     a.n_chunks = static_cast<uint32_t>(chunks_of_tiles(tiles, a.chunk_tiles));
     a.use_inline = 1;
-    return run_fused(a, args, a.n_chunks, stats_out, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
+    return run_fused(a, args, tiles, a.n_chunks, stats_out, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
 }
 
 // --- the entry point that allocates nothing -------------------------------------------------

@@ -560,11 +560,12 @@ __device__ __forceinline__ void workgroup_chunk(const KArgs& a, const A& s, uint
     constexpr int BS = launch_block(K, DT, OPT, SL);
     constexpr uint32_t CT = launch_chunk_tiles(K, DT, OPT, SL);     // the host cuts the chunk table for the same shape
     constexpr uint64_t TE = static_cast<uint64_t>(BS) * Grad<DT>::EPT;
+    const uint32_t per = CT >> a.split_log2;     // tiles of this workgroup
     if (a.use_inline) {
         const SpanDev& sp = a.span0;
         const uint32_t tiles = static_cast<uint32_t>((sp.hi + TE - 1) / TE);
-        const uint32_t lt0 = b * CT;
-        const uint32_t lt1 = lt0 + CT < tiles ? lt0 + CT : tiles;
+        const uint32_t lt0 = b * per;
+        const uint32_t lt1 = lt0 + per < tiles ? lt0 + per : tiles;
         uint32_t j0 = 0;
         if (sp.bound_count) {                  // largest j with bounds[j].start <= first live element
             ConstBounds bd = const_bounds(a.bounds + sp.bound_begin);
@@ -584,12 +585,13 @@ __device__ __forceinline__ void workgroup_chunk(const KArgs& a, const A& s, uint
         // repeat or keep as it likes) instead of being fetched again after every store that might alias them.
         typedef const __attribute__((address_space(4))) ChunkDesc* ConstChunk;
         typedef __attribute__((address_space(4))) SpanDev ConstSpan;
-        ConstChunk cp = (ConstChunk)(a.chunks + b);
-        const uint32_t c_span = cp->span, c_tile0 = cp->tile0, c_bound0 = cp->bound0;
+        ConstChunk cp = (ConstChunk)(a.chunks + (b >> a.split_log2));
+        const uint32_t c_span = cp->span, c_bound0 = cp->bound0;
+        const uint32_t lt0 = cp->tile0 + (b & ((1u << a.split_log2) - 1u)) * per;     // at or beyond the span's end: nothing to do
         const ConstSpan& sp = *(const ConstSpan*)(a.spans + c_span);
         const uint32_t tiles = static_cast<uint32_t>((sp.hi + TE - 1) / TE);
-        const uint32_t lt1 = c_tile0 + CT < tiles ? c_tile0 + CT : tiles;
-        run_chunk<K, DT, OPT, SL>(sp, c_tile0, lt1, c_bound0, s, acc);
+        const uint32_t lt1 = lt0 + per < tiles ? lt0 + per : tiles;
+        run_chunk<K, DT, OPT, SL>(sp, lt0, lt1, c_bound0, s, acc);
     }
 }
 

@@ -15,14 +15,8 @@ namespace jabas {
 // buffer compact (higher HBM rate) and cut the ramp-up / drain of a launch; kernels that carry many
 // statistics have low occupancy and a long epilogue, and do better with more work per workgroup.
 // Measured per kernel family (A/B builds of the whole library, every shape passes the parity suite):
-//   full statistics rows          256 threads x 2 tiles (K <= 4) or 4 tiles (K = 5..8); 64, 128, 512 and
-//                                 1024 threads were all slower (-2 ... -15 %). K = 5..8 with full rows alone would be
-//                                 2-3 % faster at 2 tiles, but shares its chunks with the pair products, whose 25..40
-//                                 sums per workgroup make 2 tiles 11-14 % slower (K = 8 bf16, 25 and 90 M elements)
-//   full rows, K > 8              256 threads x 2 tiles: these kernels hold one tile in flight and two or three waves
-//                                 per SIMD, and half the work per workgroup keeps the streamed window compact and
-//                                 the last round of workgroups short: ResNet-50 K = 16 bf16 254 -> 232 us, K = 12
-//                                 fp32 SGD 25 M elements 307 -> 291, K = 16 fp32 Adam 60 M 957 -> 940 (1 tile: K = 16 bf16 240)
+//   full statistics rows          256 threads x 2 tiles (K <= 4) or 4 tiles (K > 4); 64, 128, 512 and
+//                                 1024 threads were all slower (-2 ... -15 %)
 //   similarity sums only          256 threads x 2 tiles: with four sums the K > 4 kernels fit 4 waves per SIMD
 //                                 with two tiles of loads in flight
 //   plain with optimizer, K > 4   256 threads x 2 tiles: +1 % over 512 x 1 and 512 x 2, +3 % over 256 x 4;
@@ -57,9 +51,6 @@ namespace jabas {
 #ifndef JABAS_CHUNK_TILES_MANYK
 #define JABAS_CHUNK_TILES_MANYK 2
 #endif
-#ifndef JABAS_CHUNK_TILES_FULL_MANYK
-#define JABAS_CHUNK_TILES_FULL_MANYK 2
-#endif
 #ifndef JABAS_CHUNK_TILES_SIM_MANYK
 #define JABAS_CHUNK_TILES_SIM_MANYK 2
 #endif
@@ -89,13 +80,40 @@ __host__ __device__ constexpr int launch_block(int K, int grad_dtype, int opt_cl
 }
 __host__ __device__ constexpr int launch_chunk_tiles(int K, int /*grad_dtype*/, int opt_class, int stats) {
     if (stats == 2) return K > 4 ? JABAS_CHUNK_TILES_SIM_MANYK : JABAS_CHUNK_TILES_SIM_LO;
-    if (stats && K > 8) return JABAS_CHUNK_TILES_FULL_MANYK;
     if (K > 4) return (stats || opt_class == 0) ? kMaxChunkTiles : JABAS_CHUNK_TILES_MANYK;
     if (!stats && opt_class >= 2) return JABAS_CHUNK_TILES_PLAIN_LO;
     return kMinChunkTiles;
 }
 // Statistics level whose launch shape (and chunk table of a plan) a level uses.
 __host__ __device__ constexpr int shape_level(int stats) { return stats == JABAS_STATS_GRAM ? JABAS_STATS_FULL : stats; }
+// log2 of the workgroups that share a chunk of a launch of n_chunks chunks: a plan's tables know whole chunks only, the
+// launch decides how many workgroups each of them gets.
+//   short launches      split down to single tiles until there are 2048 workgroups (512 with statistics, whose epilogue is paid
+//                       per workgroup): below that compute units idle and a workgroup takes its tiles in turn, each at the
+//                       latency of memory. GPU time, whole chunks -> split: fp32 K = 4 Adam 0.1 / 0.3 / 0.7 / 1.5 M elements
+//                       10.7 / 16.1 / 14.9 / 20.4 -> 7.0 / 8.4 / 11.2 / 16.4 us (512 workgroups: 17.5), 6 M 51.3 -> 48.7
+//                       (1024: 51.9), bf16 K = 8 full rows 0.3 /
+//                       1.5 M 23.3 / 27.0 -> 13.0 / 22.4 (1024: 23.4), pair products 1.2 M 28.2 -> 24.5 (1024: 25.0)
+//   full rows, K > 8    two workgroups per chunk at any size: these kernels hold one tile in flight and two or three waves per
+//                       SIMD, and half the work per workgroup keeps the streamed window compact and the last round of
+//                       workgroups short: ResNet-50 K = 16 bf16 254 -> 231 us (four: 240), K = 12 fp32 SGD 25 M elements
+//                       307 -> 291, K = 16 fp32 Adam 60 M 957 -> 940. K = 5..8 would gain 2-3 % with full rows and lose
+//                       11-14 % with pair products (25..40 sums per workgroup), and both levels cut their sums alike
+#ifndef JABAS_SPLIT_BELOW
+#define JABAS_SPLIT_BELOW 2048
+#endif
+#ifndef JABAS_SPLIT_BELOW_STATS
+#define JABAS_SPLIT_BELOW_STATS 512
+#endif
+#ifndef JABAS_SPLIT_MANYK
+#define JABAS_SPLIT_MANYK 1
+#endif
+inline uint32_t launch_split_log2(int K, int grad_dtype, int opt_class, int stats, uint64_t n_chunks) {
+    const uint32_t tiles = static_cast<uint32_t>(launch_chunk_tiles(K, grad_dtype, opt_class, stats));
+    uint32_t s = stats == JABAS_STATS_FULL && K > 8 ? JABAS_SPLIT_MANYK : 0;
+    while ((2u << s) <= tiles && (n_chunks << s) < (stats ? JABAS_SPLIT_BELOW_STATS : JABAS_SPLIT_BELOW)) ++s;
+    return s;
+}
 // Width of the partial rows of a launch: 4 similarity sums, + K norms, + K(K-1)/2 pair products.
 __host__ __device__ constexpr int stats_row_width(int K, int stats) {
     return stats == JABAS_STATS_FULL ? 4 + K : (stats == JABAS_STATS_GRAM ? 4 + K + K * (K - 1) / 2 : (stats ? 4 : 1));
@@ -103,8 +121,7 @@ __host__ __device__ constexpr int stats_row_width(int K, int stats) {
 constexpr int imin(int a, int b) { return a < b ? a : b; }
 // Fewest elements a chunk of a launch with statistics covers (one partial row per chunk): sizes workspaces.
 constexpr int kMinStatsChunkElems = 4 * imin(imin(JABAS_BLOCK * JABAS_CHUNK_TILES_LO, JABAS_BLOCK * JABAS_CHUNK_TILES_SIM_LO),
-                                             imin(JABAS_BLOCK_SIM_MANYK * JABAS_CHUNK_TILES_SIM_MANYK,
-                                                  JABAS_BLOCK * JABAS_CHUNK_TILES_FULL_MANYK));
+                                             JABAS_BLOCK_SIM_MANYK * JABAS_CHUNK_TILES_SIM_MANYK);
 // Fewest elements any chunk covers, over all shapes: sizes blobs that must fit every launch.
 constexpr int kMinChunkElems = imin(imin(kMinStatsChunkElems, 4 * JABAS_BLOCK_SGD * JABAS_CHUNK_TILES_LO),
                                     4 * imin(imin(JABAS_BLOCK * JABAS_CHUNK_TILES_PLAIN_LO, JABAS_BLOCK * JABAS_CHUNK_TILES_LO),
@@ -190,7 +207,7 @@ struct KArgs {
     uint32_t chunk_tiles;                    // tiles per workgroup (the kernel's own shape; checked on the host)
     uint32_t use_inline;                     // 1: the only span is `span0`, chunk b starts at tile b*chunk_tiles
     uint32_t half_mask;                      // bit k set: VSW k belongs to half B
-    uint32_t pad0;
+    uint32_t split_log2;                     // 2^split_log2 workgroups share a chunk (launch_split_log2)
     SpanDev span0;
     float w[JABAS_MAX_K];
     float wh[JABAS_MAX_K];

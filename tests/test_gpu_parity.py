@@ -1106,7 +1106,7 @@ def test_statistics_over_many_chunks_are_exact(gpu, K, level, rows):
     the integer result whatever the number of chunk rows (the edges of the second level's batches and of its split into
     stripes) and the width of the row; scratch and output start as NaN."""
     from jabas_amd import sync, _lib as L
-    chunk = 1024 * (4 if 4 < K <= 8 else 2)                    # 256 threads x 4 elements x tiles
+    chunk = 1024 * (2 if K <= 4 else 4)                        # 256 threads x 4 elements x tiles, no optimizer
     n = chunk * (rows - 1) + 5
     n = min(n, 1 << 24)
     gen = torch.Generator(device=gpu).manual_seed(rows + K)
@@ -1131,3 +1131,63 @@ def test_statistics_over_many_chunks_are_exact(gpu, K, level, rows):
             for b in range(a + 1, K):
                 want[L.stat_pair(K, a, b)] = (g[a].double() * g[b].double()).sum()
     assert torch.equal(row, want)
+
+
+@pytest.mark.parametrize("K,dtype,level", [(1, torch.float32, None), (4, torch.float32, None), (4, torch.float32, "full"),
+                                           (8, torch.bfloat16, "gram"), (9, torch.float32, "full"), (16, torch.bfloat16, "full")])
+@pytest.mark.parametrize("numel", [1, 1023, 1025, 5 * 1024 + 3, 512 * 1024, 1024 * 1024 + 1, 2100 * 1024])
+def test_short_launches_give_the_result_of_whole_chunks(gpu, K, dtype, level, numel):
+    """How many workgroups share a chunk moves no element and no weight by a bit, whether the span comes by value or from a
+    plan, in spans that end inside a tile: against K one-span launches, each with the elements of one chunk at most, where
+    nothing is left to share. With scratch for a row per chunk only the launch takes whole chunks: same sums but for their order."""
+    from jabas_amd import sync, _lib as L
+    gen = torch.Generator(device=gpu).manual_seed(numel + K)
+    grads = [torch.randn(numel, generator=gen, device=gpu).to(dtype) for _ in range(K)]
+    p0, m0, v0 = (torch.randn(numel, generator=gen, device=gpu), torch.randn(numel, generator=gen, device=gpu) * 0.1,
+                  torch.rand(numel, generator=gen, device=gpu))
+    opt = dict(kind="adamw", betas=(0.9, 0.999), eps=1e-8, groups=[dict(lr=1e-2, weight_decay=0.0), dict(lr=2e-2, weight_decay=0.05)])
+    args = sync.make_step_args((1,) * K, dtype, stats=level or False, opt=opt, step=3)
+    cut = numel // 3
+    bounds = [(0, 1)] if cut == 0 else [(0, 1), (cut, 0)]
+
+    def launch(kind):
+        p, m, v, agg = p0.clone(), m0.clone(), v0.clone(), torch.zeros(numel, device=gpu)
+        span = sync.SpanSpec(grads, agg_out=agg, param=p, state1=m, state2=v, bounds=bounds)
+        row = None
+        if kind == "plan":
+            row = sync.SyncPlan([span], sync.opt_kind(opt)).run(args)
+        elif kind == "tight":
+            ws = sync.Workspace.for_span(numel, dtype, gpu)
+            tiles = -(-(numel + 63) // 1024)
+            chunks = -(-tiles // (2 if K <= 4 and level else 4))
+            width = {None: 1, "full": 4 + K, "gram": 4 + K + K * (K - 1) // 2}[level]
+            ws.nbytes = (chunks + 33) * width * 8
+            row = sync.sync_bucket(span, args, workspace=ws)
+        elif kind == "span":
+            row = sync.sync_bucket(span, args, workspace=sync.Workspace.for_span(numel, dtype, gpu))
+        else:                                                   # one tile a launch
+            for a in range(0, numel, 256):
+                b = min(numel, a + 256)
+                sl = slice(a, b)
+                inner = [(0, 1 if a < cut or cut == 0 else 0)] + ([(cut - a, 0)] if a < cut < b else [])
+                part = sync.make_step_args((1,) * K, dtype, opt=opt, step=3)
+                sync.sync_bucket(sync.SpanSpec([g[sl] for g in grads], agg_out=agg[sl], param=p[sl], state1=m[sl], state2=v[sl],
+                                               bounds=inner), part)
+        return agg, p, m, v, None if row is None else row.reshape(-1).clone()
+
+    ways = [launch("span"), launch("plan"), launch("tight")]
+    if numel <= 8192:
+        ways.append(launch("tiles"))
+    for other in ways[1:]:
+        for x, y in zip(ways[0][:4], other[:4]):
+            assert torch.equal(x.view(torch.int32), y.view(torch.int32))
+        if level and other[4] is not None:
+            # fp64 sums of fp32 gradients: 2^-53 per addition of a chain of at most 700; bf16 gradients: fp32 chains of at
+            # most 16 products per thread and 4 more over a row of lanes, 20 * 2^-24 of the sum of magnitudes
+            tol = 700 * 2.0 ** -53 if dtype == torch.float32 else 20 * 2.0 ** -24
+            norm = float(ways[0][4].abs().max())
+            assert float((ways[0][4] - other[4]).abs().max()) <= tol * norm
+    if level:
+        norms = torch.stack([(g.double() ** 2).sum() for g in grads])
+        tol = 1e-12 if dtype == torch.float32 else 20 * 2.0 ** -24
+        torch.testing.assert_close(ways[0][4][4:4 + K], norms, rtol=tol, atol=0.0)
