@@ -1191,3 +1191,39 @@ def test_short_launches_give_the_result_of_whole_chunks(gpu, K, dtype, level, nu
         norms = torch.stack([(g.double() ** 2).sum() for g in grads])
         tol = 1e-12 if dtype == torch.float32 else 20 * 2.0 ** -24
         torch.testing.assert_close(ways[0][4][4:4 + K], norms, rtol=tol, atol=0.0)
+
+
+@pytest.mark.parametrize("numel", [3, 1024, 1025, 70001])
+@pytest.mark.parametrize("kind", ["sgd", "adamw", None])
+@pytest.mark.parametrize("weight,scale,out", [(1.0, None, "own"), (1.0, 1.0, "own"), (1.0, 2.5, "own"), (1.0, float("nan"), "own"),
+                                              (1.0, 0.37, "own"), (0.5, None, "own"), (0.5, 0.37, "own"), (1.0, None, "other"),
+                                              (1.0, 2.5, "other")])
+def test_aggregate_of_one_worker_over_its_own_buffer(gpu, numel, kind, weight, scale, out):
+    """One fp32 worker of weight 1 that nothing scales is its own aggregate, and the launch writes none; any other weight, a
+    coefficient under 1 and an output elsewhere are written. Every buffer against the oracle, bit for bit; infinities,
+    negative zeros and denormals among the gradients."""
+    from jabas_amd import sync
+    gen = torch.Generator().manual_seed(numel)
+    g = torch.randn(numel, generator=gen)
+    g[:3] = torch.tensor([-0.0, float("-inf"), 1e-40])
+    p0, m0, v0 = torch.randn(numel, generator=gen), torch.randn(numel, generator=gen), torch.rand(numel, generator=gen)
+    opt = None if kind is None else dict(kind=kind, momentum=0.9, betas=(0.9, 0.999), eps=1e-8, groups=[dict(lr=1e-2, weight_decay=0.1)])
+    want = g * weight
+    if scale is not None and scale < 1.0:
+        want = want * torch.tensor(scale)
+    g_dev, res = g.to(gpu), []
+    for own in (out == "own", False):                          # the second time out of place: the update is the same
+        grad = g_dev.clone()
+        agg = grad if own else torch.full((numel,), 7.0, device=gpu)
+        state = [t.to(gpu).clone() for t in (p0, m0, v0)]
+        coef = None if scale is None else torch.tensor([scale], device=gpu)
+        args = sync.make_step_args((1,), torch.float32, opt=opt, step=2, grad_scale=coef)
+        args.weight[0] = weight
+        kw = {} if kind is None else dict(param=state[0], state1=state[1], state2=state[2] if kind == "adamw" else None)
+        sync.sync_bucket(sync.SpanSpec([grad], agg_out=agg, **kw), args)
+        res.append([agg, *state])
+        if not own:
+            assert torch.equal(grad.view(torch.int32), g_dev.view(torch.int32))
+    for a, b in zip(*res):
+        assert torch.equal(a.view(torch.int32), b.view(torch.int32))
+    assert torch.equal(res[0][0].cpu().view(torch.int32), want.view(torch.int32))
