@@ -8,6 +8,7 @@ bucket) for which K gradient buffers, the aggregated-gradient output and the par
 optimizer-state buffers are indexed alike; a *plan* is a launch-invariant table of spans.
 """
 import ctypes as C
+import struct
 
 import numpy as np
 import torch
@@ -32,29 +33,34 @@ def batch_weights(batches, half_id=None, accumulations=1):
     (jabas/train/trainer.py:594-599: global batch = local batch x decoupled workers), so
     w_k = fp32(b_k / (B * accumulations)).
     """
+    w, half_id, hw = _weights(batches, half_id, accumulations)
+    return np.array(w, dtype=np.float32), np.array(half_id, dtype=np.uint8), np.array(hw, dtype=np.float32)
+
+
+def _weights(batches, half_id, accumulations):
+    """``batch_weights`` as lists of Python floats, not yet rounded to fp32 (a C float field rounds them once, as
+    numpy does): a handful of numbers per step, for which arrays cost more than the step's launch."""
     if int(accumulations) < 1:
         raise ValueError("accumulations must be a positive integer")
     b = [float(x) for x in batches]
     K = len(b)
     if not 1 <= K <= L.MAX_K:
         raise ValueError(f"number of VSWs must be in 1..{L.MAX_K}, got {K}")
-    if any(x <= 0 for x in b):
-        raise ValueError(f"local batch sizes must be positive: {batches}")
+    for x in b:
+        if x <= 0:
+            raise ValueError(f"local batch sizes must be positive: {batches}")
     acc = float(int(accumulations))
-    total = sum(b) * acc
-    w = np.array([x / total for x in b], dtype=np.float64).astype(np.float32)
     if half_id is None:
-        half_id = [k % 2 for k in range(K)]
-    half_id = np.array(half_id, dtype=np.uint8)
-    if half_id.shape != (K,) or np.any(half_id > 1):
-        raise ValueError("half_id must hold K entries of 0 or 1")
-    hw = np.zeros(K, dtype=np.float32)
-    for h in (0, 1):
-        tot = sum(x for x, hid in zip(b, half_id) if hid == h) * acc
-        for k in range(K):
-            if half_id[k] == h:
-                hw[k] = np.float32(b[k] / tot)
-    return w, half_id, hw
+        half_id = [k & 1 for k in range(K)]
+        totals = [sum(b[::2]) * acc, sum(b[1::2]) * acc]
+    else:
+        half_id = np.array(half_id, dtype=np.uint8)
+        if half_id.shape != (K,) or np.any(half_id > 1):
+            raise ValueError("half_id must hold K entries of 0 or 1")
+        half_id = half_id.tolist()
+        totals = [sum(x for x, hid in zip(b, half_id) if hid == h) * acc for h in (0, 1)]
+    total = sum(b) * acc
+    return [x / total for x in b], half_id, [x / totals[h] for x, h in zip(b, half_id)]
 
 
 _KIND = {None: L.OPT_NONE, "none": L.OPT_NONE, "sgd": L.OPT_SGD, "adam": L.OPT_ADAM, "adamw": L.OPT_ADAMW}
@@ -98,6 +104,14 @@ def grad_dtype_code(dtype):
     raise TypeError(f"gradient dtype must be float32 or bfloat16, got {dtype}")
 
 
+# JabasStepArgs up to its groups, and one group, as one write each: a foreign assignment per field and numpy arrays for
+# the weights cost more than the launches of a short step (two VSWs with SGD 16.5 us a call -> 6.5, eight 33 -> 7.9).
+_ARGS_HEAD = struct.Struct(f"2i{L.MAX_K}fi{L.MAX_K}B{L.MAX_K}f4i5d")
+_ARGS_GROUP = struct.Struct("2dQ")               # step: the low 64 bits, as the struct's own field keeps them
+assert _ARGS_HEAD.size == L.JabasStepArgs.groups.offset and _ARGS_GROUP.size == C.sizeof(L.JabasGroup)
+_NO_WEIGHTS, _NO_HALVES = [0.0] * L.MAX_K, [0] * L.MAX_K
+
+
 def make_step_args(batches, grad_dtype, stats=False, opt=None, step=1, first_step=False, half_id=None,
                    lr_scale=1.0, grad_scale=None, accumulations=1):
     """Builds the JabasStepArgs of one call.
@@ -106,32 +120,28 @@ def make_step_args(batches, grad_dtype, stats=False, opt=None, step=1, first_ste
     momentum/dampening/nesterov or betas/eps). ``step`` is the 1-based Adam step count,
     ``lr_scale`` the adaptive-batching LR modifier (jabas/train/trainer.py:693-700).
     """
-    w, hid, hw = batch_weights(batches, half_id, accumulations)
+    w, hid, hw = _weights(batches, half_id, accumulations)
+    K = len(w)
+    w += _NO_WEIGHTS[K:]
+    hw += _NO_WEIGHTS[K:]
+    hid += _NO_HALVES[K:]
     a = L.JabasStepArgs()
-    a.K = len(w)
-    a.grad_dtype = grad_dtype_code(grad_dtype)
-    for k in range(a.K):
-        a.weight[k] = float(w[k])
-        a.half_id[k] = int(hid[k])
-        a.half_weight[k] = float(hw[k])
-    a.stats = stats_level(stats)
-    a.opt_kind = opt_kind(opt)
-    if opt is not None and a.opt_kind != L.OPT_NONE:
+    dtype_code, level, kind = grad_dtype_code(grad_dtype), stats_level(stats), opt_kind(opt)
+    if opt is not None and kind != L.OPT_NONE:
         groups = opt["groups"]
         if not 1 <= len(groups) <= L.MAX_GROUPS:
             raise ValueError(f"1..{L.MAX_GROUPS} parameter groups supported, got {len(groups)}")
-        a.n_groups = len(groups)
-        for i, g in enumerate(groups):
-            a.groups[i].lr = float(g["lr"]) * float(lr_scale)
-            a.groups[i].weight_decay = float(g.get("weight_decay", 0.0))
-            a.groups[i].step = int(g.get("step", step))
-        a.first_step = 1 if first_step else 0
-        a.nesterov = 1 if opt.get("nesterov", False) else 0
-        a.momentum = float(opt.get("momentum", 0.0))
-        a.dampening = float(opt.get("dampening", 0.0))
+        at, scale = _ARGS_HEAD.size, float(lr_scale)
+        for g in groups:
+            _ARGS_GROUP.pack_into(a, at, float(g["lr"]) * scale, float(g.get("weight_decay", 0.0)),
+                                  int(g.get("step", step)) & 0xFFFFFFFFFFFFFFFF)
+            at += _ARGS_GROUP.size
         b1, b2 = opt.get("betas", (0.9, 0.999))
-        a.beta1, a.beta2 = float(b1), float(b2)
-        a.eps = float(opt.get("eps", 1e-8))
+        tail = (len(groups), 1 if first_step else 0, 1 if opt.get("nesterov", False) else 0, float(opt.get("momentum", 0.0)),
+                float(opt.get("dampening", 0.0)), float(b1), float(b2), float(opt.get("eps", 1e-8)))
+    else:
+        tail = (0, 0, 0, 0.0, 0.0, 0.0, 0.0, 0.0)
+    _ARGS_HEAD.pack_into(a, 0, K, dtype_code, *w, level, *hid, *hw, kind, *tail)
     if grad_scale is not None:
         if grad_scale.dtype != torch.float32 or not grad_scale.is_cuda:
             raise TypeError("grad_scale must be an fp32 scalar on the GPU")

@@ -583,6 +583,34 @@ def test_rendezvous_calls_validate_their_arguments():
     assert b"rendezvous" in lib.jabas_status_string(L.ERR_STATE)
 
 
+@pytest.mark.parametrize("K", (1, 2, 5, 16))
+@pytest.mark.parametrize("half", (None, "blocks"))
+def test_step_args_hold_every_field_in_its_place(K, half):
+    """The arguments are written as packed bytes: every field of the struct read back, the weights against numpy's
+    rounding, the first and the last parameter group, a step beyond 32 bits."""
+    import torch
+    from jabas_amd import sync
+    batches = tuple(3 + 7 * k % 31 for k in range(K))
+    half_id = None if half is None else [int(k >= K // 2) for k in range(K)]
+    groups = [dict(lr=0.1 * (i + 1), weight_decay=1e-4 * i, step=2 ** 40 + i) for i in range(L.MAX_GROUPS)]
+    opt = dict(kind="sgd", momentum=0.9, dampening=0.1, nesterov=True, betas=(0.8, 0.98), eps=1e-6, groups=groups)
+    a = sync.make_step_args(batches, torch.bfloat16, stats="full", opt=opt, first_step=True, half_id=half_id, lr_scale=0.5,
+                            accumulations=3)
+    hid = [k % 2 for k in range(K)] if half_id is None else half_id
+    tot = [3.0 * sum(b for b, h in zip(batches, hid) if h == x) for x in (0, 1)]
+    w = np.array([b / (3.0 * sum(batches)) for b in batches]).astype(np.float32)
+    hw = np.array([b / tot[h] for b, h in zip(batches, hid)]).astype(np.float32)
+    zeros = [0] * (L.MAX_K - K)
+    assert (a.K, a.grad_dtype, a.stats, a.opt_kind, a.n_groups) == (K, L.BF16, L.STATS_FULL, L.OPT_SGD, L.MAX_GROUPS)
+    assert list(a.weight) == w.tolist() + zeros and list(a.half_weight) == hw.tolist() + zeros and list(a.half_id) == hid + zeros
+    assert (a.first_step, a.nesterov, a.momentum, a.dampening) == (1, 1, 0.9, 0.1)
+    assert (a.beta1, a.beta2, a.eps, a.grad_scale, a.scalars_dev) == (0.8, 0.98, 1e-6, None, None)
+    assert [(g.lr, g.weight_decay, g.step) for g in a.groups] == [(g["lr"] * 0.5, g["weight_decay"], g["step"]) for g in groups]
+    got = sync.batch_weights(batches, half_id, 3)
+    assert [x.dtype for x in got] == [np.float32, np.uint8, np.float32]
+    assert np.array_equal(got[0], w) and got[1].tolist() == hid and np.array_equal(got[2], hw)
+
+
 def test_step_scalar_block_holds_the_constants_a_plain_call_derives():
     """jabas_step_scalars_encode is host code: its block is compared, slot by slot, with the constants derived
     here in Python doubles and rounded once to fp32 (what a Python float becomes as an fp32 kernel scalar)."""
