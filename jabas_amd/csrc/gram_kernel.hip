@@ -7,7 +7,7 @@
 //                  from registers (gram_mfma_kernel below), still exact products and fp64 sums;
 //                  bf16 gradients: bf16 matrix cores, exact fp32 products, fp32 running sums over short runs,
 //                  then fp64 (gram_bf16_mfma_kernel).
-// Then a single-workgroup finalize that sums the workgroup rows in a fixed order.
+// Then a finalize that sums the workgroup rows in a fixed order, four entries of the rows per workgroup.
 #include "jabas_internal.h"
 
 #ifndef JABAS_GRAM_VALU_MAX_K
@@ -130,42 +130,70 @@ __global__ void __launch_bounds__(kBlock) gram_kernel(const SpanDev sp, double* 
     }
 }
 
-// Sums the workgroup rows and writes the symmetric matrix. E is the power of two that holds a row's products: thread
-// (part, entry) adds packed entry `entry` of rows part, part + 1024 / E, ... in that order, the parts of a wave are added
-// by a fixed butterfly and the 16 waves in order: the result does not depend on timing. Neighbouring lanes read
-// neighbouring entries of one row; with lanes along the rows a load touched as many lines as lanes, and 1024 rows of 28
-// entries cost one compute unit about 10 us (1.2 M elements, K = 7 bf16, whole call: 24.4 -> 13.7 us).
-constexpr int kGramFinalizeBlock = 1024, kGramFinalizeWaves = kGramFinalizeBlock / 64;
-static_assert(JABAS_GRAM_VALU_MAX_K * (JABAS_GRAM_VALU_MAX_K + 1) / 2 <= 32, "one slot per product");
-static_assert(JABAS_GRAM_VALU_MAX_K_BF16 * (JABAS_GRAM_VALU_MAX_K_BF16 + 1) / 2 <= 32, "one slot per product");
-template <int E>
+// Sums the workgroup rows and writes the symmetric matrix, four neighbouring entries of the rows per workgroup: lane =
+// entry + 4 * row, so a wave's load covers 32 contiguous bytes of sixteen rows, every thread has four loads in flight (1024
+// rows: all of them) and a wider row only adds workgroups. Thread (entry, class) adds rows class, class + 256, ... in order;
+// the 256 sums of an entry meet by row rotations, one LDS table and a second round of the same: the order depends on the
+// number of rows alone, the result not on timing.
+// BLOCKS: rows of the matrix-core kernels, entry [p][4 i + j] is the product of workers 4 ga + i and 4 gb + j of pair
+// p = (ga <= gb); otherwise packed rows, entry a (a + 1) / 2 + b of workers b <= a.
+// Bound by its launch and one trip to memory. One workgroup for all entries (packed rows), and two launches, a fold to 32
+// rows and one workgroup (blocks), cost more; whole calls on 0.3 / 0.7 / 1.2 / 25.6 M elements, us, before -> now:
+//   fp32 K = 2   7.9 / 7.9 / 8.9 / 36.1  ->  7.6 / 7.5 / 7.5 / 34.9       fp32 K = 8    10.0 / 11.6 / 13.6 / 122.8  ->  8.8 / 10.2 / 12.4 / 122.6
+//   fp32 K = 5   8.8 / 10.7 / 11.1 / 85.6  ->  8.2 / 8.9 / 10.3 / 84.4     fp32 K = 16   13.7 / 17.4 / 22.6 / 257.3  ->  12.1 / 15.9 / 21.7 / 257.7
+//   bf16 K = 7   11.4 / 11.9 / 13.7 / 65.6  ->  9.4 / 9.5 / 11.1 / 63.0    bf16 K = 16   14.8 / 18.8 / 22.3 / 133.6  ->  12.9 / 17.1 / 21.4 / 132.8
+constexpr int kGramFinalizeBlock = 1024, kGramFinalizeSlots = 4;
+constexpr unsigned kGramFinalizeClasses = kGramFinalizeBlock / kGramFinalizeSlots;
+template <bool BLOCKS>
 __global__ void __launch_bounds__(kGramFinalizeBlock) gram_finalize_kernel(int K, const double* partials, unsigned grid,
                                                                          double* gram_out) {
-    constexpr unsigned kParts = kGramFinalizeBlock / E;
-    __shared__ double wave_sum[kGramFinalizeWaves][E];
-    const int np = K * (K + 1) / 2;
-    const int t = threadIdx.x, v = t % E;
+    __shared__ double table[kGramFinalizeBlock / 16][kGramFinalizeSlots];
+    const int G = (K + 3) / 4;
+    const int width = BLOCKS ? G * (G + 1) / 2 * 16 : K * (K + 1) / 2;
+    const int t = threadIdx.x, entry = static_cast<int>(blockIdx.x) * kGramFinalizeSlots + (t & (kGramFinalizeSlots - 1));
+    const double* col = partials + (entry < width ? entry : width - 1);
     double s = 0.0;
-    if (v < np) {
-#pragma unroll 16
-        for (unsigned b = t / E; b < grid; b += kParts) s += partials[static_cast<uint64_t>(b) * JABAS_GRAM_STRIDE + v];
+    for (unsigned r = t / kGramFinalizeSlots; r < grid; r += 4 * kGramFinalizeClasses) {
+        double v[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {            // a row beyond the last repeats the last and is dropped
+            const unsigned c = r + i * kGramFinalizeClasses;
+            v[i] = col[static_cast<uint64_t>(c < grid ? c : grid - 1) * JABAS_GRAM_STRIDE];
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) s += r + i * kGramFinalizeClasses < grid ? v[i] : 0.0;
     }
-#pragma unroll
-    for (int off = 32; off >= E; off >>= 1) s += __shfl_xor(s, off, 64);
-    if ((t & 63) < E) wave_sum[t >> 6][v] = s;
-    if (t < JABAS_GRAM_STRIDE) gram_out[t] = 0.0;
+    s += dpp_move<0x128, 0xf>(s);                // row_ror:8, row_ror:4: the four classes of a 16-lane row, per entry
+    s += dpp_move<0x124, 0xf>(s);
+    if ((t & 15) < kGramFinalizeSlots) table[t >> 4][t & 15] = s;
     __syncthreads();
-    if (t < np) {
-        s = wave_sum[0][t];
-#pragma unroll
-        for (int w = 1; w < kGramFinalizeWaves; ++w) s += wave_sum[w][t];
-        int a = 0;
-        while ((a + 1) * (a + 2) / 2 <= t) ++a;          // packed index t = a*(a+1)/2 + b, b <= a
-        const int b = t - a * (a + 1) / 2;
-        gram_out[a * JABAS_GRAM_MAX_K + b] = s;
-        gram_out[b * JABAS_GRAM_MAX_K + a] = s;
+    if (t < 64) {                                // one wave: 64 sums of an entry, four per lane, then over the lanes
+        const int c = t >> 2, v = t & (kGramFinalizeSlots - 1);
+        double sum = ((table[c][v] + table[16 + c][v]) + table[32 + c][v]) + table[48 + c][v];
+        sum += dpp_move<0x128, 0xf>(sum);
+        sum += dpp_move<0x124, 0xf>(sum);
+        sum += __shfl_xor(sum, 16);
+        sum += __shfl_xor(sum, 32);
+        int lo = 0, hi = 0;
+        if constexpr (BLOCKS) {                  // the workgroup holds row i of pair p: p, then ga, from its index
+            int p = static_cast<int>(blockIdx.x) >> 2, ga = 0;
+            while (p >= G - ga) p -= G - ga++;
+            lo = 4 * ga + (static_cast<int>(blockIdx.x) & 3);
+            hi = 4 * (ga + p) + v;
+        } else {
+            while ((hi + 1) * (hi + 2) / 2 <= entry) ++hi;
+            lo = entry - hi * (hi + 1) / 2;
+        }
+        if (t < kGramFinalizeSlots && lo <= hi && hi < K) {      // one triangle, mirrored: symmetric bit for bit
+            gram_out[lo * JABAS_GRAM_MAX_K + hi] = sum;
+            gram_out[hi * JABAS_GRAM_MAX_K + lo] = sum;
+        }
+    } else if (blockIdx.x == 0 && t - 64 < JABAS_GRAM_STRIDE) {
+        const int o = t - 64;
+        if (o / JABAS_GRAM_MAX_K >= K || o % JABAS_GRAM_MAX_K >= K) gram_out[o] = 0.0;
     }
 }
+static_assert(kGramFinalizeBlock >= 64 + JABAS_GRAM_STRIDE, "one thread per entry of the matrix beside the summing wave");
 
 
 // ---- K >= 6: fp64 matrix cores, 4 x 4 blocks ----------------------------------------------------------
@@ -284,54 +312,6 @@ __global__ void __launch_bounds__(kBlock) gram_mfma_kernel(const SpanDev sp, int
         for (int w = 0; w < kWaves; ++w) s += ((red[w][p][l0] + red[w][p][l0 + 4]) + red[w][p][l0 + 8]) + red[w][p][l0 + 12];
         partials[static_cast<uint64_t>(blockIdx.x) * JABAS_GRAM_STRIDE + t] = s;
     }
-}
-
-// Sums the workgroup rows (1024 threads: thread (entry, part) adds rows part, part + 4, ... in order, then
-// the four parts in order) and unfolds the blocks: entry [p][4 i + j] of pair p = (ga, gb) is the product sum
-// of workers 4 ga + i and 4 gb + j.
-constexpr int kGramMfmaFinalizeBlock = 1024;
-__global__ void __launch_bounds__(kGramMfmaFinalizeBlock) gram_mfma_finalize_kernel(int K, const double* partials, unsigned grid,
-                                                                                    double* gram_out) {
-    __shared__ double part_sum[4][256];
-    __shared__ double tile[256];
-    const int t = threadIdx.x, e = t & 255, part = t >> 8;
-    const int G = (K + 3) / 4, P = G * (G + 1) / 2;
-    double s = 0.0;
-    if (e < P * 16) {
-#pragma unroll 8
-        for (unsigned b = part; b < grid; b += 4) s += partials[static_cast<uint64_t>(b) * JABAS_GRAM_STRIDE + e];
-    }
-    part_sum[part][e] = s;
-    __syncthreads();
-    if (t < 256) tile[t] = ((part_sum[0][t] + part_sum[1][t]) + part_sum[2][t]) + part_sum[3][t];
-    __syncthreads();
-    if (t < JABAS_GRAM_STRIDE) {
-        const int a = t / JABAS_GRAM_MAX_K, b = t % JABAS_GRAM_MAX_K;
-        double out = 0.0;
-        if (a < K && b < K) {
-            const int lo = a < b ? a : b, hi = a < b ? b : a;      // one triangle, mirrored: symmetric bit for bit
-            const int ga = lo >> 2, gb = hi >> 2;
-            const int p = ga * G - ga * (ga - 1) / 2 + (gb - ga);  // index of pair (ga, gb), ga <= gb
-            out = tile[p * 16 + 4 * (lo & 3) + (hi & 3)];
-        }
-        gram_out[t] = out;
-    }
-}
-
-// One workgroup on one compute unit pulls 1024 rows of up to 160 doubles (1.3 MB) in 12-29 us, a tenth of the
-// bf16 K = 8 Gram launch itself. When the workspace has room for kGramFoldRows more rows, kGramFoldRows
-// workgroups first fold rows j, j + kGramFoldRows, ... (in that order) into row j of that room and the finalize
-// sums those. Which of the two forms runs depends on the sizes the caller passes only: same call, same bits.
-constexpr unsigned kGramFoldRows = 32;
-__global__ void __launch_bounds__(JABAS_GRAM_STRIDE) gram_mfma_fold_kernel(int K, const double* partials, unsigned grid, double* folded) {
-    const int G = (K + 3) / 4, E = G * (G + 1) / 2 * 16;
-    const int e = threadIdx.x;
-    double s = 0.0;
-    if (e < E) {
-#pragma unroll 8
-        for (unsigned b = blockIdx.x; b < grid; b += kGramFoldRows) s += partials[static_cast<uint64_t>(b) * JABAS_GRAM_STRIDE + e];
-    }
-    folded[static_cast<uint64_t>(blockIdx.x) * JABAS_GRAM_STRIDE + e] = s;
 }
 
 // ---- bf16 gradients: bf16 matrix cores ------------------------------------------------------------------
@@ -505,28 +485,14 @@ int launch_gram(int K, int grad_dtype, const SpanDev& sp, double* partials, unsi
     }
 }
 
-unsigned gram_fold_rows() { return kGramFoldRows; }
-
-// spare_rows: rows of JABAS_GRAM_STRIDE doubles the workspace holds beyond the `grid` partial rows
-int launch_gram_finalize(int K, int grad_dtype, double* partials, unsigned grid, unsigned spare_rows, double* gram_out,
-                         hipStream_t stream) {
-    if (K > gram_valu_max_k(grad_dtype)) {
-        if (grid > 4 * kGramFoldRows && spare_rows >= kGramFoldRows) {
-            double* folded = partials + static_cast<uint64_t>(grid) * JABAS_GRAM_STRIDE;
-            if (launch_kernel(gram_mfma_fold_kernel, dim3(kGramFoldRows), dim3(JABAS_GRAM_STRIDE), 0, stream, K,
-                              static_cast<const double*>(partials), grid, folded) != 0)
-                return -1;
-            return static_cast<int>(launch_kernel(gram_mfma_finalize_kernel, dim3(1), dim3(kGramMfmaFinalizeBlock), 0, stream, K,
-                                                  static_cast<const double*>(folded), kGramFoldRows, gram_out));
-        }
-        return static_cast<int>(launch_kernel(gram_mfma_finalize_kernel, dim3(1), dim3(kGramMfmaFinalizeBlock), 0, stream, K,
-                                              static_cast<const double*>(partials), grid, gram_out));
-    }
-    const double* rows = partials;
-    const dim3 one(1), block(kGramFinalizeBlock);
-    if (K <= 3) return static_cast<int>(launch_kernel(gram_finalize_kernel<8>, one, block, 0, stream, K, rows, grid, gram_out));
-    if (K <= 5) return static_cast<int>(launch_kernel(gram_finalize_kernel<16>, one, block, 0, stream, K, rows, grid, gram_out));
-    return static_cast<int>(launch_kernel(gram_finalize_kernel<32>, one, block, 0, stream, K, rows, grid, gram_out));
+int launch_gram_finalize(int K, int grad_dtype, const double* partials, unsigned grid, double* gram_out, hipStream_t stream) {
+    const unsigned G = (K + 3) / 4;
+    const dim3 block(kGramFinalizeBlock);
+    if (K > gram_valu_max_k(grad_dtype))
+        return static_cast<int>(launch_kernel(gram_finalize_kernel<true>, dim3(G * (G + 1) / 2 * 16 / kGramFinalizeSlots), block, 0,
+                                              stream, K, partials, grid, gram_out));
+    return static_cast<int>(launch_kernel(gram_finalize_kernel<false>, dim3((K * (K + 1) / 2 + kGramFinalizeSlots - 1) / kGramFinalizeSlots),
+                                          block, 0, stream, K, partials, grid, gram_out));
 }
 
 }  // namespace jabas

@@ -542,13 +542,12 @@ def gradient_stats(grads, batches, half_id=None, workspace=None, stream=None):
 
 def gram(grads, stream=None, workspace=None):
     """K x K Gram matrix (float64, device) of the worker gradients. ``workspace``: a float64 device tensor of
-    at least 1024 * GRAM_STRIDE elements (1056 * GRAM_STRIDE for the faster two-stage sum of the partial rows);
-    allocated per call when None."""
+    at least 1024 * GRAM_STRIDE elements; allocated per call when None."""
     span = SpanSpec(grads)
     n, dev, gdt = span.validate()
     K = len(grads)
     if workspace is None:
-        ws = torch.empty(1056 * L.GRAM_STRIDE, dtype=torch.float64, device=dev)
+        ws = torch.empty(1024 * L.GRAM_STRIDE, dtype=torch.float64, device=dev)
     else:
         ws = workspace
         if ws.dtype != torch.float64 or ws.device != dev or not ws.is_contiguous():

@@ -323,6 +323,29 @@ def test_gram_at_the_edges_of_runs_and_routes(gpu, dtype, K):
         assert bool(G[w].isnan().all()) and bool(G[:, w].isnan().all())
 
 
+@pytest.mark.parametrize("dtype,K", [(torch.float32, 1), (torch.float32, 2), (torch.float32, 5), (torch.float32, 6), (torch.float32, 9),
+                                     (torch.float32, 16), (torch.bfloat16, 7), (torch.bfloat16, 8), (torch.bfloat16, 11), (torch.bfloat16, 13)])
+def test_gram_sum_of_the_workgroup_rows(gpu, dtype, K):
+    """A workgroup of the finalize holds four entries and takes the rows in classes of 256: one row, one class short, full and
+    one over, three and four rows per class. Every entry of the 16 x 16 result is written: the product, mirrored, or zero
+    beyond the workers. Integers of at most 3 in size: every product and sum is exact, in fp32 as in fp64."""
+    from jabas_amd import sync, _lib as L
+    ws = torch.empty(1024 * L.GRAM_STRIDE, dtype=torch.float64, device=gpu)
+    for rows in (1, 2, 255, 256, 257, 767, 769, 1023, 1024):
+        n = rows * 1024 - 5
+        gen = torch.Generator().manual_seed(rows + K)
+        hg = [torch.randint(-3, 4, (n,), generator=gen).to(dtype) for _ in range(K)]
+        dg = [t.to(gpu) for t in hg]
+        out = torch.full((L.GRAM_STRIDE,), float("nan"), dtype=torch.float64, device=gpu)
+        ws.fill_(float("nan"))
+        L.check(L.lib().jabas_gram(sync._ptr_array(dg), K, sync.grad_dtype_code(dtype), n, out.data_ptr(), ws.data_ptr(),
+                                   ws.numel() * 8, sync._stream_ptr()), "jabas_gram")
+        wide = torch.stack([t.double() for t in hg])
+        want = torch.zeros(L.GRAM_MAX_K, L.GRAM_MAX_K, dtype=torch.float64)
+        want[:K, :K] = wide @ wide.t()
+        assert torch.equal(out.cpu().view(L.GRAM_MAX_K, L.GRAM_MAX_K), want), f"K={K} rows={rows}"
+
+
 def test_gram_limits_and_determinism(gpu):
     from jabas_amd import sync, _lib as L
     g = [torch.zeros(4096, device=gpu) for _ in range(17)]
@@ -337,7 +360,7 @@ def test_gram_limits_and_determinism(gpu):
     # the diagonal is the per-worker norm row of the statistics kernel's full level
     row = sync.gradient_stats(dg, BATCHES[11]).cpu()
     assert torch.allclose(torch.diagonal(a), row[4:4 + 11], rtol=1e-12, atol=0.0)
-    # a workspace without room for the two-stage sum of the partial rows: same values within rounding
+    # a workspace of exactly the rows the call needs: the same values
     small = torch.empty(1024 * L.GRAM_STRIDE, dtype=torch.float64, device=gpu)
     b = sync.gram(dg, workspace=small).cpu()
     assert torch.allclose(a, b, rtol=1e-13, atol=1e-24)
