@@ -13,14 +13,12 @@
 namespace jabas {
 
 int launch_gram(int K, int grad_dtype, const SpanDev& sp, double* partials, unsigned grid, hipStream_t stream);
+unsigned gram_grid(int K, int grad_dtype, uint64_t hi);
 int launch_gram_finalize(int K, int grad_dtype, const double* partials, unsigned grid, double* gram_out, hipStream_t stream);
 
 namespace {
 
-#ifndef JABAS_GRAM_GRID
-#define JABAS_GRAM_GRID 1024
-#endif
-constexpr uint64_t kGramGrid = JABAS_GRAM_GRID;     // persistent workgroups of the Gram kernel
+constexpr uint64_t kGramRows = 1024;         // rows of JABAS_GRAM_STRIDE doubles a Gram call over many tiles asks of its workspace
 constexpr uint32_t kPlanMagic = 0x4a425359u;  // "JBSY"
 constexpr uint32_t kPlanVersion = 8;
 
@@ -900,10 +898,10 @@ JABAS_API int jabas_gram(const void* const* grads, int32_t K, int32_t grad_dtype
     uint32_t tiles = 0;
     const int rc = encode_span(sp, K, grad_dtype, JABAS_OPT_NONE, kBlock, &sd, &tiles);
     if (rc != JABAS_OK) return rc;
-    uint64_t g = kGramGrid;
-    if (g > tiles) g = tiles;
-    if (g < 1) g = 1;
-    if (workspace_bytes < g * JABAS_GRAM_STRIDE * sizeof(double)) return JABAS_ERR_WORKSPACE;
+    uint64_t rows = tiles < kGramRows ? tiles : kGramRows;
+    if (rows < 1) rows = 1;
+    if (workspace_bytes < rows * JABAS_GRAM_STRIDE * sizeof(double)) return JABAS_ERR_WORKSPACE;
+    const uint64_t most = gram_grid(K, grad_dtype, sd.hi), g = rows < most ? rows : most;     // persistent workgroups
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (launch_gram(K, grad_dtype, sd, static_cast<double*>(workspace), static_cast<unsigned>(g), st) != 0)
         return JABAS_ERR_LAUNCH;

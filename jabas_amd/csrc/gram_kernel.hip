@@ -14,6 +14,10 @@
 #define JABAS_GRAM_VALU_MAX_K 5
 #endif
 
+#ifndef JABAS_GRAM_GRID
+#define JABAS_GRAM_GRID 1024
+#endif
+
 namespace jabas {
 namespace {
 
@@ -213,6 +217,7 @@ static_assert(kGramFinalizeBlock >= 64 + JABAS_GRAM_STRIDE, "one thread per entr
 #endif
 // 64-element blocks in a run of a wave
 constexpr int kGramRunBlocks = JABAS_GRAM_RUN_F32;
+constexpr uint64_t kGramShortF32 = 1u << 21;           // fewer elements: half the workgroups (gram_grid)
 
 template <int G>
 __global__ void __launch_bounds__(kBlock) gram_mfma_kernel(const SpanDev sp, int K, double* partials) {
@@ -322,7 +327,7 @@ __global__ void __launch_bounds__(kBlock) gram_mfma_kernel(const SpanDev sp, int
 // lane. A lane loads 16 bytes (two operands) per group; a wave reads 256 contiguous bytes of each worker.
 // Products of bf16 values are exact in fp32; the instruction adds four of them to an fp32 running sum, which
 // is moved into fp64 sums (LDS, per wave) after at most kGramBf16FlushRuns runs, i.e. after at most
-// 4 * 2 * RUN * kGramBf16FlushRuns elements: fp32 rounding stays near 1e-6 of |g_a| |g_b|, the order is fixed.
+// 4 * 2 * kGramBf16FlushRuns elements of either of its two blocks (and those of the span's ends): fp32 rounding stays near 1e-6 of |g_a| |g_b|, the order is fixed.
 // Lanes beyond the last worker multiply worker 0's values into entries the finalize never reads.
 template <int CTRL> __device__ __forceinline__ float gram_dpp_f32(float v) {
     return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, false));
@@ -331,35 +336,21 @@ typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef u32x4 __attribute__((aligned(8))) u32x4_a8;     // element 0 of a bf16 buffer is 8-byte aligned, not more
 
-// 128-element blocks a wave loads before it multiplies, by number of groups
-#ifndef JABAS_GRAM_RUN_BF16_G2
-#define JABAS_GRAM_RUN_BF16_G2 2
-#endif
-#ifndef JABAS_GRAM_RUN_BF16_G3
-#define JABAS_GRAM_RUN_BF16_G3 2
-#endif
-#ifndef JABAS_GRAM_RUN_BF16_G4
-#define JABAS_GRAM_RUN_BF16_G4 4
-#endif
-constexpr int gram_bf16_run(int G) {
-    return G == 2 ? JABAS_GRAM_RUN_BF16_G2 : G == 3 ? JABAS_GRAM_RUN_BF16_G3 : JABAS_GRAM_RUN_BF16_G4;
-}
 constexpr int kGramBf16FlushRuns = 128;
 
-template <int G>
+// U: 128-element blocks in a run of a wave. S: running sums per pair of groups, which the blocks take in turn. EDGES: the
+// loop takes the runs across the span's ends as well; otherwise it holds whole runs and the ends follow it, which keeps the
+// conditional loads of single elements (U * G * 8 of them) out of its code: a cold launch fetches that code from memory.
+template <int G, int U, int S, bool EDGES>
 __global__ void __launch_bounds__(kBlock) gram_bf16_mfma_kernel(const SpanDev sp, int K, double* partials) {
     constexpr int P = G * (G + 1) / 2;
-    constexpr int U = gram_bf16_run(G);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    constexpr uint64_t kRun = static_cast<uint64_t>(U) * 128;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wi = lane & 3;
     const uint32_t lane_off = static_cast<uint32_t>(lane >> 2) * 8u;
     const uint16_t* base[G];
-    bool live[G];
 #pragma unroll
-    for (int g = 0; g < G; ++g) {
-        live[g] = g * 4 + wi < K;
-        base[g] = static_cast<const uint16_t*>(sp.g[live[g] ? g * 4 + wi : 0]);
-    }
+    for (int g = 0; g < G; ++g) base[g] = static_cast<const uint16_t*>(sp.g[g * 4 + wi < K ? g * 4 + wi : 0]);
     // fp64 sums of the wave: [pair * 4 + i][16-lane row * 4 + j]
     __shared__ double sums[kWaves][P * 4][16];
     double* const wave_sums = &sums[0][0][0] + static_cast<size_t>(wave) * (P * 64);     // this wave's P * 64 sums, flat
@@ -368,9 +359,11 @@ __global__ void __launch_bounds__(kBlock) gram_bf16_mfma_kernel(const SpanDev sp
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    f32x4 acc[P];
+    f32x4 acc[S][P];
 #pragma unroll
-    for (int p = 0; p < P; ++p) acc[p] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int u = 0; u < S; ++u)
+#pragma unroll
+        for (int p = 0; p < P; ++p) acc[u][p] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     // entry (i, j) of a product sits in register i of lane j + 4 * product: a rotation by 4 and by 8 inside the
     // 16-lane row adds the row's four products; lanes 0..3 of every row then own one fp64 sum each per register
     const bool owner = ((lane >> 2) & 3) == 0;
@@ -380,53 +373,93 @@ __global__ void __launch_bounds__(kBlock) gram_bf16_mfma_kernel(const SpanDev sp
         for (int p = 0; p < P; ++p)
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                float v = acc[p][i];
-                v += gram_dpp_f32<0x124>(v);        // row_ror:4
-                v += gram_dpp_f32<0x128>(v);        // row_ror:8
-                if (owner) sums[wave][p * 4 + i][col] += static_cast<double>(v);
-                acc[p][i] = 0.0f;
+                double sum = 0.0;
+#pragma unroll
+                for (int u = 0; u < S; ++u) {
+                    float v = acc[u][p][i];
+                    v += gram_dpp_f32<0x124>(v);    // row_ror:4
+                    v += gram_dpp_f32<0x128>(v);    // row_ror:8
+                    sum += static_cast<double>(v);
+                }
+                if (owner) sums[wave][p * 4 + i][col] += sum;
+#pragma unroll
+                for (int u = 0; u < S; ++u) acc[u][p][i] = 0.0f;
             }
     };
-    const uint64_t n_blocks = (sp.hi + 127) / 128;
-    const uint64_t n_runs = (n_blocks + U - 1) / U;
-    const uint64_t n_waves = static_cast<uint64_t>(gridDim.x) * kWaves;
-    int pending = 0;
-    for (uint64_t run = static_cast<uint64_t>(blockIdx.x) * kWaves + wave; run < n_runs; run += n_waves) {
-        u32x4 x[U][G];
+    auto load_edge = [&](uint64_t e, u32x4 (&v)[G]) {        // zeros for the elements beyond the span's ends, which are not read
+        const bool whole = e >= sp.lo && e + 8 <= sp.hi;
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const uint64_t e = (run * U + u) * 128 + lane_off;
-            const bool whole = e >= sp.lo && e + 8 <= sp.hi;
+        for (int g = 0; g < G; ++g) {
+            if (whole) {
+                v[g] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_a8*>(base[g] + e));
+            } else {
+                uint32_t h[8];
 #pragma unroll
-            for (int g = 0; g < G; ++g) {
-                if (whole) {
-                    x[u][g] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_a8*>(base[g] + e));
-                } else {                             // a vector across the span's first or last element
-                    uint32_t h[8];
-#pragma unroll
-                    for (int i = 0; i < 8; ++i) h[i] = (e + i >= sp.lo && e + i < sp.hi) ? base[g][e + i] : 0u;
-                    x[u][g] = u32x4{h[0] | (h[1] << 16), h[2] | (h[3] << 16), h[4] | (h[5] << 16), h[6] | (h[7] << 16)};
-                }
+                for (int i = 0; i < 8; ++i) h[i] = (e + i >= sp.lo && e + i < sp.hi) ? base[g][e + i] : 0u;
+                v[g] = u32x4{h[0] | (h[1] << 16), h[2] | (h[3] << 16), h[4] | (h[5] << 16), h[6] | (h[7] << 16)};
             }
         }
+    };
+    auto load = [&](uint64_t run, u32x4 (&x)[U][G]) {
 #pragma unroll
-        for (int u = 0; u < U; ++u)
+        for (int u = 0; u < U; ++u) {
+            const uint64_t e = run * kRun + u * 128 + lane_off;
+            if constexpr (EDGES) {
+                load_edge(e, x[u]);
+            } else {
 #pragma unroll
-            for (int half = 0; half < 2; ++half) {
-                s16x4 d[G];
-#pragma unroll
-                for (int g = 0; g < G; ++g)
-                    d[g] = __builtin_bit_cast(s16x4, half ? u32x2{x[u][g].z, x[u][g].w} : u32x2{x[u][g].x, x[u][g].y});
-                int p = 0;
-#pragma unroll
-                for (int ga = 0; ga < G; ++ga)
-#pragma unroll
-                    for (int gb = ga; gb < G; ++gb, ++p)
-                        acc[p] = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(d[ga], d[gb], acc[p], 0, 0, 0);
+                for (int g = 0; g < G; ++g) x[u][g] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_a8*>(base[g] + e));
             }
-        if (++pending == kGramBf16FlushRuns) { flush(); pending = 0; }
-    }
-    flush();
+        }
+    };
+    auto multiply_block = [&](const u32x4 (&v)[G], f32x4 (&sum)[P]) {
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+            s16x4 d[G];
+#pragma unroll
+            for (int g = 0; g < G; ++g)
+                d[g] = __builtin_bit_cast(s16x4, half ? u32x2{v[g].z, v[g].w} : u32x2{v[g].x, v[g].y});
+            int p = 0;
+#pragma unroll
+            for (int ga = 0; ga < G; ++ga)
+#pragma unroll
+                for (int gb = ga; gb < G; ++gb, ++p) sum[p] = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(d[ga], d[gb], sum[p], 0, 0, 0);
+        }
+    };
+    auto multiply = [&](const u32x4 (&x)[U][G]) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) multiply_block(x[u], acc[u % S]);
+    };
+    // The loop's runs are [first, last); at most two others hold the span's ends, taken block by block after it.
+    const uint64_t n_runs = (sp.hi + kRun - 1) / kRun, first = EDGES ? 0 : (sp.lo + kRun - 1) / kRun;
+    const uint64_t last = EDGES ? n_runs : sp.hi / kRun > first ? sp.hi / kRun : first;
+    const uint64_t n_waves = static_cast<uint64_t>(gridDim.x) * kWaves;
+    const uint64_t id = static_cast<uint64_t>(blockIdx.x) * kWaves + wave;
+    const uint64_t n_ends = first + (n_runs > last ? n_runs - last : 0);
+    auto ends = [&]() {                              // to the last waves, which have a run less when the runs do not come out even
+        for (uint64_t r = n_waves - 1 - id; r < n_ends; r += n_waves) {
+            const uint64_t e0 = (r < first ? r : last + (r - first)) * kRun + lane_off;
+#pragma unroll 1
+            for (int u = 0; u < U; ++u) {
+                u32x4 v[G];
+                load_edge(e0 + static_cast<uint64_t>(u) * 128, v);
+                multiply_block(v, acc[0]);
+            }
+        }
+    };
+    // Bound by HBM reads from about 5 M elements on, below by the trips to memory and the epilogue.
+    u32x4 x[U][G];
+    uint64_t run = first + id;
+    do {
+        for (int n = 0; run < last && n < kGramBf16FlushRuns; ++n, run += n_waves) {
+            load(run, x);
+            multiply(x);
+        }
+        if constexpr (!EDGES) {
+            if (run >= last) ends();
+        }
+        flush();                                     // the one copy of it: the code of a cold launch is fetched too
+    } while (run < last);
     __syncthreads();
     // row of the workgroup, the format of gram_mfma_kernel: entry [p][4 i + j], rows then waves in order
     for (int t = threadIdx.x; t < P * 16; t += kBlock) {
@@ -440,11 +473,43 @@ __global__ void __launch_bounds__(kBlock) gram_bf16_mfma_kernel(const SpanDev sp
 }
 
 static_assert(JABAS_GRAM_VALU_MAX_K >= 4 && JABAS_GRAM_VALU_MAX_K_BF16 >= 4, "the matrix-core kernels start at two groups");
+// Shapes of the bf16 matrix-core kernels. Whole calls in us, K = 8 / 12 / 16, before (one sum, ends in the loop, 1024
+// workgroups, runs of 2 / 2 / 4 blocks) -> now:
+//   0.3 M  8.8 / 10.5 / 12.9 -> 8.3 / 10.4 / 13.3      5 M   20.7 / 28.9 / 39.4 -> 19.1 / 27.1 / 35.4
+//   1.2 M  9.9 / 13.9 / 21.4 -> 9.9 / 13.5 / 16.3      25 M  69.1 / 97.5 / 132.8 -> 65.4 / 95.0 / 128.0
+//   four groups            two waves per SIMD fit, so 512 workgroups are resident: 1024 run in two rounds. Two sums per pair
+//                          keep the fp32 chains as short as they were.
+//   up to three groups     from kGramLongBf16 elements on the same with runs of four blocks; below, two blocks and one sum,
+//                          1024 workgroups: longer runs leave waves idle (0.3 M, K = 8: 9.2), and two sums of two products
+//                          each are 6 % further from the 64-bit result there than one of four.
+//   four groups, very long from kGramVeryLongBf16 on the loop with the ends in it and 1024 workgroups, two resident per CU by
+//                          idle LDS: 100 M elements of thirteen / fourteen / sixteen workers 405 / 431 / 478 us against
+//                          408 / 438 / 488 with the shape above, three resident 438 / 451 / 494; 40 M 174 / 183 / 200 against
+//                          165 / 177 / 197, 66 M 274 / 291 / 319 against 268 / 289 / 321.
+#ifndef JABAS_GRAM_LONG_BF16
+#define JABAS_GRAM_LONG_BF16 (1u << 21)
+#endif
+#ifndef JABAS_GRAM_VERY_LONG_BF16
+#define JABAS_GRAM_VERY_LONG_BF16 (1u << 26)
+#endif
+constexpr uint64_t kGramLongBf16 = JABAS_GRAM_LONG_BF16, kGramVeryLongBf16 = JABAS_GRAM_VERY_LONG_BF16;
+
+template <int G, int U, int S, bool EDGES>
+int launch_gram_bf16_shape(int K, const SpanDev& sp, double* partials, unsigned grid, hipStream_t stream) {
+    constexpr unsigned idle = EDGES ? 36 * 1024 : 0;     // beside the 20 KB of sums: two workgroups per CU of 160 KB
+    return static_cast<int>(launch_kernel(gram_bf16_mfma_kernel<G, U, S, EDGES>, dim3(grid), dim3(kBlock), idle, stream, sp, K, partials));
+}
+
 int launch_gram_bf16_mfma(int K, const SpanDev& sp, double* partials, unsigned grid, hipStream_t stream) {
+    const bool long_span = sp.hi >= kGramLongBf16;
     switch ((K + 3) / 4) {
-        case 2: return static_cast<int>(launch_kernel(gram_bf16_mfma_kernel<2>, dim3(grid), dim3(kBlock), 0, stream, sp, K, partials));
-        case 3: return static_cast<int>(launch_kernel(gram_bf16_mfma_kernel<3>, dim3(grid), dim3(kBlock), 0, stream, sp, K, partials));
-        case 4: return static_cast<int>(launch_kernel(gram_bf16_mfma_kernel<4>, dim3(grid), dim3(kBlock), 0, stream, sp, K, partials));
+        case 2: return long_span ? launch_gram_bf16_shape<2, 4, 2, false>(K, sp, partials, grid, stream)
+                                 : launch_gram_bf16_shape<2, 2, 1, false>(K, sp, partials, grid, stream);
+        case 3: return long_span ? launch_gram_bf16_shape<3, 4, 2, false>(K, sp, partials, grid, stream)
+                                 : launch_gram_bf16_shape<3, 2, 1, false>(K, sp, partials, grid, stream);
+        case 4: return sp.hi >= kGramVeryLongBf16 ? launch_gram_bf16_shape<4, 4, 1, true>(K, sp, partials, grid, stream)
+                       : long_span                ? launch_gram_bf16_shape<4, 4, 2, false>(K, sp, partials, grid, stream)
+                                                  : launch_gram_bf16_shape<4, 2, 2, false>(K, sp, partials, grid, stream);
         default: return -1;
     }
 }
@@ -468,6 +533,21 @@ int launch_gram_mfma(int K, const SpanDev& sp, double* partials, unsigned grid, 
 }
 
 }  // namespace
+
+// Most workgroups of a launch; hi: end of the span's element grid. 1024 unless half of them are faster:
+//   bf16 matrix cores      with the shapes above
+//   fp32 vector ALU        three to five workers: K = 5, 25 M / 100 M elements 84.3 / 322 -> 80.8 / 291 us, K = 4 65.5 / 243 ->
+//                          63.8 / 232, K = 3 50.1 / 178 -> 47.5 / 171, equal below 2 M (K = 1 and 2 lose 10-50 %, bf16 up to 30 %)
+//   fp32 matrix cores      short spans, whose waves have two or three runs each: K = 9 / 13 / 16, 1.2 M elements 15.5 / 20.4 /
+//                          21.7 -> 14.3 / 19.2 / 20.8 us, equal from 2.5 to 10 M; 25 M K = 8 122 -> 124, K = 9 151 -> 154
+unsigned gram_grid(int K, int grad_dtype, uint64_t hi) {
+    const int groups = (K + 3) / 4;
+    bool half;
+    if (K <= gram_valu_max_k(grad_dtype)) half = grad_dtype == JABAS_F32 && K >= 3;
+    else if (grad_dtype == JABAS_F32) half = hi < kGramShortF32;
+    else half = groups == 4 ? hi < kGramVeryLongBf16 : hi >= kGramLongBf16;
+    return half ? JABAS_GRAM_GRID / 2 : JABAS_GRAM_GRID;
+}
 
 int launch_gram(int K, int grad_dtype, const SpanDev& sp, double* partials, unsigned grid, hipStream_t stream) {
     if (K > gram_valu_max_k(grad_dtype))

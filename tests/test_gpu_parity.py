@@ -346,6 +346,41 @@ def test_gram_sum_of_the_workgroup_rows(gpu, dtype, K):
         assert torch.equal(out.cpu().view(L.GRAM_MAX_K, L.GRAM_MAX_K), want), f"K={K} rows={rows}"
 
 
+@pytest.mark.parametrize("K", [8, 9, 12, 13, 16])
+def test_gram_bf16_runs_and_ends(gpu, K):
+    """The bf16 matrix-core kernels take whole runs of a wave (256 elements, 512 from 2**21 elements on) in their loop and the
+    span's ends after it: one element, one off a vector, a block and a run, starts inside a vector, a block and a line; one
+    run per wave of 512 and of 1024 workgroups, one more, a second round with and without an end; and both sides of the
+    line between the two shapes, by elements and by where the span starts. Integers of at most 3 in size: every product and
+    sum is exact."""
+    from jabas_amd import sync
+    run, far = 256, 1 << 21
+    for n, skew in ((1, 0), (1, 3), (7, 1), (9, 61), (127, 0), (129, 2), (run - 1, 0), (run, 0), (run, 1), (run + 1, 3), (2 * run, 61),
+                    (3 * run - 3, 3), (2048 * run, 0), (2048 * run, 1), (2049 * run + 5, 2), (4096 * run - 1, 0), (4097 * run + 9, 61),
+                    (far - 1, 0), (far - 1, 1), (far, 0), (far + 1, 3), (far + 512, 0), (far + 513, 2), (3 * far + 517, 61)):
+        gen = torch.Generator().manual_seed(n + K)
+        hg = [torch.randint(-3, 4, (n,), generator=gen, dtype=torch.int8).to(torch.bfloat16) for _ in range(K)]
+        G = sync.gram([_dev(t, gpu, skew) for t in hg]).cpu()
+        wide = torch.stack([t.double() for t in hg])
+        assert torch.equal(G, wide @ wide.t()), f"K={K} n={n} skew={skew}"
+
+
+@pytest.mark.parametrize("n", [(1 << 26) - 70, 1 << 26, (1 << 26) + 77])
+def test_gram_bf16_four_groups_of_very_long_spans(gpu, n):
+    """Both sides of the line at 2**26 elements beyond which the kernel of thirteen and more bf16 workers takes the span's ends in
+    its loop, and its sums move to fp64 on the way. Integers: exact."""
+    from jabas_amd import sync
+    gen = torch.Generator(device=gpu).manual_seed(n)
+    flat = [torch.randint(-3, 4, (n,), generator=gen, device=gpu, dtype=torch.int8).to(torch.bfloat16) for _ in range(3)]
+    grads = [flat[k % 3][:n] for k in range(13)]                     # thirteen workers over three buffers
+    want = torch.zeros(3, 3, dtype=torch.float64, device=gpu)
+    for i in range(3):
+        for j in range(3):
+            want[i, j] = (flat[i][:n].float() * flat[j][:n].float()).double().sum()      # |product| <= 9: exact
+    index = [k % 3 for k in range(13)]
+    assert torch.equal(sync.gram(grads).cpu(), want.cpu()[index][:, index])
+
+
 def test_gram_limits_and_determinism(gpu):
     from jabas_amd import sync, _lib as L
     g = [torch.zeros(4096, device=gpu) for _ in range(17)]
