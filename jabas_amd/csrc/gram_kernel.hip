@@ -25,7 +25,7 @@ namespace {
 #define JABAS_GRAM_VALU_MAX_K_BF16 7
 #endif
 // Up to here the vector-ALU kernel, beyond it the matrix cores. Both on fp32 gradients of 65 k / 300 k / 1.2 M / 25.6 M /
-// 67 M / 100 M elements, whole call in us, vector ALU against matrix cores:
+// 67 M / 100 M elements, whole call in us, vector ALU against matrix cores (1024 workgroups and an earlier finalize on both sides):
 //   K = 4   5.9 / 7.1 /  9.3 /  68.5 / 165.5 / 244.3   against   5.9 / 8.1 / 10.2 /  69.7 / 180.6 / 260.9
 //   K = 5   5.9 / 7.6 / 10.2 /  85.6 / 218.6 / 327.1   against   6.2 / 9.0 / 11.9 /  90.1 / 227.7 / 329.0
 //   K = 6   6.1 / 9.6 / 13.4 / 101.1 / 260.1 / 395.5   against   6.3 / 9.2 / 12.2 / 102.5 / 261.0 / 381.8
@@ -115,7 +115,7 @@ __global__ void __launch_bounds__(kBlock) gram_kernel(const SpanDev sp, double* 
     // adds lanes 16 apart (entry (j, *) of its result is the sum over i), the second the four j: every lane then holds the
     // sum of the 16 lanes with its b, and lanes 0, 4, 8 and 12 write the four. Multiplying by one is exact, the sums are
     // fp64. Two instructions per product, where a tree of wave shuffles takes twelve LDS permutations: 1.2 M elements,
-    // whole call, K = 5 fp32 22.0 -> 16.5 us, K = 7 bf16 34.8 -> 24.4 (10.2 and 13.5 with the finalize below).
+    // whole call, K = 5 fp32 22.0 -> 16.5 us, K = 7 bf16 34.8 -> 24.4 (9.4 and 11.4 with the finalize below and 512 workgroups for K = 5).
     __shared__ double red[kWaves][4][NP];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
