@@ -30,7 +30,7 @@ namespace {
 //   K = 5   5.9 / 7.6 / 10.2 /  85.6 / 218.6 / 327.1   against   6.2 / 9.0 / 11.9 /  90.1 / 227.7 / 329.0
 //   K = 6   6.1 / 9.6 / 13.4 / 101.1 / 260.1 / 395.5   against   6.3 / 9.2 / 12.2 / 102.5 / 261.0 / 381.8
 //   K = 7   6.5 / 10.2 / 14.8 / 117.8 / 325.8 / 473.3  against   6.4 / 9.3 / 12.7 / 116.7 / 298.2 / 440.1
-// The vector ALU also sums in chains a sixteenth as long: 100 M elements are 1e-16 off against 5e-15. bf16 gradients change
+// The vector ALU also sums in chains a sixteenth as long: on 100 M elements the diagonal is 7e-16 off against 7e-15. bf16 gradients change
 // at eight workers, where the matrix cores' sums are fp32 over short runs: up to seven every sum stays fp64.
 constexpr int gram_valu_max_k(int grad_dtype) { return grad_dtype == JABAS_BF16 ? JABAS_GRAM_VALU_MAX_K_BF16 : JABAS_GRAM_VALU_MAX_K; }
 
@@ -72,18 +72,25 @@ template <> struct GramLoad<JABAS_BF16> {
     }
 };
 
+// Running sums per product, and 1024 / sums workgroups: the vectors of a thread go to its sums in turn, so a sum is a chain of
+// as many additions as with 1024 workgroups and one. Half the workgroups with one sum were 1.2 to 3.7 times as far from the
+// exact sums from 12 M elements on.
+constexpr int gram_valu_sums(int K, int grad_dtype) { return grad_dtype == JABAS_F32 && K >= 3 ? 2 : 1; }
+
 template <int K, int DT>
 __global__ void __launch_bounds__(kBlock) gram_kernel(const SpanDev sp, double* partials) {
     using L = GramLoad<DT>;
-    constexpr int EPT = L::EPT;
+    constexpr int EPT = L::EPT, S = gram_valu_sums(K, DT);
     constexpr int NP = K * (K + 1) / 2;
-    double acc[NP];
+    double acc[S][NP];
 #pragma unroll
-    for (int i = 0; i < NP; ++i) acc[i] = 0.0;
+    for (int u = 0; u < S; ++u)
+#pragma unroll
+        for (int i = 0; i < NP; ++i) acc[u][i] = 0.0;
 
     const uint64_t nvec = (sp.hi + EPT - 1) / EPT;
     const uint64_t stride = static_cast<uint64_t>(gridDim.x) * kBlock;
-    for (uint64_t v = static_cast<uint64_t>(blockIdx.x) * kBlock + threadIdx.x; v < nvec; v += stride) {
+    auto add = [&](uint64_t v, double (&sum)[NP]) {
         const uint64_t e = v * EPT;
         float g[K][EPT];
         if (e >= sp.lo && e + EPT <= sp.hi) {
@@ -106,8 +113,18 @@ __global__ void __launch_bounds__(kBlock) gram_kernel(const SpanDev sp, double* 
 #pragma unroll
             for (int a = 0; a < K; ++a)
 #pragma unroll
-                for (int b = 0; b <= a; ++b, ++idx) acc[idx] = __builtin_fma(d[a], d[b], acc[idx]);
+                for (int b = 0; b <= a; ++b, ++idx) sum[idx] = __builtin_fma(d[a], d[b], sum[idx]);
         }
+    };
+    for (uint64_t v = static_cast<uint64_t>(blockIdx.x) * kBlock + threadIdx.x; v < nvec; v += S * stride) {
+        add(v, acc[0]);
+        if constexpr (S == 2) {
+            if (v + stride < nvec) add(v + stride, acc[1]);
+        }
+    }
+    if constexpr (S == 2) {
+#pragma unroll
+        for (int i = 0; i < NP; ++i) acc[0][i] += acc[1][i];
     }
 
     // Sum of every product over the wave's lanes on the fp64 matrix cores: lane j + 4 b + 16 i supplies entry (j, i) of
@@ -120,7 +137,7 @@ __global__ void __launch_bounds__(kBlock) gram_kernel(const SpanDev sp, double* 
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
     for (int i = 0; i < NP; ++i) {
-        const double q = __builtin_amdgcn_mfma_f64_4x4x4f64(acc[i], 1.0, 0.0, 0, 0, 0);
+        const double q = __builtin_amdgcn_mfma_f64_4x4x4f64(acc[0][i], 1.0, 0.0, 0, 0, 0);
         const double v = __builtin_amdgcn_mfma_f64_4x4x4f64(1.0, q, 0.0, 0, 0, 0);
         if ((lane & 51) == 0) red[wave][lane >> 2][i] = v;
     }
@@ -219,7 +236,9 @@ static_assert(kGramFinalizeBlock >= 64 + JABAS_GRAM_STRIDE, "one thread per entr
 constexpr int kGramRunBlocks = JABAS_GRAM_RUN_F32;
 constexpr uint64_t kGramShortF32 = 1u << 21;           // fewer elements: half the workgroups (gram_grid)
 
-template <int G>
+// S: running sums per pair of groups; a wave's runs go to them in turn. Two with half the workgroups (gram_grid): as many runs per
+// sum as with all of them and one, which half the workgroups and one sum were 1.2 to 2.3 times as far from the exact sums as.
+template <int G, int S>
 __global__ void __launch_bounds__(kBlock) gram_mfma_kernel(const SpanDev sp, int K, double* partials) {
     using L = GramLoad<JABAS_F32>;
     constexpr int P = G * (G + 1) / 2;
@@ -234,9 +253,11 @@ __global__ void __launch_bounds__(kBlock) gram_mfma_kernel(const SpanDev sp, int
         live[g] = g * 4 + wi < K;
         base[g] = sp.g[live[g] ? g * 4 + wi : 0];
     }
-    double acc[P];
+    double acc[S][P];
 #pragma unroll
-    for (int p = 0; p < P; ++p) acc[p] = 0.0;
+    for (int u = 0; u < S; ++u)
+#pragma unroll
+        for (int p = 0; p < P; ++p) acc[u][p] = 0.0;
     // Runs that lie wholly in the span are [first, last); at most two others hold its ends.
     const uint64_t n_runs = (sp.hi + kRun - 1) / kRun, first = (sp.lo + kRun - 1) / kRun;
     const uint64_t last = sp.hi / kRun > first ? sp.hi / kRun : first;
@@ -249,7 +270,7 @@ __global__ void __launch_bounds__(kBlock) gram_mfma_kernel(const SpanDev sp, int
             // wave reads anyway) and drops it when it multiplies: no load waits for another
             for (int g = 0; g < G; ++g) x[u][g] = L::raw(base[g], run * kRun + u * 64 + lane_off);
     };
-    auto multiply = [&](const L::Raw (&x)[kGramRunBlocks][G]) {
+    auto multiply = [&](const L::Raw (&x)[kGramRunBlocks][G], double (&sum)[P]) {
 #pragma unroll
         for (int u = 0; u < kGramRunBlocks; ++u)
 #pragma unroll
@@ -262,7 +283,7 @@ __global__ void __launch_bounds__(kBlock) gram_mfma_kernel(const SpanDev sp, int
                 for (int ga = 0; ga < G; ++ga)
 #pragma unroll
                     for (int gb = ga; gb < G; ++gb, ++p)
-                        acc[p] = __builtin_amdgcn_mfma_f64_4x4x4f64(d[ga], d[gb], acc[p], 0, 0, 0);
+                        sum[p] = __builtin_amdgcn_mfma_f64_4x4x4f64(d[ga], d[gb], sum[p], 0, 0, 0);
             }
     };
     // Bound by HBM reads. Two runs in flight per wave, the next one's loads issued before this one is multiplied; only whole
@@ -279,11 +300,11 @@ __global__ void __launch_bounds__(kBlock) gram_mfma_kernel(const SpanDev sp, int
         while (true) {
             const bool more = (run += n_waves) < last;
             if (more) load(run, y);
-            multiply(x);
+            multiply(x, acc[0]);
             if (!more) break;
             const bool again = (run += n_waves) < last;
             if (again) load(run, x);
-            multiply(y);
+            multiply(y, acc[S - 1]);
             if (!again) break;
         }
     }
@@ -298,7 +319,7 @@ __global__ void __launch_bounds__(kBlock) gram_mfma_kernel(const SpanDev sp, int
 #pragma unroll
             for (int g = 0; g < G; ++g) x[u][g] = whole ? L::raw(base[g], e) : L::edge(base[g], e, sp.lo, sp.hi);
         }
-        multiply(x);
+        multiply(x, acc[0]);
     }
     // The instruction's contraction index is lane / 16 and its four independent products are indexed by
     // (lane / 4) % 4; entry (i, j) of product b sits in lane j + 4 b + 16 i. Which of a lane's elements meets
@@ -307,7 +328,7 @@ __global__ void __launch_bounds__(kBlock) gram_mfma_kernel(const SpanDev sp, int
     // [p][4 i + j] is the sum over the four products and the four waves (in that order) for pair p.
     __shared__ double red[kWaves][P][64];
 #pragma unroll
-    for (int p = 0; p < P; ++p) red[wave][p][lane] = acc[p];
+    for (int p = 0; p < P; ++p) red[wave][p][lane] = S == 2 ? acc[0][p] + acc[S - 1][p] : acc[0][p];
     __syncthreads();
     for (int t = threadIdx.x; t < P * 16; t += kBlock) {
         const int p = t >> 4, i = (t >> 2) & 3, j = t & 3;
@@ -523,11 +544,12 @@ int launch_gram_k(int grad_dtype, const SpanDev& sp, double* partials, unsigned 
     return -1;
 }
 
+template <int S>
 int launch_gram_mfma(int K, const SpanDev& sp, double* partials, unsigned grid, hipStream_t stream) {
     switch ((K + 3) / 4) {
-        case 2: return static_cast<int>(launch_kernel(gram_mfma_kernel<2>, dim3(grid), dim3(kBlock), 0, stream, sp, K, partials));
-        case 3: return static_cast<int>(launch_kernel(gram_mfma_kernel<3>, dim3(grid), dim3(kBlock), 0, stream, sp, K, partials));
-        case 4: return static_cast<int>(launch_kernel(gram_mfma_kernel<4>, dim3(grid), dim3(kBlock), 0, stream, sp, K, partials));
+        case 2: return static_cast<int>(launch_kernel(gram_mfma_kernel<2, S>, dim3(grid), dim3(kBlock), 0, stream, sp, K, partials));
+        case 3: return static_cast<int>(launch_kernel(gram_mfma_kernel<3, S>, dim3(grid), dim3(kBlock), 0, stream, sp, K, partials));
+        case 4: return static_cast<int>(launch_kernel(gram_mfma_kernel<4, S>, dim3(grid), dim3(kBlock), 0, stream, sp, K, partials));
         default: return -1;
     }
 }
@@ -536,14 +558,17 @@ int launch_gram_mfma(int K, const SpanDev& sp, double* partials, unsigned grid, 
 
 // Most workgroups of a launch; hi: end of the span's element grid. 1024 unless half of them are faster:
 //   bf16 matrix cores      with the shapes above
-//   fp32 vector ALU        three to five workers: K = 5, 25 M / 100 M elements 84.3 / 322 -> 80.8 / 291 us, K = 4 65.5 / 243 ->
-//                          63.8 / 232, K = 3 50.1 / 178 -> 47.5 / 171, equal below 2 M (K = 1 and 2 lose 10-50 %, bf16 up to 30 %)
-//   fp32 matrix cores      short spans, whose waves have two or three runs each: K = 9 / 13 / 16, 1.2 M elements 15.5 / 20.4 /
-//                          21.7 -> 14.3 / 19.2 / 20.8 us, equal from 2.5 to 10 M; 25 M K = 8 122 -> 124, K = 9 151 -> 154
+//   fp32 vector ALU        three to five workers, two sums each: K = 5, 25 M / 100 M elements 84.3 / 322 -> 80.3 / 304 us, K = 4
+//                          65.5 / 243 -> 65.5 / 239, K = 3 equal, all equal below 2 M (K = 1 and 2 lose 10-50 %, bf16 up to 30 %)
+//   fp32 matrix cores      short spans, whose waves have two or three runs each, two sums each: K = 9 / 13 / 16, 1.2 M elements
+//                          15.5 / 20.4 / 21.7 -> 14.3 / 19.4 / 20.9 us, equal from 2.5 to 10 M; 25 M K = 8 122 -> 124, K = 9 151 -> 154
+// Distance of the diagonal from the exact sums, 1024 workgroups / half of them with one sum / with two (mean over seeds):
+//   K = 5   12 M 1.8 / 2.2 / 1.2e-16   25.6 M 2.6 / 5.9 / 2.1e-16   100 M 6.9 / 10.6 / 7.2e-16
+//   K = 9   0.7 M 2.0 / 2.5 / 1.5e-16   1.2 M 3.1 / 4.6 / 2.2e-16   2.0 M 3.5 / 7.6 / 3.1e-16
 unsigned gram_grid(int K, int grad_dtype, uint64_t hi) {
     const int groups = (K + 3) / 4;
     bool half;
-    if (K <= gram_valu_max_k(grad_dtype)) half = grad_dtype == JABAS_F32 && K >= 3;
+    if (K <= gram_valu_max_k(grad_dtype)) half = gram_valu_sums(K, grad_dtype) == 2;
     else if (grad_dtype == JABAS_F32) half = hi < kGramShortF32;
     else half = groups == 4 ? hi < kGramVeryLongBf16 : hi >= kGramLongBf16;
     return half ? JABAS_GRAM_GRID / 2 : JABAS_GRAM_GRID;
@@ -552,7 +577,8 @@ unsigned gram_grid(int K, int grad_dtype, uint64_t hi) {
 int launch_gram(int K, int grad_dtype, const SpanDev& sp, double* partials, unsigned grid, hipStream_t stream) {
     if (K > gram_valu_max_k(grad_dtype))
         return grad_dtype == JABAS_BF16 ? launch_gram_bf16_mfma(K, sp, partials, grid, stream)
-                                        : launch_gram_mfma(K, sp, partials, grid, stream);
+               : sp.hi < kGramShortF32      ? launch_gram_mfma<2>(K, sp, partials, grid, stream)
+                                          : launch_gram_mfma<1>(K, sp, partials, grid, stream);
     switch (K) {
         case 1: return launch_gram_k<1>(grad_dtype, sp, partials, grid, stream);
         case 2: return launch_gram_k<2>(grad_dtype, sp, partials, grid, stream);

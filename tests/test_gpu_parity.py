@@ -1144,10 +1144,10 @@ def test_gram_from_rows_that_hold_no_memory(gpu):
 
 @pytest.mark.parametrize("K", [3, 4, 5])
 def test_gram_of_few_workers_rounds_in_short_chains(gpu, K):
-    """2**25 elements of 1 + d and 1 - d, d = 2**-22: products 1 +- 2**-21 + 2**-44 and 1 - 2**-44. A thread sums 128 of
-    them, exactly (seven bits and 45). What follows rounds at most 50 times (wave 8, workgroup 8, rows of a part 16, parts
-    of a wave 2, waves 16). In chains of 2048 products, as long as a wave's sums on the matrix cores are, the 2**-44 is lost
-    from a sum of 512 on: 4e-14 off."""
+    """2**25 elements of 1 + d and 1 - d, d = 2**-22: products 1 +- 2**-21 + 2**-44 and 1 - 2**-44. A running sum of a thread
+    holds 128 of them (two sums of 64 vectors each, 2**17 threads), exactly (seven bits and 45). What follows rounds at most
+    36 times (two sums 1, wave 8, workgroup 16, rows of a class 2, classes 9): 50 are allowed. In chains of 2048
+    products, as long as a wave's sums on the matrix cores are, the 2**-44 is lost from a sum of 512 on: 4e-14 off."""
     from jabas_amd import sync
     n, d = 1 << 25, 2.0 ** -22
     G = sync.gram([torch.full((n,), 1 - d if k % 2 else 1 + d, dtype=torch.float32, device=gpu) for k in range(K)]).cpu()
@@ -1155,6 +1155,29 @@ def test_gram_of_few_workers_rounds_in_short_chains(gpu, K):
         for b in range(K):
             exact = n * (1 - d * d if (a + b) % 2 else 1 - 2 * d + d * d if a % 2 else 1 + 2 * d + d * d)
             assert abs(float(G[a, b]) - exact) <= 50 * 2.0 ** -53 * exact, (a, b)
+
+
+def _chain(c, m):
+    """m products c * c (exact in fp64) added one after the other."""
+    s, c2 = 0.0, float(c) * float(c)
+    for _ in range(m):
+        s += c2
+    return s
+
+
+@pytest.mark.parametrize("K,vectors", [(3, 24), (4, 24), (5, 24), (6, 24), (9, 24), (13, 24), (16, 24)])
+def test_gram_fp32_sums_are_as_short_with_half_the_workgroups(gpu, K, vectors):
+    """Equal elements: every running sum of the kernel is the same chain of additions, and their number is a power of two, so
+    what follows adds equal numbers, exactly, and the result tells how long the chains were. fp32 on the vector ALU (K <= 5): 2**18
+    sums of 24 vectors of four; on the matrix cores 2**14 sums of 96 products, in spans under 2**21 elements, where half as
+    many waves keep two sums each. Chains of 192 products, one sum per thread or wave, give another number."""
+    from jabas_amd import sync
+    sums = 1 << (18 if K <= 5 else 14)
+    m = 4 * vectors
+    rng = np.random.default_rng(K)
+    c = next(x for x in rng.uniform(1.0, 2.0, 200).astype(np.float32) if abs(_chain(x, 2 * m) - 2 * _chain(x, m)) > 10 * 2.0 ** -53 * m)
+    G = sync.gram([torch.full((sums * m,), float(c), dtype=torch.float32, device=gpu)] * K).cpu()
+    assert torch.equal(G, torch.full((K, K), sums * _chain(c, m), dtype=torch.float64))
 
 
 @pytest.mark.parametrize("rows", [1, 255, 257, 1024, 1025, 4097, 6144, 6145])
