@@ -474,9 +474,9 @@ int run_fused(KArgs& a, const JabasStepArgs* s, uint32_t tiles, uint32_t max_spa
         if (!workspace || reinterpret_cast<uintptr_t>(workspace) % 8) return JABAS_ERR_WORKSPACE;
         // one compact partial row per workgroup and per (span, stripe), as wide as the level's rows are; scratch that holds
         // a row per chunk only gets one workgroup per chunk
-        const auto fits = [&] { return workspace_bytes >= workspace_rows(workgroups(), a.n_span) * ns * sizeof(double); };
-        if (!fits()) a.split_log2 = 0;
-        if (!fits()) return JABAS_ERR_WORKSPACE;
+        const auto fits = [&](size_t width) { return workspace_bytes >= workspace_rows(workgroups(), a.n_span) * width * sizeof(double); };
+        if (!fits(shared_row_width(s->K, s->grad_dtype, oc, stats))) a.split_log2 = 0;
+        if (!fits(ns)) return JABAS_ERR_WORKSPACE;
         if (reinterpret_cast<uintptr_t>(stats_out) % 8) return JABAS_ERR_ALIGN;
     }
     if (workgroups() > 0x7fffffffull) a.split_log2 = 0;

@@ -118,6 +118,19 @@ inline uint32_t launch_split_log2(int K, int grad_dtype, int opt_class, int stat
 __host__ __device__ constexpr int stats_row_width(int K, int stats) {
     return stats == JABAS_STATS_FULL ? 4 + K : (stats == JABAS_STATS_GRAM ? 4 + K + K * (K - 1) / 2 : (stats ? 4 : 1));
 }
+// Widest rows of the statistics levels that are launched in the same chunks as `stats`: whether a launch is split further is
+// asked of scratch for these, so that levels with sums in common cut them alike on any scratch and keep the same bits.
+inline int shared_row_width(int K, int grad_dtype, int opt_class, int stats) {
+    int width = 0;
+    for (int level = JABAS_STATS_FULL; level <= JABAS_STATS_GRAM; ++level) {
+        if (level == JABAS_STATS_GRAM && K > JABAS_STATS_GRAM_MAX_K) continue;
+        if (launch_block(K, grad_dtype, opt_class, level) == launch_block(K, grad_dtype, opt_class, stats) &&
+            launch_chunk_tiles(K, grad_dtype, opt_class, level) == launch_chunk_tiles(K, grad_dtype, opt_class, stats) &&
+            stats_row_width(K, level) > width)
+            width = stats_row_width(K, level);
+    }
+    return width;
+}
 constexpr int imin(int a, int b) { return a < b ? a : b; }
 // Fewest elements a chunk of a launch with statistics covers (one partial row per chunk): sizes workspaces.
 constexpr int kMinStatsChunkElems = 4 * imin(imin(JABAS_BLOCK * JABAS_CHUNK_TILES_LO, JABAS_BLOCK * JABAS_CHUNK_TILES_SIM_LO),

@@ -1274,6 +1274,34 @@ def test_short_launches_give_the_result_of_whole_chunks(gpu, K, dtype, level, nu
         torch.testing.assert_close(ways[0][4][4:4 + K], norms, rtol=tol, atol=0.0)
 
 
+@pytest.mark.parametrize("K,dtype,numel,levels", [(8, torch.bfloat16, 1_200_011, ("full", "gram")),
+                                                  (4, torch.float32, 700_001, ("similarity", "full", "gram"))])
+def test_levels_share_their_bits_on_any_scratch(gpu, K, dtype, numel, levels):
+    """The sums that two statistics levels share are the same bits whatever scratch a call brings: what the sizing function
+    returns, the least that every level takes, and sizes in between, which hold the rows of one level's split launch and only
+    the whole chunks of a wider one."""
+    from jabas_amd import sync, _lib as L
+    gen = torch.Generator(device=gpu).manual_seed(numel)
+    grads = [(torch.randn(numel, generator=gen, device=gpu) * 0.3 + 0.1).to(dtype) for _ in range(K)]
+    span = sync.SpanSpec(grads)
+    full_size = sync.Workspace.for_span(numel, dtype, gpu).nbytes
+    chunks = -(-(-(-numel // 1024)) // (2 if K <= 4 else 4))
+    widths = [{"similarity": 4, "full": 4 + K, "gram": 4 + K + K * (K - 1) // 2}[x] for x in levels]
+    least = (chunks + 33) * widths[-1] * 8
+    between = [(2 * chunks + 33) * w * 8 for w in widths[:-1]]
+    for nbytes in (full_size, least, *(b for b in between if b > least), least + 4096):
+        rows = []
+        for level in levels:
+            ws = sync.Workspace.for_span(numel, dtype, gpu)
+            ws.nbytes = nbytes
+            rows.append(sync.sync_bucket(span, sync.make_step_args((1,) * K, dtype, stats=level), workspace=ws).clone())
+        for row, width in zip(rows[:-1], widths):
+            assert torch.equal(row[:width].view(torch.int64), rows[-1][:width].view(torch.int64)), nbytes
+    ws.nbytes = least - 8
+    with pytest.raises(L.JabasSyncError):
+        sync.sync_bucket(span, sync.make_step_args((1,) * K, dtype, stats=levels[-1]), workspace=ws)
+
+
 @pytest.mark.parametrize("numel", [3, 1024, 1025, 70001])
 @pytest.mark.parametrize("kind", ["sgd", "adamw", None])
 @pytest.mark.parametrize("weight,scale,out", [(1.0, None, "own"), (1.0, 1.0, "own"), (1.0, 2.5, "own"), (1.0, float("nan"), "own"),
