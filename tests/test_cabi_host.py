@@ -96,6 +96,34 @@ def test_plan_encode_counts_chunks():
     assert rc == L.OK and lib.jabas_plan_chunks(blob.ctypes.data, 0) == 3
 
 
+@pytest.mark.parametrize("K,sizes,rows", [
+    # rows of the level with the most workgroups: chunks of four tiles for full rows and K > 4, else two (similarity sums)
+    (8, [700] * 300, 300), (8, [5] * 511, 511), (16, [700] * 5000, 5000), (2, [1000] * 200, 200),      # one tile in every chunk
+    (8, [1500] * 200, 400), (16, [3000] * 3000, 6000),                   # two and three tiles
+    (8, [4096] * 200, 800), (8, [1 << 20], 512), (16, [1 << 24], 8192), (4, [1 << 18], 256),       # whole chunks
+    (8, [700] * 12, 48), (8, [5000], 8),                                 # a few empty workgroups are left
+    (8, [300] * 100 + [60000] * 27, 1010)])                              # 100 + 27 * 15 chunks, 910 of 1010 workgroups with a tile
+def test_plan_splits_chunks_that_hold_tiles_for_it(K, sizes, rows):
+    """A launch with statistics shares its chunks between workgroups until there are 512 (full rows of more than eight workers:
+    always two), but not where more than a quarter of them would find no tile: scratch holds one row per workgroup. A blob
+    that does not record this (encoded before it was) is launched as it was."""
+    lib = L.lib()
+    rc, blob, _ = _encode([_span(n, K=K) for n in sizes], K=K)
+    assert rc == L.OK
+    stripes = 32 * len(sizes) + 1
+    assert lib.jabas_plan_workspace_bytes(blob.ctypes.data) == (rows + stripes) * L.STATS_STRIDE * 8
+    old = blob.copy()
+    old.view(np.uint32)[9] = 0
+    unlimited = []
+    for level, split in ((L.STATS_FULL, int(K > 8)), (L.STATS_SIMILARITY, 0)):
+        n = lib.jabas_plan_chunks(blob.ctypes.data, level)
+        tiles = 4 if K > 4 and level == L.STATS_FULL else 2
+        while 2 << split <= tiles and n << split < 512:
+            split += 1
+        unlimited.append(n << split)
+    assert lib.jabas_plan_workspace_bytes(old.ctypes.data) == (max(unlimited) + stripes) * L.STATS_STRIDE * 8
+
+
 def test_plan_encode_starts_the_element_grid_at_a_256_byte_line_when_all_buffers_allow_it():
     """2048 elements per workgroup here (K = 2, no optimizer). With every buffer 61 elements into a
     256-byte line the grid starts at that line: 61 + 4036 elements still fit two workgroups, one
