@@ -320,45 +320,56 @@ const LaunchFn kLaunch[JABAS_MAX_K] = {launch_fused_k1,  launch_fused_k2,  launc
 
 // Second level of the statistics reduction: sums partial rows in a fixed order.
 //   stripes == 0  rows [s*in_stripes, (s+1)*in_stripes) of `in` -> row s of `out`
-//   stripes >= 1  stripe j = blockIdx.z of the chunk rows of span s = blockIdx.y -> row s*stripes + j
-// A workgroup sums four neighbouring slots (blockIdx.x) of its rows: lane = slot + 4 * row, so a wave's load covers
-// 32 contiguous bytes of sixteen rows, and a row of any width costs the time of its four widest. Thread (slot, class)
-// adds rows class, class + 256, ... in increasing order, sixteen loads in flight; the 256 sums of a slot meet by row
-// rotations, one LDS table and a second round of the same. The order depends on the number of rows alone, so the sums
-// that two statistics levels share are the same bits, on any machine.
-// Bound by latency: one trip to memory per sixteen (or four) rows of a class and the launch. Lanes along the rows with a
-// wave tree per slot, as it was, cost 2.1 us for 147 rows of 4 doubles, 5.6 us for 294 rows of 40, 9.4 us in two launches
-// beyond 2560 rows; this one 2.4, 3.8 and (3200 rows of 4, one launch) 4.5. Fourteen buckets through the hooks, fp32 K = 4:
-// 960 -> 897 us, 25 M elements, K = 6 with pair products: 243 -> 226 us.
-constexpr int kFinalizeBlock = 1024;
+//   stripes >= 1  stripe j of the rows of span s -> row s*stripes + j, kStripeRows rows or more in each that has any
+// An item is four neighbouring slots of the rows of one (span, stripe), summed by WAVES waves: lane = slot + 4 * row, so a
+// wave's load covers 32 contiguous bytes of sixteen rows, and a row of any width costs the time of its four widest. Thread
+// (slot, class) of C = 16 * WAVES classes adds rows class, class + C, ... in increasing order, sixteen loads in flight; the C
+// sums of a slot meet by row rotations and, with several waves, one LDS table and a second round of the same. The order
+// depends on the numbers of rows alone, so the sums that two statistics levels share are the same bits, on any machine.
+// Bound by latency: one trip to memory per sixteen (or fewer) rows of a class, and the launch of its waves.
+//   waves per item   sixteen for every item (before) cost many short spans the launch of waves without rows: 5000 spans of 700
+//                    elements K = 1 similarity sums 26.3 -> 10.7 us (whole launches), K = 8 pair products 208 -> 58, 60 rows of 4
+//                    doubles 5.1 -> 4.8; and the item of up to 1024 rows, one stripe of the split form, the same: 150 tensors of 1 k to
+//                    20 M elements, one span each, K = 1 42.8 -> 41.2, K = 4 full rows 142 -> 136
+//   batches          sixteen rows at once read rows beyond the last again where six are left (1500 rows 7.5 -> 6.5 us): eight too
 constexpr int kFinalizeSlots = 4;
-constexpr uint32_t kFinalizeClasses = kFinalizeBlock / kFinalizeSlots;
-constexpr uint32_t kStripeRows = 1024;        // chunk rows one workgroup sums in the striped launch
+constexpr uint32_t kStripeRows = 512;
 constexpr uint32_t kMaxStripes = 32;
-constexpr uint32_t kSingleLaunchRows = 6144;  // up to here one workgroup per span and four slots (15.4 k rows: 9.9 us)
-constexpr uint32_t kMaxStatsSpans = 65535;    // spans index the y dimension of the finalize grid
+constexpr uint32_t kMaxStatsSpans = 65535;    // spans index a dimension of the finalize grid
+// Up to here one launch: one batch of sixteen waves. Rows of 4 doubles, whole call, one launch / two: 4000 9.9 / 10.8 us,
+// 5000 12.0 / 11.8, 6000 14.2 / 13.1, 8000 16.7 / 15.0; stripes of 256 or 1024 rows the same.
+constexpr uint32_t kSingleLaunchRows = 4096;
 
-// Adds U rows of a class to acc, first row r, no row at or beyond c1 (c1 > 0): the loads are issued together, those beyond
-// the end repeat the last row and are dropped.
-template <int U>
+// Adds U rows of a class to acc, first row r, C rows apart, no row at or beyond c1 (c1 > 0): the loads are issued together,
+// those beyond the end repeat the last row and are dropped.
+template <int U, uint32_t C>
 __device__ __forceinline__ void add_rows(const double* col, uint32_t ns, uint32_t r, uint32_t c1, double& acc) {
     double v[U];
 #pragma unroll
     for (int i = 0; i < U; ++i) {
-        const uint32_t c = r + i * kFinalizeClasses;
+        const uint32_t c = r + i * C;
         v[i] = col[static_cast<uint64_t>(c < c1 ? c : c1 - 1) * ns];
     }
 #pragma unroll
-    for (int i = 0; i < U; ++i) acc += r + i * kFinalizeClasses < c1 ? v[i] : 0.0;
+    for (int i = 0; i < U; ++i) acc += r + i * C < c1 ? v[i] : 0.0;
 }
 
-__global__ void __launch_bounds__(kFinalizeBlock) finalize_stats_kernel(const uint32_t* chunk_prefix, uint32_t n_rows,
-                                                                        uint32_t split_log2, uint32_t use_inline, uint32_t stripes,
-                                                                        uint32_t in_stripes, uint32_t ns, uint32_t out_stride,
-                                                                        const double* in, double* out) {
+constexpr int finalize_block(int waves) { return waves == 1 ? 256 : 64 * waves; }     // one wave per item: four items
+template <int WAVES>
+__global__ void __launch_bounds__(finalize_block(WAVES)) finalize_stats_kernel(const uint32_t* chunk_prefix, uint32_t n_span, uint32_t n_rows,
+                                                                               uint32_t split_log2, uint32_t use_inline, uint32_t stripes,
+                                                                               uint32_t in_stripes, uint32_t ns, uint32_t out_stride,
+                                                                               const double* in, double* out) {
     // input rows are compact (ns doubles each, the width of the level); output rows have out_stride slots, the unused ones 0
-    __shared__ double table[kFinalizeBlock / 16][kFinalizeSlots];
-    const uint32_t s = blockIdx.y, j = blockIdx.z, t = threadIdx.x;
+    constexpr uint32_t kThreads = 64 * WAVES, kClasses = kThreads / kFinalizeSlots;
+    const uint32_t t = threadIdx.x % kThreads, j = blockIdx.z;
+    uint32_t s = blockIdx.y, group = blockIdx.x;
+    if constexpr (WAVES == 1) {                  // four items per workgroup, whole waves, no barrier below
+        const uint32_t groups = (ns + kFinalizeSlots - 1) / kFinalizeSlots, item = blockIdx.x * 4 + threadIdx.x / 64;
+        s = item / groups;
+        group = item % groups;
+        if (s >= n_span) return;
+    }
     uint32_t c0, c1, o;
     if (stripes == 0) {
         c0 = s * in_stripes;
@@ -367,54 +378,81 @@ __global__ void __launch_bounds__(kFinalizeBlock) finalize_stats_kernel(const ui
     } else {
         uint32_t b0 = 0, b1 = n_rows;
         if (!use_inline) { b0 = chunk_prefix[s] << split_log2; b1 = chunk_prefix[s + 1] << split_log2; }
-        const uint32_t per = (b1 - b0 + stripes - 1) / stripes;
+        uint32_t per = (b1 - b0 + stripes - 1) / stripes;
+        if (stripes > 1 && per < kStripeRows) per = kStripeRows;
         c0 = b0 + j * per < b1 ? b0 + j * per : b1;
         c1 = c0 + per < b1 ? c0 + per : b1;
         o = s * stripes + j;
     }
-    const uint32_t slot = blockIdx.x * kFinalizeSlots + (t & (kFinalizeSlots - 1));
+    const uint32_t slot = group * kFinalizeSlots + (t & (kFinalizeSlots - 1));
     const double* col = in + (slot < ns ? slot : ns - 1);
     double acc = 0.0;
-    for (uint32_t base = c0; base < c1;) {       // uniform over the workgroup
+    for (uint32_t base = c0; base < c1;) {       // uniform over the item's waves
         const uint32_t r = base + t / kFinalizeSlots;
-        if (c1 - base > 4 * kFinalizeClasses) {
-            add_rows<16>(col, ns, r, c1, acc);
-            base += 16 * kFinalizeClasses;
+        if (c1 - base > 8 * kClasses) {
+            add_rows<16, kClasses>(col, ns, r, c1, acc);
+            base += 16 * kClasses;
+        } else if (c1 - base > 4 * kClasses) {
+            add_rows<8, kClasses>(col, ns, r, c1, acc);
+            base += 8 * kClasses;
         } else {
-            add_rows<4>(col, ns, r, c1, acc);
-            base += 4 * kFinalizeClasses;
+            add_rows<4, kClasses>(col, ns, r, c1, acc);
+            base += 4 * kClasses;
         }
     }
     acc += dpp_move<0x128, 0xf>(acc);            // row_ror:8, row_ror:4: the four classes of a 16-lane row, per slot
     acc += dpp_move<0x124, 0xf>(acc);
-    if ((t & 15) < kFinalizeSlots) table[t >> 4][t & 15] = acc;
-    __syncthreads();
-    double* row = out + static_cast<uint64_t>(o) * out_stride;
-    if (t < 64) {                                // one wave: 64 entries of a slot, four per lane, then over the lanes
-        const int e = t >> 2, v = t & (kFinalizeSlots - 1);
-        double sum = table[e][v];
+    if constexpr (WAVES > 1) {
+        __shared__ double table[4 * WAVES][kFinalizeSlots];
+        if ((t & 15) < kFinalizeSlots) table[t >> 4][t & 15] = acc;
+        __syncthreads();
+        if (t < 64) {                            // one wave: the entries of a slot, WAVES / 4 per lane, then over the lanes
+            const int e = t >> 2, v = t & (kFinalizeSlots - 1);
+            acc = table[e][v];
 #pragma unroll
-        for (int i = 1; i < kFinalizeBlock / 256; ++i) sum += table[16 * i + e][v];
-        sum += dpp_move<0x128, 0xf>(sum);
-        sum += dpp_move<0x124, 0xf>(sum);
-        sum += __shfl_xor(sum, 16);
-        sum += __shfl_xor(sum, 32);
-        if (t < kFinalizeSlots && slot < ns) row[slot] = sum;
-    } else if (blockIdx.x == 0) {
-        for (uint32_t i = ns + t - 64; i < out_stride; i += kFinalizeBlock - 64) row[i] = 0.0;
+            for (int i = 1; i < WAVES / 4; ++i) acc += table[16 * i + e][v];
+            acc += dpp_move<0x128, 0xf>(acc);
+            acc += dpp_move<0x124, 0xf>(acc);
+        }
+    }
+    double* row = out + static_cast<uint64_t>(o) * out_stride;
+    if (t < 64) {
+        acc += __shfl_xor(acc, 16);
+        acc += __shfl_xor(acc, 32);
+        if (t < kFinalizeSlots && slot < ns) row[slot] = acc;
+    }
+    if (group == 0) {
+        for (uint32_t i = ns + t; i < out_stride; i += kThreads) row[i] = 0.0;
     }
 }
 
-hipError_t finalize(uint32_t ns, uint32_t grid_stripes, hipStream_t stream, const KArgs& a, uint32_t n_rows, uint32_t stripes, uint32_t in_stripes,
-                    uint32_t out_stride, const double* in, double* out) {
-    const dim3 grid((ns + kFinalizeSlots - 1) / kFinalizeSlots, a.n_span, grid_stripes);
-    return launch_kernel(finalize_stats_kernel, grid, dim3(kFinalizeBlock), 0, stream, a.chunk_prefix, n_rows, a.split_log2,
-                         a.use_inline, stripes, in_stripes, ns, out_stride, in, out);
+// By the most rows of an item: one wave up to one batch of four, where its four items share a workgroup and none waits.
+inline int finalize_waves(uint32_t max_rows) {
+    if (max_rows <= 64) return 1;
+    return max_rows <= 1024 ? 4 : 16;
 }
 
-inline uint32_t stripes_for(uint32_t max_span_chunks) {
-    if (max_span_chunks <= kSingleLaunchRows) return 1;      // a second launch costs more than it saves
-    const uint32_t st = (max_span_chunks + kStripeRows - 1) / kStripeRows;
+template <int WAVES>
+hipError_t launch_finalize(uint32_t ns, uint32_t grid_stripes, hipStream_t stream, const KArgs& a, uint32_t n_rows, uint32_t stripes,
+                           uint32_t in_stripes, uint32_t out_stride, const double* in, double* out) {
+    const uint32_t groups = (ns + kFinalizeSlots - 1) / kFinalizeSlots;
+    const dim3 grid = WAVES == 1 ? dim3((a.n_span * groups + 3) / 4, 1, grid_stripes) : dim3(groups, a.n_span, grid_stripes);
+    return launch_kernel(finalize_stats_kernel<WAVES>, grid, dim3(finalize_block(WAVES)), 0, stream, a.chunk_prefix, a.n_span, n_rows,
+                         a.split_log2, a.use_inline, stripes, in_stripes, ns, out_stride, in, out);
+}
+// max_rows: most rows of an item
+hipError_t finalize(uint32_t ns, uint32_t max_rows, uint32_t grid_stripes, hipStream_t stream, const KArgs& a, uint32_t n_rows, uint32_t stripes,
+                    uint32_t in_stripes, uint32_t out_stride, const double* in, double* out) {
+    switch (finalize_waves(max_rows)) {
+        case 1: return launch_finalize<1>(ns, grid_stripes, stream, a, n_rows, stripes, in_stripes, out_stride, in, out);
+        case 4: return launch_finalize<4>(ns, grid_stripes, stream, a, n_rows, stripes, in_stripes, out_stride, in, out);
+        default: return launch_finalize<16>(ns, grid_stripes, stream, a, n_rows, stripes, in_stripes, out_stride, in, out);
+    }
+}
+
+inline uint32_t stripes_for(uint32_t max_rows) {
+    if (max_rows <= kSingleLaunchRows) return 1;
+    const uint32_t st = (max_rows + kStripeRows - 1) / kStripeRows;
     return st > kMaxStripes ? kMaxStripes : st;
 }
 // workspace rows: one per chunk, then one per (span, stripe)
@@ -486,14 +524,15 @@ int run_fused(KArgs& a, const JabasStepArgs* s, uint32_t tiles, uint32_t max_spa
         if (err != 0) return JABAS_ERR_LAUNCH;
     }
     if (stats) {
-        const uint32_t st = stripes_for(a.use_inline ? n_rows : max_span_chunks << a.split_log2);
+        const uint32_t max_rows = a.use_inline ? n_rows : max_span_chunks << a.split_log2;     // of a span
+        const uint32_t st = stripes_for(max_rows);
         hipError_t err;
         if (st == 1) {
-            err = finalize(ns, 1, stream, a, n_rows, 1u, 0u, kStatsStride, a.partials, stats_out);
+            err = finalize(ns, max_rows, 1, stream, a, n_rows, 1u, 0u, kStatsStride, a.partials, stats_out);
         } else {
             double* level2 = a.partials + static_cast<uint64_t>(n_rows) * ns;
-            err = finalize(ns, st, stream, a, n_rows, st, 0u, ns, a.partials, level2);
-            if (err == hipSuccess) err = finalize(ns, 1, stream, a, n_rows, 0u, st, kStatsStride, level2, stats_out);
+            err = finalize(ns, (max_rows + st - 1) / st, st, stream, a, n_rows, st, 0u, ns, a.partials, level2);
+            if (err == hipSuccess) err = finalize(ns, st, 1, stream, a, n_rows, 0u, st, kStatsStride, level2, stats_out);
         }
         if (err != hipSuccess) return JABAS_ERR_LAUNCH;
     }

@@ -1180,38 +1180,82 @@ def test_gram_fp32_sums_are_as_short_with_half_the_workgroups(gpu, K, vectors):
     assert torch.equal(G, torch.full((K, K), sums * _chain(c, m), dtype=torch.float64))
 
 
-@pytest.mark.parametrize("rows", [1, 255, 257, 1024, 1025, 4097, 6144, 6145])
-@pytest.mark.parametrize("K,level", [(4, "similarity"), (5, "full"), (8, "gram"), (16, "full")])
-def test_statistics_over_many_chunks_are_exact(gpu, K, level, rows):
-    """Small whole numbers and weights that are powers of two: every sum is exact in fp64 in any order, so the row has to be
-    the integer result whatever the number of chunk rows (the edges of the second level's batches and of its split into
-    stripes) and the width of the row; scratch and output start as NaN."""
-    from jabas_amd import sync, _lib as L
-    chunk = 1024 * (2 if K <= 4 else 4)                        # 256 threads x 4 elements x tiles, no optimizer
-    n = chunk * (rows - 1) + 5
-    n = min(n, 1 << 24)
-    gen = torch.Generator(device=gpu).manual_seed(rows + K)
-    grads = [torch.randint(-3, 4, (n,), generator=gen, device=gpu).to(torch.bfloat16) for _ in range(K)]
-    batches = (4, 2, 1, 3, 2)[:K] if K == 5 else (1,) * K
-    args = sync.make_step_args(batches, torch.bfloat16, stats=level)
+def _exact_row(grads, level):
+    """Statistics row of whole numbers under weights of a quarter: every sum is exact in fp64 (and fp32) in any order."""
+    from jabas_amd import _lib as L
+    K = len(grads)
+    want = torch.zeros(L.STATS_STRIDE, dtype=torch.float64, device=grads[0].device)
+    quarter = [sum(g.float() for g in grads[h::2]) * 0.25 if K > h else torch.zeros_like(grads[0], dtype=torch.float32) for h in (0, 1)]
+    agg = sum(g.float() for g in grads) * 0.25
+    want[0] = (quarter[0] * quarter[1]).sum(dtype=torch.float64)
+    for slot, x in ((1, quarter[0]), (2, quarter[1]), (3, agg)):
+        want[slot] = (x * x).sum(dtype=torch.float64)
+    if level != "similarity":
+        for k, g in enumerate(grads):
+            want[4 + k] = g.float().square().sum(dtype=torch.float64)
+    if level == "gram":
+        for i in range(K):
+            for j in range(i + 1, K):
+                want[L.stat_pair(K, i, j)] = (grads[i].float() * grads[j].float()).sum(dtype=torch.float64)
+    return want
+
+
+def _quarter_args(K, dtype, level):
+    from jabas_amd import sync
+    args = sync.make_step_args((1,) * K, dtype, stats=level)
     for k in range(K):                                         # powers of two instead of the batch quotients
         args.weight[k] = args.half_weight[k] = 0.25
-    ws = sync.Workspace.for_span(n, torch.bfloat16, gpu)
-    ws.buf.fill_(float("nan"))
-    ws.stats.fill_(float("nan"))
-    row = sync.sync_bucket(sync.SpanSpec(grads), args, workspace=ws)
-    g = torch.stack(grads).float()
-    quarter = [(g[h::2].sum(0) * 0.25).double() for h in (0, 1)]
-    agg = (g.sum(0) * 0.25).double()
-    want = torch.zeros(L.STATS_STRIDE, dtype=torch.float64, device=gpu)
-    want[:4] = torch.stack([(quarter[0] * quarter[1]).sum(), (quarter[0] ** 2).sum(), (quarter[1] ** 2).sum(), (agg ** 2).sum()])
-    if level != "similarity":
-        want[4:4 + K] = torch.stack([(x.double() ** 2).sum() for x in g])
-    if level == "gram":
-        for a in range(K):
-            for b in range(a + 1, K):
-                want[L.stat_pair(K, a, b)] = (g[a].double() * g[b].double()).sum()
-    assert torch.equal(row, want)
+    return args
+
+
+def _whole_numbers(gpu, n, K, dtype, seed):
+    gen = torch.Generator(device=gpu).manual_seed(seed)
+    return [torch.randint(-3, 4, (n,), generator=gen, device=gpu, dtype=torch.int8).to(dtype) for _ in range(K)]
+
+
+@pytest.mark.parametrize("rows", [1, 64, 65, 255, 256, 257, 512, 1024, 1025, 2049, 4096, 4097, 5000, 16900])
+@pytest.mark.parametrize("K,level", [(4, "similarity"), (5, "full"), (8, "gram"), (16, "full")])
+def test_statistics_over_many_chunks_are_exact(gpu, K, level, rows):
+    """The row has to be the integer result whatever the number of partial rows (edges of the second level's waves per span, of
+    its batches, of its classes and of its split into stripes, stripes of 512 rows and 32 longer ones) and the width of the row.
+    Scratch and output start as NaN, which tells how many rows the launch wrote; the number of tiles per workgroup is the
+    launch's own, so the size that gives the wanted rows is looked for among one, two and four, then among whole chunks."""
+    from jabas_amd import sync
+    width = {"similarity": 4, "full": 4 + K, "gram": 4 + K + K * (K - 1) // 2}[level]
+    stripes = 0 if rows <= 4096 else min(32, -(-rows // 512))
+    args = _quarter_args(K, torch.bfloat16, level)
+    for tight in (False, True):                                # scratch of whole chunks: the launch is not split
+        for tiles in (1, 2, 4):
+            n = 1024 * tiles * (rows - 1) + 5
+            grads = _whole_numbers(gpu, n, min(K, 4), torch.bfloat16, rows + K)
+            grads = [grads[k % len(grads)] for k in range(K)]  # the kernel only reads
+            ws = sync.Workspace.for_span(n, torch.bfloat16, gpu)
+            ws.buf.fill_(float("nan"))
+            ws.stats.fill_(float("nan"))
+            if tight:
+                ws.nbytes = min(ws.nbytes, (-(-n // (2048 if K <= 4 else 4096)) + 33) * width * 8)
+            row = sync.sync_bucket(sync.SpanSpec(grads), args, workspace=ws)
+            assert torch.equal(row, _exact_row(grads, level))
+            if int((~ws.buf.isnan()).sum()) == (rows + stripes) * width:
+                return
+    pytest.fail(f"no launch wrote {rows} rows")
+
+
+@pytest.mark.parametrize("K,level,sizes", [
+    (9, "full", [700, 13_000_123, 3000]),                      # two workgroups per chunk and stripes, short spans beside them
+    (4, "similarity", [5, 9_000_001, 1 << 20, 1]), (4, "gram", [300_001, 1025, 1024, 70_000]), (1, "similarity", [1 << 20] * 2),
+    (3, "full", [1000] * 301), (8, "gram", [1 + 37 * i for i in range(130)]), (8, "full", [4097] * 67 + [400_000]), (2, "similarity", [9])])
+def test_statistics_of_plans_are_exact(gpu, K, level, sizes):
+    """Every span's row of a plan is the integer result: rows of split chunks behind the spans' table of whole ones, the second
+    level in one launch and in stripes, one, four and sixteen waves per span, full and ragged groups of four spans."""
+    from jabas_amd import sync
+    sets = [_whole_numbers(gpu, n, K, torch.float32, 7 * i + K) for i, n in enumerate(sizes)]
+    plan = sync.SyncPlan([sync.SpanSpec(g) for g in sets])
+    plan.ws.buf.fill_(float("nan"))
+    plan.ws.stats.fill_(float("nan"))
+    rows = plan.run(_quarter_args(K, torch.float32, level))
+    for g, row in zip(sets, rows):
+        assert torch.equal(row, _exact_row(g, level))
 
 
 @pytest.mark.parametrize("K,dtype,level", [(1, torch.float32, None), (4, torch.float32, None), (4, torch.float32, "full"),
