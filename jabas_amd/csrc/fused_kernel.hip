@@ -457,6 +457,7 @@ __device__ __forceinline__ void span_range(const SP& sp, uint32_t lt0, uint32_t 
             const uint64_t fit = (stretch_end - e0) / TE;
             const uint32_t left = lt1 - lt;
             nfull = fit < left ? static_cast<uint32_t>(fit) : left;
+            __builtin_assume(nfull <= CT);       // lt1 - lt0 is a chunk's share: the cascade below has at most CT / U rounds
         }
         if (nfull) {
             const GroupDev G = a.groups[gid];
