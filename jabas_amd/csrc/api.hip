@@ -37,7 +37,7 @@ struct PlanHeader {
     int32_t K, grad_dtype, opt_kind;
     uint32_t max_group;       // largest group index any bound names
     uint32_t all_have_s1;     // every non-empty span carries a state1 pointer
-    uint32_t most_split;      // byte v: 1 + the most split_log2 that pays for shape v's chunks (useful_split); 0: not recorded
+    uint32_t split;           // byte v: 1 + split_log2 of launches of shape v (launch_split_log2); 0: not recorded
     PlanShape shape[3];
     uint64_t off_spans, off_bounds, total_bytes;
 };
@@ -632,27 +632,14 @@ JABAS_API size_t jabas_plan_bytes(const JabasSpan* spans, uint32_t n_span, uint3
 }
 
 namespace {
-// Most workgroups (log2) per chunk of a shape of which at least three in four have a tile, a few dozen aside: the last chunk of a
-// span holds the tiles that are left, and where most spans are shorter than a chunk (one span per small tensor) more workgroups
-// are mostly ones without work, which still write a row each. Spans of 700 elements, all splits -> these: 500, K = 1 AdamW
-// without statistics 7.7 -> 4.3 us, 500, K = 8 bf16 pair products 31.5 -> 26.3, 20000, K = 16 bf16 full rows 651 -> 502.
-uint32_t useful_split(const SpanDev* sd, uint32_t n_span, const PlanShape& ps) {
-    uint32_t s = 0;
-    for (; (2u << s) <= ps.chunk_tiles; ++s) {
-        uint64_t live = 0, all = 0;
-        for (uint32_t i = 0; i < n_span; ++i) {
-            const uint64_t tiles = tiles_of(sd[i].hi, static_cast<int>(ps.block));
-            live += chunks_of_tiles(tiles, ps.chunk_tiles >> (s + 1));
-            all += chunks_of_tiles(tiles, ps.chunk_tiles) << (s + 1);
-        }
-        if (4 * live < 3 * all && all - live > 64) break;
-    }
-    return s;
-}
+// Workgroups of a launch over `tiles` tiles of one span that have one, with 2^s workgroups per chunk of ct tiles.
+inline uint64_t live_workgroups(uint64_t tiles, uint32_t ct, uint32_t s) { return chunks_of_tiles(tiles, ct >> s); }
 uint32_t plan_split_log2(const PlanHeader& h, int stats) {
-    const uint32_t s = launch_split_log2(h.K, h.grad_dtype, opt_class_of(h.opt_kind), stats, h.shape[shape_level(stats)].n_chunks);
-    const uint32_t most = h.most_split >> (8 * shape_level(stats)) & 0xff;
-    return most && s >= most ? most - 1 : s;
+    const int v = shape_level(stats);
+    const uint32_t recorded = h.split >> (8 * v) & 0xff;
+    if (recorded) return recorded - 1;
+    const uint64_t n = h.shape[v].n_chunks;
+    return launch_split_log2(h.K, h.grad_dtype, opt_class_of(h.opt_kind), stats, n, [&](uint32_t s) { return n << s; });
 }
 }  // namespace
 
@@ -702,7 +689,6 @@ JABAS_API int jabas_plan_encode(const JabasSpan* spans, uint32_t n_span, const J
         if (rc != JABAS_OK) return rc;
         if (spans[i].numel && !spans[i].state1) h.all_have_s1 = 0;
     }
-    for (int v = 0; v < 3; ++v) h.most_split |= (1u + useful_split(sd, n_span, h.shape[v])) << (8 * v);
     size_t cursor = fixed;
     int table_of[3];                             // level -> the level whose table it uses (itself when it owns one)
     for (int v = 0; v < 3; ++v) {
@@ -756,8 +742,16 @@ JABAS_API int jabas_plan_encode(const JabasSpan* spans, uint32_t n_span, const J
         prefix[n_span] = c;
         if (c != ps.n_chunks) return JABAS_ERR_PLAN;
     }
-    for (int v = 0; v < 3; ++v)
+    for (int v = 0; v < 3; ++v) {
         if (table_of[v] != v) h.shape[v] = h.shape[table_of[v]];
+        const auto live = [&](uint32_t s) {
+            uint64_t n = 0;
+            for (uint32_t i = 0; i < n_span; ++i)
+                n += live_workgroups(tiles_of(sd[i].hi, static_cast<int>(h.shape[v].block)), h.shape[v].chunk_tiles, s);
+            return n;
+        };
+        h.split |= (1u + launch_split_log2(K, grad_dtype, oc, v, h.shape[v].n_chunks, live)) << (8 * v);
+    }
     if (n_bounds) memcpy(base + h.off_bounds, bounds, static_cast<size_t>(n_bounds) * sizeof(JabasBound));
     memcpy(base, &h, sizeof(h));
     return JABAS_OK;
@@ -854,7 +848,8 @@ JABAS_API int jabas_sync_bucket(const JabasSpan* span, const JabasBound* bounds_
     a.chunk_tiles = launch_chunk_tiles(args->K, args->grad_dtype, oc, stats);
     a.n_chunks = static_cast<uint32_t>(chunks_of_tiles(tiles, a.chunk_tiles));
     a.use_inline = 1;
-    a.split_log2 = launch_split_log2(args->K, args->grad_dtype, oc, stats, a.n_chunks);
+    a.split_log2 = launch_split_log2(args->K, args->grad_dtype, oc, stats, a.n_chunks,
+                                     [&](uint32_t s) { return live_workgroups(tiles, a.chunk_tiles, s); });
     return run_fused(a, args, tiles, a.n_chunks, stats_out, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
 }
 

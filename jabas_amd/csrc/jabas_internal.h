@@ -86,32 +86,41 @@ __host__ __device__ constexpr int launch_chunk_tiles(int K, int /*grad_dtype*/, 
 }
 // Statistics level whose launch shape (and chunk table of a plan) a level uses.
 __host__ __device__ constexpr int shape_level(int stats) { return stats == JABAS_STATS_GRAM ? JABAS_STATS_FULL : stats; }
-// log2 of the workgroups that share a chunk of a launch of n_chunks chunks: a plan's tables know whole chunks only, the
-// launch decides how many workgroups each of them gets.
-//   short launches      split down to single tiles until there are 2048 workgroups (512 with statistics, whose epilogue is paid
-//                       per workgroup): below that compute units idle and a workgroup takes its tiles in turn, each at the
-//                       latency of memory. GPU time, whole chunks -> split: fp32 K = 4 Adam 0.1 / 0.3 / 0.7 / 1.5 M elements
-//                       10.7 / 16.1 / 14.9 / 20.4 -> 7.0 / 8.4 / 11.2 / 16.4 us (512 workgroups: 17.5), 6 M 51.3 -> 48.7
-//                       (1024: 51.9), bf16 K = 8 full rows 0.3 /
-//                       1.5 M 23.3 / 27.0 -> 13.0 / 22.4 (1024: 23.4), pair products 1.2 M 28.2 -> 24.5 (1024: 25.0)
+// log2 of the workgroups that share a chunk of a launch of n_chunks chunks, live(s) of them with a tile to work on at split s: a
+// plan's tables know whole chunks only, the launch decides how many workgroups each of them gets. All figures: spans by value
+// over buffers that rotate through more than the last-level cache; one set of buffers that stays there misleads.
+//   short launches      below about 400 workgroups compute units idle and a workgroup takes its tiles in turn, each at the latency
+//                       of memory. Whole chunks -> split: fp32 K = 4 AdamW 0.1 / 0.5 / 1.5 M elements 7.4 / 8.2 / 13.0 -> 4.1 / 6.0 /
+//                       10.6 us, bf16 K = 8 AdamW full rows 0.1 / 0.5 M 12.0 / 13.1 -> 7.8 / 10.2. Split while there are fewer than
+//                       2048 without statistics, as it was, 1 to 4 M elements lose: K = 4 AdamW 2 / 3 / 4 M 17.9 / 25.1 / 32.7 ->
+//                       19.0 / 27.5 / 35.8, K = 8 bf16 aggregate 4 M 15.4 -> 18.0; while fewer than 512, 2 M 18.9, and K = 8 pair
+//                       products 0.9 M 0.90 of the time of whole chunks against 0.74
+//   without a tile      at most a quarter, or 64 with statistics (each still runs its epilogue and writes a row) and 256 without, or as
+//                       many as there are compute units for: plans over short spans, one per small tensor, whose last chunk is
+//                       mostly their only one. All splits -> these: 500 spans of 700 elements, K = 1 AdamW 7.7 -> 4.4 us, 5000, K = 16
+//                       bf16 full rows 88.5 -> 52.0
 //   full rows, K > 8    two workgroups per chunk at any size: these kernels hold one tile in flight and two or three waves per
 //                       SIMD, and half the work per workgroup keeps the streamed window compact and the last round of
-//                       workgroups short: ResNet-50 K = 16 bf16 254 -> 231 us (four: 240), K = 12 fp32 SGD 25 M elements
-//                       307 -> 291, K = 16 fp32 Adam 60 M 957 -> 940. K = 5..8 would gain 2-3 % with full rows and lose
-//                       11-14 % with pair products (25..40 sums per workgroup), and both levels cut their sums alike
+//                       workgroups short: ResNet-50 K = 16 bf16 254 -> 231 us (four: 240), 25 M elements K = 12 fp32 SGD
+//                       302 -> 284, K = 16 fp32 AdamW 406 -> 390. Not bf16 gradients without an optimizer, whose reads alone are
+//                       at the rate of memory: K = 12 / 16, 25 M 102 / 138 -> 113 / 162. K = 5..8 would gain 2-3 % with full
+//                       rows and lose 11-14 % with pair products (25..40 sums per workgroup), and both levels cut their sums alike
 #ifndef JABAS_SPLIT_BELOW
-#define JABAS_SPLIT_BELOW 2048
+#define JABAS_SPLIT_BELOW 448
 #endif
 #ifndef JABAS_SPLIT_BELOW_STATS
-#define JABAS_SPLIT_BELOW_STATS 512
+#define JABAS_SPLIT_BELOW_STATS 384
 #endif
-#ifndef JABAS_SPLIT_MANYK
-#define JABAS_SPLIT_MANYK 1
-#endif
-inline uint32_t launch_split_log2(int K, int grad_dtype, int opt_class, int stats, uint64_t n_chunks) {
+template <class Live>
+inline uint32_t launch_split_log2(int K, int grad_dtype, int opt_class, int stats, uint64_t n_chunks, const Live& live) {
     const uint32_t tiles = static_cast<uint32_t>(launch_chunk_tiles(K, grad_dtype, opt_class, stats));
-    uint32_t s = stats == JABAS_STATS_FULL && K > 8 ? JABAS_SPLIT_MANYK : 0;
-    while ((2u << s) <= tiles && (n_chunks << s) < (stats ? JABAS_SPLIT_BELOW_STATS : JABAS_SPLIT_BELOW)) ++s;
+    const uint64_t below = stats ? JABAS_SPLIT_BELOW_STATS : JABAS_SPLIT_BELOW, empty = stats ? 64 : 256;
+    const auto pays = [&](uint32_t s) {
+        const uint64_t idle = (n_chunks << s) - live(s);
+        return (n_chunks << s) <= 256 || idle <= empty || 3 * idle <= live(s);
+    };
+    uint32_t s = stats == JABAS_STATS_FULL && K > 8 && (opt_class != 0 || grad_dtype == JABAS_F32) && pays(1) ? 1 : 0;
+    while ((2u << s) <= tiles && live(s) < below && pays(s + 1)) ++s;
     return s;
 }
 // Width of the partial rows of a launch: 4 similarity sums, + K norms, + K(K-1)/2 pair products.

@@ -98,15 +98,15 @@ def test_plan_encode_counts_chunks():
 
 @pytest.mark.parametrize("K,sizes,rows", [
     # rows of the level with the most workgroups: chunks of four tiles for full rows and K > 4, else two (similarity sums)
-    (8, [700] * 300, 300), (8, [5] * 511, 511), (16, [700] * 5000, 5000), (2, [1000] * 200, 200),      # one tile in every chunk
-    (8, [1500] * 200, 400), (16, [3000] * 3000, 6000),                   # two and three tiles
-    (8, [4096] * 200, 800), (8, [1 << 20], 512), (16, [1 << 24], 8192), (4, [1 << 18], 256),       # whole chunks
-    (8, [700] * 12, 48), (8, [5000], 8),                                 # a few empty workgroups are left
-    (8, [300] * 100 + [60000] * 27, 1010)])                              # 100 + 27 * 15 chunks, 910 of 1010 workgroups with a tile
+    (8, [700] * 200, 200), (8, [5] * 211, 211), (16, [700] * 5000, 5000), (2, [1000] * 210, 210),      # one tile in every chunk
+    (8, [1500] * 210, 420), (16, [3000] * 3000, 6000),                   # two and three tiles
+    (8, [4096] * 200, 400), (8, [1 << 20], 512), (16, [1 << 24], 8192), (4, [1 << 18], 256), (8, [4096] * 145, 580),       # whole chunks
+    (8, [700] * 12, 48), (8, [5000], 5 + 3), (8, [700] * 64, 256),       # empty workgroups on compute units that are left
+    (8, [300] * 50 + [60000] * 13, 490)])                                # 50 + 13 * 15 chunks, 440 of 490 workgroups with a tile
 def test_plan_splits_chunks_that_hold_tiles_for_it(K, sizes, rows):
-    """A launch with statistics shares its chunks between workgroups until there are 512 (full rows of more than eight workers:
-    always two), but not where more than a quarter of them would find no tile: scratch holds one row per workgroup. A blob
-    that does not record this (encoded before it was) is launched as it was."""
+    """A launch with statistics shares its chunks between workgroups until there are enough of them (full rows of more than eight
+    workers: always two), but not where more than a quarter of them would find no tile: scratch holds one row per workgroup. A
+    blob that does not record this (encoded before it was) is launched by the number of chunks alone."""
     lib = L.lib()
     rc, blob, _ = _encode([_span(n, K=K) for n in sizes], K=K)
     assert rc == L.OK
@@ -118,7 +118,7 @@ def test_plan_splits_chunks_that_hold_tiles_for_it(K, sizes, rows):
     for level, split in ((L.STATS_FULL, int(K > 8)), (L.STATS_SIMILARITY, 0)):
         n = lib.jabas_plan_chunks(blob.ctypes.data, level)
         tiles = 4 if K > 4 and level == L.STATS_FULL else 2
-        while 2 << split <= tiles and n << split < 512:
+        while 2 << split <= tiles and n << split < 384:
             split += 1
         unlimited.append(n << split)
     assert lib.jabas_plan_workspace_bytes(old.ctypes.data) == (max(unlimited) + stripes) * L.STATS_STRIDE * 8
