@@ -637,7 +637,7 @@ inline uint64_t live_workgroups(uint64_t tiles, uint32_t ct, uint32_t s) { retur
 uint32_t plan_split_log2(const PlanHeader& h, int stats) {
     const int v = shape_level(stats);
     const uint32_t recorded = h.split >> (8 * v) & 0xff;
-    if (recorded) return recorded - 1;
+    if (recorded && 1u << ((recorded - 1) & 31) <= h.shape[v].chunk_tiles && recorded <= 31) return recorded - 1;
     const uint64_t n = h.shape[v].n_chunks;
     return launch_split_log2(h.K, h.grad_dtype, opt_class_of(h.opt_kind), stats, n, [&](uint32_t s) { return n << s; });
 }

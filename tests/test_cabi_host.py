@@ -122,6 +122,9 @@ def test_plan_splits_chunks_that_hold_tiles_for_it(K, sizes, rows):
             split += 1
         unlimited.append(n << split)
     assert lib.jabas_plan_workspace_bytes(old.ctypes.data) == (max(unlimited) + stripes) * L.STATS_STRIDE * 8
+    for junk in (0x04040404, 0x20202020, 0x21212121, 0xffffffff):                # more workgroups than a chunk has tiles: not taken
+        old.view(np.uint32)[9] = junk
+        assert lib.jabas_plan_workspace_bytes(old.ctypes.data) == (max(unlimited) + stripes) * L.STATS_STRIDE * 8
 
 
 def test_plan_encode_starts_the_element_grid_at_a_256_byte_line_when_all_buffers_allow_it():
