@@ -251,9 +251,10 @@ def test_gnmt_embedding_rows_with_independent_masks(gpu):
 
 @pytest.mark.parametrize("K", [8, 13])
 def test_gram_bf16_long_span(gpu, K):
-    """bf16 Gram over a span long enough (2^28 + 77 elements) that every wave moves its fp32 running sums
-    into the fp64 sums several times before the last one. The K workers point at three distinct buffers
-    (the kernel only reads), so every entry is one of six dot products, which a float64 library reduction gives."""
+    """bf16 Gram over a span long enough (2^28 + 77 elements) that the waves move their fp32 running sums
+    into the fp64 sums on the way: K = 8 after 128 of 256 runs, K = 13 after 128, of which the first wave has
+    one more. The K workers point at three distinct buffers (the kernel only reads), so every entry is one of
+    six dot products, which a float64 library reduction gives."""
     from jabas_amd import sync
     n = (1 << 28) + 77
     gen = torch.Generator(device=gpu).manual_seed(99)

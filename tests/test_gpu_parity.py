@@ -297,15 +297,19 @@ def test_gram(gpu, K, dtype):
                                      (torch.float32, 6), (torch.float32, 8), (torch.float32, 12), (torch.float32, 13),
                                      (torch.float32, 16), (torch.bfloat16, 2), (torch.bfloat16, 5), (torch.bfloat16, 7)])
 def test_gram_at_the_edges_of_runs_and_routes(gpu, dtype, K):
-    """One element, one less and one more than a run of a wave (128 elements), starts inside a vector; then a full grid (1024
-    workgroups: 4096 waves, 2**18 threads): one vector more than it holds at a time, a third and a fourth run of the first
-    wave, with and without an end; and a worker with infinities and NaN reaches no product but its own (the first worker's
+    """One element, one less and one more than a run of a wave (128 elements), starts inside a vector; then a full grid: one run per
+    wave of 512 workgroups (2048 waves; fp32 matrix cores below 2**21 elements, with two sums, whose runs alternate) and of 1024,
+    one vector more than a grid of 2**18 threads holds at a time, a third and a fourth run of the first wave, with and without an
+    end; both sides of the line at 2**21 elements and a fifth round of runs beyond it; and a worker with infinities and NaN reaches no product but its own (the first worker's
     values stand in for the missing ones of a group of four). fp64 sums of n exact products in any order: n * 2**-53 *
     |g_a| |g_b| apart at most."""
     from jabas_amd import sync
-    grid = 1024 * 1024
-    for n, skew in ((1, 0), (1, 3), (127, 0), (128, 0), (129, 1), (253, 3), (257, 0), (4096 * 128 + 1, 0), (4097 * 128 + 3, 3),
-                    (grid + 1, 0), (grid + 128, 0), (grid + 129, 3), (grid + 4097 * 128 + 3, 1)):
+    grid, far = 1024 * 1024, 1 << 21
+    sizes = [(1, 0), (1, 3), (127, 0), (128, 0), (129, 1), (253, 3), (257, 0), (2048 * 128 + 1, 0), (2049 * 128 + 3, 3),
+             (4096 * 128 + 1, 0), (4097 * 128 + 3, 3), (grid + 1, 0), (grid + 128, 0), (grid + 129, 3), (grid + 4097 * 128 + 3, 1)]
+    if dtype == torch.float32 and K > 5:
+        sizes += [(far - 1, 0), (far - 1, 1), (far, 0), (far + 1, 3), (far + 4096 * 128 + 1, 0), (far + 4097 * 128 + 3, 3)]
+    for n, skew in sizes:
         hg = _host_grads(K, n, 70 + K, dtype=dtype)
         G = sync.gram([_dev(t, gpu, skew) for t in hg]).cpu()
         wide = torch.stack([t.double() for t in hg])
@@ -327,12 +331,17 @@ def test_gram_at_the_edges_of_runs_and_routes(gpu, dtype, K):
                                      (torch.float32, 16), (torch.bfloat16, 7), (torch.bfloat16, 8), (torch.bfloat16, 11), (torch.bfloat16, 13)])
 def test_gram_sum_of_the_workgroup_rows(gpu, dtype, K):
     """A workgroup of the finalize holds four entries and takes the rows in classes of 256: one row, one class short, full and
-    one over, three and four rows per class. Every entry of the 16 x 16 result is written: the product, mirrored, or zero
+    one over, two rows per class, and three and four where the launch has more than 512 workgroups (fp32 of six workers and more
+    only from 2**21 elements on); scratch that starts as NaN tells how many rows there were. Every entry of the 16 x 16 result is written: the product, mirrored, or zero
     beyond the workers. Integers of at most 3 in size: every product and sum is exact, in fp32 as in fp64."""
     from jabas_amd import sync, _lib as L
     ws = torch.empty(1024 * L.GRAM_STRIDE, dtype=torch.float64, device=gpu)
-    for rows in (1, 2, 255, 256, 257, 767, 769, 1023, 1024):
-        n = rows * 1024 - 5
+    sizes = [(rows, rows * 1024 - 5) for rows in (1, 2, 255, 256, 257, 511, 512)]
+    if dtype == torch.float32 and K > 5:
+        sizes.append((1024, (1 << 21) + 5))
+    elif K < (3 if dtype == torch.float32 else 13):
+        sizes += [(rows, rows * 1024 - 5) for rows in (767, 769, 1023, 1024)]
+    for rows, n in sizes:
         gen = torch.Generator().manual_seed(rows + K)
         hg = [torch.randint(-3, 4, (n,), generator=gen).to(dtype) for _ in range(K)]
         dg = [t.to(gpu) for t in hg]
@@ -344,6 +353,7 @@ def test_gram_sum_of_the_workgroup_rows(gpu, dtype, K):
         want = torch.zeros(L.GRAM_MAX_K, L.GRAM_MAX_K, dtype=torch.float64)
         want[:K, :K] = wide @ wide.t()
         assert torch.equal(out.cpu().view(L.GRAM_MAX_K, L.GRAM_MAX_K), want), f"K={K} rows={rows}"
+        assert int((~ws.view(1024, L.GRAM_STRIDE)[:, 0].isnan()).sum()) == rows
 
 
 @pytest.mark.parametrize("K", [8, 9, 12, 13, 16])
@@ -365,10 +375,11 @@ def test_gram_bf16_runs_and_ends(gpu, K):
         assert torch.equal(G, wide @ wide.t()), f"K={K} n={n} skew={skew}"
 
 
-@pytest.mark.parametrize("n", [(1 << 26) - 70, 1 << 26, (1 << 26) + 77])
+@pytest.mark.parametrize("n", [(1 << 26) - 70, 1 << 26, (1 << 26) + 77, 3 * (1 << 27) + 77])
 def test_gram_bf16_four_groups_of_very_long_spans(gpu, n):
     """Both sides of the line at 2**26 elements beyond which the kernel of thirteen and more bf16 workers takes the span's ends in
-    its loop, and its sums move to fp64 on the way. Integers: exact."""
+    its loop; and a span whose waves have 192 runs, so that their sums move to fp64 once on the way (after 128) and once at the
+    end. Integers: exact."""
     from jabas_amd import sync
     gen = torch.Generator(device=gpu).manual_seed(n)
     flat = [torch.randint(-3, 4, (n,), generator=gen, device=gpu, dtype=torch.int8).to(torch.bfloat16) for _ in range(3)]
@@ -1316,6 +1327,56 @@ def test_short_launches_give_the_result_of_whole_chunks(gpu, K, dtype, level, nu
         norms = torch.stack([(g.double() ** 2).sum() for g in grads])
         tol = 1e-12 if dtype == torch.float32 else 20 * 2.0 ** -24
         torch.testing.assert_close(ways[0][4][4:4 + K], norms, rtol=tol, atol=0.0)
+
+
+@pytest.mark.parametrize("K,dtype,kind,level", [
+    (2, torch.float32, "sgd", None), (4, torch.float32, "sgd", "similarity"), (4, torch.bfloat16, "sgd", None), (8, torch.float32, "sgd", "similarity"),
+    (1, torch.float32, "adam", "full"), (4, torch.bfloat16, "adamw_amsgrad", None), (8, torch.bfloat16, "adamw_amsgrad", "gram"),
+    (12, torch.bfloat16, "adamw", "full"), (16, torch.float32, "adam", "similarity"), (16, torch.bfloat16, None, "full"), (6, torch.float32, None, None)])
+@pytest.mark.parametrize("numel", [517, 2049, 90_001, 400_003])
+def test_split_launches_of_every_kind(gpu, K, dtype, kind, level, numel):
+    """Every optimizer, block size and level under a split: aggregate, weights and state against the first elements of a span too
+    long to be split, bit for bit; by value, as a plan of spans of unequal length (one of a single element, most shorter than a
+    chunk) and with the step's scalars in device memory."""
+    from jabas_amd import sync, _lib as L
+    far = numel + 4_000_000
+    gen = torch.Generator(device=gpu).manual_seed(numel + K)
+    grads = [torch.randn(far, generator=gen, device=gpu).to(dtype) for _ in range(K)]
+    start = [torch.randn(far, generator=gen, device=gpu) * 0.1 for _ in range(2)] + [torch.rand(far, generator=gen, device=gpu) * 0.1 for _ in range(2)]
+    n_state = {None: 0, "sgd": 2, "adam": 3, "adamw": 3, "adamw_amsgrad": 4}[kind]
+    opt = None if kind is None else dict(kind=kind.replace("_amsgrad", ""), amsgrad="amsgrad" in kind, momentum=0.9, betas=(0.9, 0.999),
+                                         eps=1e-8, groups=[dict(lr=1e-2, weight_decay=0.05)])
+
+    def launch(cuts, stats, dyn=False):
+        n = cuts[-1]
+        state, agg = [t[:n].clone() for t in start[:n_state]], torch.zeros(n, device=gpu)
+        args = sync.make_step_args((1,) * K, dtype, stats=stats or False, opt=opt, step=3)
+        if dyn:
+            scalars = sync.StepScalars(gpu)
+            scalars.update(args)
+            scalars.attach(args)
+        spans = [sync.SpanSpec([g[a:b] for g in grads], agg_out=agg[a:b], **dict(zip(("param", "state1", "state2", "state3"), (t[a:b] for t in state))))
+                 for a, b in zip(cuts, cuts[1:])]
+        if len(spans) > 1:
+            rows = sync.SyncPlan(spans, sync.opt_kind(opt)).run(args)
+        else:
+            rows = sync.sync_bucket(spans[0], args, workspace=sync.Workspace.for_span(n, dtype, gpu))
+        return [agg, *state], None if not stats else rows.reshape(-1, L.STATS_STRIDE).sum(0)
+
+    want, _ = launch((0, far), None)
+    ways = [launch((0, numel), level), launch((0, 256, 257, 300, 2 * numel // 3, numel), level)]
+    if kind in ("sgd", "adam", "adamw"):
+        ways.append(launch((0, numel), level, dyn=True))
+    for got, row in ways:
+        for x, y in zip(got, want):
+            assert torch.equal(x.view(torch.int32), y[:numel].view(torch.int32))
+        if level:
+            # fp32 gradients: fp64 sums; bf16 gradients: fp32 chains of at most 16 products per thread and 4 more over a row of lanes
+            tol = 1e-12 if dtype == torch.float32 else 20 * 2.0 ** -24
+            torch.testing.assert_close(row[3], (got[0].double() ** 2).sum(), rtol=tol, atol=0.0)
+            if level != "similarity":
+                norms = torch.stack([(g[:numel].double() ** 2).sum() for g in grads])
+                torch.testing.assert_close(row[4:4 + K], norms, rtol=tol, atol=0.0)
 
 
 @pytest.mark.parametrize("K,dtype,numel,levels", [(8, torch.bfloat16, 1_200_011, ("full", "gram")),
