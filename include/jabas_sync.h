@@ -217,7 +217,10 @@ int jabas_step_scalars_upload(const JabasStepArgs* args, void* scalars_dev, jaba
 
 /* Bytes of device workspace a single-span call (jabas_sync_bucket, jabas_stats) over
  * numel elements needs when statistics are requested: one partial row per workgroup of
- * the two-level reduction. No reference counterpart. */
+ * the two-level reduction. A call also takes less, down to one row of the level's width per
+ * chunk (jabas_plan_chunks) and 33 more; it then launches whole chunks, which is slower for short
+ * spans and adds the sums in another order: the last bits of the statistics depend on whether
+ * the scratch has this size. No reference counterpart. */
 size_t jabas_sync_workspace_bytes(uint64_t numel, int32_t grad_dtype);
 
 /* --- multi-span plan --------------------------------------------------------------
@@ -240,17 +243,21 @@ int jabas_plan_encode(const JabasSpan* spans, uint32_t n_span,
                       const JabasBound* bounds, uint32_t n_bounds,
                       int32_t K, int32_t grad_dtype, int32_t opt_kind,
                       void* host_blob, size_t blob_bytes);
-/* Number of workgroups (chunks) one launch of the plan uses at statistics level `stats`
- * (JABAS_STATS_*): the levels may run different workgroup shapes, the plan holds a chunk
- * table for each shape. Negative JabasStatus on a malformed blob or an unknown level. */
+/* Number of chunks of the plan at statistics level `stats` (JABAS_STATS_*): the levels may run
+ * different workgroup shapes, the plan holds a chunk table for each shape. A launch has one, two or
+ * four workgroups per chunk, recorded in the blob, by how many it takes to fill the GPU; a blob
+ * that does not record it is launched by the number of chunks. Negative JabasStatus on a malformed
+ * blob or an unknown level. */
 int64_t jabas_plan_chunks(const void* host_blob, int32_t stats);
 /* Bytes of device workspace jabas_sync_fused needs for this plan when statistics are
- * requested (0 on a malformed blob). */
+ * requested (0 on a malformed blob): a row per workgroup. Less is taken as by
+ * jabas_sync_bucket, see jabas_sync_workspace_bytes (32 rows more per span and one, not 33). */
 size_t jabas_plan_workspace_bytes(const void* host_blob);
 
 /* --- the fused sync step ------------------------------------------------------------
  * Aggregate + statistics + optimizer (+ fan-out) over every span of a plan, one
- * launch (plus a one-workgroup-per-span finalize launch when args->stats is set).
+ * launch (plus a launch that sums the workgroups' rows of every span when args->stats is set,
+ * two when a span has more than 4096).
  * stats_out: n_span * JABAS_STATS_STRIDE doubles (device), required when stats != 0.
  * A launch with statistics takes a plan of at most 65535 spans (JABAS_ERR_SIZE beyond,
  * returned before anything is launched); without statistics up to 2^24.
@@ -296,7 +303,8 @@ int jabas_sync_bucket(const JabasSpan* span, const JabasBound* bounds_dev,
  * five VSWs (rows of more than 4 + JABAS_MAX_K sums, wider than the array is sized for). All calls on one GPU share that GPU's
  * array: calls with statistics that overlap in time on one GPU (different streams or
  * threads) race on it and must be serialised by the caller; calls without statistics do
- * not touch it. Results are those of jabas_sync_bucket, bit for bit. */
+ * not touch it. Results are those of jabas_sync_bucket with a workspace of the size
+ * jabas_sync_workspace_bytes returns, bit for bit. */
 int jabas_sync_bucket_static(const JabasSpan* span, const JabasBound* bounds_dev,
                              const JabasStepArgs* args, double* stats_out,
                              jabas_stream_t stream);

@@ -26,9 +26,9 @@ constexpr uint32_t kPlanVersion = 8;
 // 1 full rows, 2 similarity sums). Levels whose shapes are the same share one table.
 struct PlanShape {
     uint32_t block;           // threads per workgroup the chunk table was cut for
-    uint32_t chunk_tiles;     // tiles per workgroup
-    uint32_t n_chunks;        // workgroups of one launch
-    uint32_t max_span_chunks; // chunks of the largest span (sizes the striped finalize)
+    uint32_t chunk_tiles;     // tiles per chunk
+    uint32_t n_chunks;        // chunks of one launch
+    uint32_t max_span_chunks; // chunks of the largest span (its rows choose the finalize's waves and stripes)
     uint64_t off_prefix, off_chunks;
 };
 struct PlanHeader {
@@ -333,7 +333,7 @@ const LaunchFn kLaunch[JABAS_MAX_K] = {launch_fused_k1,  launch_fused_k2,  launc
 //                    20 M elements, one span each, K = 1 42.8 -> 41.2, K = 4 full rows 142 -> 136
 //   batches          sixteen rows at once read rows beyond the last again where six are left (1500 rows 7.5 -> 6.5 us): eight too
 constexpr int kFinalizeSlots = 4;
-constexpr uint32_t kStripeRows = 512;
+constexpr uint32_t kStripeRows = 512;         // partial rows of a stripe, more where there are kMaxStripes of them
 constexpr uint32_t kMaxStripes = 32;
 constexpr uint32_t kMaxStatsSpans = 65535;    // spans index a dimension of the finalize grid
 // Up to here one launch: one batch of sixteen waves. Rows of 4 doubles, whole call, one launch / two: 4000 9.9 / 10.8 us,
@@ -455,8 +455,8 @@ inline uint32_t stripes_for(uint32_t max_rows) {
     const uint32_t st = (max_rows + kStripeRows - 1) / kStripeRows;
     return st > kMaxStripes ? kMaxStripes : st;
 }
-// workspace rows: one per chunk, then one per (span, stripe)
-constexpr size_t workspace_rows(uint64_t n_chunks, uint64_t n_span) { return n_chunks + n_span * kMaxStripes + 1; }
+// workspace rows: one per workgroup, then one per (span, stripe)
+constexpr size_t workspace_rows(uint64_t workgroups, uint64_t n_span) { return workgroups + n_span * kMaxStripes + 1; }
 
 // One wave: fixed-order sum of slot NORM_AGG over the rows, then the coefficient.
 __global__ void __launch_bounds__(64) clip_coef_kernel(const double* rows, uint32_t n_rows, double max_norm, double eps,
@@ -600,8 +600,8 @@ JABAS_API int jabas_step_scalars_upload(const JabasStepArgs* args, void* scalars
 }
 
 JABAS_API size_t jabas_sync_workspace_bytes(uint64_t numel, int32_t grad_dtype) {
-    // chunks of a single span whose first element may sit anywhere in the line the grid starts at,
-    // under the launch shape with the smallest chunks
+    // workgroups of a single span whose first element may sit anywhere in the line the grid starts at: kMinChunkElems is a
+    // tile of the launches with statistics too
     (void)grad_dtype;
     const uint64_t chunks = (numel + kWideElems - 1 + kMinChunkElems - 1) / kMinChunkElems;
     return workspace_rows(chunks, 1) * kStatsStride * sizeof(double);
@@ -860,7 +860,7 @@ JABAS_API int jabas_sync_bucket(const JabasSpan* span, const JabasBound* bounds_
 // made with that device current.
 namespace {
 constexpr uint64_t kStaticMaxNumel = JABAS_STATIC_MAX_NUMEL;
-constexpr uint64_t kStaticMinChunkElems = kMinStatsChunkElems;    // one partial row per chunk of a statistics launch
+constexpr uint64_t kStaticMinChunkElems = kMinStatsChunkElems;    // one partial row per chunk of a statistics launch, or more that fit
 constexpr int kStaticRowDoubles = 4 + JABAS_MAX_K;            // the widest rows it serves: full rows of 16 VSWs
 constexpr size_t kStaticScratchBytes =
     workspace_rows((kStaticMaxNumel + kWideElems - 1 + kStaticMinChunkElems - 1) / kStaticMinChunkElems, 1) *

@@ -3,7 +3,8 @@
 // streams are fully unrolled into independent 128-bit loads.
 //
 // Execution shape
-//   - one workgroup per chunk of consecutive tiles of one span; a tile is one 16-byte vector of
+//   - one workgroup per chunk of consecutive tiles of one span, two or four where that leaves compute
+//     units idle (launch_split_log2); a tile is one 16-byte vector of
 //     every fp32 buffer (one 8-byte vector of a bf16 gradient buffer) per thread. Threads per
 //     workgroup and tiles per chunk depend on the kernel family (launch_block / launch_chunk_tiles):
 //     256 threads x 2 or 4 tiles with statistics, 128 x 2, 256 x 2 or 256 x 4 without. Small,
@@ -457,7 +458,7 @@ __device__ __forceinline__ void span_range(const SP& sp, uint32_t lt0, uint32_t 
             const uint64_t fit = (stretch_end - e0) / TE;
             const uint32_t left = lt1 - lt;
             nfull = fit < left ? static_cast<uint32_t>(fit) : left;
-            __builtin_assume(nfull <= CT);       // lt1 - lt0 is a chunk's share: the cascade below has at most CT / U rounds
+            __builtin_assume(nfull <= CT);       // a workgroup's tiles are a chunk's or a part of them: one worker's statistics +5-10 %
         }
         if (nfull) {
             const GroupDev G = a.groups[gid];

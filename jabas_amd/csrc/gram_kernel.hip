@@ -347,8 +347,10 @@ __global__ void __launch_bounds__(kBlock) gram_mfma_kernel(const SpanDev sp, int
 // the operands: no widening, no conversion, one instruction per pair of groups and four elements of every
 // lane. A lane loads 16 bytes (two operands) per group; a wave reads 256 contiguous bytes of each worker.
 // Products of bf16 values are exact in fp32; the instruction adds four of them to an fp32 running sum, which
-// is moved into fp64 sums (LDS, per wave) after at most kGramBf16FlushRuns runs, i.e. after at most
-// 4 * 2 * kGramBf16FlushRuns elements of either of its two blocks (and those of the span's ends): fp32 rounding stays near 1e-6 of |g_a| |g_b|, the order is fixed.
+// is moved into fp64 sums (LDS, per wave) after at most kGramBf16FlushRuns runs. A sum then holds at most 4 * 2 * (U / S) *
+// kGramBf16FlushRuns products (U blocks of a run go to S sums; two vectors of four per block) and, in the first of them, those of
+// the span's ends: 1024 to 2048, 4096 in the shape of four groups and very long spans. fp32 rounding stays near 1e-6 of
+// |g_a| |g_b|, the order is fixed.
 // Lanes beyond the last worker multiply worker 0's values into entries the finalize never reads.
 template <int CTRL> __device__ __forceinline__ float gram_dpp_f32(float v) {
     return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, false));

@@ -11,7 +11,8 @@
 namespace jabas {
 
 // Launch shape: threads per workgroup and tiles per workgroup (a tile = one 16-byte fp32 vector per
-// thread; a chunk = the tiles one workgroup processes). Small chunks keep the streamed window of every
+// thread; a chunk = consecutive tiles of a span, the share of one workgroup or, where that leaves compute
+// units idle, of two or four: launch_split_log2). Small chunks keep the streamed window of every
 // buffer compact (higher HBM rate) and cut the ramp-up / drain of a launch; kernels that carry many
 // statistics have low occupancy and a long epilogue, and do better with more work per workgroup.
 // Measured per kernel family (A/B builds of the whole library, every shape passes the parity suite):
@@ -97,8 +98,8 @@ __host__ __device__ constexpr int shape_level(int stats) { return stats == JABAS
 //                       products 0.9 M 0.90 of the time of whole chunks against 0.74
 //   without a tile      at most a quarter, or 64 with statistics (each still runs its epilogue and writes a row) and 256 without, or as
 //                       many as there are compute units for: plans over short spans, one per small tensor, whose last chunk is
-//                       mostly their only one. All splits -> these: 500 spans of 700 elements, K = 1 AdamW 7.7 -> 4.4 us, 5000, K = 16
-//                       bf16 full rows 88.5 -> 52.0
+//                       mostly their only one. All splits -> these: 500 spans of 700 elements, K = 1 AdamW 7.7 -> 4.4 us, 20000, K = 16
+//                       bf16 full rows 651 -> 502 (193 with the finalize of short spans)
 //   full rows, K > 8    two workgroups per chunk at any size: these kernels hold one tile in flight and two or three waves per
 //                       SIMD, and half the work per workgroup keeps the streamed window compact and the last round of
 //                       workgroups short: ResNet-50 K = 16 bf16 254 -> 231 us (four: 240), 25 M elements K = 12 fp32 SGD
@@ -141,10 +142,12 @@ inline int shared_row_width(int K, int grad_dtype, int opt_class, int stats) {
     return width;
 }
 constexpr int imin(int a, int b) { return a < b ? a : b; }
-// Fewest elements a chunk of a launch with statistics covers (one partial row per chunk): sizes workspaces.
+// Fewest elements a chunk of a launch with statistics covers: one partial row per chunk at least, sizes the static scratch, in
+// which only launches short enough to leave room are split.
 constexpr int kMinStatsChunkElems = 4 * imin(imin(JABAS_BLOCK * JABAS_CHUNK_TILES_LO, JABAS_BLOCK * JABAS_CHUNK_TILES_SIM_LO),
                                              JABAS_BLOCK_SIM_MANYK * JABAS_CHUNK_TILES_SIM_MANYK);
-// Fewest elements any chunk covers, over all shapes: sizes blobs that must fit every launch.
+// Fewest elements any chunk covers, over all shapes: sizes blobs that must fit every launch, and workspaces (a tile of a launch
+// with statistics, the least its workgroups take, is as long).
 constexpr int kMinChunkElems = imin(imin(kMinStatsChunkElems, 4 * JABAS_BLOCK_SGD * JABAS_CHUNK_TILES_LO),
                                     4 * imin(imin(JABAS_BLOCK * JABAS_CHUNK_TILES_PLAIN_LO, JABAS_BLOCK * JABAS_CHUNK_TILES_LO),
                                              imin(JABAS_BLOCK_MANYK * JABAS_CHUNK_TILES_MANYK, JABAS_BLOCK * JABAS_CHUNK_TILES_HI)));
@@ -209,7 +212,7 @@ struct OptDev {
     int32_t has_momentum, first_step, nesterov, adamw;
 };
 
-// One workgroup's share of a planned launch: chunk_tiles consecutive tiles of one span.
+// chunk_tiles consecutive tiles of one span of a planned launch.
 struct ChunkDesc {
     uint32_t span;                           // index into the span table
     uint32_t tile0;                          // first tile, local to the span
@@ -219,15 +222,15 @@ struct ChunkDesc {
 
 struct KArgs {
     const SpanDev* spans;                    // device table (planned launch)
-    const ChunkDesc* chunks;                 // one per workgroup (planned launch)
+    const ChunkDesc* chunks;                 // one per 2^split_log2 workgroups (planned launch)
     const uint32_t* chunk_prefix;            // n_span + 1 entries: first chunk of each span (planned launch)
     const BoundDev* bounds;                  // device, may be NULL
-    double* partials;                        // one row of kStatsStride doubles per workgroup
+    double* partials;                        // one row of the level's width per workgroup
     const float* grad_scale;                 // device scalar or NULL (clipping)
     uint32_t n_span;
     uint32_t n_chunks;
-    uint32_t chunk_tiles;                    // tiles per workgroup (the kernel's own shape; checked on the host)
-    uint32_t use_inline;                     // 1: the only span is `span0`, chunk b starts at tile b*chunk_tiles
+    uint32_t chunk_tiles;                    // tiles per chunk (the kernel's own shape; checked on the host)
+    uint32_t use_inline;                     // 1: the only span is `span0`, workgroup b starts at tile b * (chunk_tiles >> split_log2)
     uint32_t half_mask;                      // bit k set: VSW k belongs to half B
     uint32_t split_log2;                     // 2^split_log2 workgroups share a chunk (launch_split_log2)
     SpanDev span0;
