@@ -388,7 +388,7 @@ def time_config(cfg, device, steps, warmup, torch, extras=True):
             from jabas_amd import sync
             ms, _ = timed_region(lambda i: engines[i % n].step(stats="gram"), steps, warmup, torch)
             res["step_with_worker_gram_in_the_launch"] = rate(bytes_per_step, ms)
-            gws = torch.empty(1056 * 256, dtype=torch.float64, device=device)
+            gws = torch.empty(1024 * 256, dtype=torch.float64, device=device)
 
             def step_then_gram(i):
                 engines[i % n].step(stats="full")
