@@ -639,7 +639,7 @@ uint32_t plan_split_log2(const PlanHeader& h, int stats) {
     const uint32_t recorded = h.split >> (8 * v) & 0xff;
     if (recorded && 1u << ((recorded - 1) & 31) <= h.shape[v].chunk_tiles && recorded <= 31) return recorded - 1;
     const uint64_t n = h.shape[v].n_chunks;
-    return launch_split_log2(h.K, h.grad_dtype, opt_class_of(h.opt_kind), stats, n, [&](uint32_t s) { return n << s; });
+    return launch_split_log2(h.K, h.grad_dtype, opt_class_of(h.opt_kind), stats, n, h.n_bounds > h.n_span, [&](uint32_t s) { return n << s; });
 }
 }  // namespace
 
@@ -742,6 +742,8 @@ JABAS_API int jabas_plan_encode(const JabasSpan* spans, uint32_t n_span, const J
         prefix[n_span] = c;
         if (c != ps.n_chunks) return JABAS_ERR_PLAN;
     }
+    bool group_changes = false;
+    for (uint32_t i = 0; i < n_span; ++i) group_changes |= spans[i].numel && spans[i].bound_count > 1;
     for (int v = 0; v < 3; ++v) {
         if (table_of[v] != v) h.shape[v] = h.shape[table_of[v]];
         const auto live = [&](uint32_t s) {
@@ -750,7 +752,7 @@ JABAS_API int jabas_plan_encode(const JabasSpan* spans, uint32_t n_span, const J
                 n += live_workgroups(tiles_of(sd[i].hi, static_cast<int>(h.shape[v].block)), h.shape[v].chunk_tiles, s);
             return n;
         };
-        h.split |= (1u + launch_split_log2(K, grad_dtype, oc, v, h.shape[v].n_chunks, live)) << (8 * v);
+        h.split |= (1u + launch_split_log2(K, grad_dtype, oc, v, h.shape[v].n_chunks, group_changes, live)) << (8 * v);
     }
     if (n_bounds) memcpy(base + h.off_bounds, bounds, static_cast<size_t>(n_bounds) * sizeof(JabasBound));
     memcpy(base, &h, sizeof(h));
@@ -848,7 +850,7 @@ JABAS_API int jabas_sync_bucket(const JabasSpan* span, const JabasBound* bounds_
     a.chunk_tiles = launch_chunk_tiles(args->K, args->grad_dtype, oc, stats);
     a.n_chunks = static_cast<uint32_t>(chunks_of_tiles(tiles, a.chunk_tiles));
     a.use_inline = 1;
-    a.split_log2 = launch_split_log2(args->K, args->grad_dtype, oc, stats, a.n_chunks,
+    a.split_log2 = launch_split_log2(args->K, args->grad_dtype, oc, stats, a.n_chunks, span->bound_count > 1,
                                      [&](uint32_t s) { return live_workgroups(tiles, a.chunk_tiles, s); });
     return run_fused(a, args, tiles, a.n_chunks, stats_out, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
 }

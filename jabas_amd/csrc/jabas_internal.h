@@ -88,14 +88,19 @@ __host__ __device__ constexpr int launch_chunk_tiles(int K, int /*grad_dtype*/, 
 // Statistics level whose launch shape (and chunk table of a plan) a level uses.
 __host__ __device__ constexpr int shape_level(int stats) { return stats == JABAS_STATS_GRAM ? JABAS_STATS_FULL : stats; }
 // log2 of the workgroups that share a chunk of a launch of n_chunks chunks, live(s) of them with a tile to work on at split s: a
-// plan's tables know whole chunks only, the launch decides how many workgroups each of them gets. All figures: spans by value
-// over buffers that rotate through more than the last-level cache; one set of buffers that stays there misleads.
+// plan's tables know whole chunks only, the launch decides how many workgroups each of them gets. All figures: spans of one
+// parameter group by value (unless stated) over buffers that rotate through more than the last-level cache; one set of buffers
+// that stays there misleads.
 //   short launches      below about 400 workgroups compute units idle and a workgroup takes its tiles in turn, each at the latency
 //                       of memory. Whole chunks -> split: fp32 K = 4 AdamW 0.1 / 0.5 / 1.5 M elements 7.4 / 8.2 / 13.0 -> 4.1 / 6.0 /
 //                       10.6 us, bf16 K = 8 AdamW full rows 0.1 / 0.5 M 12.0 / 13.1 -> 7.8 / 10.2. Split while there are fewer than
-//                       2048 without statistics, as it was, 1 to 4 M elements lose: K = 4 AdamW 2 / 3 / 4 M 17.9 / 25.1 / 32.7 ->
-//                       19.0 / 27.5 / 35.8, K = 8 bf16 aggregate 4 M 15.4 -> 18.0; while fewer than 512, 2 M 18.9, and K = 8 pair
-//                       products 0.9 M 0.90 of the time of whole chunks against 0.74
+//                       2048 without statistics, 1 to 4 M elements lose: K = 4 AdamW 2 / 3 / 4 M 17.9 / 25.1 / 32.7 -> 19.0 / 27.5 /
+//                       35.8, K = 8 bf16 aggregate 4 M 15.4 -> 18.0; while fewer than 512, 2 M 18.9, and K = 8 pair products 0.9 M
+//                       0.90 of the time of whole chunks against 0.74
+//   group changes       in a span (norms and biases between the weights): up to 2048 and 512. A tile with a change takes the careful
+//                       path, three others of its workgroup wait for it, and the slowest workgroups make the launch. Engine steps,
+//                       up to 448 -> up to 2048: K = 2 fp32 AdamW 2.3 M in 293 tensors 26.1 -> 20.0 us, K = 1 4.0 M in 85 30.5 -> 25.7, K = 4
+//                       6.4 M in 117 71.1 -> 66.1, K = 4 3.0 M in 23 26.1 -> 24.9; K = 6 full rows 1.0 M in 153 20.7 -> 18.6
 //   without a tile      at most a quarter, or 64 with statistics (each still runs its epilogue and writes a row) and 256 without, or as
 //                       many as there are compute units for: plans over short spans, one per small tensor, whose last chunk is
 //                       mostly their only one. All splits -> these: 500 spans of 700 elements, K = 1 AdamW 7.7 -> 4.4 us, 20000, K = 16
@@ -112,10 +117,18 @@ __host__ __device__ constexpr int shape_level(int stats) { return stats == JABAS
 #ifndef JABAS_SPLIT_BELOW_STATS
 #define JABAS_SPLIT_BELOW_STATS 384
 #endif
+#ifndef JABAS_SPLIT_BELOW_GROUPS
+#define JABAS_SPLIT_BELOW_GROUPS 2048
+#endif
+#ifndef JABAS_SPLIT_BELOW_GROUPS_STATS
+#define JABAS_SPLIT_BELOW_GROUPS_STATS 512
+#endif
 template <class Live>
-inline uint32_t launch_split_log2(int K, int grad_dtype, int opt_class, int stats, uint64_t n_chunks, const Live& live) {
+inline uint32_t launch_split_log2(int K, int grad_dtype, int opt_class, int stats, uint64_t n_chunks, bool group_changes, const Live& live) {
     const uint32_t tiles = static_cast<uint32_t>(launch_chunk_tiles(K, grad_dtype, opt_class, stats));
-    const uint64_t below = stats ? JABAS_SPLIT_BELOW_STATS : JABAS_SPLIT_BELOW, empty = stats ? 64 : 256;
+    const uint64_t below = group_changes ? (stats ? JABAS_SPLIT_BELOW_GROUPS_STATS : JABAS_SPLIT_BELOW_GROUPS)
+                                         : (stats ? JABAS_SPLIT_BELOW_STATS : JABAS_SPLIT_BELOW);
+    const uint64_t empty = stats ? 64 : 256;
     const auto pays = [&](uint32_t s) {
         const uint64_t idle = (n_chunks << s) - live(s);
         return (n_chunks << s) <= 256 || idle <= empty || 3 * idle <= live(s);

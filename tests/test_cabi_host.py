@@ -127,6 +127,19 @@ def test_plan_splits_chunks_that_hold_tiles_for_it(K, sizes, rows):
         assert lib.jabas_plan_workspace_bytes(old.ctypes.data) == (max(unlimited) + stripes) * L.STATS_STRIDE * 8
 
 
+@pytest.mark.parametrize("groups,rows", [((0,), 450), ((0, 1), 900)])
+def test_plan_splits_further_where_parameter_groups_change(groups, rows):
+    """Tiles with a change of parameter group hold up the others of their workgroup: 450 chunks are shared where there are any
+    (up to 512 with statistics), not where there are none (up to 384)."""
+    lib = L.lib()
+    span = _span(900 * 1024, K=4, opt=True)
+    span.bound_count = len(groups)
+    bounds = [(i * 70_001, g) for i, g in enumerate(groups)]
+    rc, blob, _ = _encode([span], bounds, K=4, opt=L.OPT_SGD)
+    assert rc == L.OK and lib.jabas_plan_chunks(blob.ctypes.data, L.STATS_FULL) == 450
+    assert lib.jabas_plan_workspace_bytes(blob.ctypes.data) == (rows + 33) * L.STATS_STRIDE * 8
+
+
 def test_plan_encode_starts_the_element_grid_at_a_256_byte_line_when_all_buffers_allow_it():
     """2048 elements per workgroup here (K = 2, no optimizer). With every buffer 61 elements into a
     256-byte line the grid starts at that line: 61 + 4036 elements still fit two workgroups, one
