@@ -37,11 +37,12 @@ struct PlanHeader {
     int32_t K, grad_dtype, opt_kind;
     uint32_t max_group;       // largest group index any bound names
     uint32_t all_have_s1;     // every non-empty span carries a state1 pointer
-    uint32_t split;           // byte v: 1 + split_log2 of launches of shape v (launch_split_log2); 0: not recorded
+    uint32_t split;           // byte v < 3: 1 + split_log2 of launches of shape v (launch_split_log2); 0: not recorded. Bit 24: a span's aggregate is written
     PlanShape shape[3];
     uint64_t off_spans, off_bounds, total_bytes;
 };
 static_assert(sizeof(PlanShape) == 32 && sizeof(PlanHeader) == 160, "plan header layout");
+constexpr uint32_t kPlanWritesAgg = 1u << 24;
 constexpr size_t kHeaderBytes = 160;
 static_assert(kHeaderBytes >= sizeof(PlanHeader) && kHeaderBytes % 16 == 0, "plan header slot");
 
@@ -742,8 +743,12 @@ JABAS_API int jabas_plan_encode(const JabasSpan* spans, uint32_t n_span, const J
         prefix[n_span] = c;
         if (c != ps.n_chunks) return JABAS_ERR_PLAN;
     }
-    bool group_changes = false;
-    for (uint32_t i = 0; i < n_span; ++i) group_changes |= spans[i].numel && spans[i].bound_count > 1;
+    bool group_changes = false, writes_agg = false;
+    for (uint32_t i = 0; i < n_span; ++i) {
+        group_changes |= spans[i].numel && spans[i].bound_count > 1;
+        writes_agg |= spans[i].numel && spans[i].agg_out;
+    }
+    h.split |= writes_agg ? kPlanWritesAgg : 0u;
     for (int v = 0; v < 3; ++v) {
         if (table_of[v] != v) h.shape[v] = h.shape[table_of[v]];
         const auto live = [&](uint32_t s) {
@@ -821,6 +826,7 @@ JABAS_API int jabas_sync_fused(const void* plan_host, const void* plan_dev, cons
     a.n_chunks = ps.n_chunks;
     a.chunk_tiles = ps.chunk_tiles;
     a.use_inline = 0;
+    a.writes_agg = (h.split & kPlanWritesAgg) != 0;
     a.split_log2 = plan_split_log2(h, stats);
     return run_fused(a, args, 0, ps.max_span_chunks, stats_out, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
 }
@@ -850,6 +856,7 @@ JABAS_API int jabas_sync_bucket(const JabasSpan* span, const JabasBound* bounds_
     a.chunk_tiles = launch_chunk_tiles(args->K, args->grad_dtype, oc, stats);
     a.n_chunks = static_cast<uint32_t>(chunks_of_tiles(tiles, a.chunk_tiles));
     a.use_inline = 1;
+    a.writes_agg = span->agg_out != nullptr;
     a.split_log2 = launch_split_log2(args->K, args->grad_dtype, oc, stats, a.n_chunks, span->bound_count > 1,
                                      [&](uint32_t s) { return live_workgroups(tiles, a.chunk_tiles, s); });
     return run_fused(a, args, tiles, a.n_chunks, stats_out, workspace, workspace_bytes, static_cast<hipStream_t>(stream));

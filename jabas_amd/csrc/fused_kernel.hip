@@ -13,9 +13,9 @@
 //     persistent grid that spreads over the whole buffers;
 //   - every global access is a vector access with the nontemporal hint (each byte is touched
 //     exactly once per step);
-//   - tiles that lie wholly inside the live range of a span and inside one parameter
-//     group take the vector path (all loads of U tiles issued before any arithmetic);
-//     the few tiles that straddle a span end or a group change take a scalar path;
+//   - tiles that lie wholly inside the live range of a span take the vector path (all loads of U tiles issued
+//     before any arithmetic, the parameter group looked up while they are under way); a tile that straddles a span
+//     end, or is the only one left, goes wave by wave (single_tile);
 //   - statistics: per-thread fp64 accumulators -> LDS -> 16-way sums in fixed order -> DPP row
 //     reduction -> one partial row of 4 + K doubles per workgroup in the workspace, summed in
 //     fixed order by the finalize kernel. The order is fixed, so results are bit-identical run to run.
@@ -69,11 +69,15 @@ template <> struct Grad<JABAS_F32> {
     template <bool NARROW> static __device__ __forceinline__ Raw load(const void* base, uint64_t e) {
         return __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(elem_addr<NARROW, 4>(base, e)));
     }
-    static __device__ __forceinline__ void widen(const Raw& r, float (&x)[4]) {
-        x[0] = r.x; x[1] = r.y; x[2] = r.z; x[3] = r.w;
-    }
-    static __device__ __forceinline__ float load1(const void* base, uint64_t e) {
-        return static_cast<const float*>(base)[e];
+    static __device__ __forceinline__ float elem(const Raw& r, int i) { return r[i]; }
+    // elements at byte addresses of one stream, the live ones of a vector that straddles a span end
+    static __device__ __forceinline__ Raw gather(const char* const (&at)[4], const bool (&live)[4]) {
+        Raw r;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) r[i] = *reinterpret_cast<const float*>(at[i]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) r[i] = live[i] ? r[i] : 0.0f;
+        return r;
     }
 };
 
@@ -84,12 +88,17 @@ template <> struct Grad<JABAS_BF16> {
         return __builtin_nontemporal_load(reinterpret_cast<const u32x2*>(elem_addr<NARROW, 2>(base, e)));
     }
     // bf16 -> fp32 is exact: the 16 bits become the high half of the fp32 pattern.
-    static __device__ __forceinline__ void widen(const Raw& r, float (&x)[4]) {
-        x[0] = bits_to_float(r.x << 16); x[1] = bits_to_float(r.x & 0xffff0000u);
-        x[2] = bits_to_float(r.y << 16); x[3] = bits_to_float(r.y & 0xffff0000u);
+    static __device__ __forceinline__ float elem(const Raw& r, int i) {
+        const uint32_t w = i < 2 ? r.x : r.y;
+        return bits_to_float(i & 1 ? w & 0xffff0000u : w << 16);
     }
-    static __device__ __forceinline__ float load1(const void* base, uint64_t e) {
-        return bits_to_float(static_cast<uint32_t>(static_cast<const uint16_t*>(base)[e]) << 16);
+    static __device__ __forceinline__ Raw gather(const char* const (&at)[4], const bool (&live)[4]) {
+        uint32_t h[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) h[i] = *reinterpret_cast<const uint16_t*>(at[i]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) h[i] = live[i] ? h[i] : 0u;
+        return Raw{h[0] | (h[1] << 16), h[2] | (h[3] << 16)};
     }
 };
 
@@ -99,7 +108,7 @@ __host__ __device__ constexpr bool is_adam(int opt) { return opt == OPT_ADAM || 
 // on the ViT-L/16 set, K = 8 bf16: +0.5 % with full rows, +2 % with similarity sums; K = 4 fp32 Adam: 8-9 fewer
 // VGPRs, full rows 131 -> 123 and 4 waves per SIMD instead of 3, ViT-B/16 +1.2 % with similarity sums, +0.4 % with
 // full rows, GNMT +-0.3 %); their spans that 32-bit byte offsets do not reach (over 4 GiB of fp32 per buffer)
-// go through the careful path tile by tile: correct but slower. The plain kernels keep 64-bit vector addresses
+// go tile by tile (single_tile): correct but slower. The plain kernels keep 64-bit vector addresses
 // (no gain there: their registers are not what limits them).
 __host__ __device__ constexpr bool narrow_addressing(int /*K*/, int SL) { return SL != 0; }
 
@@ -201,23 +210,26 @@ __device__ __forceinline__ void opt_elem(float g, float& p, float& s1, float& s2
     }
 }
 
-// Aggregate, statistics and optimizer for N consecutive elements held in registers.
-template <int K, int N, int DT, int OPT, int SL, bool HD, class A>
-__device__ __forceinline__ void compute(const float (&g)[K][N], float (&p)[N], float (&s1)[N],
-                                        float (&s2)[N], float (&s3)[N], float (&agg)[N], const A& a,
-                                        const GroupDev& G, float clip, typename StatAcc<DT>::type (&acc)[NStats<K, SL>::value]) {
+// Aggregate and statistics of a thread's four elements of a tile, out of the vectors as loaded. They are widened one element
+// at a time: all four at once keep 4 K floats alive beside the vectors.
+template <int K, int DT, int SL, bool HD, class A>
+__device__ __forceinline__ void aggregate(const typename Grad<DT>::Raw (&raw)[K], float (&agg)[4], const A& a, float clip,
+                                          typename StatAcc<DT>::type (&acc)[NStats<K, SL>::value]) {
 #pragma unroll
-    for (int i = 0; i < N; ++i) {
-        float s = g[0][i] * a.w[0];
+    for (int i = 0; i < 4; ++i) {
+        float g[K];
 #pragma unroll
-        for (int k = 1; k < K; ++k) s = s + g[k][i] * a.w[k];
+        for (int k = 0; k < K; ++k) g[k] = Grad<DT>::elem(raw[k], i);
+        float s = g[0] * a.w[0];
+#pragma unroll
+        for (int k = 1; k < K; ++k) s = s + g[k] * a.w[k];
         if (clip < 1.0f) s = s * clip;         // global-norm clipping: only ever scales down
         agg[i] = s;
         if constexpr (SL) {
             float ga = 0.0f, gb = 0.0f;
 #pragma unroll
             for (int k = 0; k < K; ++k) {
-                const float t = g[k][i] * a.wh[k];
+                const float t = g[k] * a.wh[k];
                 if constexpr (HD) {            // default halves: even worker -> A, odd -> B
                     if (k & 1) gb = gb + t; else ga = ga + t;
                 } else {
@@ -226,11 +238,11 @@ __device__ __forceinline__ void compute(const float (&g)[K][N], float (&p)[N], f
                     ga = in_b ? ga : ga + t;
                 }
                 if constexpr (per_vsw_norms(SL))
-                    acc[JABAS_STAT_NORM_VSW0 + k] = stat_fma(g[k][i], g[k][i], acc[JABAS_STAT_NORM_VSW0 + k]);
+                    acc[JABAS_STAT_NORM_VSW0 + k] = stat_fma(g[k], g[k], acc[JABAS_STAT_NORM_VSW0 + k]);
                 if constexpr (SL == JABAS_STATS_GRAM) {
 #pragma unroll
                     for (int b = k + 1; b < K; ++b)
-                        acc[JABAS_STAT_PAIR(K, k, b)] = stat_fma(g[k][i], g[b][i], acc[JABAS_STAT_PAIR(K, k, b)]);
+                        acc[JABAS_STAT_PAIR(K, k, b)] = stat_fma(g[k], g[b], acc[JABAS_STAT_PAIR(K, k, b)]);
                 }
             }
             // fp64 sums: fp32 x fp32 products are exact in fp64, so fma == mul followed by add there.
@@ -238,184 +250,275 @@ __device__ __forceinline__ void compute(const float (&g)[K][N], float (&p)[N], f
             acc[JABAS_STAT_NORM_A] = stat_fma(ga, ga, acc[JABAS_STAT_NORM_A]);
             acc[JABAS_STAT_NORM_B] = stat_fma(gb, gb, acc[JABAS_STAT_NORM_B]);
             acc[JABAS_STAT_NORM_AGG] = stat_fma(s, s, acc[JABAS_STAT_NORM_AGG]);
+            // keep the elements' dependency chains apart: interleaving them costs the statistics
+            // kernels a third of their occupancy in registers and buys nothing in a memory-bound loop
+            __builtin_amdgcn_sched_barrier(0);
         }
-        if constexpr (OPT != OPT_NONE) opt_elem<OPT>(s, p[i], s1[i], s2[i], s3[i], G, a.opt);
-        // keep the elements' dependency chains apart: interleaving them costs the statistics
-        // kernels a third of their occupancy in registers and buys nothing in a memory-bound loop
-        if constexpr (SL) __builtin_amdgcn_sched_barrier(0);
     }
 }
 
-template <int NV, bool NARROW> __device__ __forceinline__ void load_vec(f32x4 (&r)[NV], const float* base, uint64_t e) {
+// The parameter group a wave is in, in scalar registers: entry j of the span's bound table, which ends at element `end` of the
+// span. Looked up while the loads of the wave's elements are under way, not before they are issued: a table read is a trip to
+// memory for the first waves of a launch.
+template <bool SEARCH> struct GroupCursor {
+    ConstBounds bd;
+    uint32_t nb, j;
+    uint64_t end;                                // 0: not looked up yet
+    GroupDev g;
+    // moves on to the group of element rel >= end. SEARCH: j is not known to be near (a span by value has no chunk table).
+    template <class A> __device__ __forceinline__ void seek(uint64_t rel, const A& a) {
+        if (SEARCH && end == 0) {                // largest j with bd[j].start <= rel
+            uint32_t lo = 0, hi = nb;
+            while (hi - lo > 1) {
+                const uint32_t mid = (lo + hi) >> 1;
+                if (bd[mid].start <= rel) lo = mid; else hi = mid;
+            }
+            j = lo;
+        }
+        while (j + 1 < nb && bd[j + 1].start <= rel) ++j;
+        g = a.groups[nb ? bd[j].group & (JABAS_MAX_GROUPS - 1) : 0];     // a bound table on the device cannot be checked by the host
+        end = j + 1 < nb ? bd[j + 1].start : ~static_cast<uint64_t>(0);
+    }
+};
+
+constexpr uint32_t kWaveElems = 256;             // of a tile: 64 lanes, four elements each
+
+// Optimizer step on the live elements [first, last) of a wave's share of a tile, group by group: almost always one. Elements of
+// another group go through the arithmetic too and keep their values (a branch per element instead saves up to ten registers and
+// loses 1 to 2.5 %: K = 1 Adam 160 M elements 717 -> 737 us). rel0: the wave's first element, in span coordinates.
+template <int OPT, int SL, class A, class C>
+__device__ __forceinline__ void update(const float (&agg)[4], f32x4& p, f32x4& s1, f32x4& s2, f32x4& s3, const A& a, C& cur,
+                                       uint64_t rel0, uint32_t first, uint32_t last) {
+    const uint32_t lane4 = (threadIdx.x & 63) * 4;
+    while (true) {
+        const uint64_t rel = rel0 + first;
+        if (rel >= cur.end) cur.seek(rel, a);
+        const uint64_t left = cur.end - rel;
+        const uint32_t upto = left < last - first ? first + static_cast<uint32_t>(left) : last;
 #pragma unroll
-    for (int v = 0; v < NV; ++v)
-        r[v] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(elem_addr<NARROW, 4>(base, e + 4 * v)));
-}
-template <int NV, bool NARROW> __device__ __forceinline__ void store_vec(const float (&x)[4 * NV], float* base, uint64_t e) {
-#pragma unroll
-    for (int v = 0; v < NV; ++v) {
-        f32x4 r = {x[4 * v], x[4 * v + 1], x[4 * v + 2], x[4 * v + 3]};
-        __builtin_nontemporal_store(r, reinterpret_cast<f32x4*>(const_cast<char*>(elem_addr<NARROW, 4>(base, e + 4 * v))));
+        for (int i = 0; i < 4; ++i) {
+            const bool in = lane4 + i - first < upto - first;
+            float np = p[i], n1 = s1[i], n2 = 0.0f, n3 = 0.0f;
+            if constexpr (is_adam(OPT)) n2 = s2[i];
+            if constexpr (OPT == OPT_AMS) n3 = s3[i];
+            opt_elem<OPT>(agg[i], np, n1, n2, n3, cur.g, a.opt);
+            p[i] = in ? np : p[i];
+            s1[i] = in ? n1 : s1[i];
+            if constexpr (is_adam(OPT)) s2[i] = in ? n2 : s2[i];
+            if constexpr (OPT == OPT_AMS) s3[i] = in ? n3 : s3[i];
+            if constexpr (SL) __builtin_amdgcn_sched_barrier(0);
+        }
+        if (upto == last) return;
+        first = upto;
     }
 }
-template <int NV> __device__ __forceinline__ void unpack_vec(const f32x4 (&r)[NV], float (&x)[4 * NV]) {
-#pragma unroll
-    for (int v = 0; v < NV; ++v) { x[4 * v] = r[v].x; x[4 * v + 1] = r[v].y; x[4 * v + 2] = r[v].z; x[4 * v + 3] = r[v].w; }
+
+template <bool NARROW> __device__ __forceinline__ f32x4 load_vec(const float* base, uint64_t e) {
+    return __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(elem_addr<NARROW, 4>(base, e)));
+}
+template <bool NARROW> __device__ __forceinline__ void store_vec(const f32x4& r, float* base, uint64_t e) {
+    __builtin_nontemporal_store(r, reinterpret_cast<f32x4*>(const_cast<char*>(elem_addr<NARROW, 4>(base, e))));
 }
 
-// Registers of U consecutive full tiles: the raw 16-byte vectors as loaded.
+// Registers of U consecutive tiles: the raw vectors as loaded.
 template <int K, int DT, int U, int OPT = OPT_ADAM> struct TileRegs {
     typename Grad<DT>::Raw g[U][K];
-    f32x4 p[U][Grad<DT>::EPT / 4], s1[U][Grad<DT>::EPT / 4], s2[U][Grad<DT>::EPT / 4];
-    f32x4 s3[OPT == OPT_AMS ? U : 1][Grad<DT>::EPT / 4];
+    f32x4 p[U], s1[U], s2[U], s3[OPT == OPT_AMS ? U : 1];
 };
 
 // Issues every load of U consecutive full tiles. e is the (rebased) index of this
 // thread's first element in the first tile.
 template <int K, int DT, int OPT, int U, int BS, bool NARROW, class SP>
 __device__ __forceinline__ void issue_loads(TileRegs<K, DT, U, OPT>& r, const SP& sp, uint64_t e, bool load_s1) {
-    using GR = Grad<DT>;
-    constexpr int EPT = GR::EPT, NV = EPT / 4;
-    constexpr uint64_t TE = static_cast<uint64_t>(BS) * EPT;
+    constexpr uint64_t TE = static_cast<uint64_t>(BS) * 4;
 #pragma unroll
     for (int u = 0; u < U; ++u) {
         const uint64_t eu = e + u * TE;
 #pragma unroll
-        for (int k = 0; k < K; ++k) r.g[u][k] = GR::template load<NARROW>(sp.g[k], eu);
+        for (int k = 0; k < K; ++k) r.g[u][k] = Grad<DT>::template load<NARROW>(sp.g[k], eu);
         if constexpr (OPT != OPT_NONE) {
-            load_vec<NV, NARROW>(r.p[u], sp.p, eu);
+            r.p[u] = load_vec<NARROW>(sp.p, eu);
             const uint64_t mu = is_adam(OPT) ? moment_index(sp, eu) : eu;
-            if (load_s1) load_vec<NV, NARROW>(r.s1[u], sp.s1, mu);
-            if constexpr (is_adam(OPT)) load_vec<NV, NARROW>(r.s2[u], sp.s2, mu);
-            if constexpr (OPT == OPT_AMS) load_vec<NV, NARROW>(r.s3[u], sp.s3, mu);
+            r.s1[u] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            if (load_s1) r.s1[u] = load_vec<NARROW>(sp.s1, mu);
+            if constexpr (is_adam(OPT)) r.s2[u] = load_vec<NARROW>(sp.s2, mu);
+            if constexpr (OPT == OPT_AMS) r.s3[u] = load_vec<NARROW>(sp.s3, mu);
         }
     }
 }
 
-// Arithmetic and stores of U tiles whose loads were issued by issue_loads.
-template <int K, int DT, int OPT, int SL, bool HD, int U, bool NARROW, class A, class SP>
-__device__ __forceinline__ void consume(const TileRegs<K, DT, U, OPT>& r, const SP& sp, uint64_t e, const A& a,
-                                        const GroupDev& G, float clip, bool use_s1, bool load_s1, float* out,
-                                        typename StatAcc<DT>::type (&acc)[NStats<K, SL>::value]) {
-    using GR = Grad<DT>;
-    constexpr int EPT = GR::EPT, NV = EPT / 4;
-    constexpr uint64_t TE = static_cast<uint64_t>(launch_block(K, DT, OPT, SL)) * EPT;
+// Arithmetic and stores of U full tiles whose loads were issued by issue_loads.
+template <int K, int DT, int OPT, int SL, bool HD, int U, bool NARROW, class A, class SP, class C>
+__device__ __forceinline__ void consume(TileRegs<K, DT, U, OPT>& r, const SP& sp, uint64_t e, uint64_t rel0, const A& a, C& cur, float clip,
+                                        bool use_s1, float* out, typename StatAcc<DT>::type (&acc)[NStats<K, SL>::value]) {
+    constexpr uint64_t TE = static_cast<uint64_t>(launch_block(K, DT, OPT, SL)) * 4;
 #pragma unroll
     for (int u = 0; u < U; ++u) {
         const uint64_t eu = e + u * TE;
-        float g[K][EPT], p[EPT], s1[EPT], s2[EPT], s3[EPT], agg[EPT];
-#pragma unroll
-        for (int k = 0; k < K; ++k) GR::widen(r.g[u][k], g[k]);
+        float agg[4];
+        aggregate<K, DT, SL, HD>(r.g[u], agg, a, clip, acc);
+        if (out) store_vec<NARROW>(f32x4{agg[0], agg[1], agg[2], agg[3]}, out, eu);
         if constexpr (OPT != OPT_NONE) {
-            unpack_vec<NV>(r.p[u], p);
-            if (load_s1) unpack_vec<NV>(r.s1[u], s1);
-            else {
-#pragma unroll
-                for (int i = 0; i < EPT; ++i) s1[i] = 0.0f;
-            }
-            if constexpr (is_adam(OPT)) unpack_vec<NV>(r.s2[u], s2);
-            if constexpr (OPT == OPT_AMS) unpack_vec<NV>(r.s3[u], s3);
-        }
-        compute<K, EPT, DT, OPT, SL, HD>(g, p, s1, s2, s3, agg, a, G, clip, acc);
-        if (out) store_vec<NV, NARROW>(agg, out, eu);
-        if constexpr (OPT != OPT_NONE) {
-            store_vec<NV, NARROW>(p, sp.p, eu);
+            f32x4& s3 = r.s3[OPT == OPT_AMS ? u : 0];
+            update<OPT, SL>(agg, r.p[u], r.s1[u], r.s2[u], s3, a, cur, rel0 + u * TE, 0u, kWaveElems);
+            store_vec<NARROW>(r.p[u], sp.p, eu);
             const uint64_t mu = is_adam(OPT) ? moment_index(sp, eu) : eu;
-            if (use_s1) store_vec<NV, NARROW>(s1, sp.s1, mu);
-            if constexpr (is_adam(OPT)) store_vec<NV, NARROW>(s2, sp.s2, mu);
-            if constexpr (OPT == OPT_AMS) store_vec<NV, NARROW>(s3, sp.s3, mu);
-            for (uint32_t f = 0; f < sp.n_fan; ++f) store_vec<NV, NARROW>(p, sp.fan[f], eu);
+            if (use_s1) store_vec<NARROW>(r.s1[u], sp.s1, mu);
+            if constexpr (is_adam(OPT)) store_vec<NARROW>(r.s2[u], sp.s2, mu);
+            if constexpr (OPT == OPT_AMS) store_vec<NARROW>(s3, sp.s3, mu);
+            for (uint32_t f = 0; f < sp.n_fan; ++f) store_vec<NARROW>(r.p[u], sp.fan[f], eu);
         }
     }
 }
 
-// Vector path over nfull consecutive full tiles of one parameter group: groups of U tiles,
-// then U/2, ... down to single tiles.
-template <int K, int DT, int OPT, int SL, bool HD, int U, class A, class SP>
-__device__ __forceinline__ void fast_run(const SP& sp, uint64_t e, uint32_t nfull, const A& a,
-                                         const GroupDev& G, float clip, float* out, typename StatAcc<DT>::type (&acc)[NStats<K, SL>::value]) {
+__device__ __forceinline__ uint32_t wave_of_workgroup() { return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); }
+
+// Vector path over nfull consecutive full tiles: groups of U tiles, then U/2, ... down to LEAST. Returns the tiles left over.
+template <int K, int DT, int OPT, int SL, bool HD, int U, int LEAST, class A, class SP, class C>
+__device__ __forceinline__ uint32_t fast_run(const SP& sp, uint64_t e0, uint32_t nfull, const A& a, C& cur, float clip, bool use_s1, bool load_s1,
+                                             float* out, typename StatAcc<DT>::type (&acc)[NStats<K, SL>::value]) {
     constexpr int BS = launch_block(K, DT, OPT, SL);
-    constexpr uint64_t TE = static_cast<uint64_t>(BS) * Grad<DT>::EPT;
-    const bool use_s1 = is_adam(OPT) || (OPT == OPT_SGD && a.opt.has_momentum);
-    const bool load_s1 = is_adam(OPT) || (OPT == OPT_SGD && a.opt.has_momentum && !a.opt.first_step);
+    constexpr uint64_t TE = static_cast<uint64_t>(BS) * 4;
     uint32_t i = 0;
-    for (; i + U <= nfull; i += U, e += U * TE) {
+    for (; i + U <= nfull; i += U, e0 += U * TE) {
+        const uint64_t e = e0 + static_cast<uint64_t>(threadIdx.x) * 4;
         TileRegs<K, DT, U, OPT> r;
         issue_loads<K, DT, OPT, U, BS, narrow_addressing(K, SL)>(r, sp, e, load_s1);
-        consume<K, DT, OPT, SL, HD, U, narrow_addressing(K, SL)>(r, sp, e, a, G, clip, use_s1, load_s1, out, acc);
+        consume<K, DT, OPT, SL, HD, U, narrow_addressing(K, SL)>(r, sp, e, e0 - sp.lo + wave_of_workgroup() * kWaveElems, a, cur, clip, use_s1, out, acc);
     }
-    if constexpr (U > 1) fast_run<K, DT, OPT, SL, HD, U / 2>(sp, e, nfull - i, a, G, clip, out, acc);
+    if constexpr (U > LEAST) return fast_run<K, DT, OPT, SL, HD, U / 2, LEAST>(sp, e0, nfull - i, a, cur, clip, use_s1, load_s1, out, acc);
+    else return nfull - i;
 }
 
-// One tile that touches a span edge or a group change. tile_e0 is the (rebased) index of the first
-// element of the tile, j the bound entry covering the first live element of the tile. Each thread
-// looks at its own four elements: all live and in one parameter group -> the vector path with that
-// group's constants (held per thread); otherwise -> element by element. Only the few threads whose
-// vector straddles the span's first or last element or a bound take the slow way, so such a tile costs
-// little more than a full one (ResNet-50's batch-norm tensors and ViT's biases put a group change
-// into roughly every hundredth tile; one span per tensor puts an edge into every tensor).
-template <int K, int DT, int OPT, int SL, class A, class SP>
-__device__ __forceinline__ void careful_tile(const SP& sp, uint64_t tile_e0, const A& a, uint32_t j,
-                                             float clip, float* out, typename StatAcc<DT>::type (&acc)[NStats<K, SL>::value]) {
+// Place of a wave's share of a tile in a span's streams: element `first`, its first live one, is the scalar base, a lane's
+// elements lie `at` elements behind it and their moments `mom` (32 bits: any length of span).
+struct WavePlace {
+    uint64_t e, m;                               // grid index and moment index of the wave's first live element
+    uint32_t first, last;                        // live elements, wave-relative
+    template <class SP> __device__ __forceinline__ WavePlace(const SP& sp, uint64_t wave_e) {
+        first = sp.lo > wave_e ? static_cast<uint32_t>(sp.lo - wave_e < kWaveElems ? sp.lo - wave_e : kWaveElems) : 0u;
+        last = sp.hi > wave_e ? static_cast<uint32_t>(sp.hi - wave_e < kWaveElems ? sp.hi - wave_e : kWaveElems) : 0u;
+        e = wave_e + first;
+        m = moment_index(sp, e);
+    }
+    template <class SP> __device__ __forceinline__ uint32_t moment_at(const SP& sp, uint32_t at) const {
+        const uint32_t t = static_cast<uint32_t>(e + sp.mom_add), mask = static_cast<uint32_t>(sp.mom_mask);
+        return at + sp.mom_mult * (((t + at) & mask) - (t & mask));
+    }
+};
+template <int ES> __device__ __forceinline__ const char* lane_addr(const void* base, uint64_t e, uint32_t at) {
+    return static_cast<const char*>(base) + e * ES + static_cast<uint64_t>(at * ES);
+}
+__device__ __forceinline__ f32x4 load_at(const float* base, uint64_t e, uint32_t at) {
+    return __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(lane_addr<4>(base, e, at)));
+}
+__device__ __forceinline__ f32x4 gather_at(const float* base, uint64_t e, const uint32_t (&at)[4], const bool (&live)[4]) {
+    const char* const p[4] = {lane_addr<4>(base, e, at[0]), lane_addr<4>(base, e, at[1]), lane_addr<4>(base, e, at[2]), lane_addr<4>(base, e, at[3])};
+    return Grad<JABAS_F32>::gather(p, live);
+}
+__device__ __forceinline__ void store_at(const f32x4& r, float* base, uint64_t e, uint32_t at) {
+    __builtin_nontemporal_store(r, reinterpret_cast<f32x4*>(const_cast<char*>(lane_addr<4>(base, e, at))));
+}
+
+// One tile, wave by wave, wherever it lies in the span. A thread whose four elements are all live takes the vector accesses; the
+// few that straddle the span's first or last element gather theirs, every load issued before any is waited for (indices of dead
+// elements are those of live ones, their values zero: nothing outside the span is touched, the sums are not changed).
+// A launch of a few hundred workgroups lasts as long as its slowest one. Before, a tile with a group change was taken by itself,
+// each thread looking up its own bounds and those that straddled one working element by element, a trip to memory each: such a
+// workgroup took 9 to 10 us where the others took 4 (K = 8 bf16 AdamW, similarity sums, 0.3 M elements), and the table was read
+// before any load was issued. Sync launch alone, 46 to 60 tensors, before -> now in us:
+//   K = 4 fp32 AdamW   0.3 M none 8.8 -> 6.2, similarity sums 10.6 -> 6.7   1.2 M 15.2 -> 13.2, 17.8 -> 14.2   5 M 40.8 -> 36.9, 42.3 -> 39.5
+//   K = 8 bf16 AdamW   0.3 M none 9.0 -> 6.2, pair products 12.4 -> 9.6     1.2 M 15.6 -> 12.8, 23.1 -> 17.6   5 M 40.9 -> 38.1, 51.1 -> 45.2
+//   K = 2 fp32 SGD     0.3 M none 5.6 -> 4.3, similarity sums 7.5 -> 5.3    1.2 M 10.8 -> 8.8, 13.9 -> 10.0    5 M 26.9 -> 24.7, 28.8 -> 26.3
+// and 25 M the same within 2 %.
+template <int K, int DT, int OPT, int SL, bool HD, class A, class SP, class C>
+__device__ __forceinline__ void single_tile(const SP& sp, uint64_t tile_e0, const A& a, C& cur, float clip, bool use_s1, bool load_s1, float* out,
+                                            typename StatAcc<DT>::type (&acc)[NStats<K, SL>::value]) {
     using GR = Grad<DT>;
-    constexpr int EPT = GR::EPT;
-    constexpr int BS = launch_block(K, DT, OPT, SL);
-    const bool use_s1 = is_adam(OPT) || (OPT == OPT_SGD && a.opt.has_momentum);
-    const bool load_s1 = is_adam(OPT) || (OPT == OPT_SGD && a.opt.has_momentum && !a.opt.first_step);
-    ConstBounds bd = sp.bound_count ? const_bounds(a.bounds + sp.bound_begin) : nullptr;
-    const uint64_t e_first = tile_e0 + static_cast<uint64_t>(threadIdx.x) * EPT;
-    const bool all_live = e_first >= sp.lo && e_first + EPT <= sp.hi;
-    bool one_group = true;
-    uint32_t gid_first = 0;
-    if (bd && all_live) {
-        const uint64_t rel = e_first - sp.lo;
-        uint32_t jj = j;
-        while (jj + 1 < sp.bound_count && bd[jj + 1].start <= rel) ++jj;
-        gid_first = bd[jj].group & (JABAS_MAX_GROUPS - 1);
-        one_group = jj + 1 >= sp.bound_count || bd[jj + 1].start >= rel + EPT;
-    }
-    if (all_live && one_group) {
-        const GroupDev G = a.groups[gid_first];
-        TileRegs<K, DT, 1, OPT> r;
-        issue_loads<K, DT, OPT, 1, BS, false>(r, sp, e_first, load_s1);
-        consume<K, DT, OPT, SL, false, 1, false>(r, sp, e_first, a, G, clip, use_s1, load_s1, out, acc);   // halves from the mask: always right
-        return;
-    }
-    for (int i = 0; i < EPT; ++i) {
-        const uint64_t e = e_first + i;
-        if (e < sp.lo || e >= sp.hi) continue;
-        uint32_t gid = 0;
-        if (bd) {
-            const uint64_t rel = e - sp.lo;
-            uint32_t jj = j;
-            while (jj + 1 < sp.bound_count && bd[jj + 1].start <= rel) ++jj;
-            gid = bd[jj].group & (JABAS_MAX_GROUPS - 1);   // a bound table on the device cannot be checked by the host
-        }
-        const GroupDev G = a.groups[gid];
-        float g[K][1], p[1] = {0.0f}, s1[1] = {0.0f}, s2[1] = {0.0f}, s3[1] = {0.0f}, agg[1];
+    constexpr int GS = DT == JABAS_BF16 ? 2 : 4;
+    const uint64_t wave_e = tile_e0 + wave_of_workgroup() * kWaveElems;
+    const WavePlace w(sp, wave_e);
+    if (w.first >= w.last) return;               // none of the wave's elements is live
+    const uint32_t lane4 = (threadIdx.x & 63) * 4;
+    const bool whole = lane4 >= w.first && lane4 + 4 <= w.last, some = lane4 + 4 > w.first && lane4 < w.last;
+    const uint32_t at = lane4 - w.first, mom = w.moment_at(sp, at);
+    uint32_t eat[4], emom[4];
+    bool live[4];
 #pragma unroll
-        for (int k = 0; k < K; ++k) g[k][0] = GR::load1(sp.g[k], e);
-        [[maybe_unused]] const uint64_t me = is_adam(OPT) ? moment_index(sp, e) : e;
+    for (int i = 0; i < 4; ++i) {
+        live[i] = lane4 + i >= w.first && lane4 + i < w.last;
+        eat[i] = live[i] ? at + i : (lane4 + i < w.first ? 0u : w.last - 1 - w.first);
+        emom[i] = w.moment_at(sp, eat[i]);
+    }
+    TileRegs<K, DT, 1, OPT> r;
+    const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (whole) {
+#pragma unroll
+        for (int k = 0; k < K; ++k)
+            r.g[0][k] = __builtin_nontemporal_load(reinterpret_cast<const typename GR::Raw*>(lane_addr<GS>(sp.g[k], w.e, at)));
         if constexpr (OPT != OPT_NONE) {
-            p[0] = sp.p[e];
-            if (load_s1) s1[0] = sp.s1[me];
-            if constexpr (is_adam(OPT)) s2[0] = sp.s2[me];
-            if constexpr (OPT == OPT_AMS) s3[0] = sp.s3[me];
+            r.p[0] = load_at(sp.p, w.e, at);
+            r.s1[0] = zero;
+            if (load_s1) r.s1[0] = is_adam(OPT) ? load_at(sp.s1, w.m, mom) : load_at(sp.s1, w.e, at);
+            if constexpr (is_adam(OPT)) r.s2[0] = load_at(sp.s2, w.m, mom);
+            if constexpr (OPT == OPT_AMS) r.s3[0] = load_at(sp.s3, w.m, mom);
         }
-        compute<K, 1, DT, OPT, SL, false>(g, p, s1, s2, s3, agg, a, G, clip, acc);
-        if (out) out[e] = agg[0];
+    } else if (some) {
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            const char* const p[4] = {lane_addr<GS>(sp.g[k], w.e, eat[0]), lane_addr<GS>(sp.g[k], w.e, eat[1]),
+                                      lane_addr<GS>(sp.g[k], w.e, eat[2]), lane_addr<GS>(sp.g[k], w.e, eat[3])};
+            r.g[0][k] = GR::gather(p, live);
+            if constexpr (K > 8) {               // a few workers at a time: sixteen streams of four elements would set the register count
+                if (k % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+            }
+        }
         if constexpr (OPT != OPT_NONE) {
-            sp.p[e] = p[0];
-            if (use_s1) sp.s1[me] = s1[0];
-            if constexpr (is_adam(OPT)) sp.s2[me] = s2[0];
-            if constexpr (OPT == OPT_AMS) sp.s3[me] = s3[0];
-            for (uint32_t r = 0; r < sp.n_fan; ++r) sp.fan[r][e] = p[0];
+            r.p[0] = gather_at(sp.p, w.e, eat, live);
+            r.s1[0] = zero;
+            if (load_s1) r.s1[0] = is_adam(OPT) ? gather_at(sp.s1, w.m, emom, live) : gather_at(sp.s1, w.e, eat, live);
+            if constexpr (is_adam(OPT)) r.s2[0] = gather_at(sp.s2, w.m, emom, live);
+            if constexpr (OPT == OPT_AMS) r.s3[0] = gather_at(sp.s3, w.m, emom, live);
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < K; ++k) r.g[0][k] = typename GR::Raw{};
+        if constexpr (OPT != OPT_NONE) {
+            r.p[0] = r.s1[0] = zero;
+            if constexpr (is_adam(OPT)) r.s2[0] = zero;
+            if constexpr (OPT == OPT_AMS) r.s3[0] = zero;
+        }
+    }
+    float agg[4];
+    aggregate<K, DT, SL, HD>(r.g[0], agg, a, clip, acc);
+    if constexpr (OPT != OPT_NONE) update<OPT, SL>(agg, r.p[0], r.s1[0], r.s2[0], r.s3[0], a, cur, wave_e - sp.lo, w.first, w.last);
+    if (whole) {
+        if (out) store_at(f32x4{agg[0], agg[1], agg[2], agg[3]}, out, w.e, at);
+        if constexpr (OPT != OPT_NONE) {
+            store_at(r.p[0], sp.p, w.e, at);
+            if (use_s1) { if constexpr (is_adam(OPT)) store_at(r.s1[0], sp.s1, w.m, mom); else store_at(r.s1[0], sp.s1, w.e, at); }
+            if constexpr (is_adam(OPT)) store_at(r.s2[0], sp.s2, w.m, mom);
+            if constexpr (OPT == OPT_AMS) store_at(r.s3[0], sp.s3, w.m, mom);
+            for (uint32_t f = 0; f < sp.n_fan; ++f) store_at(r.p[0], sp.fan[f], w.e, at);
+        }
+    } else if (some) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            if (!live[i]) continue;
+            if (out) out[w.e + eat[i]] = agg[i];
+            if constexpr (OPT != OPT_NONE) {
+                sp.p[w.e + eat[i]] = r.p[0][i];
+                if (use_s1) sp.s1[is_adam(OPT) ? w.m + emom[i] : w.e + eat[i]] = r.s1[0][i];
+                if constexpr (is_adam(OPT)) sp.s2[w.m + emom[i]] = r.s2[0][i];
+                if constexpr (OPT == OPT_AMS) sp.s3[w.m + emom[i]] = r.s3[0][i];
+                for (uint32_t f = 0; f < sp.n_fan; ++f) sp.fan[f][w.e + eat[i]] = r.p[0][i];
+            }
         }
     }
 }
 
-// Tiles [lt0, lt1) of one span (tile indices local to the span).
-template <int K, int DT, int OPT, int SL, bool HD, class A, class SP>
+// Tiles [lt0, lt1) of one span (tile indices local to the span). SEARCH: no bound entry near their first element is known.
+template <int K, int DT, int OPT, int SL, bool HD, bool SEARCH, class A, class SP>
 __device__ __forceinline__ void span_range(const SP& sp, uint32_t lt0, uint32_t lt1, uint32_t j0,
                                            const A& a, typename StatAcc<DT>::type (&acc)[NStats<K, SL>::value]) {
     const float clip = a.grad_scale ? *a.grad_scale : 1.0f;      // uniform: one scalar load per workgroup
@@ -428,46 +531,35 @@ __device__ __forceinline__ void span_range(const SP& sp, uint32_t lt0, uint32_t 
     if constexpr (K == 1 && DT == JABAS_F32) {
         if (static_cast<const void*>(out) == sp.g[0] && a.w[0] == 1.0f && !(clip < 1.0f)) out = nullptr;
     }
-    using GR = Grad<DT>;
-    constexpr int EPT = GR::EPT;
-    constexpr uint64_t TE = static_cast<uint64_t>(launch_block(K, DT, OPT, SL)) * EPT;
+    constexpr uint64_t TE = static_cast<uint64_t>(launch_block(K, DT, OPT, SL)) * 4;
     constexpr int UW = SL ? JABAS_UNROLL_STATS : JABAS_UNROLL_PLAIN;
     constexpr int CT = launch_chunk_tiles(K, DT, OPT, SL);
     constexpr int U0 = UW < CT ? UW : CT;     // never more than a chunk holds
     // 9..16 gradient streams: one tile's loads fill the registers; so do eight fp32 ones beside the 28 fp64 pair
     // sums of the Gram level (two tiles in flight: 256 registers and one wave per SIMD, 13 % slower)
     constexpr int U = (K > 8 || (SL == JABAS_STATS_GRAM && DT == JABAS_F32 && K > 7)) ? 1 : U0;
-    static_assert((U & (U - 1)) == 0, "the unroll cascade halves U down to 1");
+    constexpr int LEAST = U > 1 ? 2 : 1;      // a single tile goes through single_tile, unless it is all that is ever in flight
+    static_assert((U & (U - 1)) == 0, "the unroll cascade halves U down to LEAST");
+    const bool use_s1 = is_adam(OPT) || (OPT == OPT_SGD && a.opt.has_momentum);
+    const bool load_s1 = is_adam(OPT) || (OPT == OPT_SGD && a.opt.has_momentum && !a.opt.first_step);
     const uint32_t nb = sp.bound_count;
-    ConstBounds bd = nb ? const_bounds(a.bounds + sp.bound_begin) : nullptr;
-    uint32_t lt = lt0, j = j0;
-    while (lt < lt1) {
+    GroupCursor<SEARCH> cur{nb ? const_bounds(a.bounds + sp.bound_begin) : nullptr, nb, j0, 0, {}};
+    for (uint32_t lt = lt0; lt < lt1;) {
         const uint64_t e0 = static_cast<uint64_t>(lt) * TE;
-        const uint64_t cur = e0 > sp.lo ? e0 : sp.lo;
-        const uint64_t rel = cur - sp.lo;
-        uint64_t stretch_end = sp.hi;
-        uint32_t gid = 0;
-        if (nb) {
-            while (j + 1 < nb && bd[j + 1].start <= rel) ++j;
-            gid = bd[j].group & (JABAS_MAX_GROUPS - 1);
-            if (j + 1 < nb) stretch_end = sp.lo + bd[j + 1].start;
-        }
         uint32_t nfull = 0;
-        // spans beyond 32-bit byte offsets take the careful path tile by tile (64-bit addresses there)
-        if (e0 >= sp.lo && stretch_end >= e0 + TE && (!narrow_addressing(K, SL) || sp.narrow_ok)) {
-            const uint64_t fit = (stretch_end - e0) / TE;
+        // spans beyond 32-bit byte offsets go tile by tile
+        if (e0 >= sp.lo && (!narrow_addressing(K, SL) || sp.narrow_ok)) {
+            const uint64_t fit = (sp.hi - e0) / TE;
             const uint32_t left = lt1 - lt;
             nfull = fit < left ? static_cast<uint32_t>(fit) : left;
             // a workgroup's tiles are a chunk's or a part of them: one worker's statistics 60 M elements 36.0 -> 32.7 us (bf16), 46.5 ->
             // 45.9 (fp32); in other kernels the registers fall out worse (K = 4 SGD with replicas 212 -> 217, clipped Adam 1390 -> 1399)
             if constexpr (K == 1 && OPT == OPT_NONE && SL != 0) __builtin_assume(nfull <= CT);
         }
-        if (nfull) {
-            const GroupDev G = a.groups[gid];
-            fast_run<K, DT, OPT, SL, HD, U>(sp, e0 + static_cast<uint64_t>(threadIdx.x) * EPT, nfull, a, G, clip, out, acc);
-            lt += nfull;
+        if (nfull >= static_cast<uint32_t>(LEAST)) {
+            lt += nfull - fast_run<K, DT, OPT, SL, HD, U, LEAST>(sp, e0, nfull, a, cur, clip, use_s1, load_s1, out, acc);
         } else {
-            careful_tile<K, DT, OPT, SL>(sp, e0, a, j, clip, out, acc);
+            single_tile<K, DT, OPT, SL, HD>(sp, e0, a, cur, clip, use_s1, load_s1, out, acc);
             lt += 1;
         }
     }
@@ -475,15 +567,15 @@ __device__ __forceinline__ void span_range(const SP& sp, uint32_t lt0, uint32_t 
 
 // Statistics kernels carry two copies of the arithmetic: one with the default halves
 // (even worker -> A, odd -> B) resolved at compile time, one driven by the half mask.
-template <int K, int DT, int OPT, int SL, class A, class SP>
+template <int K, int DT, int OPT, int SL, bool SEARCH, class A, class SP>
 __device__ __forceinline__ void run_chunk(const SP& sp, uint32_t lt0, uint32_t lt1, uint32_t j0, const A& a,
                                           typename StatAcc<DT>::type (&acc)[NStats<K, SL>::value]) {
     if constexpr (SL) {
         constexpr uint32_t kDefaultMask = 0xAAAAu & ((1u << K) - 1u);
-        if (a.half_mask == kDefaultMask) span_range<K, DT, OPT, SL, true>(sp, lt0, lt1, j0, a, acc);
-        else span_range<K, DT, OPT, SL, false>(sp, lt0, lt1, j0, a, acc);
+        if (a.half_mask == kDefaultMask) span_range<K, DT, OPT, SL, true, SEARCH>(sp, lt0, lt1, j0, a, acc);
+        else span_range<K, DT, OPT, SL, false, SEARCH>(sp, lt0, lt1, j0, a, acc);
     } else {
-        span_range<K, DT, OPT, 0, true>(sp, lt0, lt1, j0, a, acc);
+        span_range<K, DT, OPT, 0, true, SEARCH>(sp, lt0, lt1, j0, a, acc);
     }
 }
 
@@ -579,19 +671,7 @@ __device__ __forceinline__ void workgroup_chunk(const KArgs& a, const A& s, uint
         const uint32_t tiles = static_cast<uint32_t>((sp.hi + TE - 1) / TE);
         const uint32_t lt0 = b * per;
         const uint32_t lt1 = lt0 + per < tiles ? lt0 + per : tiles;
-        uint32_t j0 = 0;
-        if (sp.bound_count) {                  // largest j with bounds[j].start <= first live element
-            ConstBounds bd = const_bounds(a.bounds + sp.bound_begin);
-            const uint64_t e0 = static_cast<uint64_t>(lt0) * TE;
-            const uint64_t rel = (e0 > sp.lo ? e0 : sp.lo) - sp.lo;
-            uint32_t lo = 0, hi = sp.bound_count;
-            while (hi - lo > 1) {
-                const uint32_t mid = (lo + hi) >> 1;
-                if (bd[mid].start <= rel) lo = mid; else hi = mid;
-            }
-            j0 = lo;
-        }
-        run_chunk<K, DT, OPT, SL>(sp, lt0, lt1, j0, s, acc);
+        run_chunk<K, DT, OPT, SL, true>(sp, lt0, lt1, 0, s, acc);
     } else {
         // The plan's tables are not written while a launch that names them runs: read through the constant
         // address space, their fields are loaded like kernel arguments (uniform loads the compiler may move,
@@ -604,7 +684,7 @@ __device__ __forceinline__ void workgroup_chunk(const KArgs& a, const A& s, uint
         const ConstSpan& sp = *(const ConstSpan*)(a.spans + c_span);
         const uint32_t tiles = static_cast<uint32_t>((sp.hi + TE - 1) / TE);
         const uint32_t lt1 = lt0 + per < tiles ? lt0 + per : tiles;
-        run_chunk<K, DT, OPT, SL>(sp, lt0, lt1, c_bound0, s, acc);
+        run_chunk<K, DT, OPT, SL, false>(sp, lt0, lt1, c_bound0, s, acc);
     }
 }
 
@@ -642,10 +722,24 @@ int launch_one(const KArgs& a, unsigned grid, hipStream_t stream, bool dyn) {
 #ifndef JABAS_STATS_LDS_BYTES
 #define JABAS_STATS_LDS_BYTES 53248u      // per workgroup, flush_stats' own table included: three workgroups per CU
 #endif
-    constexpr bool capped = OPT == OPT_ADAM && K <= 4 && DT == JABAS_F32;
+    // An aggregate with statistics and no optimizer, K <= 4 with fp32 gradients, five workgroups per CU where it is written and six
+    // where the gradients are only read (their registers allow seven or eight). 160 M elements, seven / five: K = 4 similarity
+    // sums 549 -> 526 us, full rows 550 -> 536, K = 3 436 -> 419, K = 2 330 -> 319, GNMT's clipped step, whose first launch this is,
+    // 1413 -> 1383; read only, no cap / six / five: K = 2 202 / 200 / 211, K = 3 303 / 301 / 304.
+#ifndef JABAS_AGG_LDS_BYTES
+#define JABAS_AGG_LDS_BYTES 32768u
+#endif
+#ifndef JABAS_AGG_READ_LDS_BYTES
+#define JABAS_AGG_READ_LDS_BYTES 26624u
+#endif
+    constexpr bool capped = OPT == OPT_ADAM && K <= 4 && DT == JABAS_F32, capped_agg = OPT == OPT_NONE && SL && K > 1 && K <= 4 && DT == JABAS_F32;
     constexpr unsigned flush_bytes = imin(NStats<K, SL>::value, launch_block(K, DT, OPT, SL) / 16) * launch_block(K, DT, OPT, SL) * 8u;   // flush_stats' fp64 table
     static_assert(!capped || !SL || flush_bytes < JABAS_STATS_LDS_BYTES, "the cap is what is left beside the table");
-    constexpr unsigned idle = !capped ? 0u : SL ? JABAS_STATS_LDS_BYTES - flush_bytes : JABAS_IDLE_LDS_BYTES;
+    const unsigned total = capped_agg ? (a.writes_agg ? JABAS_AGG_LDS_BYTES : JABAS_AGG_READ_LDS_BYTES)
+                         : !capped    ? 0u
+                         : SL         ? JABAS_STATS_LDS_BYTES
+                                      : JABAS_IDLE_LDS_BYTES;
+    const unsigned table = SL ? flush_bytes : 0u, idle = total > table ? total - table : 0u;
     const dim3 block(launch_block(K, DT, OPT, SL));
     if constexpr (SL == JABAS_STATS_GRAM && K > JABAS_STATS_GRAM_MAX_K) {
         return static_cast<int>(hipErrorInvalidValue);              // refused by the front before it gets here

@@ -97,9 +97,8 @@ __host__ __device__ constexpr int shape_level(int stats) { return stats == JABAS
 //                       2048 without statistics, 1 to 4 M elements lose: K = 4 AdamW 2 / 3 / 4 M 17.9 / 25.1 / 32.7 -> 19.0 / 27.5 /
 //                       35.8, K = 8 bf16 aggregate 4 M 15.4 -> 18.0; while fewer than 512, 2 M 18.9, and K = 8 pair products 0.9 M
 //                       0.90 of the time of whole chunks against 0.74
-//   group changes       in a span (norms and biases between the weights): up to 2048 and 512. A tile with a change takes the careful
-//                       path, three others of its workgroup wait for it, and the slowest workgroups make the launch. Engine steps,
-//                       up to 448 -> up to 2048: K = 2 fp32 AdamW 2.3 M in 293 tensors 26.1 -> 20.0 us, K = 1 4.0 M in 85 30.5 -> 25.7, K = 4
+//   group changes       in a span (norms and biases between the weights): up to 2048 and 512. Engine steps while a tile
+//                       with a change took many times as long as the others, up to 448 -> up to 2048: K = 2 fp32 AdamW 2.3 M in 293 tensors 26.1 -> 20.0 us, K = 1 4.0 M in 85 30.5 -> 25.7, K = 4
 //                       6.4 M in 117 71.1 -> 66.1, K = 4 3.0 M in 23 26.1 -> 24.9; K = 6 full rows 1.0 M in 153 20.7 -> 18.6
 //   without a tile      at most a quarter, or 64 with statistics (each still runs its epilogue and writes a row) and 256 without, or as
 //                       many as there are compute units for: plans over short spans, one per small tensor, whose last chunk is
@@ -246,6 +245,8 @@ struct KArgs {
     uint32_t use_inline;                     // 1: the only span is `span0`, workgroup b starts at tile b * (chunk_tiles >> split_log2)
     uint32_t half_mask;                      // bit k set: VSW k belongs to half B
     uint32_t split_log2;                     // 2^split_log2 workgroups share a chunk (launch_split_log2)
+    uint32_t writes_agg;                     // 1: a span's aggregate is written (the host's choice of residency; no kernel reads it)
+    uint32_t pad;
     SpanDev span0;
     float w[JABAS_MAX_K];
     float wh[JABAS_MAX_K];

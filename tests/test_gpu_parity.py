@@ -1441,3 +1441,45 @@ def test_aggregate_of_one_worker_over_its_own_buffer(gpu, numel, kind, weight, s
     for a, b in zip(*res):
         assert torch.equal(a.view(torch.int32), b.view(torch.int32))
     assert torch.equal(res[0][0].cpu().view(torch.int32), want.view(torch.int32))
+
+
+@pytest.mark.parametrize("K,dtype,kind,level", [(1, torch.float32, "adam", None), (3, torch.float32, "sgd", None), (4, torch.float32, "adamw", "similarity"),
+                                                (8, torch.bfloat16, "adamw", "gram"), (8, torch.float32, "sgd", "gram"),
+                                                (13, torch.float32, "adam", "full"), (16, torch.bfloat16, "adamw_amsgrad", "full")])
+@pytest.mark.parametrize("skew", [0, 1, 63])
+def test_group_changes_and_ends_anywhere_in_a_wave(gpu, K, dtype, kind, level, skew):
+    """Parameter groups that change at every place a wave's 256 elements can have it (inside a thread's four elements, between
+    threads, waves and tiles, several times in one wave, every element), and spans that begin and end inside a wave, inside a
+    thread's four elements or within one of them: aggregate, weights and state bit for bit, as one span by value and as a plan,
+    nothing written beyond the span."""
+    from jabas_amd import sync
+    groups = [dict(lr=1e-2, weight_decay=0.05), dict(lr=3e-3, weight_decay=0.0), dict(lr=5e-2, weight_decay=0.01)]
+    opt = dict(kind=kind.replace("_amsgrad", ""), amsgrad="amsgrad" in kind, momentum=0.9, betas=(0.9, 0.999), eps=1e-8, groups=groups)
+    n_state = 1 if kind == "sgd" else 3 if "amsgrad" in kind else 2
+    every = tuple(range(700, 720))
+    for n, starts in ((1, ()), (2, (1,)), (3, (1, 2)), (255, (254,)), (257, (3, 4, 256)), (1021, (253, 255, 256, 257, 258, 511, 1020)),
+                      (5003, (1, 2, 5, 1023, 1024, 1025, 2047, 2050, 4095, 4097, 5002)), (9001, every + (3001, 8191, 8192, 8999, 9000))):
+        bounds = tuple((s, i % 3) for i, s in enumerate((0,) + starts))
+        hg = _host_grads(K, n, 400 + K, dtype=dtype)
+        p_h, state_h = _host_state(n, 11), [_host_state(n, 12, 1e-3), _host_state(n, 13, 1e-3).abs(), _host_state(n, 14, 1e-3).abs()][:n_state]
+        start = [p_h.clone()] + [t.clone() for t in state_h]
+        agg_h, rows_h = O.sync_step(hg, BATCHES[K], [(0, n, bounds)], opt, p_h, *state_h[:2], step=3, want_stats=True,
+                                    **({"state3": state_h[2]} if n_state == 3 else {}))
+        for plan in (False, True):
+            def place(t):
+                buf = torch.full((n + 192,), 7.25, dtype=t.dtype, device=gpu)
+                buf[skew:skew + n].copy_(t)
+                return buf
+            whole = [place(t) for t in hg] + [place(torch.zeros(n))] + [place(t) for t in start]
+            views = [b[skew:skew + n] for b in whole]
+            span = sync.SpanSpec(views[:K], agg_out=views[K], param=views[K + 1], bounds=bounds,
+                                 **{f"state{j + 1}": t for j, t in enumerate(views[K + 2:])})
+            args = sync.make_step_args(BATCHES[K], dtype, stats=level or False, opt=opt, step=3)
+            row = sync.SyncPlan([span], sync.opt_kind(opt)).run(args) if plan else sync.sync_bucket(span, args)
+            for got, want in zip(views[K:], [agg_h, p_h, *state_h]):
+                assert torch.equal(_bits(got), _bits(want)), (n, plan)
+            for b in whole:
+                assert bool((b[:skew] == 7.25).all()) and bool((b[skew + n:] == 7.25).all())
+            if level:
+                tol = 1e-11 if dtype == torch.float32 else 20 * 2.0 ** -24      # bf16: as in the test of split launches above
+                torch.testing.assert_close(row.reshape(-1)[1:4].cpu(), rows_h[0][1:4], rtol=tol, atol=0.0)
