@@ -128,7 +128,13 @@ enum {
  * t + (ways - 1) * (t - t mod T), t = state_block_pos + i, from the start of the block group, ways = 2 or 3.
  * The alias rule treats everything from state1 to the last element's last moment as one written buffer.
  * No reference counterpart (torch keeps one tensor per parameter and moment,
- * examples/gnmt/seq2seq/train/shard_optimizer.py:50-66). */
+ * examples/gnmt/seq2seq/train/shard_optimizer.py:50-66).
+ *
+ * JABAS_SPAN_LOOSE_GRADS (in `reserved`; fp32 gradients only, no effect on bf16 ones): the gradient buffers, and an
+ * agg_out that is one of them, may sit at any element, also at another position of a 16-byte line than the buffers
+ * they update, as the views of a packed bucket sit next to weights that an allocator placed. They cost a line more
+ * per wave and access where they do. */
+#define JABAS_SPAN_LOOSE_GRADS 1u
 typedef struct JabasSpan {
     const void* grads[JABAS_MAX_K];     /* K gradient buffers (fp32 or bf16)           */
     float*      agg_out;                /* aggregated fp32 gradient, or NULL           */
@@ -143,7 +149,7 @@ typedef struct JabasSpan {
     uint32_t    bound_count;            /* 0: the whole span is parameter group 0      */
     uint32_t    state_block_log2;       /* 0: state1/2/3 are arrays of their own; else interleaved moments */
     uint32_t    state_block_pos;        /* interleaved moments: position of the first element in its block */
-    uint32_t    reserved;
+    uint32_t    reserved;               /* 0, or JABAS_SPAN_... bits                   */
 } JabasSpan;
 
 /* Parameter-group change inside a span: elements [start, next start) use `group`.

@@ -21,6 +21,7 @@ STATIC_MAX_NUMEL = 1 << 26
 STEP_SCALARS_BYTES = 688
 
 F32, BF16 = 0, 1
+SPAN_LOOSE_GRADS = 1
 OPT_NONE, OPT_SGD, OPT_ADAM, OPT_ADAMW, OPT_ADAM_AMSGRAD, OPT_ADAMW_AMSGRAD = 0, 1, 2, 3, 4, 5
 STATS_NONE, STATS_FULL, STATS_SIMILARITY, STATS_GRAM = 0, 1, 2, 3
 

@@ -118,7 +118,17 @@ int encode_span(const JabasSpan& in, int K, int grad_dtype, int opt_kind, int bl
         il_bytes = 4 * (tl + (il_ways - 1) * (tl & ~(il_T - 1)) + (il_ways - 1) * il_T + 1 - in.state_block_pos);
     }
 
-    const uintptr_t g0 = reinterpret_cast<uintptr_t>(in.grads[0]);
+    // The element grid starts at a line of the gradients, or, where those may sit at any element, of the weights (the aggregate,
+    // where there are none).
+    const auto is_grad = [&](const void* p) {
+        for (int k = 0; k < K; ++k)
+            if (p == in.grads[k]) return true;
+        return false;
+    };
+    const bool loose = (in.reserved & JABAS_SPAN_LOOSE_GRADS) && grad_dtype == JABAS_F32;
+    const bool loose_out = loose && is_grad(in.agg_out);
+    const void* first = !loose ? in.grads[0] : oc != 0 ? in.param : in.agg_out && !loose_out ? in.agg_out : in.grads[0];
+    const uintptr_t g0 = reinterpret_cast<uintptr_t>(first);
     if (g0 % gs) return JABAS_ERR_ALIGN;
     const uint32_t wide_skew = static_cast<uint32_t>((g0 / gs) % kWideElems);
     bool wide = true;
@@ -126,8 +136,8 @@ int encode_span(const JabasSpan& in, int K, int grad_dtype, int opt_kind, int bl
         const uintptr_t a = reinterpret_cast<uintptr_t>(p);
         if (p && (a % es || (a / es) % kWideElems != wide_skew)) wide = false;
     };
-    for (int k = 0; k < K; ++k) same_wide(in.grads[k], gs);
-    same_wide(in.agg_out, 4);
+    for (int k = 0; k < K && !loose; ++k) same_wide(in.grads[k], gs);
+    if (!loose_out) same_wide(in.agg_out, 4);
     if (oc != 0) {
         same_wide(in.param, 4);
         same_wide(in.state1, 4);
@@ -141,21 +151,21 @@ int encode_span(const JabasSpan& in, int K, int grad_dtype, int opt_kind, int bl
     const uint32_t skew = wide ? wide_skew : static_cast<uint32_t>((g0 / gs) % ept);
     auto rebase_g = [&](const void* p, const void** dst) -> bool {
         const uintptr_t a = reinterpret_cast<uintptr_t>(p);
-        if (a % gs || (a / gs) % ept != skew % ept) return false;
+        if (a % gs || (!loose && (a / gs) % ept != skew % ept)) return false;
         *dst = reinterpret_cast<const void*>(a - static_cast<uintptr_t>(skew) * gs);
         return true;
     };
-    auto rebase_f = [&](float* p, float** dst) -> bool {
+    auto rebase_f = [&](float* p, float** dst, bool any = false) -> bool {
         if (!p) { *dst = nullptr; return true; }
         const uintptr_t a = reinterpret_cast<uintptr_t>(p);
-        if (a % 4 || (a / 4) % 4 != skew % 4) return false;
+        if (a % 4 || (!any && (a / 4) % 4 != skew % 4)) return false;
         *dst = reinterpret_cast<float*>(a - static_cast<uintptr_t>(skew) * 4);
         return true;
     };
     memset(out, 0, sizeof(*out));
     for (int k = 0; k < K; ++k)
         if (!rebase_g(in.grads[k], &out->g[k])) return JABAS_ERR_ALIGN;
-    if (!rebase_f(in.agg_out, &out->out)) return JABAS_ERR_ALIGN;
+    if (!rebase_f(in.agg_out, &out->out, loose_out)) return JABAS_ERR_ALIGN;
     if (oc != 0) {
         if (!rebase_f(in.param, &out->p) || !rebase_f(in.state1, &out->s1)) return JABAS_ERR_ALIGN;
         if (il_log2) {

@@ -43,6 +43,11 @@ namespace jabas {
 namespace {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+// fp32 gradients and the aggregate may sit at any element (JABAS_SPAN_LOOSE_GRADS). The access is the same instruction, which takes
+// any multiple of 4 bytes; a wave whose vectors straddle lines touches nine of 128 bytes instead of eight. ShardAdamW.step over
+// gradients packed at odd elements, an aligned copy of each such tensor before -> now: 1 M elements in 100 tensors 310 -> 50 us (then
+// bound by its host side), 25.6 M in 60 219 -> 124, 80 M in 150 656 -> 385, 3 % over the rate of a copy.
+typedef f32x4 __attribute__((aligned(4))) f32x4_a4;
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 __device__ __forceinline__ float bits_to_float(uint32_t u) { return __builtin_bit_cast(float, u); }
@@ -64,10 +69,10 @@ template <bool NARROW, int ES> __device__ __forceinline__ const char* elem_addr(
 template <int DT> struct Grad;
 
 template <> struct Grad<JABAS_F32> {
-    static constexpr int EPT = 4;
     using Raw = f32x4;
+    using Mem = f32x4_a4;
     template <bool NARROW> static __device__ __forceinline__ Raw load(const void* base, uint64_t e) {
-        return __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(elem_addr<NARROW, 4>(base, e)));
+        return __builtin_nontemporal_load(reinterpret_cast<const f32x4_a4*>(elem_addr<NARROW, 4>(base, e)));
     }
     static __device__ __forceinline__ float elem(const Raw& r, int i) { return r[i]; }
     // elements at byte addresses of one stream, the live ones of a vector that straddles a span end
@@ -82,8 +87,8 @@ template <> struct Grad<JABAS_F32> {
 };
 
 template <> struct Grad<JABAS_BF16> {
-    static constexpr int EPT = 4;
     using Raw = u32x2;
+    using Mem = u32x2;
     template <bool NARROW> static __device__ __forceinline__ Raw load(const void* base, uint64_t e) {
         return __builtin_nontemporal_load(reinterpret_cast<const u32x2*>(elem_addr<NARROW, 2>(base, e)));
     }
@@ -316,8 +321,8 @@ __device__ __forceinline__ void update(const float (&agg)[4], f32x4& p, f32x4& s
 template <bool NARROW> __device__ __forceinline__ f32x4 load_vec(const float* base, uint64_t e) {
     return __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(elem_addr<NARROW, 4>(base, e)));
 }
-template <bool NARROW> __device__ __forceinline__ void store_vec(const f32x4& r, float* base, uint64_t e) {
-    __builtin_nontemporal_store(r, reinterpret_cast<f32x4*>(const_cast<char*>(elem_addr<NARROW, 4>(base, e))));
+template <bool NARROW, class MEM = f32x4> __device__ __forceinline__ void store_vec(const f32x4& r, float* base, uint64_t e) {
+    __builtin_nontemporal_store(r, reinterpret_cast<MEM*>(const_cast<char*>(elem_addr<NARROW, 4>(base, e))));
 }
 
 // Registers of U consecutive tiles: the raw vectors as loaded.
@@ -357,7 +362,7 @@ __device__ __forceinline__ void consume(TileRegs<K, DT, U, OPT>& r, const SP& sp
         const uint64_t eu = e + u * TE;
         float agg[4];
         aggregate<K, DT, SL, HD>(r.g[u], agg, a, clip, acc);
-        if (out) store_vec<NARROW>(f32x4{agg[0], agg[1], agg[2], agg[3]}, out, eu);
+        if (out) store_vec<NARROW, f32x4_a4>(f32x4{agg[0], agg[1], agg[2], agg[3]}, out, eu);
         if constexpr (OPT != OPT_NONE) {
             f32x4& s3 = r.s3[OPT == OPT_AMS ? u : 0];
             update<OPT, SL>(agg, r.p[u], r.s1[u], r.s2[u], s3, a, cur, rel0 + u * TE, 0u, kWaveElems);
@@ -416,8 +421,8 @@ __device__ __forceinline__ f32x4 gather_at(const float* base, uint64_t e, const 
     const char* const p[4] = {lane_addr<4>(base, e, at[0]), lane_addr<4>(base, e, at[1]), lane_addr<4>(base, e, at[2]), lane_addr<4>(base, e, at[3])};
     return Grad<JABAS_F32>::gather(p, live);
 }
-__device__ __forceinline__ void store_at(const f32x4& r, float* base, uint64_t e, uint32_t at) {
-    __builtin_nontemporal_store(r, reinterpret_cast<f32x4*>(const_cast<char*>(lane_addr<4>(base, e, at))));
+template <class MEM = f32x4> __device__ __forceinline__ void store_at(const f32x4& r, float* base, uint64_t e, uint32_t at) {
+    __builtin_nontemporal_store(r, reinterpret_cast<MEM*>(const_cast<char*>(lane_addr<4>(base, e, at))));
 }
 
 // One tile, wave by wave, wherever it lies in the span. A thread whose four elements are all live takes the vector accesses; the
@@ -455,7 +460,7 @@ __device__ __forceinline__ void single_tile(const SP& sp, uint64_t tile_e0, cons
     if (whole) {
 #pragma unroll
         for (int k = 0; k < K; ++k)
-            r.g[0][k] = __builtin_nontemporal_load(reinterpret_cast<const typename GR::Raw*>(lane_addr<GS>(sp.g[k], w.e, at)));
+            r.g[0][k] = __builtin_nontemporal_load(reinterpret_cast<const typename GR::Mem*>(lane_addr<GS>(sp.g[k], w.e, at)));
         if constexpr (OPT != OPT_NONE) {
             r.p[0] = load_at(sp.p, w.e, at);
             r.s1[0] = zero;
@@ -493,7 +498,7 @@ __device__ __forceinline__ void single_tile(const SP& sp, uint64_t tile_e0, cons
     aggregate<K, DT, SL, HD>(r.g[0], agg, a, clip, acc);
     if constexpr (OPT != OPT_NONE) update<OPT, SL>(agg, r.p[0], r.s1[0], r.s2[0], r.s3[0], a, cur, wave_e - sp.lo, w.first, w.last);
     if (whole) {
-        if (out) store_at(f32x4{agg[0], agg[1], agg[2], agg[3]}, out, w.e, at);
+        if (out) store_at<f32x4_a4>(f32x4{agg[0], agg[1], agg[2], agg[3]}, out, w.e, at);
         if constexpr (OPT != OPT_NONE) {
             store_at(r.p[0], sp.p, w.e, at);
             if (use_s1) { if constexpr (is_adam(OPT)) store_at(r.s1[0], sp.s1, w.m, mom); else store_at(r.s1[0], sp.s1, w.e, at); }
@@ -664,7 +669,7 @@ __device__ __forceinline__ void workgroup_chunk(const KArgs& a, const A& s, uint
                                                 typename StatAcc<DT>::type (&acc)[NStats<K, SL>::value]) {
     constexpr int BS = launch_block(K, DT, OPT, SL);
     constexpr uint32_t CT = launch_chunk_tiles(K, DT, OPT, SL);     // the host cuts the chunk table for the same shape
-    constexpr uint64_t TE = static_cast<uint64_t>(BS) * Grad<DT>::EPT;
+    constexpr uint64_t TE = static_cast<uint64_t>(BS) * 4;
     const uint32_t per = CT >> a.split_log2;     // tiles of this workgroup
     if (a.use_inline) {
         const SpanDev& sp = a.span0;

@@ -176,6 +176,7 @@ __host__ __device__ constexpr int tile_elems_of(int block) { return block * 4; }
 // A span as the kernels see it. Pointers are rebased downwards by `lo` elements so that
 // element index 0 of every buffer is 16-byte aligned (256-byte aligned when the buffers allow
 // it, lo < 64 then, else lo < 4); [lo, hi) is the live range. Nothing below `lo` is accessed.
+// Loose fp32 gradients (JABAS_SPAN_LOOSE_GRADS), and an aggregate in one of them, are 4-byte aligned only.
 struct SpanDev {
     const void* g[JABAS_MAX_K];
     float* out;

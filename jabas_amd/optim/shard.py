@@ -94,10 +94,10 @@ class _ShardOptimizer(torch.optim.Optimizer):
         return tuple([(p.data_ptr(), g.data_ptr(), g.numel()) + tuple(q.data_ptr() for q in rep.get(id(p), ()))
                       for _, p, g in pairs])
 
-    def _remember(self, sig, launches, copies):
+    def _remember(self, sig, launches):
         if len(self._recipes) >= self._max_cached_plans:
             self._recipes.clear()
-        self._recipes[sig] = (launches, copies, list(self._late_copies))
+        self._recipes[sig] = (launches, list(self._late_copies))
 
     _late_copies = ()
 
@@ -143,17 +143,7 @@ class _ShardOptimizer(torch.optim.Optimizer):
         if not g.is_contiguous():
             g = g.contiguous()
             self._volatile = True                 # a fresh copy every call: nothing to remember
-        g = g.view(-1)
-        if not self._congruent(g, p):
-            # a bucket view that starts off the weight's position in a 16-byte line: realign a copy
-            skew = (p.data_ptr() // 4) % 4
-            buf = torch.empty(g.numel() + 4, dtype=torch.float32, device=g.device)
-            base = (buf.data_ptr() // 4) % 4
-            tmp = buf[(skew - base) % 4:][:g.numel()]
-            tmp.copy_(g)
-            self._copies.append((tmp, g))
-            g = tmp
-        return g
+        return g.view(-1)           # wherever a bucket put it: the spans below take loose gradients
 
     def _launch(self, spans, args):
         key = (args.opt_kind,) + tuple((s.grads[0].data_ptr(), s.param.data_ptr(), s.grads[0].numel(), s.bounds[0][1],
@@ -199,7 +189,7 @@ class ShardSGD(_ShardOptimizer):
         sig = self._signature(pairs)
         if self._replay(self._recipes.get(sig)):
             return loss
-        self._copies, self._volatile, launches, self._late_copies = [], False, [], []
+        self._volatile, launches, self._late_copies = False, [], []
         # launches are split by (momentum, dampening, nesterov, first-step): launch-wide scalars
         batches = {}
         for gi, p, g in pairs:
@@ -218,7 +208,7 @@ class ShardSGD(_ShardOptimizer):
                 if slot >= L.MAX_GROUPS:
                     raise RuntimeError(f"more than {L.MAX_GROUPS} parameter groups in one launch")
                 spans.append(sync.SpanSpec([g], param=p.data.view(-1), state1=None if buf is None else buf.view(-1),
-                                           fanout=self._fanout(p), bounds=((0, slot),)))
+                                           fanout=self._fanout(p), bounds=((0, slot),), loose_grads=True))
             for gi, slot in slots.items():
                 args.groups[slot].lr = float(self.param_groups[gi]["lr"])
                 args.groups[slot].weight_decay = float(self.param_groups[gi]["weight_decay"])
@@ -231,7 +221,7 @@ class ShardSGD(_ShardOptimizer):
             self._volatile = self._volatile or first
         self._copy_late(self._late_copies)
         if not self._volatile:
-            self._remember(sig, launches, self._copies)
+            self._remember(sig, launches)
         return loss
 
     def _replay(self, recipe):
@@ -239,14 +229,12 @@ class ShardSGD(_ShardOptimizer):
         nothing done) when a group changed a scalar the launches were split by."""
         if recipe is None:
             return False
-        launches, copies, late = recipe
+        launches, late = recipe
         for _, _, key, slots in launches:
             for gi, _ in slots:
                 group = self.param_groups[gi]
                 if (group["momentum"], group["dampening"], bool(group["nesterov"])) != key:
                     return False
-        for tmp, g in copies:
-            tmp.copy_(g)
         for plan, args, _, slots in launches:
             for gi, slot in slots:
                 args.groups[slot].lr = float(self.param_groups[gi]["lr"])
@@ -279,7 +267,7 @@ class ShardAdam(_ShardOptimizer):
         sig = self._signature(pairs)
         if self._replay(self._recipes.get(sig)):
             return loss
-        self._copies, self._volatile, launches, self._late_copies = [], False, [], []
+        self._volatile, launches, self._late_copies = False, [], []
         batches = {}
         write_back = getattr(self, "_grad_scale", None) is not None     # a clipped step leaves the clipped gradients behind
         for gi, p, g in pairs:
@@ -311,7 +299,7 @@ class ShardAdam(_ShardOptimizer):
                 spans.append(sync.SpanSpec([g], agg_out=g if write_back else None, param=p.data.view(-1),
                                            state1=st["exp_avg"].view(-1), state2=st["exp_avg_sq"].view(-1),
                                            state3=st["max_exp_avg_sq"].view(-1) if amsgrad else None,
-                                           fanout=self._fanout(p), bounds=((0, slot),)))
+                                           fanout=self._fanout(p), bounds=((0, slot),), loose_grads=True))
             for (gi, step), slot in slots.items():
                 args.groups[slot].lr = float(self.param_groups[gi]["lr"])
                 args.groups[slot].weight_decay = float(self.param_groups[gi]["weight_decay"])
@@ -325,12 +313,9 @@ class ShardAdam(_ShardOptimizer):
                 reps.setdefault(slots[(gi, step)], (gi, st))
             launches.append((plan, args, (betas, eps, amsgrad), sorted(reps.items()),
                              [(st, slots[(gi, step)]) for gi, step, p, g, st in items]))
-        if write_back:
-            for tmp, g in self._copies:           # gradients that were realigned into a copy: the clipped values go back
-                g.copy_(tmp)
         self._copy_late(self._late_copies)
         if not self._volatile:
-            self._remember(sig, launches, self._copies)
+            self._remember(sig, launches)
         return loss
 
     def _replay(self, recipe):
@@ -339,7 +324,7 @@ class ShardAdam(_ShardOptimizer):
         step count no longer do (they were stepped apart in between)."""
         if recipe is None:
             return False
-        launches, copies, late = recipe
+        launches, late = recipe
         for _, _, key, reps, items in launches:
             for _, (gi, _) in reps:
                 group = self.param_groups[gi]
@@ -349,8 +334,6 @@ class ShardAdam(_ShardOptimizer):
             for st, slot in items:
                 if st["step"] != steps[slot]:
                     return False
-        for tmp, g in copies:
-            tmp.copy_(g)
         for plan, args, _, reps, items in launches:
             for st, _ in items:
                 st["step"] += 1
@@ -359,9 +342,6 @@ class ShardAdam(_ShardOptimizer):
                 args.groups[slot].weight_decay = float(self.param_groups[gi]["weight_decay"])
                 args.groups[slot].step = int(st["step"])
             plan.run(args)
-        if getattr(self, "_grad_scale", None) is not None:
-            for tmp, g in copies:
-                g.copy_(tmp)
         self._copy_late(late)
         return True
 

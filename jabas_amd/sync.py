@@ -267,15 +267,17 @@ class MomentArena:
 class SpanSpec:
     """Tensors of one span. All 1-D (or contiguous) with the same number of elements. ``moments=(arena,
     first)``: Adam's moments of the span are elements [first, first + n) of a ``MomentArena`` instead of the
-    tensors state1 / state2 / state3."""
+    tensors state1 / state2 / state3. ``loose_grads``: fp32 gradients (and an aggregate that is one of them) may sit at
+    any element, not only at the other buffers' position of a 16-byte line."""
 
     def __init__(self, grads, agg_out=None, param=None, state1=None, state2=None, fanout=(), bounds=(), state3=None,
-                 moments=None):
+                 moments=None, loose_grads=False):
         self.grads = list(grads)
         self.agg_out, self.param, self.state1, self.state2, self.state3 = agg_out, param, state1, state2, state3
         self.fanout = list(fanout)
         self.bounds = list(bounds)          # [(start_element, group), ...], first start 0
         self.moments = moments
+        self.loose_grads = loose_grads
         if moments is not None and (state1 is not None or state2 is not None or state3 is not None):
             raise ValueError("moments= stands for state1, state2 and state3: pass one or the other")
 
@@ -326,6 +328,7 @@ class SpanSpec:
         s.n_fanout = len(self.fanout)
         s.bound_begin = bound_begin
         s.bound_count = len(self.bounds)
+        s.reserved = L.SPAN_LOOSE_GRADS if self.loose_grads else 0
         return s
 
 

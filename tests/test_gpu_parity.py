@@ -1483,3 +1483,48 @@ def test_group_changes_and_ends_anywhere_in_a_wave(gpu, K, dtype, kind, level, s
             if level:
                 tol = 1e-11 if dtype == torch.float32 else 20 * 2.0 ** -24      # bf16: as in the test of split launches above
                 torch.testing.assert_close(row.reshape(-1)[1:4].cpu(), rows_h[0][1:4], rtol=tol, atol=0.0)
+
+
+@pytest.mark.parametrize("K,kind,level", [(1, "adamw", None), (1, "sgd", None), (3, "adam", "full"), (4, "adamw", "gram"), (12, "sgd", "similarity"),
+                                          (2, None, "similarity")])
+@pytest.mark.parametrize("n", [1, 5, 255, 1027, 70_003, 3_000_001])
+def test_loose_gradients_at_any_element(gpu, K, kind, level, n):
+    """Gradients (and an aggregate in one of them) at other positions of a 16-byte line than the buffers they update: aggregate,
+    weights and state bit for bit those of aligned ones, by value and as a plan; refused without the flag and for bf16."""
+    from jabas_amd import sync, _lib as L
+    opt = None if kind is None else dict(kind=kind, momentum=0.9, betas=(0.9, 0.999), eps=1e-8,
+                                         groups=[dict(lr=1e-2, weight_decay=0.05), dict(lr=3e-3, weight_decay=0.0)])
+    bounds = ((0, 0), (n // 3, 1)) if kind and n > 3 else ((0, 0),)
+    hg = _host_grads(K, n, 7)
+    start = [_host_state(n, 21 + j).abs() for j in range({None: 0, "sgd": 2}.get(kind, 3))]
+    args = sync.make_step_args(BATCHES[K], torch.float32, stats=level or False, opt=opt, step=3)
+
+    def step(at, out_at, plan, loose=True, dtype=torch.float32):
+        grads = [_dev(t.to(dtype), gpu, (at + 3 * k) % 7 if at else 0) for k, t in enumerate(hg)]
+        state = [_dev(t, gpu, 5 if at else 0) for t in start]
+        agg = grads[out_at] if isinstance(out_at, int) else _dev(torch.zeros(n), gpu, 5 if at else 0) if out_at else None
+        span = sync.SpanSpec(grads, agg_out=agg, bounds=bounds if kind else (), loose_grads=loose,
+                             **dict(zip(("param", "state1", "state2"), state)))
+        a = args if dtype == torch.float32 else sync.make_step_args(BATCHES[K], dtype, stats=level or False, opt=opt, step=3)
+        rows = sync.SyncPlan([span], sync.opt_kind(opt)).run(a) if plan else sync.sync_bucket(span, a)
+        torch.cuda.synchronize()
+        return [t for t in (agg, *state) if t is not None], rows, grads
+
+    for out_at in ("own", 0, K - 1, None) if kind else ("own", 0, K - 1):
+        want, rows, _ = step(0, out_at, False)
+        for at in (1, 2, 6):
+            for plan in (False, True):
+                got, loose_rows, grads = step(at, out_at, plan)
+                assert all(torch.equal(_bits(x), _bits(y)) for x, y in zip(got, want)), (out_at, at, plan)
+                if level:
+                    torch.testing.assert_close(loose_rows.reshape(-1), rows.reshape(-1), rtol=1e-11, atol=1e-25)
+                for k, t in enumerate(grads):
+                    if k != out_at:
+                        assert torch.equal(_bits(t), _bits(hg[k]))
+    with pytest.raises(L.JabasSyncError) as e:
+        step(2, "own", False, loose=False)
+    assert e.value.status == L.ERR_ALIGN
+    if K > 1:
+        with pytest.raises(L.JabasSyncError) as e:
+            step(2, "own", True, dtype=torch.bfloat16)
+        assert e.value.status == L.ERR_ALIGN
