@@ -136,8 +136,10 @@ JABAS_API int jabas_rdv_publish(JabasRendezvous* r, int32_t k, uint32_t bucket, 
             if (hipEventRecord(b->events[k], mine) != hipSuccess) return JABAS_ERR_LAUNCH;
             // The event covers what the stream's earlier ones cover: the launch waits once per stream. Four VSWs on one stream, the
             // 14 buckets of ViT-B/16: 836 -> 802 us.
-            for (int j = 0; j < r->K; ++j)
-                if ((b->recorded >> j & 1u) && b->streams[j] == mine) b->recorded &= ~(1u << j);
+            // Not for hipStreamPerThread: one handle, a stream of its own on every thread.
+            if (mine != hipStreamPerThread)
+                for (int j = 0; j < r->K; ++j)
+                    if ((b->recorded >> j & 1u) && b->streams[j] == mine) b->recorded &= ~(1u << j);
             b->recorded |= bit;
         }
         b->streams[k] = mine;
@@ -156,7 +158,7 @@ JABAS_API int jabas_rdv_publish(JabasRendezvous* r, int32_t k, uint32_t bucket, 
     }
     hipStream_t main = static_cast<hipStream_t>(launch_stream);
     for (int j = 0; j < r->K; ++j)
-        if ((recorded >> j & 1u) && snap.streams[j] != main)
+        if ((recorded >> j & 1u) && (snap.streams[j] != main || main == hipStreamPerThread))
             if (hipStreamWaitEvent(main, snap.events[j], 0) != hipSuccess) return JABAS_ERR_LAUNCH;
     JabasStepArgs a = *args;
     a.stats = want ? static_cast<uint32_t>(stats_level) : static_cast<uint32_t>(JABAS_STATS_NONE);

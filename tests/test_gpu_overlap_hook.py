@@ -716,3 +716,45 @@ def test_vsws_that_share_streams_are_waited_for(gpu, on):
         torch.cuda.synchronize()
         assert local.native_launches == step
         assert _same(bufs[0], O.aggregate(host, batches)), step
+
+
+@pytest.mark.parametrize("own_launch_stream", [True, False])
+def test_vsws_on_the_stream_of_their_thread_are_all_waited_for(gpu, own_launch_stream):
+    """hipStreamPerThread is one handle and a stream per thread: an event on one thread's covers nothing of another's, and a launch
+    on the completing thread's follows that one alone. Every gradient but the last is written late."""
+    import ctypes as C
+    from jabas_amd import _lib as L, sync
+    K, batches, n, per_thread = 3, (3, 2, 1), 300_001, 2
+    lib = L.lib()
+    bufs = [torch.zeros(n, device=gpu) for _ in range(K)]
+    busy = [torch.zeros(1 << 25, device=gpu) for _ in range(K)]
+    host = [torch.randn(n, generator=torch.Generator().manual_seed(k)) * 1e-3 for k in range(K)]
+    ready = [t.to(gpu) for t in host]
+    launch = torch.cuda.Stream(gpu).cuda_stream if own_launch_stream else per_thread
+    span, args, rdv = sync.SpanSpec(bufs, agg_out=bufs[0]).to_c(), sync.make_step_args(batches, torch.float32), C.c_void_p()
+    L.check(lib.jabas_rdv_create(K, C.byref(rdv)), "jabas_rdv_create")
+    L.check(lib.jabas_rdv_set_bucket(rdv, 0, C.byref(span), None, None, None, 0, 0), "jabas_rdv_set_bucket")
+    torch.cuda.synchronize()
+    codes, done = [], [threading.Event() for _ in range(K + 1)]
+
+    def vsw(k):
+        torch.cuda.set_device(gpu)
+        with torch.cuda.stream(torch.cuda.ExternalStream(per_thread, device=gpu)):
+            for _ in range(40 if k < K - 1 else 0):
+                busy[k].add_(1.0)
+            bufs[k].copy_(ready[k])
+            codes.append(lib.jabas_rdv_publish(rdv, k, 0, 0, per_thread, launch, C.byref(args), L.STATS_SIMILARITY))
+        done[k].set()
+        done[K].wait(60)                 # the thread's stream lives until the launch has run
+
+    threads = [threading.Thread(target=vsw, args=(k,)) for k in range(K)]
+    for k, t in enumerate(threads):
+        t.start()
+        assert done[k].wait(60)
+    torch.cuda.synchronize()
+    done[K].set()
+    for t in threads:
+        t.join()
+    lib.jabas_rdv_destroy(rdv)
+    assert codes == [L.RDV_WAITING] * (K - 1) + [L.RDV_LAUNCHED]
+    assert _same(bufs[0], O.aggregate(host, batches))
