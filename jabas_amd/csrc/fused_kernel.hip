@@ -288,10 +288,18 @@ template <bool SEARCH> struct GroupCursor {
 
 constexpr uint32_t kWaveElems = 256;             // of a tile: 64 lanes, four elements each
 
+// Whether elements of another group are jumped over, a branch per element, instead of going through the arithmetic and keeping
+// their values. That takes 5 to 15 registers less and 1 to 2.5 % more time (K = 1 Adam 160 M elements 717 -> 737 us; K = 5 and 6 bf16
+// with statistics, 40 M, 1 %), so only where it decides between one wave per SIMD and two: amsgrad with the pair products of eight
+// fp32 workers, 263 -> 248 registers, 40 M elements 576 -> 474 us, without an aggregate 518 -> 436.
+constexpr bool update_branches(int K, int DT, int OPT, int SL) {
+    return OPT == OPT_AMS && SL == JABAS_STATS_GRAM && DT == JABAS_F32 && K > 7;
+}
+
 // Optimizer step on the live elements [first, last) of a wave's share of a tile, group by group: almost always one. Elements of
-// another group go through the arithmetic too and keep their values (a branch per element instead saves up to ten registers and
-// loses 1 to 2.5 %: K = 1 Adam 160 M elements 717 -> 737 us). rel0: the wave's first element, in span coordinates.
-template <int OPT, int SL, class A, class C>
+// another group go through the arithmetic too and keep their values; BRANCH: they jump over it. rel0: the wave's first element, in
+// span coordinates.
+template <bool BRANCH, int OPT, int SL, class A, class C>
 __device__ __forceinline__ void update(const float (&agg)[4], f32x4& p, f32x4& s1, f32x4& s2, f32x4& s3, const A& a, C& cur,
                                        uint64_t rel0, uint32_t first, uint32_t last) {
     const uint32_t lane4 = (threadIdx.x & 63) * 4;
@@ -303,14 +311,16 @@ __device__ __forceinline__ void update(const float (&agg)[4], f32x4& p, f32x4& s
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const bool in = lane4 + i - first < upto - first;
-            float np = p[i], n1 = s1[i], n2 = 0.0f, n3 = 0.0f;
-            if constexpr (is_adam(OPT)) n2 = s2[i];
-            if constexpr (OPT == OPT_AMS) n3 = s3[i];
-            opt_elem<OPT>(agg[i], np, n1, n2, n3, cur.g, a.opt);
-            p[i] = in ? np : p[i];
-            s1[i] = in ? n1 : s1[i];
-            if constexpr (is_adam(OPT)) s2[i] = in ? n2 : s2[i];
-            if constexpr (OPT == OPT_AMS) s3[i] = in ? n3 : s3[i];
+            if (!BRANCH || in) {
+                float np = p[i], n1 = s1[i], n2 = 0.0f, n3 = 0.0f;
+                if constexpr (is_adam(OPT)) n2 = s2[i];
+                if constexpr (OPT == OPT_AMS) n3 = s3[i];
+                opt_elem<OPT>(agg[i], np, n1, n2, n3, cur.g, a.opt);
+                p[i] = in ? np : p[i];
+                s1[i] = in ? n1 : s1[i];
+                if constexpr (is_adam(OPT)) s2[i] = in ? n2 : s2[i];
+                if constexpr (OPT == OPT_AMS) s3[i] = in ? n3 : s3[i];
+            }
             if constexpr (SL) __builtin_amdgcn_sched_barrier(0);
         }
         if (upto == last) return;
@@ -365,7 +375,7 @@ __device__ __forceinline__ void consume(TileRegs<K, DT, U, OPT>& r, const SP& sp
         if (out) store_vec<NARROW, f32x4_a4>(f32x4{agg[0], agg[1], agg[2], agg[3]}, out, eu);
         if constexpr (OPT != OPT_NONE) {
             f32x4& s3 = r.s3[OPT == OPT_AMS ? u : 0];
-            update<OPT, SL>(agg, r.p[u], r.s1[u], r.s2[u], s3, a, cur, rel0 + u * TE, 0u, kWaveElems);
+            update<update_branches(K, DT, OPT, SL), OPT, SL>(agg, r.p[u], r.s1[u], r.s2[u], s3, a, cur, rel0 + u * TE, 0u, kWaveElems);
             store_vec<NARROW>(r.p[u], sp.p, eu);
             const uint64_t mu = is_adam(OPT) ? moment_index(sp, eu) : eu;
             if (use_s1) store_vec<NARROW>(r.s1[u], sp.s1, mu);
@@ -496,7 +506,7 @@ __device__ __forceinline__ void single_tile(const SP& sp, uint64_t tile_e0, cons
     }
     float agg[4];
     aggregate<K, DT, SL, HD>(r.g[0], agg, a, clip, acc);
-    if constexpr (OPT != OPT_NONE) update<OPT, SL>(agg, r.p[0], r.s1[0], r.s2[0], r.s3[0], a, cur, wave_e - sp.lo, w.first, w.last);
+    if constexpr (OPT != OPT_NONE) update<update_branches(K, DT, OPT, SL), OPT, SL>(agg, r.p[0], r.s1[0], r.s2[0], r.s3[0], a, cur, wave_e - sp.lo, w.first, w.last);
     if (whole) {
         if (out) store_at<f32x4_a4>(f32x4{agg[0], agg[1], agg[2], agg[3]}, out, w.e, at);
         if constexpr (OPT != OPT_NONE) {

@@ -1445,7 +1445,7 @@ def test_aggregate_of_one_worker_over_its_own_buffer(gpu, numel, kind, weight, s
 
 @pytest.mark.parametrize("K,dtype,kind,level", [(1, torch.float32, "adam", None), (3, torch.float32, "sgd", None), (4, torch.float32, "adamw", "similarity"),
                                                 (8, torch.bfloat16, "adamw", "gram"), (8, torch.float32, "sgd", "gram"),
-                                                (13, torch.float32, "adam", "full"), (16, torch.bfloat16, "adamw_amsgrad", "full")])
+                                                (8, torch.float32, "adamw_amsgrad", "gram"), (13, torch.float32, "adam", "full"), (16, torch.bfloat16, "adamw_amsgrad", "full")])
 @pytest.mark.parametrize("skew", [0, 1, 63])
 def test_group_changes_and_ends_anywhere_in_a_wave(gpu, K, dtype, kind, level, skew):
     """Parameter groups that change at every place a wave's 256 elements can have it (inside a thread's four elements, between
