@@ -110,6 +110,18 @@ __host__ __device__ constexpr int shape_level(int stats) { return stats == JABAS
 //                       302 -> 284, K = 16 fp32 AdamW 406 -> 390. Not bf16 gradients without an optimizer, whose reads alone are
 //                       at the rate of memory: K = 12 / 16, 25 M 102 / 138 -> 113 / 162. K = 5..8 would gain 2-3 % with full
 //                       rows and lose 11-14 % with pair products (25..40 sums per workgroup), and both levels cut their sums alike
+//   with an optimizer,  the same for the same reason (one tile in flight, a chunk of two tiles) without statistics from 2048 chunks
+//   K > 8               and with similarity sums from 4096 on. Engine steps of 100 tensors, whole chunks -> two workgroups each, fp32 K = 9 /
+//                       12 / 16 AdamW with an aggregate, 6 M elements 67 / 80 / 98 -> 65 / 77 / 95 us, 20 M 216 / 259 / 319 -> 210 / 253 / 314,
+//                       K = 16 SGD 100 M 1500 -> 1440; bf16 K = 16 AdamW amsgrad 40 M 463 -> 446; similarity sums, K = 12 fp32 SGD 20 M
+//                       248 -> 240, bf16 K = 16 SGD 40 M 365 -> 353. Below, nothing is gained (plain 3 M) or bf16 loses up to 4 %
+//                       (similarity sums 6 M, AdamW 68.5 -> 70.5)
+#ifndef JABAS_SPLIT_FROM_PLAIN
+#define JABAS_SPLIT_FROM_PLAIN 2048
+#endif
+#ifndef JABAS_SPLIT_FROM_SIM
+#define JABAS_SPLIT_FROM_SIM 4096
+#endif
 #ifndef JABAS_SPLIT_BELOW
 #define JABAS_SPLIT_BELOW 448
 #endif
@@ -132,7 +144,10 @@ inline uint32_t launch_split_log2(int K, int grad_dtype, int opt_class, int stat
         const uint64_t idle = (n_chunks << s) - live(s);
         return (n_chunks << s) <= 256 || idle <= empty || 3 * idle <= live(s);
     };
-    uint32_t s = stats == JABAS_STATS_FULL && K > 8 && (opt_class != 0 || grad_dtype == JABAS_F32) && pays(1) ? 1 : 0;
+    const bool rows = stats == JABAS_STATS_FULL && (opt_class != 0 || grad_dtype == JABAS_F32);
+    const bool long_step = opt_class != 0 && ((stats == JABAS_STATS_NONE && n_chunks >= JABAS_SPLIT_FROM_PLAIN) ||
+                                              (stats == JABAS_STATS_SIMILARITY && n_chunks >= JABAS_SPLIT_FROM_SIM));
+    uint32_t s = K > 8 && (rows || long_step) && pays(1) ? 1 : 0;
     while ((2u << s) <= tiles && live(s) < below && pays(s + 1)) ++s;
     return s;
 }

@@ -1379,6 +1379,54 @@ def test_split_launches_of_every_kind(gpu, K, dtype, kind, level, numel):
                 torch.testing.assert_close(row[4:4 + K], norms, rtol=tol, atol=0.0)
 
 
+@pytest.mark.parametrize("K,dtype,kind,level", [(9, torch.float32, "adam", None), (16, torch.bfloat16, "sgd", None), (12, torch.bfloat16, "adamw_amsgrad", None),
+                                                (9, torch.bfloat16, "adamw", "similarity"), (16, torch.float32, "sgd", "similarity")])
+@pytest.mark.parametrize("off_by", [-1, 1, 2049])
+def test_long_steps_of_many_workers(gpu, K, dtype, kind, level, off_by):
+    """On both sides of the length from which two workgroups share a chunk (2048 elements; from 2048 chunks on, with similarity sums
+    4096): weights, state and aggregate bit for bit those of three shorter launches, by value and as a plan, on the scratch that the
+    sizing function names and on the least, which holds whole chunks only."""
+    from jabas_amd import sync, _lib as L
+    chunks = 4096 if level else 2048
+    n = (chunks - 1) * 2048 + off_by
+    gen = torch.Generator(device=gpu).manual_seed(K + off_by)
+    grads = [torch.randn(n, generator=gen, device=gpu).to(dtype) for _ in range(K)]
+    start = [torch.randn(n, generator=gen, device=gpu) * 0.1 for _ in range(2)] + [torch.rand(n, generator=gen, device=gpu) * 0.1 for _ in range(2)]
+    start = start[:{"sgd": 2, "adamw_amsgrad": 4}.get(kind, 3)]
+    opt = dict(kind=kind.replace("_amsgrad", ""), amsgrad="amsgrad" in kind, momentum=0.9, betas=(0.9, 0.999), eps=1e-8,
+               groups=[dict(lr=1e-2, weight_decay=0.05), dict(lr=3e-3, weight_decay=0.0)])
+    change = n // 2 + 77
+
+    def launch(cuts, plan, scratch=None):
+        state, agg, rows = [t.clone() for t in start], torch.zeros(n, device=gpu), []
+        args = sync.make_step_args((1,) * K, dtype, stats=level or False, opt=opt, step=3)
+        for a, b in zip(cuts, cuts[1:]):
+            bounds = ((0, 0), (change - a, 1)) if a < change < b else ((0, int(a >= change)),)
+            span = sync.SpanSpec([g[a:b] for g in grads], agg_out=agg[a:b], bounds=bounds,
+                                 **dict(zip(("param", "state1", "state2", "state3"), (t[a:b] for t in state))))
+            if plan:
+                row = sync.SyncPlan([span], sync.opt_kind(opt)).run(args)
+            else:
+                ws = sync.Workspace.for_span(b - a, dtype, gpu)
+                ws.nbytes = scratch or ws.nbytes
+                row = sync.sync_bucket(span, args, workspace=ws)
+            if level:
+                rows.append(row.reshape(-1)[:4].clone())
+        return [agg, *state], sum(rows) if level else None
+
+    want, sums = launch((0, n // 3 + 1, 2 * n // 3 + 2, n), False)
+    ways = [launch((0, n), False), launch((0, n), True)]
+    if level:
+        ways.append(launch((0, n), False, scratch=(-(-n // 2048) + 33) * 4 * 8))    # a row per chunk, 33 for the finalize
+    for got, row in ways:
+        assert all(torch.equal(_bits(x), _bits(y)) for x, y in zip(got, want))
+        if level:
+            # as in the test of split launches above; the product of the halves against the size of its terms
+            tol = 1e-12 if dtype == torch.float32 else 20 * 2.0 ** -24
+            torch.testing.assert_close(row[1:], sums[1:], rtol=tol, atol=0.0)
+            assert abs(float(row[0] - sums[0])) <= tol * float((sums[1] * sums[2]).sqrt())
+
+
 @pytest.mark.parametrize("K,dtype,numel,levels", [(8, torch.bfloat16, 1_200_011, ("full", "gram")),
                                                   (4, torch.float32, 700_001, ("similarity", "full", "gram"))])
 def test_levels_share_their_bits_on_any_scratch(gpu, K, dtype, numel, levels):
