@@ -97,9 +97,11 @@ __host__ __device__ constexpr int shape_level(int stats) { return stats == JABAS
 //                       2048 without statistics, 1 to 4 M elements lose: K = 4 AdamW 2 / 3 / 4 M 17.9 / 25.1 / 32.7 -> 19.0 / 27.5 /
 //                       35.8, K = 8 bf16 aggregate 4 M 15.4 -> 18.0; while fewer than 512, 2 M 18.9, and K = 8 pair products 0.9 M
 //                       0.90 of the time of whole chunks against 0.74
-//   group changes       in a span (norms and biases between the weights): up to 2048 and 512. Engine steps while a tile
-//                       with a change took many times as long as the others, up to 448 -> up to 2048: K = 2 fp32 AdamW 2.3 M in 293 tensors 26.1 -> 20.0 us, K = 1 4.0 M in 85 30.5 -> 25.7, K = 4
-//                       6.4 M in 117 71.1 -> 66.1, K = 4 3.0 M in 23 26.1 -> 24.9; K = 6 full rows 1.0 M in 153 20.7 -> 18.6
+//   group changes       in a span (norms and biases between the weights): up to 512 with statistics; without, up to 640 where chunks
+//                       are whole loads of few streams (up to four fp32 workers, three or four bf16 ones), 2048 otherwise. Up to 2048
+//                       for all, from when a tile with a change took many times as long as the others -> these, engine steps of
+//                       100 tensors: K = 1 fp32 AdamW 3 M 18.6 -> 17.0 us, K = 2 amsgrad 4 M without an aggregate 33.7 -> 30.7, K = 4 fp32 AdamW 2 M 18.7 -> 18.2,
+//                       bf16 amsgrad 3 M 26.9 -> 23.8. With 640 for the others K = 16 4 M loses 5 %, K = 1 bf16 amsgrad 4 M 8 %
 //   without a tile      at most a quarter, or 64 with statistics (each still runs its epilogue and writes a row) and 256 without, or as
 //                       many as there are compute units for: plans over short spans, one per small tensor, whose last chunk is
 //                       mostly their only one. All splits -> these: 500 spans of 700 elements, K = 1 AdamW 7.7 -> 4.4 us, 20000, K = 16
@@ -129,7 +131,10 @@ __host__ __device__ constexpr int shape_level(int stats) { return stats == JABAS
 #define JABAS_SPLIT_BELOW_STATS 384
 #endif
 #ifndef JABAS_SPLIT_BELOW_GROUPS
-#define JABAS_SPLIT_BELOW_GROUPS 2048
+#define JABAS_SPLIT_BELOW_GROUPS 640
+#endif
+#ifndef JABAS_SPLIT_BELOW_GROUPS_MANYK
+#define JABAS_SPLIT_BELOW_GROUPS_MANYK 2048
 #endif
 #ifndef JABAS_SPLIT_BELOW_GROUPS_STATS
 #define JABAS_SPLIT_BELOW_GROUPS_STATS 512
@@ -137,7 +142,8 @@ __host__ __device__ constexpr int shape_level(int stats) { return stats == JABAS
 template <class Live>
 inline uint32_t launch_split_log2(int K, int grad_dtype, int opt_class, int stats, uint64_t n_chunks, bool group_changes, const Live& live) {
     const uint32_t tiles = static_cast<uint32_t>(launch_chunk_tiles(K, grad_dtype, opt_class, stats));
-    const uint64_t below = group_changes ? (stats ? JABAS_SPLIT_BELOW_GROUPS_STATS : JABAS_SPLIT_BELOW_GROUPS)
+    const bool few = K <= 4 && (grad_dtype == JABAS_F32 || K > 2);
+    const uint64_t below = group_changes ? (stats ? JABAS_SPLIT_BELOW_GROUPS_STATS : few ? JABAS_SPLIT_BELOW_GROUPS : JABAS_SPLIT_BELOW_GROUPS_MANYK)
                                          : (stats ? JABAS_SPLIT_BELOW_STATS : JABAS_SPLIT_BELOW);
     const uint64_t empty = stats ? 64 : 256;
     const auto pays = [&](uint32_t s) {
