@@ -18,11 +18,6 @@ from .. import _lib as L
 from .. import sync
 
 
-def _index_of(t):
-    idx = getattr(t, "index", None)       # the attribute the reference sets; anything callable is not it
-    return idx if isinstance(idx, int) else None
-
-
 class _ShardOptimizer(torch.optim.Optimizer):
     _kind = None
     _max_cached_plans = 1024       # one per distinct call (a DDP bucket each in the overlap mode): a few KB of tables apiece
@@ -86,13 +81,23 @@ class _ShardOptimizer(torch.optim.Optimizer):
     # A training loop hands step() the same parameters and the same gradient buffers every iteration
     # (DDP bucket views keep their addresses). Matching, validating and marshalling ~150 tensors costs
     # more host time than the launch takes on the GPU, so a call that found every state in place is
-    # remembered under its signature, and repeated calls only refresh the launch scalars.
-    def _signature(self, pairs):
-        rep = self._replicas
-        if not rep:
-            return tuple([(p.data_ptr(), g.data_ptr(), g.numel()) for _, p, g in pairs])
-        return tuple([(p.data_ptr(), g.data_ptr(), g.numel()) + tuple(q.data_ptr() for q in rep.get(id(p), ()))
-                      for _, p, g in pairs])
+    # remembered under its signature, and repeated calls only refresh the launch scalars. The signature
+    # names everything else that the launches were prepared from: each parameter's group, the memory of
+    # the weight, the gradient, the state and the replicas, and the clipping coefficient. The state is looked
+    # up anew by every call (``states``, one per pair) and nothing of it is kept.
+    def _signature(self, pairs, states):
+        scale, memory = getattr(self, "_grad_scale", None), torch.Tensor.data_ptr
+        params, grads = [p for _, p, _ in pairs], [g for _, _, g in pairs]
+        sig = [None if scale is None else scale.data_ptr(), tuple([gi for gi, _, _ in pairs]), *map(memory, params), *map(memory, grads),
+               *map(torch.Tensor.numel, grads), *map(torch.Tensor.is_contiguous, grads)]
+        for name in self._state_names():
+            try:
+                sig += list(map(memory, [st[name] for st in states]))
+            except (KeyError, TypeError):         # not every parameter has one
+                sig += [memory(st[name]) if st and st.get(name) is not None else None for st in states]
+        if self._replicas:
+            sig += [tuple([q.data_ptr() for q in self._replicas.get(id(p), ())]) for p in params]
+        return tuple(sig)
 
     def _remember(self, sig, launches):
         if len(self._recipes) >= self._max_cached_plans:
@@ -117,15 +122,15 @@ class _ShardOptimizer(torch.optim.Optimizer):
             return out
         by_index = {}
         for g in gradients:
-            idx = _index_of(g)
-            if idx is None:
+            idx = getattr(g, "index", None)       # the attribute the reference sets; anything callable is not it
+            if not isinstance(idx, int):
                 raise ValueError("step(gradients): every gradient needs an .index attribute naming its parameter")
             by_index[idx] = g
         for gi, group in enumerate(self.param_groups):
             for p in group["params"]:
-                g = by_index.get(_index_of(p))
-                if g is not None and _index_of(p) is not None:
-                    out.append((gi, p, g))
+                idx = getattr(p, "index", None)
+                if isinstance(idx, int) and idx in by_index:
+                    out.append((gi, p, by_index[idx]))
         return out
 
     @staticmethod
@@ -147,7 +152,8 @@ class _ShardOptimizer(torch.optim.Optimizer):
 
     def _launch(self, spans, args):
         key = (args.opt_kind,) + tuple((s.grads[0].data_ptr(), s.param.data_ptr(), s.grads[0].numel(), s.bounds[0][1],
-                                         s.agg_out is not None) + tuple(f.data_ptr() for f in s.fanout) for s in spans)
+                                         s.agg_out is not None, *[t.data_ptr() for t in (s.state1, s.state2, s.state3) if t is not None])
+                                        + tuple(f.data_ptr() for f in s.fanout) for s in spans)
         plan = self._plans.get(key)
         if plan is None:
             if len(self._plans) >= self._max_cached_plans:
@@ -170,6 +176,9 @@ class _ShardOptimizer(torch.optim.Optimizer):
 
 
 class ShardSGD(_ShardOptimizer):
+    def _state_names(self):
+        return ("momentum_buffer",)
+
     def __init__(self, params, lr, momentum=0, dampening=0, weight_decay=0, nesterov=False):
         if lr < 0.0:
             raise ValueError("Invalid learning rate: {}".format(lr))
@@ -186,8 +195,9 @@ class ShardSGD(_ShardOptimizer):
     def step(self, gradients=None, closure=None):
         loss = closure() if closure is not None else None
         pairs = self._pairs(gradients)
-        sig = self._signature(pairs)
-        if self._replay(self._recipes.get(sig)):
+        states = list(map(self.state.get, [p for _, p, _ in pairs]))
+        sig = self._signature(pairs, states)
+        if self._replay(self._recipes.get(sig), states):
             return loss
         self._volatile, launches, self._late_copies = False, [], []
         # launches are split by (momentum, dampening, nesterov, first-step): launch-wide scalars
@@ -224,7 +234,7 @@ class ShardSGD(_ShardOptimizer):
             self._remember(sig, launches)
         return loss
 
-    def _replay(self, recipe):
+    def _replay(self, recipe, states):
         """Repeats a remembered call with the hyperparameters as the groups hold them now. False (and
         nothing done) when a group changed a scalar the launches were split by."""
         if recipe is None:
@@ -260,17 +270,21 @@ class ShardAdam(_ShardOptimizer):
             raise ValueError("Invalid weight_decay value: {}".format(weight_decay))
         super().__init__(params, dict(lr=lr, betas=betas, eps=eps, weight_decay=weight_decay, amsgrad=amsgrad))
 
+    def _state_names(self):
+        return ("exp_avg", "exp_avg_sq", "max_exp_avg_sq") if any(g["amsgrad"] for g in self.param_groups) else ("exp_avg", "exp_avg_sq")
+
     @torch.no_grad()
     def step(self, gradients=None, closure=None):
         loss = closure() if closure is not None else None
         pairs = self._pairs(gradients)
-        sig = self._signature(pairs)
-        if self._replay(self._recipes.get(sig)):
+        states = list(map(self.state.get, [p for _, p, _ in pairs]))
+        sig = self._signature(pairs, states)
+        if self._replay(self._recipes.get(sig), states):
             return loss
         self._volatile, launches, self._late_copies = False, [], []
         batches = {}
         write_back = getattr(self, "_grad_scale", None) is not None     # a clipped step leaves the clipped gradients behind
-        for gi, p, g in pairs:
+        for at, (gi, p, g) in enumerate(pairs):
             group = self.param_groups[gi]
             amsgrad = bool(group["amsgrad"])
             st = self.state[p]
@@ -285,14 +299,14 @@ class ShardAdam(_ShardOptimizer):
                 raise RuntimeError("amsgrad was switched on after the state was created: no max_exp_avg_sq to continue from")
             st["step"] += 1
             key = (tuple(group["betas"]), group["eps"], amsgrad)
-            batches.setdefault(key, []).append((gi, int(st["step"]), p, self._prepare(p, g), st))
+            batches.setdefault(key, []).append((gi, int(st["step"]), p, self._prepare(p, g), st, at))
         for (betas, eps, amsgrad), items in batches.items():
             slots, spans = {}, []
             if amsgrad:
                 args = self._new_args(L.OPT_ADAMW_AMSGRAD if self._adamw else L.OPT_ADAM_AMSGRAD)
             else:
                 args = self._new_args(L.OPT_ADAMW if self._adamw else L.OPT_ADAM)
-            for gi, step, p, g, st in items:
+            for gi, step, p, g, st, _ in items:
                 slot = slots.setdefault((gi, step), len(slots))
                 if slot >= L.MAX_GROUPS:
                     raise RuntimeError(f"more than {L.MAX_GROUPS} (group, step) combinations in one launch")
@@ -307,40 +321,39 @@ class ShardAdam(_ShardOptimizer):
             args.n_groups = len(slots)
             args.beta1, args.beta2, args.eps = float(betas[0]), float(betas[1]), float(eps)
             plan = self._launch(spans, args)
-            # per slot: its group and one state that carries the slot's step count; per item: state and slot
-            reps = {}
-            for gi, step, p, g, st in items:
-                reps.setdefault(slots[(gi, step)], (gi, st))
-            launches.append((plan, args, (betas, eps, amsgrad), sorted(reps.items()),
-                             [(st, slots[(gi, step)]) for gi, step, p, g, st in items]))
+            # per slot: its group and the places among the pairs of the parameters that share its step count
+            places = {}
+            for gi, step, p, g, st, at in items:
+                places.setdefault(slots[(gi, step)], (gi, []))[1].append(at)
+            launches.append((plan, args, (betas, eps, amsgrad), [(slot, gi, at) for slot, (gi, at) in places.items()]))
         self._copy_late(self._late_copies)
         if not self._volatile:
             self._remember(sig, launches)
         return loss
 
-    def _replay(self, recipe):
+    def _replay(self, recipe, states):
         """Repeats a remembered call: bumps every parameter's step count and refreshes the launch scalars.
         False (and nothing done) when betas / eps of a group changed or when parameters that shared a
         step count no longer do (they were stepped apart in between)."""
         if recipe is None:
             return False
         launches, late = recipe
-        for _, _, key, reps, items in launches:
-            for _, (gi, _) in reps:
+        for _, _, key, slots in launches:
+            for _, gi, places in slots:
                 group = self.param_groups[gi]
                 if (tuple(group["betas"]), group["eps"], bool(group["amsgrad"])) != key:
                     return False
-            steps = [st["step"] for _, (_, st) in reps]
-            for st, slot in items:
-                if st["step"] != steps[slot]:
+                steps = [states[at]["step"] for at in places]
+                if steps.count(steps[0]) != len(steps):
                     return False
-        for plan, args, _, reps, items in launches:
-            for st, _ in items:
-                st["step"] += 1
-            for slot, (gi, st) in reps:
+        for plan, args, _, slots in launches:
+            for slot, gi, places in slots:
+                step = states[places[0]]["step"] + 1
+                for at in places:
+                    states[at]["step"] = step
                 args.groups[slot].lr = float(self.param_groups[gi]["lr"])
                 args.groups[slot].weight_decay = float(self.param_groups[gi]["weight_decay"])
-                args.groups[slot].step = int(st["step"])
+                args.groups[slot].step = int(step)
             plan.run(args)
         self._copy_late(late)
         return True

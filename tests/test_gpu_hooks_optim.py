@@ -903,3 +903,70 @@ def test_trainer_parameter_that_no_micro_batch_reaches(gpu):
     for p, b, buf in zip(main.idle.parameters(), idle_before, momentum):
         want = b.reshape(-1) - 0.05 * (0.9 * buf) - 0.05 * (0.81 * buf)
         assert torch.allclose(p.reshape(-1), want, rtol=1e-5, atol=1e-8)
+
+
+@pytest.mark.parametrize("bounds", [(float("inf"), 1e-2, float("inf"), 3e-3), (1e-2, float("inf"), 1e-2, float("inf"))])
+def test_shard_optimizer_remembered_calls_follow_the_norm_bound(gpu, bounds):
+    """grad_clip switched on and off between calls over the same buffers: a remembered call is not repeated for another kind of
+    step (torch.nn.utils.clip_grad_norm_ and torch.optim.Adam on a twin; a step without a bound leaves its gradients alone)."""
+    from jabas_amd import optim
+    model, ref_model = _mlp(5).to(gpu), _mlp(5).to(gpu)
+    mine = optim.ShardGNMTAdam(model.parameters(), lr=2e-3)
+    ref = torch.optim.Adam(ref_model.parameters(), lr=2e-3, foreach=False)
+    for p in model.parameters():
+        p.grad = torch.empty_like(p)
+    for step in range(4 * len(bounds)):
+        mine.grad_clip = bounds[step // 4]
+        for i, (p, rp) in enumerate(zip(model.parameters(), ref_model.parameters())):
+            p.grad.copy_(torch.randn(p.shape, generator=torch.Generator().manual_seed(50 * step + i)) * 1e-2)
+            rp.grad = p.grad.clone()
+        if mine.grad_clip != float("inf"):
+            torch.nn.utils.clip_grad_norm_(ref_model.parameters(), mine.grad_clip, foreach=False)
+        ref.step()
+        mine.step()
+        torch.cuda.synchronize()
+        for p, rp in zip(model.parameters(), ref_model.parameters()):
+            assert _close(p.grad, rp.grad, 1e-6, 1e-12), (step, mine.grad_clip)
+            assert _close(p, rp, 1e-6, 1e-8), (step, mine.grad_clip)
+
+
+@pytest.mark.parametrize("kind", ["sgd", "adamw", "adamw_amsgrad"])
+def test_shard_optimizer_remembered_calls_follow_the_state(gpu, kind):
+    """State cleared, replaced tensor by tensor, replaced as a whole, and moved to other memory by .data, between calls over the same
+    buffers: the next call works on the state as it is then (torch.optim on a twin whose state is handled alike)."""
+    from jabas_amd import optim
+    model, ref_model = _mlp(6).to(gpu), _mlp(6).to(gpu)
+    if kind == "sgd":
+        mine, ref = optim.ShardSGD(model.parameters(), lr=0.05, momentum=0.9), torch.optim.SGD(ref_model.parameters(), lr=0.05, momentum=0.9, foreach=False)
+    else:
+        mine = optim.ShardAdamW(model.parameters(), lr=1e-3, amsgrad=kind.endswith("amsgrad"))
+        ref = torch.optim.AdamW(ref_model.parameters(), lr=1e-3, amsgrad=kind.endswith("amsgrad"), foreach=False)
+    names = ("momentum_buffer",) if kind == "sgd" else ("exp_avg", "exp_avg_sq") + (("max_exp_avg_sq",) if kind.endswith("amsgrad") else ())
+    for p in model.parameters():
+        p.grad = torch.empty_like(p)
+    for step in range(16):
+        for i, (p, rp) in enumerate(zip(model.parameters(), ref_model.parameters())):
+            p.grad.copy_(torch.randn(p.shape, generator=torch.Generator().manual_seed(70 * step + i)) * 1e-2)
+            rp.grad = p.grad.clone()
+        for opt in (mine, ref):
+            if step == 4:
+                opt.state.clear()
+            for p in opt.param_groups[0]["params"] if step in (8, 11, 13) else ():
+                if step == 8:
+                    for name in names:
+                        opt.state[p][name] = opt.state[p][name] * 0.5
+                elif step == 11:
+                    opt.state[p] = dict(opt.state[p])
+                else:
+                    for name in names:
+                        opt.state[p][name].data = opt.state[p][name].data * 2.0
+        ref.step()
+        mine.step()
+        torch.cuda.synchronize()
+        for p, rp in zip(model.parameters(), ref_model.parameters()):
+            assert _close(p, rp, 1e-6, 1e-8), (kind, step)
+            for name in names:
+                # first moments cancel: three roundings of up to 0.02 * 2^-24 a step, each forgotten by 0.9 a step
+                assert _close(mine.state[p][name], ref.state[rp][name], 1e-6, 4e-8 if name == "exp_avg" else 1e-14), (kind, step, name)
+        if kind != "sgd":
+            assert all(int(mine.state[p]["step"]) == int(ref.state[rp]["step"]) for p, rp in zip(model.parameters(), ref_model.parameters()))
