@@ -392,24 +392,23 @@ class SyncPlan:
             all_bounds += sp.bounds
         c_bounds = _bounds_array(all_bounds)
         nbytes = lib.jabas_plan_bytes(c_spans, n_span, len(all_bounds), grad_dtype_code(gdt))
-        self._host = np.zeros((nbytes + 7) // 8, dtype=np.uint64)        # 8-byte aligned blob
+        self._host = torch.from_numpy(np.zeros((nbytes + 7) // 8, dtype=np.int64))       # 8-byte aligned blob
         L.check(lib.jabas_plan_encode(c_spans, n_span, c_bounds if all_bounds else None, len(all_bounds),
                                       self.K, grad_dtype_code(gdt), opt_kind_code,
-                                      self._host.ctypes.data, nbytes), "jabas_plan_encode")
+                                      self._host.data_ptr(), nbytes), "jabas_plan_encode")
         # chunks, of which the launch gives each one, two or four workgroups
-        self.n_chunks = int(lib.jabas_plan_chunks(self._host.ctypes.data, 0))            # of a plain launch
-        self.n_chunks_stats = int(lib.jabas_plan_chunks(self._host.ctypes.data, 1))      # of a launch with full statistics rows
-        self.n_chunks_similarity = int(lib.jabas_plan_chunks(self._host.ctypes.data, 2)) # of a launch with similarity sums
-        self._dev = torch.from_numpy(self._host.view(np.int64)).to(dev)
-        self.ws = Workspace(lib.jabas_plan_workspace_bytes(self._host.ctypes.data), n_span, dev)
+        self.n_chunks = int(lib.jabas_plan_chunks(self._host.data_ptr(), 0))            # of a plain launch
+        self.n_chunks_stats = int(lib.jabas_plan_chunks(self._host.data_ptr(), 1))      # of a launch with full statistics rows
+        self.n_chunks_similarity = int(lib.jabas_plan_chunks(self._host.data_ptr(), 2)) # of a launch with similarity sums
+        self._dev = self._host.to(dev)
+        self.ws = Workspace(lib.jabas_plan_workspace_bytes(self._host.data_ptr()), n_span, dev)
         self.n_span = n_span
-        self._ptrs = (self._host.ctypes.data, self._dev.data_ptr())
 
     def run(self, args, stream=None):
         """Queues aggregate (+stats, +optimizer) over every span. Returns the stats tensor
         (n_span x STATS_STRIDE doubles, device) when args.stats is set, else None."""
         ws = self.ws
-        L.check(L.lib().jabas_sync_fused(*self._ptrs, C.byref(args), ws.stats.data_ptr() if args.stats else None,
+        L.check(L.lib().jabas_sync_fused(self._host.data_ptr(), self._dev.data_ptr(), C.byref(args), ws.stats.data_ptr() if args.stats else None,
                                          ws.buf.data_ptr(), ws.nbytes, _stream_ptr(stream)), "jabas_sync_fused")
         return ws.stats if args.stats else None
 

@@ -1576,3 +1576,28 @@ def test_loose_gradients_at_any_element(gpu, K, kind, level, n):
         with pytest.raises(L.JabasSyncError) as e:
             step(2, "own", True, dtype=torch.bfloat16)
         assert e.value.status == L.ERR_ALIGN
+
+
+def test_a_copy_of_a_plan_outlives_the_plan(gpu):
+    """copy.deepcopy of a plan carries its own tables, on the host and on the device: it runs after the plan it was made of is gone
+    and its memory holds something else."""
+    import copy
+    import gc
+    from jabas_amd import sync
+    K, n = 3, 70_001
+    hg = _host_grads(K, n, 3)
+    grads, out = [_dev(t, gpu) for t in hg], torch.zeros(n, device=gpu)
+    plan = sync.SyncPlan([sync.SpanSpec([g[a:b] for g in grads], agg_out=out[a:b]) for a, b in ((0, 30_004), (30_004, n))])
+    size = plan._dev.numel()
+    twin = copy.deepcopy(plan)
+    del plan
+    gc.collect()
+    torch.cuda.synchronize()
+    overwritten = [torch.zeros(size, dtype=torch.int64, device=gpu) for _ in range(64)]
+    for seed in (3, 4):
+        for g, t in zip(grads, _host_grads(K, n, seed)):
+            g.copy_(t)
+        twin.run(sync.make_step_args(BATCHES[K], torch.float32))
+        torch.cuda.synchronize()
+        assert torch.equal(_bits(out), _bits(O.aggregate(_host_grads(K, n, seed), BATCHES[K])))
+    assert all(not bool(t.any()) for t in overwritten)
