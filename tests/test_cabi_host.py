@@ -627,6 +627,66 @@ def test_rendezvous_calls_validate_their_arguments():
     assert b"rendezvous" in lib.jabas_status_string(L.ERR_STATE)
 
 
+_HIP_RECORDER = r"""
+#include "rendezvous.hip"
+#include <string>
+static std::string g_log;
+static long g_events = 0;
+extern "C" {
+hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
+hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) { *e = reinterpret_cast<hipEvent_t>(++g_events); return hipSuccess; }
+hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
+    g_log += "record " + std::to_string(reinterpret_cast<long>(e)) + " " + std::to_string(reinterpret_cast<long>(s)) + "\n"; return hipSuccess; }
+hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t e, unsigned) {
+    g_log += "wait " + std::to_string(reinterpret_cast<long>(e)) + " " + std::to_string(reinterpret_cast<long>(s)) + "\n"; return hipSuccess; }
+int jabas_sync_bucket(const JabasSpan*, const JabasBound*, const JabasStepArgs*, double*, void*, size_t, jabas_stream_t s) {
+    g_log += "launch 0 " + std::to_string(reinterpret_cast<long>(s)) + "\n"; return 0; }
+const char* take_log() { static std::string out; out = g_log; g_log.clear(); return out.c_str(); }
+}
+"""
+
+
+def test_rendezvous_waits_for_every_hand_over_whatever_the_streams_are_called(tmp_path):
+    """The host code of the meeting point over a recorder in place of the HIP runtime: the launch is preceded by a wait for the event
+    of every hand-over, also where hand-overs, or one of them and the launch, name the same stream handle. The handle of a stream that
+    was destroyed after its hand-over may name a new stream by then, and hipStreamPerThread (2) names one per thread."""
+    import itertools
+    import shutil
+    import subprocess
+    if shutil.which("g++") is None:
+        pytest.skip("no g++")
+    src, so = tmp_path / "recorder.cpp", str(tmp_path / "recorder.so")
+    src.write_text(_HIP_RECORDER)
+    r = subprocess.run(["g++", "-std=c++17", "-shared", "-fPIC", "-Wno-attributes", "-D__HIP_PLATFORM_AMD__", "-I", "/opt/rocm/include",
+                        "-I", os.path.join(ROOT, "include"), "-I", os.path.join(ROOT, "jabas_amd", "csrc"), str(src), "-o", so,
+                        "-Wl,-Bsymbolic"], capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr
+    rec = C.CDLL(so)
+    for name, (res, argtypes) in L.SIGNATURES.items():
+        if name.startswith("jabas_rdv_"):
+            getattr(rec, name).restype, getattr(rec, name).argtypes = res, argtypes
+    rec.take_log.restype = C.c_char_p
+    K, rdv, span, args = 3, C.c_void_p(), L.JabasSpan(), L.JabasStepArgs()
+    args.K = K
+    assert rec.jabas_rdv_create(K, C.byref(rdv)) == 0
+    assert rec.jabas_rdv_set_bucket(rdv, 0, C.byref(span), None, None, None, 0, 0) == 0
+    for streams in itertools.product((16, 32, 2), repeat=K):
+        for launch in (16, 64, 2):
+            for order in itertools.permutations(range(K)):
+                codes = [rec.jabas_rdv_publish(rdv, k, 0, 0, streams[k], launch, C.byref(args), L.STATS_SIMILARITY) for k in order]
+                assert codes == [L.RDV_WAITING] * (K - 1) + [L.RDV_LAUNCHED]
+                log = [line.split() for line in rec.take_log().decode().splitlines()]
+                assert log[-1] == ["launch", "0", str(launch)]
+                recorded = {int(e): int(s) for what, e, s in log if what == "record"}
+                # the completing hand-over on the launch's own stream, the same one in the same call, needs none
+                needed = [k for k in order if not (k == order[-1] and streams[k] == launch)]
+                assert recorded == {k + 1: streams[k] for k in needed}
+                assert sorted(int(e) for what, e, s in log if what == "wait" and int(s) == launch) == sorted(recorded)
+                assert [what for what, _, _ in log] == ["record"] * len(needed) + ["wait"] * len(needed) + ["launch"]
+    rec.jabas_rdv_destroy(rdv)
+
+
 @pytest.mark.parametrize("K", (1, 2, 5, 16))
 @pytest.mark.parametrize("half", (None, "blocks"))
 def test_step_args_hold_every_field_in_its_place(K, half):

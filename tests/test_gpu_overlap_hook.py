@@ -693,8 +693,8 @@ def test_optimizer_load_state_dict_after_the_buckets_are_bound(gpu, kind, interl
 
 @pytest.mark.parametrize("on", [(0, 0, 0, 0), (0, 1, 0, 1), (1, 1, 0, 0), (0, 1, 1, 2)])
 def test_vsws_that_share_streams_are_waited_for(gpu, on):
-    """VSWs on shared streams, handed over in every rotation: the launch waits once per stream, for the last of its hand-overs.
-    Each gradient is written late (behind a long chain of work on its stream)."""
+    """VSWs on shared streams, handed over in every rotation: the launch waits for each of them. Each gradient is
+    written late (behind a long chain of work on its stream)."""
     from jabas_amd.local_sync import LocalBucketSync
     K, batches, n = 4, (4, 3, 2, 1), 300_001
     local = LocalBucketSync(batches, stream=torch.cuda.Stream(gpu))
