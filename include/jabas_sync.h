@@ -104,7 +104,7 @@ enum {
  * 16-byte line, and of every bf16 gradient buffer at the same position of an 8-byte line
  * ((address / element size) mod 4 equal for all buffers), which holds whenever they are
  * views at one element offset into 16-byte aligned arenas. That much is required
- * (JABAS_ERR_ALIGN otherwise). Spans run fastest when the same holds within 64 elements
+ * (JABAS_ERR_ALIGN otherwise), of fp32 gradients unless JABAS_SPAN_LOOSE_GRADS says that they may sit anywhere. Spans run fastest when the same holds within 64 elements
  * ((address / element size) mod 64 equal for all buffers: views at one element offset into
  * 256-byte aligned arenas, which allocators of device memory give): the launch then starts its
  * element grid at that 256-byte line and moves whole cache lines; spans that start at arbitrary
@@ -130,7 +130,7 @@ enum {
  * No reference counterpart (torch keeps one tensor per parameter and moment,
  * examples/gnmt/seq2seq/train/shard_optimizer.py:50-66).
  *
- * JABAS_SPAN_LOOSE_GRADS (in `reserved`; fp32 gradients only, no effect on bf16 ones): the gradient buffers, and an
+ * JABAS_SPAN_LOOSE_GRADS (`reserved` equal to it; fp32 gradients only, no effect on bf16 ones): the gradient buffers, and an
  * agg_out that is one of them, may sit at any element, also at another position of a 16-byte line than the buffers
  * they update, as the views of a packed bucket sit next to weights that an allocator placed. They cost a line more
  * per wave and access where they do. */
@@ -149,7 +149,7 @@ typedef struct JabasSpan {
     uint32_t    bound_count;            /* 0: the whole span is parameter group 0      */
     uint32_t    state_block_log2;       /* 0: state1/2/3 are arrays of their own; else interleaved moments */
     uint32_t    state_block_pos;        /* interleaved moments: position of the first element in its block */
-    uint32_t    reserved;               /* 0, or JABAS_SPAN_... bits                   */
+    uint32_t    reserved;               /* 0 or JABAS_SPAN_LOOSE_GRADS; anything else counts as 0 */
 } JabasSpan;
 
 /* Parameter-group change inside a span: elements [start, next start) use `group`.

@@ -125,7 +125,8 @@ int encode_span(const JabasSpan& in, int K, int grad_dtype, int opt_kind, int bl
             if (p == in.grads[k]) return true;
         return false;
     };
-    const bool loose = (in.reserved & JABAS_SPAN_LOOSE_GRADS) && grad_dtype == JABAS_F32;
+    // The word exactly: other values were never read and still are not, so what an older caller left there relaxes nothing.
+    const bool loose = in.reserved == JABAS_SPAN_LOOSE_GRADS && grad_dtype == JABAS_F32;
     const bool loose_out = loose && is_grad(in.agg_out);
     const void* first = !loose ? in.grads[0] : oc != 0 ? in.param : in.agg_out && !loose_out ? in.agg_out : in.grads[0];
     const uintptr_t g0 = reinterpret_cast<uintptr_t>(first);

@@ -199,6 +199,25 @@ def test_plan_encode_rejects_bad_spans():
     assert _encode([s], opt=L.OPT_SGD)[0] == L.ERR_SIZE
 
 
+@pytest.mark.parametrize("word,loose", [(0, False), (1, True), (2, False), (3, False), (0x80000001, False), (0xCDCDCDCD, False), (0xFFFFFFFF, False)])
+def test_loose_gradients_are_asked_for_by_one_value_of_the_word(word, loose):
+    """The span's last word was not read before it came to say that fp32 gradients may sit at any element: whatever else a caller
+    left in it changes nothing, neither for a span that is accepted nor for one that is refused."""
+    for dtype, gs in ((L.F32, 4), (L.BF16, 2)):
+        aligned, off = _span(4096, gs=gs, opt=True), _span(4096, gs=gs, opt=True)
+        off.grads[1] += gs
+        aligned.reserved = off.reserved = word
+        if dtype == L.BF16:
+            aligned.agg_out = off.agg_out = None
+        plain = _span(4096, gs=gs, opt=True)
+        plain.agg_out = aligned.agg_out
+        rc, blob, _ = _encode([aligned], dtype=dtype, opt=L.OPT_ADAMW)
+        rc0, blob0, _ = _encode([plain], dtype=dtype, opt=L.OPT_ADAMW)
+        assert rc == rc0 == L.OK and np.array_equal(blob, blob0)
+        rc, _, _ = _encode([off], dtype=dtype, opt=L.OPT_ADAMW)
+        assert rc == (L.OK if loose and dtype == L.F32 else L.ERR_ALIGN)
+
+
 def test_plan_encode_checks_bounds():
     def with_bounds(bounds, count=None, begin=0):
         s = _span(10000, opt=True)
