@@ -19,6 +19,7 @@ GRAM_STRIDE = 256
 STATS_GRAM_MAX_K = 8
 STATIC_MAX_NUMEL = 1 << 26
 STEP_SCALARS_BYTES = 688
+MIN_VERSION = (0, 8)               # JABAS_SPAN_LOOSE_GRADS, which no symbol tells of
 
 F32, BF16 = 0, 1
 SPAN_LOOSE_GRADS = 1
@@ -162,6 +163,10 @@ def lib():
                                    "(`make -C jabas_amd/csrc`)") from None
             fn.restype = res
             fn.argtypes = args
+        version = handle.jabas_sync_version().decode()
+        if tuple(int(x) for x in version.split()[1].split(".")) < MIN_VERSION:
+            raise RuntimeError(f"{LIB_PATH} is {version}, older than {MIN_VERSION[0]}.{MIN_VERSION[1]}: it was built from older sources; "
+                               "build it again (`make -C jabas_amd/csrc`)")
         _lib = handle
     return _lib
 

@@ -556,7 +556,7 @@ int run_fused(KArgs& a, const JabasStepArgs* s, uint32_t tiles, uint32_t max_spa
 
 using namespace jabas;
 
-JABAS_API const char* jabas_sync_version(void) { return "jabas_sync 0.7 (gfx950)"; }
+JABAS_API const char* jabas_sync_version(void) { return "jabas_sync 0.8 (gfx950)"; }
 
 JABAS_API const char* jabas_status_string(int status) {
     switch (status) {

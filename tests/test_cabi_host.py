@@ -861,3 +861,12 @@ def test_library_without_an_entry_point_is_refused_by_name(monkeypatch):
     with pytest.raises(RuntimeError, match="jabas_of_a_later_build.*build it again"):
         L.lib()
     assert L._lib is None
+
+
+def test_library_of_an_older_version_is_refused_by_its_version(monkeypatch):
+    """An older library may have every entry point and still not know a flag that the package passes."""
+    monkeypatch.setattr(L, "_lib", None)
+    monkeypatch.setattr(L, "MIN_VERSION", (99, 0))
+    with pytest.raises(RuntimeError, match="older than 99.0.*build it again"):
+        L.lib()
+    assert L._lib is None
