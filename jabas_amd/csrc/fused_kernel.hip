@@ -737,20 +737,26 @@ int launch_one(const KArgs& a, unsigned grid, hipStream_t stream, bool dyn) {
 #ifndef JABAS_STATS_LDS_BYTES
 #define JABAS_STATS_LDS_BYTES 53248u      // per workgroup, flush_stats' own table included: three workgroups per CU
 #endif
-    // An aggregate with statistics and no optimizer, K <= 4 with fp32 gradients, five workgroups per CU where it is written and six
-    // where the gradients are only read (their registers allow seven or eight). 160 M elements, seven / five: K = 4 similarity
-    // sums 549 -> 526 us, full rows 550 -> 536, K = 3 436 -> 419, K = 2 330 -> 319, GNMT's clipped step, whose first launch this is,
-    // 1413 -> 1383; read only, no cap / six / five: K = 2 202 / 200 / 211, K = 3 303 / 301 / 304.
+    // An aggregate with statistics and no optimizer, K = 2..4 with fp32 gradients, where it reads 340 MB of them or more (their
+    // registers allow seven or eight workgroups per CU): five where four workers' aggregate is written, six otherwise. Time against no
+    // cap, aggregate in place, full rows / similarity sums: K = 4 five 25 M elements 0.984 / 0.973, 95 M 0.965 / 0.953; K = 3 six
+    // 37 M 0.983 / 0.983, 119 M 0.970 / 0.972; K = 2 six 50 M 1.005 / 1.000, 158 M 0.974 / 0.961, read only 75 M 0.971 / 0.964; GNMT's
+    // clipped step, whose first launch this is, 1413 -> 1383 us. Shorter launches wait for their last workgroups instead and lose:
+    // 12 M elements K = 2 six 1.03 / 1.06, 9 M K = 3 five 1.06 / 1.08; and two workers' aggregate loses at five at any length (158 M 1.04).
 #ifndef JABAS_AGG_LDS_BYTES
 #define JABAS_AGG_LDS_BYTES 32768u
 #endif
-#ifndef JABAS_AGG_READ_LDS_BYTES
-#define JABAS_AGG_READ_LDS_BYTES 26624u
+#ifndef JABAS_AGG_FEW_LDS_BYTES
+#define JABAS_AGG_FEW_LDS_BYTES 26624u
+#endif
+#ifndef JABAS_AGG_CAP_FROM
+#define JABAS_AGG_CAP_FROM 40960u         // gradient streams times workgroups of 2048 elements
 #endif
     constexpr bool capped = OPT == OPT_ADAM && K <= 4 && DT == JABAS_F32, capped_agg = OPT == OPT_NONE && SL && K > 1 && K <= 4 && DT == JABAS_F32;
     constexpr unsigned flush_bytes = imin(NStats<K, SL>::value, launch_block(K, DT, OPT, SL) / 16) * launch_block(K, DT, OPT, SL) * 8u;   // flush_stats' fp64 table
     static_assert(!capped || !SL || flush_bytes < JABAS_STATS_LDS_BYTES, "the cap is what is left beside the table");
-    const unsigned total = capped_agg ? (a.writes_agg ? JABAS_AGG_LDS_BYTES : JABAS_AGG_READ_LDS_BYTES)
+    const bool long_agg = capped_agg && static_cast<uint64_t>(grid) * K >= JABAS_AGG_CAP_FROM;
+    const unsigned total = long_agg   ? (K > 3 && a.writes_agg ? JABAS_AGG_LDS_BYTES : JABAS_AGG_FEW_LDS_BYTES)
                          : !capped    ? 0u
                          : SL         ? JABAS_STATS_LDS_BYTES
                                       : JABAS_IDLE_LDS_BYTES;
