@@ -97,11 +97,12 @@ __host__ __device__ constexpr int shape_level(int stats) { return stats == JABAS
 //                       2048 without statistics, 1 to 4 M elements lose: K = 4 AdamW 2 / 3 / 4 M 17.9 / 25.1 / 32.7 -> 19.0 / 27.5 /
 //                       35.8, K = 8 bf16 aggregate 4 M 15.4 -> 18.0; while fewer than 512, 2 M 18.9, and K = 8 pair products 0.9 M
 //                       0.90 of the time of whole chunks against 0.74
-//   group changes       in a span (norms and biases between the weights): up to 512 with statistics; without, up to 640 where chunks
-//                       are whole loads of few streams (up to four fp32 workers, three or four bf16 ones), 2048 otherwise. Up to 2048
-//                       for all, from when a tile with a change took many times as long as the others -> these, engine steps of
-//                       100 tensors: K = 1 fp32 AdamW 3 M 18.6 -> 17.0 us, K = 2 amsgrad 4 M without an aggregate 33.7 -> 30.7, K = 4 fp32 AdamW 2 M 18.7 -> 18.2,
-//                       bf16 amsgrad 3 M 26.9 -> 23.8. With 640 for the others K = 16 4 M loses 5 %, K = 1 bf16 amsgrad 4 M 8 %
+//   group changes       in a span (norms and biases between the weights): up to 512 with statistics; without, up to 2048, or 640 where a
+//                       chunk is 1024 elements (SGD of up to four fp32 workers), whose halves are one tile of two waves.
+//                       640 -> 2048 for the others, a change every 40000 elements, time in us: K = 1 fp32 amsgrad 1.7 / 4.5 / 6.5 M 14.3 / 32.5 /
+//                       44.3 -> 13.4 / 30.7 / 42.1, K = 4 AdamW 3 / 4.5 / 6.5 M 25.7 / 37.7 / 52.9 -> 25.2 / 35.5 / 49.8, K = 3 bf16 AdamW 6.5 M
+//                       42.0 -> 39.8; 1.4 M loses (K = 1 / 4 AdamW 9.5 / 13.5 -> 9.8 / 13.9); the same on buffers that stay in the
+//                       last-level cache. SGD would lose with 2048: K = 2 fp32 1 M 6.8 -> 7.6, K = 1 5.8 -> 6.1, longer ones the same
 //   without a tile      at most a quarter, or 64 with statistics (each still runs its epilogue and writes a row) and 256 without, or as
 //                       many as there are compute units for: plans over short spans, one per small tensor, whose last chunk is
 //                       mostly their only one. All splits -> these: 500 spans of 700 elements, K = 1 AdamW 7.7 -> 4.4 us, 20000, K = 16
@@ -113,11 +114,13 @@ __host__ __device__ constexpr int shape_level(int stats) { return stats == JABAS
 //                       at the rate of memory: K = 12 / 16, 25 M 102 / 138 -> 113 / 162. K = 5..8 would gain 2-3 % with full
 //                       rows and lose 11-14 % with pair products (25..40 sums per workgroup), and both levels cut their sums alike
 //   with an optimizer,  the same for the same reason (one tile in flight, a chunk of two tiles) without statistics from 2048 chunks
-//   K > 8               and with similarity sums from 4096 on. Engine steps of 100 tensors, whole chunks -> two workgroups each, fp32 K = 9 /
+//   K > 8               and with similarity sums from 4096 on, whether or not the group changes; where it does, plain launches are split
+//                       below 2048 too, by the rule above, so that whole chunks are left to spans of one group of 448 to 2047 and to similarity
+//                       sums of 512 to 4095. Engine steps of 100 tensors, whole chunks -> two workgroups each, fp32 K = 9 /
 //                       12 / 16 AdamW with an aggregate, 6 M elements 67 / 80 / 98 -> 65 / 77 / 95 us, 20 M 216 / 259 / 319 -> 210 / 253 / 314,
 //                       K = 16 SGD 100 M 1500 -> 1440; bf16 K = 16 AdamW amsgrad 40 M 463 -> 446; similarity sums, K = 12 fp32 SGD 20 M
-//                       248 -> 240, bf16 K = 16 SGD 40 M 365 -> 353. Below, nothing is gained (plain 3 M) or bf16 loses up to 4 %
-//                       (similarity sums 6 M, AdamW 68.5 -> 70.5)
+//                       248 -> 240, bf16 K = 16 SGD 40 M 365 -> 353. Below, bf16 similarity sums lose up to 4 % (6 M, AdamW 68.5 -> 70.5)
+//                       and plain launches of 3 M gain nothing
 #ifndef JABAS_SPLIT_FROM_PLAIN
 #define JABAS_SPLIT_FROM_PLAIN 2048
 #endif
@@ -131,10 +134,10 @@ __host__ __device__ constexpr int shape_level(int stats) { return stats == JABAS
 #define JABAS_SPLIT_BELOW_STATS 384
 #endif
 #ifndef JABAS_SPLIT_BELOW_GROUPS
-#define JABAS_SPLIT_BELOW_GROUPS 640
+#define JABAS_SPLIT_BELOW_GROUPS 2048
 #endif
-#ifndef JABAS_SPLIT_BELOW_GROUPS_MANYK
-#define JABAS_SPLIT_BELOW_GROUPS_MANYK 2048
+#ifndef JABAS_SPLIT_BELOW_GROUPS_SHORT
+#define JABAS_SPLIT_BELOW_GROUPS_SHORT 640
 #endif
 #ifndef JABAS_SPLIT_BELOW_GROUPS_STATS
 #define JABAS_SPLIT_BELOW_GROUPS_STATS 512
@@ -142,8 +145,8 @@ __host__ __device__ constexpr int shape_level(int stats) { return stats == JABAS
 template <class Live>
 inline uint32_t launch_split_log2(int K, int grad_dtype, int opt_class, int stats, uint64_t n_chunks, bool group_changes, const Live& live) {
     const uint32_t tiles = static_cast<uint32_t>(launch_chunk_tiles(K, grad_dtype, opt_class, stats));
-    const bool few = K <= 4 && (grad_dtype == JABAS_F32 || K > 2);
-    const uint64_t below = group_changes ? (stats ? JABAS_SPLIT_BELOW_GROUPS_STATS : few ? JABAS_SPLIT_BELOW_GROUPS : JABAS_SPLIT_BELOW_GROUPS_MANYK)
+    const bool short_chunks = 4 * static_cast<uint32_t>(launch_block(K, grad_dtype, opt_class, stats)) * tiles <= 1024;
+    const uint64_t below = group_changes ? (stats ? JABAS_SPLIT_BELOW_GROUPS_STATS : short_chunks ? JABAS_SPLIT_BELOW_GROUPS_SHORT : JABAS_SPLIT_BELOW_GROUPS)
                                          : (stats ? JABAS_SPLIT_BELOW_STATS : JABAS_SPLIT_BELOW);
     const uint64_t empty = stats ? 64 : 256;
     const auto pays = [&](uint32_t s) {

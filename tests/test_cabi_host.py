@@ -129,8 +129,8 @@ def test_plan_splits_chunks_that_hold_tiles_for_it(K, sizes, rows):
 
 @pytest.mark.parametrize("groups,rows", [((0,), 450), ((0, 1), 900)])
 def test_plan_splits_further_where_parameter_groups_change(groups, rows):
-    """Tiles with a change of parameter group hold up the others of their workgroup: 450 chunks are shared where there are any
-    (up to 512 with statistics), not where there are none (up to 384)."""
+    """With statistics, 450 chunks are shared where the parameter group changes inside a span (up to 512 workgroups), not where it
+    does not (up to 384)."""
     lib = L.lib()
     span = _span(900 * 1024, K=4, opt=True)
     span.bound_count = len(groups)
@@ -216,6 +216,35 @@ def test_loose_gradients_are_asked_for_by_one_value_of_the_word(word, loose):
         assert rc == rc0 == L.OK and np.array_equal(blob, blob0)
         rc, _, _ = _encode([off], dtype=dtype, opt=L.OPT_ADAMW)
         assert rc == (L.OK if loose and dtype == L.F32 else L.ERR_ALIGN)
+
+
+_CASES_OF_SPLITS = [
+    # K, dtype, optimizer, level, elements of a chunk, {(chunks, group change): log2 of the workgroups that share one}
+    (4, L.F32, L.OPT_ADAMW, 0, 4096, {(1023, True): 2, (1024, True): 1, (2047, True): 1, (2048, True): 0, (447, False): 1, (448, False): 0}),
+    (1, L.F32, L.OPT_ADAM_AMSGRAD, 0, 4096, {(1023, True): 2, (2047, True): 1, (2048, True): 0}),
+    (2, L.F32, L.OPT_SGD, 0, 1024, {(639, True): 1, (640, True): 0, (447, False): 1, (448, False): 0}),
+    (2, L.BF16, L.OPT_SGD, 0, 2048, {(2047, True): 1, (2048, True): 0}),
+    (9, L.F32, L.OPT_ADAM, 0, 2048, {(447, False): 1, (448, False): 0, (2047, False): 0, (2048, False): 1, (2047, True): 1, (2048, True): 1}),
+    (16, L.BF16, L.OPT_SGD, 0, 2048, {(2047, False): 0, (2048, False): 1, (2047, True): 1}),
+    (9, L.BF16, L.OPT_ADAMW, 2, 2048, {(511, True): 1, (512, True): 0, (4095, False): 0, (4096, False): 1, (4095, True): 0, (4096, True): 1}),
+    (16, L.F32, L.OPT_SGD, 2, 2048, {(4095, False): 0, (4096, False): 1}),
+]
+
+
+@pytest.mark.parametrize("K,dtype,opt,level,chunk,splits", _CASES_OF_SPLITS)
+def test_recorded_splits_on_both_sides_of_every_limit(K, dtype, opt, level, chunk, splits):
+    """How many workgroups share a chunk, as the plan records it (byte `level` of the header's word 9: 1 + its log2), on both sides of the
+    lengths at which that changes, for spans of one parameter group and with a change inside."""
+    for (chunks, change), want in splits.items():
+        n = chunks * chunk
+        s = _span(n, K=K, gs=4 if dtype == L.F32 else 2, opt=True)
+        s.state3 = s.state2 + (1 << 32) if opt == L.OPT_ADAM_AMSGRAD else None
+        bounds = [(0, 0), (n // 2 + 77, 1)] if change else [(0, 0)]
+        s.bound_count = len(bounds)
+        rc, blob, _ = _encode([s], bounds, K=K, dtype=dtype, opt=opt)
+        assert rc == L.OK
+        assert L.lib().jabas_plan_chunks(blob.ctypes.data, level) == chunks
+        assert int(blob.view(np.uint8)[36 + level]) == 1 + want, (chunks, change)
 
 
 def test_plan_encode_checks_bounds():
