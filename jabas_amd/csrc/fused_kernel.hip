@@ -586,11 +586,16 @@ __device__ __forceinline__ void span_range(const SP& sp, uint32_t lt0, uint32_t 
     const bool load_s1 = is_adam(OPT) || (OPT == OPT_SGD && a.opt.has_momentum && !a.opt.first_step);
     const uint32_t nb = sp.bound_count;
     GroupCursor<SEARCH> cur{nb ? const_bounds(a.bounds + sp.bound_begin) : nullptr, nb, j0, 0, 0, JABAS_MAX_GROUPS, {}};
+    // Eight fp32 workers with pair products, one tile in flight, take every tile by itself: the path over full tiles beside it costs 80
+    // registers, for SGD (235 -> 154) and without an optimizer (230 -> 145) one wave per SIMD of three, for AdamW (250 -> 169) a third of the
+    // spilled scalars. 3 M elements, both paths -> this: SGD 40.2 -> 35.0 us, AdamW 43.5 -> 41.2, no optimizer 30.2 -> 26.4; 12 M 122.5 -> 119.2,
+    // 136.3 -> 133.5, 88.5 -> 83.6; 40 M SGD 369 -> 366, AdamW 426 -> 431. Not amsgrad: 3 M 47.5 -> 45.3, but 12 M 152.2 -> 155.3, 40 M 488 -> 499.
+    constexpr bool ONE_BY_ONE = K <= 8 && U == 1 && OPT != OPT_AMS;
     for (uint32_t lt = lt0; lt < lt1;) {
         const uint64_t e0 = static_cast<uint64_t>(lt) * TE;
         uint32_t nfull = 0;
         // spans beyond 32-bit byte offsets go tile by tile
-        if (e0 >= sp.lo && (!narrow_addressing(K, SL) || sp.narrow_ok)) {
+        if (!ONE_BY_ONE && e0 >= sp.lo && (!narrow_addressing(K, SL) || sp.narrow_ok)) {
             const uint64_t fit = (sp.hi - e0) / TE;
             const uint32_t left = lt1 - lt;
             nfull = fit < left ? static_cast<uint32_t>(fit) : left;

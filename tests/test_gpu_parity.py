@@ -1639,6 +1639,44 @@ def test_dense_group_changes(gpu, K, dtype, kind, level, every):
             assert torch.equal(row.reshape(-1), row_1.reshape(-1))
 
 
+@pytest.mark.parametrize("kind", [None, "sgd", "adamw", "adamw_amsgrad"])
+@pytest.mark.parametrize("n", [1, 3, 1023, 1024, 1025, 4099, 70_003])
+def test_pair_products_of_eight_fp32_workers(gpu, kind, n):
+    """The kernels that take every tile by itself, on both sides of a tile and of a workgroup's four, default halves and others:
+    aggregate, weights and state bit for bit, every sum of the row against fp64, by value and as a plan."""
+    from jabas_amd import sync
+    K = 8
+    opt = None if kind is None else dict(kind=kind.replace("_amsgrad", ""), amsgrad="amsgrad" in kind, momentum=0.9, betas=(0.9, 0.999), eps=1e-8,
+                                         groups=[dict(lr=1e-2, weight_decay=0.05), dict(lr=3e-3, weight_decay=0.0)])
+    bounds = ((0, 0), (n // 2, 1)) if kind and n > 1 else ((0, 0),)
+    hg, n_state = _host_grads(K, n, 5), {None: 0, "sgd": 1, "adamw": 2, "adamw_amsgrad": 3}[kind]
+    start = [_host_state(n, 11)] + [_host_state(n, 12 + j, 1e-3).abs() for j in range(n_state)]
+    want = [t.clone() for t in start]
+    if kind:
+        agg_h, _ = O.sync_step(hg, BATCHES[K], [(0, n, bounds)], opt, *want[:3], step=3, **({"state3": want[3]} if n_state == 3 else {}))
+    else:
+        agg_h = O.aggregate(hg, BATCHES[K])
+    products = torch.stack([t.double() for t in hg]) @ torch.stack([t.double() for t in hg]).t()
+    size = products.diagonal().sqrt()
+    for half in (None, (0, 1, 1, 0, 1, 0, 0, 1)):
+        args = sync.make_step_args(BATCHES[K], torch.float32, stats="gram", opt=opt, step=3, half_id=half)
+        for plan in (False, True):
+            grads, agg, state = [_dev(t, gpu, 5) for t in hg], _dev(torch.zeros(n), gpu, 5), [_dev(t, gpu, 5) for t in start]
+            span = sync.SpanSpec(grads, agg_out=agg, bounds=bounds if kind else (),
+                                 **(dict(zip(("param", "state1", "state2", "state3"), state)) if kind else {}))
+            row = (sync.SyncPlan([span], sync.opt_kind(opt)).run(args) if plan else sync.sync_bucket(span, args)).reshape(-1).cpu()
+            assert torch.equal(_bits(agg), _bits(agg_h))
+            if kind:
+                assert all(torch.equal(_bits(x), _bits(y)) for x, y in zip(state, want))
+            # fp64 sums of exact products: 2^-53 per addition, a thread's 16 and 256 threads of 18 workgroups
+            tol = 1e-12
+            torch.testing.assert_close(row[4:4 + K], products.diagonal(), rtol=tol, atol=0.0)
+            pairs = [(i, j) for i in range(K) for j in range(i + 1, K)]
+            for at, (i, j) in enumerate(pairs):
+                assert abs(float(row[4 + K + at] - products[i, j])) <= tol * float(size[i] * size[j])
+            torch.testing.assert_close(row[3], (agg_h.double() ** 2).sum(), rtol=tol, atol=0.0)
+
+
 def test_dense_group_changes_cost_a_pass_per_group(gpu):
     """Two groups that change every 16 elements take two passes over the arithmetic, not one per change: 50 us against 30 for one
     group, of three million elements of four workers with similarity sums (107 with a pass per change, 3.6 times)."""
