@@ -27,7 +27,8 @@ struct JabasRendezvous {
         size_t workspace_bytes = 0;
         hipEvent_t events[JABAS_MAX_K] = {};
         uint32_t arrived = 0;                   // bit k: VSW k handed its buffer over in this step
-        uint32_t recorded = 0;                  // bit k: events[k] was recorded in this step
+        uint32_t recorded = 0;                  // bit k: events[k] was recorded in this step and is to be waited for
+        uint32_t on_null = 0;                   // of these, recorded on the null stream
         int want_stats = 0;                     // VSW 0's word
         int flip = 0;
     };
@@ -94,7 +95,7 @@ JABAS_API int jabas_rdv_set_bucket(JabasRendezvous* r, uint32_t bucket, const Ja
     b.rows = stats_rows;
     b.workspace = workspace;
     b.workspace_bytes = workspace_bytes;
-    b.recorded = 0;
+    b.recorded = b.on_null = 0;
     b.want_stats = 0;
     b.flip = last_row;                          // the next statistics launch takes the other row
     b.set = true;
@@ -108,7 +109,7 @@ JABAS_API int jabas_rdv_drop_bucket(JabasRendezvous* r, uint32_t bucket) {
     JabasRendezvous::Bucket& b = r->buckets[bucket];
     const int arrived = __builtin_popcount(b.arrived);
     b.set = false;
-    b.arrived = b.recorded = 0;
+    b.arrived = b.recorded = b.on_null = 0;
     return arrived;
 }
 
@@ -133,6 +134,14 @@ JABAS_API int jabas_rdv_publish(JabasRendezvous* r, int32_t k, uint32_t bucket, 
         // event, and the completing one does unless the launch follows its own work on its own stream.
         if (!complete || vsw_stream != launch_stream) {
             if (hipEventRecord(b->events[k], mine) != hipSuccess) return JABAS_ERR_LAUNCH;
+            // The null stream is one stream for as long as the process runs, so its last event covers the earlier ones. No other handle
+            // is a stream's name for good: that of a destroyed stream is given out again, hipStreamPerThread is another stream on
+            // every thread. Four VSWs on the null stream, the 14 buckets of ViT-B/16 with similarity sums, a step: 951 us with a wait per
+            // event, 833 and 873 with one per bucket (processes differ by up to 9 %).
+            if (!mine) {
+                b->recorded &= ~b->on_null;
+                b->on_null = bit;
+            }
             b->recorded |= bit;
         }
         b->arrived |= bit;
@@ -145,13 +154,10 @@ JABAS_API int jabas_rdv_publish(JabasRendezvous* r, int32_t k, uint32_t bucket, 
         want = b->want_stats && b->rows != nullptr;
         if (want) flip = (b->flip ^= 1);
         snap = *b;
-        b->arrived = b->recorded = 0;
+        b->arrived = b->recorded = b->on_null = 0;
         b->want_stats = 0;
     }
     hipStream_t main = static_cast<hipStream_t>(launch_stream);
-    // Every event, also where two hand-overs or the launch name the same handle: a handle is no stream's name for good (that of a
-    // destroyed stream is given out again, hipStreamPerThread is another stream on every thread). One wait per handle measured the
-    // same: four VSWs on one stream, the 14 buckets of ViT-B/16 with similarity sums, 930 us a step both ways.
     for (int j = 0; j < r->K; ++j)
         if (recorded >> j & 1u)
             if (hipStreamWaitEvent(main, snap.events[j], 0) != hipSuccess) return JABAS_ERR_LAUNCH;
@@ -170,7 +176,7 @@ JABAS_API int jabas_rdv_reset(JabasRendezvous* r) {
     int pending = 0;
     for (auto& b : r->buckets) {
         if (b.arrived) ++pending;
-        b.arrived = b.recorded = 0;
+        b.arrived = b.recorded = b.on_null = 0;
         b.want_stats = 0;
     }
     return pending;

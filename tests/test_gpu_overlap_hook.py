@@ -691,14 +691,14 @@ def test_optimizer_load_state_dict_after_the_buckets_are_bound(gpu, kind, interl
                     assert _same(state["max_exp_avg_sq"], s3_h[sl]), (b, i, "maximum")
 
 
-@pytest.mark.parametrize("on", [(0, 0, 0, 0), (0, 1, 0, 1), (1, 1, 0, 0), (0, 1, 1, 2)])
+@pytest.mark.parametrize("on", [(0, 0, 0, 0), (0, 1, 0, 1), (1, 1, 0, 0), (0, 1, 1, 2), (-1, -1, -1, -1), (-1, 0, -1, 1), (0, -1, -1, 0)])
 def test_vsws_that_share_streams_are_waited_for(gpu, on):
     """VSWs on shared streams, handed over in every rotation: the launch waits for each of them. Each gradient is
     written late (behind a long chain of work on its stream)."""
     from jabas_amd.local_sync import LocalBucketSync
     K, batches, n = 4, (4, 3, 2, 1), 300_001
     local = LocalBucketSync(batches, stream=torch.cuda.Stream(gpu))
-    streams = [torch.cuda.Stream(gpu) for _ in range(max(on) + 1)]
+    streams = [torch.cuda.Stream(gpu) for _ in range(max(on) + 1)] + [torch.cuda.default_stream(gpu)]      # -1: the null stream
     bufs = [torch.zeros(n, device=gpu) for _ in range(K)]
     busy = [torch.full((2048, 2048), 1e-3, device=gpu) for _ in streams]
     for step in range(5):
