@@ -85,14 +85,15 @@ class _ShardOptimizer(torch.optim.Optimizer):
     # names everything else that the launches were prepared from: each parameter's group, the memory of
     # the weight, the gradient, the state and the replicas, and the clipping coefficient. The state is looked
     # up anew by every call (``states``, one per pair) and nothing of it is kept.
-    def _signature(self, pairs, states):
+    def _signature(self, counts, params, grads, where, states):
         scale, memory = getattr(self, "_grad_scale", None), torch.Tensor.data_ptr
-        params, grads = [p for _, p, _ in pairs], [g for _, _, g in pairs]
-        sig = [None if scale is None else scale.data_ptr(), tuple([gi for gi, _, _ in pairs]), *map(memory, params), *map(memory, grads),
-               *map(torch.Tensor.numel, grads), *map(torch.Tensor.is_contiguous, grads)]
+        sig = [None if scale is None else scale.data_ptr(), *counts, *where]
+        sig += map(memory, params)
+        sig += map(torch.Tensor.numel, grads)
+        sig += map(torch.Tensor.is_contiguous, grads)
         for name in self._state_names():
             try:
-                sig += list(map(memory, [st[name] for st in states]))
+                sig += [*map(memory, [st[name] for st in states])]
             except (KeyError, TypeError):         # not every parameter has one
                 sig += [memory(st[name]) if st and st.get(name) is not None else None for st in states]
         if self._replicas:
@@ -111,27 +112,51 @@ class _ShardOptimizer(torch.optim.Optimizer):
             q.data.copy_(p.data)
 
     # -- matching ---------------------------------------------------------------------
-    def _pairs(self, gradients):
-        """[(group_index, param, grad)] for this call."""
-        out = []
+    def _matched(self, gradients):
+        """This call's parameters per group, its parameters, their gradients, and the gradients' memory, group by group."""
+        counts, params, grads, where = [], [], [], []
         if gradients is None:
-            for gi, group in enumerate(self.param_groups):
-                for p in group["params"]:
-                    if p.grad is not None:
-                        out.append((gi, p, p.grad))
-            return out
+            for group in self.param_groups:
+                mine = group["params"]
+                theirs = [p.grad for p in mine]
+                try:
+                    at = self._memory(theirs)
+                except TypeError:                 # one of them is None
+                    mine = [p for p, g in zip(mine, theirs) if g is not None]
+                    theirs = [g for g in theirs if g is not None]
+                    at = self._memory(theirs)
+                counts.append(len(mine))
+                params += mine
+                grads += theirs
+                where += at
+            return counts, params, grads, where
         by_index = {}
         for g in gradients:
             idx = getattr(g, "index", None)       # the attribute the reference sets; anything callable is not it
             if not isinstance(idx, int):
                 raise ValueError("step(gradients): every gradient needs an .index attribute naming its parameter")
             by_index[idx] = g
-        for gi, group in enumerate(self.param_groups):
+        for group in self.param_groups:
+            before = len(params)
             for p in group["params"]:
                 idx = getattr(p, "index", None)
                 if isinstance(idx, int) and idx in by_index:
-                    out.append((gi, p, by_index[idx]))
-        return out
+                    params.append(p)
+                    grads.append(by_index[idx])
+            counts.append(len(params) - before)
+        return counts, params, grads, self._memory(grads)
+
+    @staticmethod
+    def _memory(grads):
+        try:
+            return [*map(torch.Tensor.data_ptr, grads)]
+        except RuntimeError:                      # a sparse one: refused further on
+            return []
+
+    @staticmethod
+    def _pairs(counts, params, grads, where):
+        """[(group_index, param, grad)] of the same."""
+        return list(zip([gi for gi, n in enumerate(counts) for _ in range(n)], params, grads))
 
     @staticmethod
     def _congruent(g, p):
@@ -194,11 +219,12 @@ class ShardSGD(_ShardOptimizer):
     @torch.no_grad()
     def step(self, gradients=None, closure=None):
         loss = closure() if closure is not None else None
-        pairs = self._pairs(gradients)
-        states = list(map(self.state.get, [p for _, p, _ in pairs]))
-        sig = self._signature(pairs, states)
+        matched = self._matched(gradients)
+        states = list(map(self.state.get, matched[1]))
+        sig = self._signature(*matched, states)
         if self._replay(self._recipes.get(sig), states):
             return loss
+        pairs = self._pairs(*matched)
         self._volatile, launches, self._late_copies = False, [], []
         # launches are split by (momentum, dampening, nesterov, first-step): launch-wide scalars
         batches = {}
@@ -276,11 +302,12 @@ class ShardAdam(_ShardOptimizer):
     @torch.no_grad()
     def step(self, gradients=None, closure=None):
         loss = closure() if closure is not None else None
-        pairs = self._pairs(gradients)
-        states = list(map(self.state.get, [p for _, p, _ in pairs]))
-        sig = self._signature(pairs, states)
+        matched = self._matched(gradients)
+        states = list(map(self.state.get, matched[1]))
+        sig = self._signature(*matched, states)
         if self._replay(self._recipes.get(sig), states):
             return loss
+        pairs = self._pairs(*matched)
         self._volatile, launches, self._late_copies = False, [], []
         batches = {}
         write_back = getattr(self, "_grad_scale", None) is not None     # a clipped step leaves the clipped gradients behind
@@ -390,7 +417,7 @@ class ShardGNMTAdam(ShardAdam):
     def step(self, gradients=None, closure=None):
         if self.grad_clip == float('inf'):
             return super().step(gradients, closure)
-        pairs = self._pairs(gradients)
+        pairs = self._pairs(*self._matched(gradients))
         if not pairs:
             return super().step(gradients, closure)
         flat = []
