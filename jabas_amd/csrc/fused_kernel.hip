@@ -3,8 +3,8 @@
 // streams are fully unrolled into independent 128-bit loads.
 //
 // Execution shape
-//   - one workgroup per chunk of consecutive tiles of one span, two or four where that leaves compute
-//     units idle (launch_split_log2); a tile is one 16-byte vector of
+//   - one workgroup per chunk of consecutive tiles of one span, two or four where the launch is short or the kernel
+//     holds one tile of many streams in flight (launch_split_log2); a tile is one 16-byte vector of
 //     every fp32 buffer (one 8-byte vector of a bf16 gradient buffer) per thread. Threads per
 //     workgroup and tiles per chunk depend on the kernel family (launch_block / launch_chunk_tiles):
 //     256 threads x 2 or 4 tiles with statistics, 128 x 2, 256 x 2 or 256 x 4 without. Small,
@@ -15,7 +15,7 @@
 //     exactly once per step);
 //   - tiles that lie wholly inside the live range of a span take the vector path (all loads of U tiles issued
 //     before any arithmetic, the parameter group looked up while they are under way); a tile that straddles a span
-//     end, or is the only one left, goes wave by wave (single_tile);
+//     end, or is the only one left, goes wave by wave (single_tile), as do all of eight fp32 workers with pair products;
 //   - statistics: per-thread fp64 accumulators -> LDS -> 16-way sums in fixed order -> DPP row
 //     reduction -> one partial row of 4 + K doubles per workgroup in the workspace, summed in
 //     fixed order by the finalize kernel. The order is fixed, so results are bit-identical run to run.
@@ -175,13 +175,13 @@ struct DynView {
     }
 };
 
-// Float index of grid element e's Adam moments from the span's moment bases: e itself when the moments are
-// arrays of their own, its place in the interleaved arena otherwise (SpanDev). Two integer operations.
 // The bound table of a launch is, like the plan's other tables, not written while the launch runs: read through
 // the constant address space (uniform loads the compiler is free to move or repeat).
 typedef const __attribute__((address_space(4))) BoundDev* ConstBounds;
 __device__ __forceinline__ ConstBounds const_bounds(const BoundDev* p) { return (ConstBounds)p; }
 
+// Float index of grid element e's Adam moments from the span's moment bases: e itself when the moments are
+// arrays of their own, its place in the interleaved arena otherwise (SpanDev). Two integer operations.
 template <class SP> __device__ __forceinline__ uint64_t moment_index(const SP& sp, uint64_t e) {
     const uint64_t t = e + sp.mom_add;
     return t + sp.mom_mult * (t & sp.mom_mask);

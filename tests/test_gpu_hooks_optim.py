@@ -752,7 +752,7 @@ def test_trainer_with_bf16_gradient_buckets(gpu):
 def test_shard_optimizer_remembered_calls_follow_every_change(gpu, kind):
     """step() remembers a call it has prepared once (same parameters, same gradient buffers) and then
     only refreshes launch scalars. Everything that may change between two such calls must still take
-    effect: gradient values, learning rate and weight decay, gradients that need a realigned copy,
+    effect: gradient values, learning rate and weight decay, gradients off their weights' 16-byte line,
     parameters stepped in different subsets (diverging Adam step counts), a changed momentum / betas,
     and load_state_dict. Checked against torch.optim on a twin model over persistent gradient buffers."""
     from jabas_amd import optim

@@ -1335,11 +1335,11 @@ def test_short_launches_give_the_result_of_whole_chunks(gpu, K, dtype, level, nu
     (12, torch.bfloat16, "adamw", "full"), (16, torch.float32, "adam", "similarity"), (16, torch.bfloat16, None, "full"), (6, torch.float32, None, None)])
 @pytest.mark.parametrize("numel", [517, 2049, 90_001, 400_003])
 def test_split_launches_of_every_kind(gpu, K, dtype, kind, level, numel):
-    """Every optimizer, block size and level under a split: aggregate, weights and state against the first elements of a span too
-    long to be split, bit for bit; by value, as a plan of spans of unequal length (one of a single element, most shorter than a
+    """Every optimizer, block size and level under a split: aggregate, weights and state against the first elements of a span that is
+    not split (too long for it, too short for the rule of long steps), bit for bit; by value, as a plan of spans of unequal length (one of a single element, most shorter than a
     chunk) and with the step's scalars in device memory."""
     from jabas_amd import sync, _lib as L
-    far = numel + 4_000_000
+    far = numel + (2_000_000 if K > 8 else 4_000_000)
     gen = torch.Generator(device=gpu).manual_seed(numel + K)
     grads = [torch.randn(far, generator=gen, device=gpu).to(dtype) for _ in range(K)]
     start = [torch.randn(far, generator=gen, device=gpu) * 0.1 for _ in range(2)] + [torch.rand(far, generator=gen, device=gpu) * 0.1 for _ in range(2)]
@@ -1363,6 +1363,9 @@ def test_split_launches_of_every_kind(gpu, K, dtype, kind, level, numel):
             rows = sync.sync_bucket(spans[0], args, workspace=sync.Workspace.for_span(n, dtype, gpu))
         return [agg, *state], None if not stats else rows.reshape(-1, L.STATS_STRIDE).sum(0)
 
+    whole = sync.SyncPlan([sync.SpanSpec(grads, agg_out=torch.zeros(far, device=gpu), **dict(zip(("param", "state1", "state2", "state3"), start[:n_state])))],
+                          sync.opt_kind(opt))
+    assert int(whole._host.view(torch.uint8)[36]) == 1          # one workgroup per chunk
     want, _ = launch((0, far), None)
     ways = [launch((0, numel), level), launch((0, 256, 257, 300, 2 * numel // 3, numel), level)]
     if kind in ("sgd", "adam", "adamw"):
@@ -1381,11 +1384,13 @@ def test_split_launches_of_every_kind(gpu, K, dtype, kind, level, numel):
 
 @pytest.mark.parametrize("K,dtype,kind,level", [(9, torch.float32, "adam", None), (16, torch.bfloat16, "sgd", None), (12, torch.bfloat16, "adamw_amsgrad", None),
                                                 (9, torch.bfloat16, "adamw", "similarity"), (16, torch.float32, "sgd", "similarity")])
+@pytest.mark.parametrize("change", [False, True])
 @pytest.mark.parametrize("off_by", [-1, 1, 2049])
-def test_long_steps_of_many_workers(gpu, K, dtype, kind, level, off_by):
+def test_long_steps_of_many_workers(gpu, K, dtype, kind, level, off_by, change):
     """On both sides of the length from which two workgroups share a chunk (2048 elements; from 2048 chunks on, with similarity sums
-    4096): weights, state and aggregate bit for bit those of three shorter launches, by value and as a plan, on the scratch that the
-    sizing function names and on the least, which holds whole chunks only."""
+    4096; plain spans in which the group changes share theirs on both sides): weights, state and aggregate bit for bit those of
+    three shorter launches, by value and as a plan, on the scratch that the sizing function names and on the least, which holds
+    whole chunks only. The plan records which of them the launch is."""
     from jabas_amd import sync, _lib as L
     chunks = 4096 if level else 2048
     n = (chunks - 1) * 2048 + off_by
@@ -1395,17 +1400,19 @@ def test_long_steps_of_many_workers(gpu, K, dtype, kind, level, off_by):
     start = start[:{"sgd": 2, "adamw_amsgrad": 4}.get(kind, 3)]
     opt = dict(kind=kind.replace("_amsgrad", ""), amsgrad="amsgrad" in kind, momentum=0.9, betas=(0.9, 0.999), eps=1e-8,
                groups=[dict(lr=1e-2, weight_decay=0.05), dict(lr=3e-3, weight_decay=0.0)])
-    change = n // 2 + 77
+    at = n // 2 + 77 if change else n
 
     def launch(cuts, plan, scratch=None):
         state, agg, rows = [t.clone() for t in start], torch.zeros(n, device=gpu), []
         args = sync.make_step_args((1,) * K, dtype, stats=level or False, opt=opt, step=3)
         for a, b in zip(cuts, cuts[1:]):
-            bounds = ((0, 0), (change - a, 1)) if a < change < b else ((0, int(a >= change)),)
+            bounds = ((0, 0), (at - a, 1)) if a < at < b else ((0, int(a >= at)),)
             span = sync.SpanSpec([g[a:b] for g in grads], agg_out=agg[a:b], bounds=bounds,
                                  **dict(zip(("param", "state1", "state2", "state3"), (t[a:b] for t in state))))
             if plan:
-                row = sync.SyncPlan([span], sync.opt_kind(opt)).run(args)
+                p = sync.SyncPlan([span], sync.opt_kind(opt))
+                assert int(p._host.view(torch.uint8)[36 + (2 if level else 0)]) == 1 + int(off_by > 0 or (change and not level))
+                row = p.run(args)
             else:
                 ws = sync.Workspace.for_span(b - a, dtype, gpu)
                 ws.nbytes = scratch or ws.nbytes
